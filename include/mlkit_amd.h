@@ -216,6 +216,19 @@ int mk_fit_scales(const float *value, long long row_stride, float *scales, float
                   int span, int group, int asym, float reciprocal, float value_minimum,
                   int scale_format, int store_zero, void *stream);
 
+/* mk_fit_scales, mk_search_scales (n_fractions > 0) and mk_scalar_encode of a contiguous [rows, width] matrix of type
+ * `dtype` in one pass over it; the same scales, zeros and codes as those calls on its fp32 copy, bit for bit.
+ *   group       8, 16, 32, 64, 128 or 256 columns (MK_ERR_UNSUPPORTED otherwise); the last one of a row may be narrower
+ *   reciprocal  fp32(1) / fp32(value range) of the grid; `minimum` is its least value
+ *   zeros       stored with their magnitude rounded to `scale_format`; written only when asym != 0
+ *   flag        device int32, set to one when a weight or a scale is not finite (never cleared here); the outputs
+ *               mean nothing then
+ * Replaces: formats/grouped_scaling.py:132-175 over kernels/scalar_encode.py:110-146,261-304. */
+int mk_round_matrix(const void *value, int dtype, const float *values, int n_values, const float *fractions,
+                    int n_fractions, float *scales, float *zeros, uint8_t *codes, int *flag, int rows,
+                    int width, int group, int asym, int integer, float minimum, float maximum,
+                    float reciprocal, int scale_format, void *stream);
+
 /* output = quantize-dequantize of `inputs` ([rows, width], fp32 / fp16 / bf16; output has the
  * same dtype and may alias) with per-group scales fitted on the fly: the result equals
  * mk_fit_scales (zeros stored rounded) + mk_scalar_encode + mk_scalar_decode on the fp32

@@ -13,45 +13,11 @@
 //   scalar_rounding.py:15-73   rounding helpers (device functions below)
 
 #include "mk_common.h"
-#include "packed_matvec_impl.h"   // lane_exchange
+#include "scalar_codec_impl.h"
+
+using namespace mk_scalar;
 
 namespace {
-
-constexpr int kMaxTable = 256;
-constexpr int kThreads = 256;
-
-// Index of the first table entry >= x by bisection over a table padded with +inf, then
-// the nearer of that entry and the one below it; equal distances pick the lower entry.
-__device__ __forceinline__ int nearest_entry(float x, const float *table, int count, int steps) {
-    int lower = 0, upper = count;
-    for (int s = 0; s < steps; ++s) {
-        const int middle = (lower + upper) >> 1;
-        const float candidate = middle < count ? table[middle] : __builtin_inff();
-        const bool right = candidate < x;
-        lower = right ? middle + 1 : lower;
-        upper = right ? upper : middle;
-    }
-    const int above = lower < count - 1 ? lower : count - 1;
-    const int below = above > 0 ? above - 1 : 0;
-    const float below_distance = fabsf(__fsub_rn(x, table[below]));
-    const float above_distance = fabsf(__fsub_rn(x, table[above]));
-    return below_distance <= above_distance ? below : above;
-}
-
-__device__ __forceinline__ float nearest_integer(float x, float minimum, float maximum) {
-    return fminf(fmaxf(rintf(x), minimum), maximum);
-}
-
-__device__ __forceinline__ int bisection_steps(int count) {
-    int steps = 0;
-    while ((1 << steps) < count + 1) ++steps;
-    return steps;
-}
-
-__device__ __forceinline__ void stage_table(float *shared, const float *values, int count) {
-    for (int i = threadIdx.x; i < count; i += blockDim.x) shared[i] = values[i];
-    __syncthreads();
-}
 
 struct CodecArgs {
     const float *value;
@@ -415,43 +381,10 @@ __device__ __forceinline__ void store_fit(const FitArgs &a, size_t slot, float l
         if (a.zeros) a.zeros[slot] = __builtin_nanf("");
         return;
     }
-    float scale, zero = 0.0f;
-    if (a.asym) {
-        scale = __fmul_rn(fmaxf(__fsub_rn(high, low), 1e-12f), a.reciprocal);
-        zero = __fsub_rn(low, __fmul_rn(a.value_minimum, scale));
-    } else {
-        scale = __fmul_rn(fmaxf(fmaxf(high, -low), 1e-12f), a.reciprocal);
-    }
+    float zero;
+    const float scale = range_scale(low, high, a.asym, a.reciprocal, a.value_minimum, zero);
     a.scales[slot] = mk_rounded_scale(scale, a.format);
-    if (a.zeros) {
-        if (a.store_zero) {
-            const float magnitude = mk_rounded_scale(fmaxf(fabsf(zero), 1e-12f), a.format);
-            zero = zero > 0.0f ? magnitude : (zero < 0.0f ? -magnitude : 0.0f);
-        }
-        a.zeros[slot] = zero;
-    }
-}
-
-// Minimum, maximum and "all finite" over the LANES adjacent lanes of a team, by vector-ALU
-// lane moves (an LDS permute per step cost more than the loads of the group).
-template <int LANES>
-__device__ __forceinline__ void team_range(float &low, float &high, bool &finite, int lane) {
-    float bad = finite ? 0.0f : 1.0f;
-    auto stage = [&](auto s) __attribute__((always_inline)) {
-        constexpr int S = decltype(s)::value;
-        if constexpr ((1 << S) < LANES) {
-            low = fminf(low, mk_matvec::lane_exchange<S>(low, lane));
-            high = fmaxf(high, mk_matvec::lane_exchange<S>(high, lane));
-            bad = fmaxf(bad, mk_matvec::lane_exchange<S>(bad, lane));
-        }
-    };
-    stage(std::integral_constant<int, 0>{});
-    stage(std::integral_constant<int, 1>{});
-    stage(std::integral_constant<int, 2>{});
-    stage(std::integral_constant<int, 3>{});
-    stage(std::integral_constant<int, 4>{});
-    stage(std::integral_constant<int, 5>{});
-    finite = bad == 0.0f;
+    if (a.zeros) a.zeros[slot] = a.store_zero ? rounded_offset(zero, a.format) : zero;
 }
 
 template <int LANES>

@@ -149,6 +149,41 @@ def fit_scales(
     return scales, zeros
 
 
+ROUND_GROUPS = frozenset({8, 16, 32, 64, 128, 256})   # the groups one pass of `round_matrix` keeps in registers
+
+
+def round_matrix(
+    value: Tensor,
+    values: Tensor,
+    fractions: Tensor | None,
+    group: int,
+    *,
+    asym: bool,
+    integer: bool,
+    minimum: float,
+    maximum: float,
+    reciprocal: float,
+    scale_format: str,
+) -> tuple[Tensor, Tensor, Tensor | None, Tensor]:
+    """``(codes, scales, zeros, flag)`` of a matrix in its own type (fp32 / fp16 / bf16): ``fit_scales``,
+    ``search_scales`` (with ``fractions``) and ``encode`` in one pass.  ``flag`` is a one-element int32
+    tensor that reads one when a weight or a scale is not finite."""
+    device = native.require_device(value, values, fractions)
+    if value.dim() != 2 or not value.is_contiguous():
+        raise ValueError("round_matrix requires a contiguous two-dimensional tensor")
+    rows, width = value.shape
+    codes = torch.empty((rows, width), device=device, dtype=torch.uint8)
+    scales = torch.empty((rows, -(-width // group)), device=device, dtype=torch.float32)
+    zeros = torch.empty_like(scales) if asym else None
+    flag = torch.zeros(1, device=device, dtype=torch.int32)
+    native.check(native.library().mk_round_matrix(
+        value.data_ptr(), native.dtype_code(value), values.data_ptr(), values.numel(), native.pointer(fractions),
+        0 if fractions is None else fractions.numel(), scales.data_ptr(), native.pointer(zeros), codes.data_ptr(),
+        flag.data_ptr(), rows, width, group, int(asym), int(integer), minimum, maximum, reciprocal,
+        native.SCALE_FORMAT_CODES[scale_format], native.current_stream(device)))
+    return codes, scales, zeros, flag
+
+
 def reconstruct(
     inputs: Tensor,
     values: Tensor,

@@ -310,6 +310,39 @@ class Scaled(Quantizer):
 
         return FittedRounder(round_columns, scalar=scalar, vector=vector)
 
+    def __call__(self, w: Tensor, ctx: Ctx | None = None) -> Q:
+        whole = self._rounded_in_one_pass(w) if type(self).fit is Scaled.fit else None
+        return super().__call__(w, ctx) if whole is None else whole
+
+    def _rounded_in_one_pass(self, w: Tensor) -> Q | None:
+        """The matrix rounded by one kernel that reads it once, in its own type; None where that kernel does not
+        apply (``fit`` and its rounder then do the same in steps)."""
+        if not (w.is_cuda and w.ndim == 2 and w.numel() and w.dtype in (torch.float32, torch.float16, torch.bfloat16)
+                and self.grid.dim == 1 and self.grid.values is not None and self.grid.bits <= 8
+                and isinstance(self.scale_fmt, str) and not callable(self.scale)):
+            return None
+        table = self.values_on(w.device)
+        width = w.shape[1]
+        group = width if self.group is None else min(self.group, width)
+        searching = self.scale == "mse"
+        from mlkit_amd.kernels import scalar_encode
+
+        if (group not in scalar_encode.ROUND_GROUPS or table.numel() > FUSED_CODEBOOK_LIMIT
+                or (searching and self.search_steps > 64)):
+            return None
+        fractions = torch.linspace(0.5, 1.0, self.search_steps, device=w.device) if searching else None
+        codes, scales, zero, flag = scalar_encode.round_matrix(
+            w.detach().contiguous(), table, fractions, group, asym=self.asym, integer=self.grid.integer,
+            minimum=self._value_minimum, maximum=self._value_maximum,
+            reciprocal=self._range_reciprocal if self.asym else self._magnitude_reciprocal, scale_format=self.scale_fmt)
+        if flag.item():
+            raise ValueError("scaled requires a finite floating-point weight matrix")
+        side_bits = scales.numel() * SCALE_FORMAT_BITS[self.scale_fmt] * (2 if zero is not None else 1)
+        return Q(bits=self.grid.bits * w.numel() + side_bits, codes=codes, decode=decode_scaled, codec="scaled",
+                 metadata={"code_bits": self.grid.bits, "scale_fmt": self.scale_fmt,
+                           "trainable": ["scales"] + (["zero"] if zero is not None else [])},
+                 params={"scales": scales, "values": table, "group": group, "offset": 0, "zero": zero})
+
     def _scalar_codes(self, value: Tensor, scalar: ScalarRounding, start: int, stop: int) -> Tensor:
         """Codes of the nearest grid values for columns ``start`` to ``stop`` of the fitted region."""
         if (value.is_cuda and start % scalar.group == 0 and self.grid.bits <= 8

@@ -233,3 +233,52 @@ def test_activation_reconstruction_matches_oracle_directly():
     dense = scaling.decode_grouped(expected["codes"], expected["scales"], INT4, 64, expected["zero"])
     result = mk.int(4, group=64, asym=True).reconstruct_activations(dev(value))
     np.testing.assert_array_equal(host(result), dense)
+
+
+TABLE9 = np.sort(np.random.default_rng(5).standard_normal(9).astype(F32))
+REPEATED = np.array([-1, -0.25, -0.25, 0.5, 0.5, 1], dtype=F32)
+
+
+@pytest.mark.parametrize("rows,width,group,values,integer,asym,scale,fmt,dtype", [
+    (3, 8, 8, INT4, True, False, "absmax", "fp16", torch.float32),           # one group of one lane
+    (37, 272, 16, INT4, True, True, "mse", "fp16", torch.bfloat16),
+    (33, 203, 64, INT3, True, True, "mse", "bf16", torch.float16),           # rows of odd width, a narrower last group
+    (65, 200, 128, INT4, True, False, "absmax", "fp16", torch.bfloat16),     # whole lanes past the row
+    (19, 1024, 256, SEVEN, False, False, "mse", "fp16", torch.float16),
+    (19, 1000, 256, SEVEN, False, True, "mse", "fp32", torch.float32),
+    (64, 512, 64, scaling.NF4_VALUES, False, False, "mse", "fp8", torch.float16),
+    (16, 96, 32, TABLE9, False, False, "absmax", "e8m0", torch.float32),
+    (16, 384, 128, TABLE256, False, True, "absmax", "fp16", torch.float32),
+    (32, 256, 64, REPEATED, False, False, "mse", "fp16", torch.float32),
+])
+def test_rounding_in_one_pass_matches_oracle(rows, width, group, values, integer, asym, scale, fmt, dtype):
+    """Codes, scales and offsets of mk_round_matrix bit for bit, on weights that include exact multiples of half
+    a step (quotients at rounding boundaries) and, in fp32, groups whose scales leave the ordinary range."""
+    from mlkit_amd.kernels import scalar_encode
+
+    weight = torch.from_numpy(helpers.normal_weight(rows, width, seed=rows + width, student_t=True))
+    weight[::3] = (weight[::3] * 64).round() / 128
+    if fmt == "fp32":
+        weight[1] *= 1e-33
+        weight[2] *= 1e33
+    weight = weight.to(dtype)
+    expected = scaling.quantize(weight.float().numpy(), values, group=group, integer=integer, asym=asym, scale=scale, fmt=fmt)
+    reciprocal = scaling.f32_reciprocal(float(values.max() - values.min()) if asym else float(np.abs(values).max()))
+    codes, scales, zeros, flag = scalar_encode.round_matrix(
+        weight.cuda(), dev(values), dev(FRACTIONS) if scale == "mse" else None, group, asym=asym, integer=integer,
+        minimum=float(values.min()), maximum=float(values.max()), reciprocal=float(reciprocal), scale_format=fmt)
+    assert flag.item() == 0
+    np.testing.assert_array_equal(host(scales), expected["scales"])
+    if asym:
+        np.testing.assert_array_equal(host(zeros), expected["zero"])
+    np.testing.assert_array_equal(host(codes), expected["codes"])
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_rounding_in_one_pass_reports_non_finite_weights(bad):
+    import mlkit_amd as mk
+
+    weight = torch.randn(40, 200, device="cuda").half()
+    weight[39, 199] = bad
+    with pytest.raises(ValueError, match="finite"):
+        mk.int(4, 64)(weight)
