@@ -60,6 +60,20 @@ int mk_packed_matvec(const void *x, int x_dtype, const uint8_t *packed, const vo
                      int input_width, int group, int bits, int uniform, float grid_min,
                      float grid_step, void *stream);
 
+/* The same product for nine rows of activations and more, on the matrix cores; arguments as mk_packed_matvec.
+ *   x_dtype, scale_dtype  MK_F16 or MK_BF16
+ *   bits                  2, 3 or 4; 8 with a uniform grid
+ *   input_width           a multiple of 32; x and packed 16-byte aligned
+ *   group                 64, a multiple of 128, or at least input_width
+ * MK_ERR_UNSUPPORTED otherwise (nothing was launched): decode the weight and multiply.
+ * Codes are exact operands and scales multiply fp32 sums, so no weight is rounded to x's type.
+ * Replaces: the decode and dense product of inference/packed_linear.py:110-154. */
+int mk_packed_matmul(const void *x, int x_dtype, const uint8_t *packed, const void *scales,
+                     int scale_dtype, const float *values, int n_values, const void *zeros,
+                     const void *bias, int bias_dtype, void *y, int samples, int output_width,
+                     int input_width, int group, int bits, int uniform, float grid_min,
+                     float grid_step, void *stream);
+
 /* mk_packed_matvec for `count` (1..8) weight matrices of one input width and one codec in a
  * single call: y[i] = x[i] @ dequant(packed[i])^T (+ bias[i]) for every i, each with
  * output_widths[i] rows.  The activation pointers may all be the same (sibling projections

@@ -32,6 +32,7 @@ COMMON_FLAGS = [
 EXACT_FLAGS = ["-ffp-contract=off"]
 
 MATVEC_WIDTHS = range(2, 9)
+MATMUL_FORMATS = range(5)
 
 
 def translation_units() -> list[tuple[str, pathlib.Path, list[str]]]:
@@ -39,9 +40,12 @@ def translation_units() -> list[tuple[str, pathlib.Path, list[str]]]:
     for width in MATVEC_WIDTHS:
         units.append((f"packed_matvec_b{width}", CSRC / "packed_matvec_bits.hip",
                       [f"-DMK_MATVEC_BITS={width}"]))
+    for code_format in MATMUL_FORMATS:
+        units.append((f"packed_matmul_f{code_format}", CSRC / "packed_matmul_kernels.hip",
+                      [f"-DMK_MATMUL_FORMAT={code_format}"]))
     exact = {"packed_decode", "scalar_codec", "scalar_round", "error_feedback", "hadamard", "vector_feedback"}
     for source in sorted(CSRC.glob("*.hip")):
-        if source.name == "packed_matvec_bits.hip":
+        if source.name in ("packed_matvec_bits.hip", "packed_matmul_kernels.hip"):
             continue
         units.append((source.stem, source, EXACT_FLAGS if source.stem in exact else []))
     return units

@@ -11,6 +11,8 @@ How a call is served here:
   has absorbed its online input rotation, one ``mk_rotated_packed_matvec`` call (rotation
   kernel and matvec enqueued back to back, the rotated activations staying in a small buffer
   of the layer);
+* up to ``maximum_product_rows`` rows of fp16 or bf16 (a batch of sequences, a short prompt): one
+  ``mk_packed_matmul`` launch that multiplies the codes on the matrix cores;
 * more rows, or a layout without a fused kernel: the weight is decoded once
   (``mk_packed_decode``) and an ordinary matrix product follows;
 * a tied embedding decodes only the requested rows (``mk_packed_decode_rows``).
@@ -33,6 +35,12 @@ from mlkit_amd.quantization.core import Q
 
 SCALE_STORAGE_DTYPES = {"fp16": torch.float16, "bf16": torch.bfloat16}
 MAXIMUM_FUSED_ROWS = 8
+# Rows up to which multiplying the codes beats decoding the weight for a library product (us, 4096 x 14336 / 14336 x 4096
+# INT4 at 128 rows 38 / 44 against 90 / 60, NF4 54 / 52 against 85 / 55; at 192 rows NF4 and INT8 14336 x 4096 lose, 74
+# and 80 against 62 and 65).  Layers of at most 2^24 weights gain up to 256 rows (4096 x 4096: INT4 23 against 35, INT8 29
+# against 34), where the decode and the product are two short launches.
+MAXIMUM_PRODUCT_ROWS, MAXIMUM_PRODUCT_ROWS_SMALL, SMALL_WEIGHTS = 128, 256, 1 << 24
+PRODUCT_DTYPES = frozenset({torch.float16, torch.bfloat16})
 _LAUNCH_BUFFERS = frozenset({"packed", "scales", "values", "zeros", "bias"})
 
 
@@ -133,12 +141,23 @@ class PackedLinear(nn.Module):
         self.uniform_grid, self.grid_minimum, self.grid_step = grid.uniform, grid.minimum, grid.step
         self.layout: PackedLayout | None = layout_for(self.code_bits, self.in_features, self.group)
         self.maximum_fused_rows = MAXIMUM_FUSED_ROWS if self.layout is not None else 0
+        self.maximum_product_rows = self._product_rows()
         self._launch: tuple | None = None
         self._rotation = None          # an absorbed OnlineRotation
         self._rotation_launch: tuple | None = None
         self._siblings: SiblingLaunch | None = None
         preserve_input_processing(original, self)
         self._absorb_rotation_hook()
+
+    def _product_rows(self) -> int:
+        """Rows up to which ``mk_packed_matmul`` serves this layer; zero when it does not take the layer."""
+        width, group, bits = self.in_features, self.group, self.code_bits
+        taken = (self.layout is not None and (bits in (2, 3, 4) or (bits == 8 and self.uniform_grid)) and width % 32 == 0
+                 and (group == 64 or group % 128 == 0 or group >= width)
+                 and self.scales.dtype in (torch.float16, torch.bfloat16) and self.packed.data_ptr() % 16 == 0)
+        if not taken:
+            return 0
+        return MAXIMUM_PRODUCT_ROWS_SMALL if width * self.out_features <= SMALL_WEIGHTS else MAXIMUM_PRODUCT_ROWS
 
     # -- online input rotation ---------------------------------------------------------------
 
@@ -227,6 +246,11 @@ class PackedLinear(nn.Module):
             else:
                 inputs = self._rotation(inputs)   # the general path: rotate, then as an unrotated layer
         if not fused:
+            if (MAXIMUM_FUSED_ROWS < rows <= self.maximum_product_rows and not compiling and self._dense_weight is None
+                    and inputs.dtype in PRODUCT_DTYPES and not (inputs.requires_grad and torch.is_grad_enabled())):
+                product = self._product(inputs, rows)
+                if product is not None:
+                    return product
             return functional.linear(inputs, self.weight.to(inputs.dtype), self.bias)
         if inputs.requires_grad and torch.is_grad_enabled():
             raise RuntimeError("packed CUDA inference does not support autograd")
@@ -302,6 +326,22 @@ class PackedLinear(nn.Module):
                 rotated = torch.empty((MAXIMUM_FUSED_ROWS, self.in_features), dtype=inputs.dtype, device=inputs.device)
                 bound = self._rotation_launch = (key, rotated, (order, power, basis, signs, scale), keep)
         return None if bound[1] is None else bound
+
+    def _product(self, inputs: Tensor, rows: int) -> Tensor | None:
+        """More rows than a matvec on the codes; None when the library refuses the call (a buffer that was moved
+        to an unaligned address, say): the caller decodes the weight then."""
+        flat = inputs.reshape(rows, self.in_features)
+        if not flat.is_contiguous():
+            flat = flat.contiguous()
+        output = inputs.new_empty((rows, self.out_features))
+        _, tensors, constants = self._bound_arguments()
+        status = native.library().mk_packed_matmul(flat.data_ptr(), native.DTYPE_CODES[flat.dtype], *tensors, output.data_ptr(),
+                                                   rows, *constants, native.current_stream(flat.device))
+        if status == native.MK_ERR_UNSUPPORTED:
+            return None
+        if status:
+            native.check(status)
+        return output.view(inputs.shape[:-1] + (self.out_features,))
 
     def _matvec(self, inputs: Tensor, output: Tensor, rows: int, rotate: bool = False) -> None:
         """One call into the C ABI on the current stream."""

@@ -1,0 +1,124 @@
+"""GPU parity (through the C ABI) of the packed product on the matrix cores, nine rows of activations and more: the
+oracle's dense reconstruction multiplied in float64."""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import scaling
+
+import helpers
+
+pytestmark = pytest.mark.gpu
+
+F32 = np.float32
+INT4 = scaling.int_values(4)
+SEVEN = np.array([-1, -0.5, -0.25, 0, 0.25, 0.5, 1], dtype=F32)
+# name -> (values, bits, integer)
+CODECS = {"int4": (INT4, 4, True), "nf4": (scaling.NF4_VALUES, 4, False), "seven": (SEVEN, 3, False),
+          "int3": (scaling.int_values(3), 3, True), "int2": (scaling.int_values(2), 2, True),
+          "int8": (scaling.int_values(8), 8, True)}
+# An output is rounded once to x's type (2^-12 / 2^-9 of it); table values are rounded to that type too.
+RANGE_TOLERANCE = {torch.float16: 1e-3, torch.bfloat16: 8e-3}
+
+
+def run(layer, x, bias=None, scale_dtype=torch.float16):
+    from mlkit_amd import native
+
+    def device(array, dtype):
+        return None if array is None else torch.from_numpy(np.ascontiguousarray(array)).to(device="cuda", dtype=dtype)
+
+    rows, width = layer["shape"]
+    packed, scales = device(layer["packed"], torch.uint8), device(layer["scales"], scale_dtype)
+    zeros, values = device(layer["zero"], scale_dtype), device(layer["values"], torch.float32)
+    y = torch.full((x.shape[0], rows), float("nan"), dtype=x.dtype, device="cuda")
+    uniform = int(np.allclose(np.diff(layer["values"]), layer["values"][1] - layer["values"][0]))
+    minimum, step = float(layer["values"][0]), float(layer["values"][1] - layer["values"][0])
+    status = native.library().mk_packed_matmul(
+        x.data_ptr(), native.dtype_code(x), packed.data_ptr(), scales.data_ptr(), native.dtype_code(scales), values.data_ptr(),
+        values.numel(), native.pointer(zeros), native.pointer(bias), 0 if bias is None else native.dtype_code(bias), y.data_ptr(),
+        x.shape[0], rows, width, layer["group"], layer["bits"], uniform, minimum, step, native.current_stream(x.device))
+    native.check(status)
+    torch.cuda.synchronize()
+    return y
+
+
+def check(y, layer, x, bias=None):
+    expected = x.double().cpu().numpy() @ layer["dense"].astype(np.float64).T
+    if bias is not None:
+        expected = expected + bias.double().cpu().numpy()
+    error = np.abs(y.double().cpu().numpy() - expected).max() / np.abs(expected).max()
+    assert error <= RANGE_TOLERANCE[y.dtype], error
+
+
+@pytest.mark.parametrize("name,rows,width,group,samples,asym", [
+    # one tile of each kind, every format, rows / columns / samples that do not fill it
+    ("int4", 1, 32, 64, 9, False),
+    ("int4", 77, 416, 128, 17, True),
+    ("int4", 130, 1056, 256, 33, False),        # a scale for two steps of 128 columns, a ragged last group
+    ("int4", 100, 160, 160, 128, True),         # one scale a row
+    ("int4", 66, 4096 + 96, 64, 40, False),     # two groups a step, the last step half empty
+    ("nf4", 31, 224, 64, 16, False),
+    ("nf4", 40, 384, 128, 65, True),            # a table with offsets
+    ("seven", 50, 672, 64, 20, False),          # 48 bits a lane, from 2-byte boundaries
+    ("int3", 35, 2080, 128, 48, True),          # three dwords a lane
+    ("int2", 48, 352, 64, 10, False),
+    ("int2", 33, 288, 128, 96, True),
+    ("int8", 47, 544, 128, 31, True),
+    ("int8", 20, 192, 64, 12, False),
+    # the tiles the launch chooses among: 2 x 1, 2 x 2, 4 x 1, 4 x 2, two workgroups of 2 x 4 on a compute unit
+    ("int4", 4096 + 5, 64, 64, 17, False),
+    ("int4", 4000, 256, 128, 64, False),
+    ("nf4", 14336, 64, 64, 16, False),
+    ("int4", 14336, 128, 128, 32, True),
+    ("int8", 8200, 128, 128, 100, False),
+    ("int4", 20000, 32, 32, 16, False),         # more tiles than compute units at 4 x 1 and at 4 x 2
+    ("int3", 20000, 64, 64, 30, False),
+    # eight wavefronts of many steps
+    ("int4", 96, 18944, 128, 24, True),
+])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_product_matches_the_dense_reconstruction(name, rows, width, group, samples, asym, dtype):
+    values, bits, integer = CODECS[name]
+    layer = helpers.quantised_layer(helpers.normal_weight(rows, width, seed=rows + width), values, bits=bits, group=group,
+                                    integer=integer, asym=asym)
+    x = helpers.activations(samples, width, seed=samples, dtype=dtype).cuda()
+    bias = torch.randn(rows, generator=torch.Generator().manual_seed(3)).to(device="cuda", dtype=dtype) if rows % 2 else None
+    check(run(layer, x, bias), layer, x, bias)
+
+
+def test_bf16_scales_and_activations_with_a_common_offset():
+    """The operands carry an offset that sums of x cancel: activations far from zero mean keep the tolerance."""
+    layer = helpers.quantised_layer(helpers.normal_weight(64, 1024, seed=5), INT4, bits=4, group=128, integer=True, fmt="bf16")
+    for dtype in (torch.float16, torch.bfloat16):
+        x = (helpers.activations(20, 1024, seed=1, dtype=torch.float32) + 3).to(dtype).cuda()
+        check(run(layer, x, scale_dtype=torch.bfloat16), layer, x)
+
+
+def test_refuses_what_it_does_not_take():
+    layer = helpers.quantised_layer(helpers.normal_weight(16, 96, seed=5), INT4, bits=4, group=32, integer=True)
+    x = helpers.activations(16, 96, seed=1).cuda()
+    with pytest.raises(ValueError, match="scale groups"):
+        run(layer, x)
+    with pytest.raises(ValueError, match="fp16 or bf16 activations"):
+        run(layer, x.float())
+
+
+@pytest.mark.parametrize("samples", [9, 128, 129, 300])
+def test_packed_linear_on_both_sides_of_the_row_limit(samples):
+    import mlkit_amd as mk
+
+    torch.manual_seed(samples)
+    linear = torch.nn.Linear(512, 320, device="cuda", dtype=torch.bfloat16)
+    packed = mk.PackedLinear(linear, mk.int(4, 128, asym=True)(linear.weight.detach()))
+    x = torch.randn(3, samples // 3, 512, device="cuda", dtype=torch.bfloat16)[:, :, :] if samples % 3 == 0 else \
+        torch.randn(1, samples, 512, device="cuda", dtype=torch.bfloat16)
+    expected = torch.nn.functional.linear(x.float(), packed.weight.float(), packed.bias.float())
+    with torch.no_grad():
+        y = packed(x)
+    assert y.shape == expected.shape
+    # the decoded weight is rounded to bf16 (2^-9 relative), the output once more
+    assert ((y.float() - expected).norm() / expected.norm()).item() < 6e-3
+    x.requires_grad_(True)
+    packed(x).float().sum().backward()     # more than eight rows stay differentiable in the input
+    assert torch.isfinite(x.grad).all()
