@@ -4,9 +4,9 @@
 // (K up to 16384).  The library factorisation spends most of its time in its small
 // unblocked panel kernel, so the blocked algorithm is driven from the host with library
 // matrix products for the trailing updates, and this file supplies the rest: a workgroup
-// factors a diagonal block of at most 128 x 128 in registers and, on request, carries 128
+// factors a diagonal block of at most 128 x 128 in registers and, on request, carries 64
 // columns of the block's rows through the same elimination, which makes them the factor's
-// block row (one workgroup per 128 columns; no triangular solve is needed).
+// block row (one workgroup per 64 columns; no triangular solve is needed).
 //
 // Replaces the `torch.linalg.cholesky_ex` call of `feedback_coefficients`
 // (quantization/algorithms/error_feedback.py:37-83 in /root/reference/src/mlkit) for large
@@ -15,8 +15,6 @@
 // by the diagonal and reversal back), one pass over the matrix each.
 
 #include "mk_common.h"
-
-#include <type_traits>
 
 namespace {
 
@@ -33,198 +31,197 @@ struct BlockArgs {
     float *factor_out;   // where the factor goes when row_columns > 0 (128 floats per row); else in place
 };
 
-constexpr int kTile = kBlock / 16;
-constexpr int kRowFloats = 2 * kBlock;   // a published row: the block's columns, then the columns carried beside it
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-// Columns 16 SIXTEEN ... 16 SIXTEEN + 15 of the factorisation below, two per step (their rows
-// sit in register row SIXTEEN of their owners).  False after a pivot that is not positive and
-// finite, which every thread sees in the same step.
-//
-// A step takes rows j and j + 1 as the updates of columns < j left them (`pivot_rows`), and
-// every thread derives what it needs of the two finished rows itself:
-//   U[j][k]     = A[j][k] / sqrt(A[j][j])
-//   U[j+1][k]   = (A[j+1][k] - U[j][j+1] U[j][k]) / sqrt(A[j+1][j+1] - U[j][j+1]^2)
-// and subtracts both outer products from its sub-block: one LDS round trip and one barrier
-// per two columns.
-//
-// ROW: the workgroup also carries 128 columns to the right of the block (`beside`), which take
-// the same row operations and so become U_jj^-T A_jr, the block row of the factor.
-template <int SIXTEEN, bool ROW, int BT>
-__device__ __forceinline__ bool sixteen_steps(const BlockArgs &a, float (&mine)[kTile][kTile], float (&beside)[kTile][BT],
-                                              float (&pivot_rows)[2][2][kRowFloats], int tx, int ty) {
-#pragma unroll 1
-    for (int lane = 0; lane < 16; lane += 2) {
-        const int j = 16 * SIXTEEN + lane;
-        const float *first = pivot_rows[(j >> 1) & 1][0], *second = pivot_rows[(j >> 1) & 1][1];
-        const float pivot = first[j];
-        if (!(pivot > 0.0f) || !(pivot - pivot == 0.0f)) {
-            if (threadIdx.x == 0) *a.status = a.first_column + j + 1;
-            return false;
-        }
-        // (one v_rsq_f32, accurate to an ulp; the IEEE square root and division were a fifth of a step's chain)
-        const float reciprocal = __builtin_amdgcn_rsqf(pivot);
-        const float link = first[j + 1] * reciprocal;                 // U[j][j+1]
-        const float next_pivot = second[j + 1] - link * link;
-        if (!(next_pivot > 0.0f) || !(next_pivot - next_pivot == 0.0f)) {
-            if (threadIdx.x == 0) *a.status = a.first_column + j + 2;
-            return false;
-        }
-        const float next_reciprocal = __builtin_amdgcn_rsqf(next_pivot);
-        // Register rows below SIXTEEN hold only rows <= j (finished); register columns below
-        // SIXTEEN only columns < j, which for the rows still changing lie below the diagonal
-        // (never read): neither takes part, so a step costs 2 (8 - SIXTEEN)^2 multiply-adds.
-        float rows_first[kTile], rows_second[kTile], columns_first[kTile], columns_second[kTile];
-#pragma unroll
-        for (int u = SIXTEEN; u < kTile; ++u) {
-            const int i = ty + 16 * u, k = tx + 16 * u;
-            const float upper = first[i] * reciprocal;                                   // U[j][i]
-            const float lower = (second[i] - link * upper) * next_reciprocal;            // U[j+1][i]
-            rows_first[u] = i > j + 1 ? upper : 0.0f;   // zero keeps rows <= j + 1 as they are
-            rows_second[u] = i > j + 1 ? lower : 0.0f;
-            columns_first[u] = first[k] * reciprocal;                                    // U[j][k]
-            columns_second[u] = (second[k] - link * columns_first[u]) * next_reciprocal; // U[j+1][k]
-        }
-        float beside_first[BT], beside_second[BT];
-        if constexpr (ROW) {
-#pragma unroll
-            for (int v = 0; v < BT; ++v) {
-                const int c = kBlock + tx + 16 * v;
-                beside_first[v] = first[c] * reciprocal;
-                beside_second[v] = (second[c] - link * beside_first[v]) * next_reciprocal;
-            }
-        }
-        // The two rows' owners keep the finished rows.
-        if (ty == lane) {
-#pragma unroll
-            for (int v = SIXTEEN; v < kTile; ++v) mine[SIXTEEN][v] = columns_first[v];
-            if constexpr (ROW) {
-#pragma unroll
-                for (int v = 0; v < BT; ++v) beside[SIXTEEN][v] = beside_first[v];
-            }
-        }
-        if (ty == lane + 1) {
-#pragma unroll
-            for (int v = SIXTEEN; v < kTile; ++v) mine[SIXTEEN][v] = columns_second[v];
-            if constexpr (ROW) {
-#pragma unroll
-                for (int v = 0; v < BT; ++v) beside[SIXTEEN][v] = beside_second[v];
-            }
-        }
-#pragma unroll
-        for (int u = SIXTEEN; u < kTile; ++u) {
-#pragma unroll
-            for (int v = SIXTEEN; v < kTile; ++v)
-                mine[u][v] -= rows_first[u] * columns_first[v] + rows_second[u] * columns_second[v];
-            if constexpr (ROW) {
-#pragma unroll
-                for (int v = 0; v < BT; ++v)
-                    beside[u][v] -= rows_first[u] * beside_first[v] + rows_second[u] * beside_second[v];
-            }
-        }
-        // Rows j + 2 and j + 3 have all their updates now: their owners publish them.
-        float (*next)[kRowFloats] = pivot_rows[((j >> 1) + 1) & 1];
-        if (lane < 14) {
-            if (ty == lane + 2 || ty == lane + 3) {
-#pragma unroll
-                for (int v = SIXTEEN; v < kTile; ++v) next[ty - lane - 2][tx + 16 * v] = mine[SIXTEEN][v];   // columns < j are not read
-                if constexpr (ROW) {
-#pragma unroll
-                    for (int v = 0; v < BT; ++v) next[ty - lane - 2][kBlock + tx + 16 * v] = beside[SIXTEEN][v];
-                }
-            }
-        } else if constexpr (SIXTEEN + 1 < kTile) {
-            if (ty < 2) {
-#pragma unroll
-                for (int v = SIXTEEN + 1; v < kTile; ++v) next[ty][tx + 16 * v] = mine[SIXTEEN + 1][v];
-                if constexpr (ROW) {
-#pragma unroll
-                    for (int v = 0; v < BT; ++v) next[ty][kBlock + tx + 16 * v] = beside[SIXTEEN + 1][v];
-                }
-            }
-        }
-        __syncthreads();
-    }
-    return true;
+constexpr int kTile = 16;                       // rows and columns of a tile
+constexpr int kTiles = kBlock / kTile;          // tile columns of the block
+constexpr int kWaves = kThreads / 64;
+constexpr int kCarried = kWaves * kTile;        // columns a workgroup carries beside the block
+constexpr int kColumnFloats = kTile + 4;        // a tile column in LDS (16-byte aligned, banks spread)
+
+__device__ __forceinline__ float lane_value(float x, int lane) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), lane));
 }
 
 // In: the upper triangle of a symmetric positive definite block.  Out: U with block = U^T U
 // in the upper triangle, zeros below it.  A pivot that is not positive (or not finite)
 // records its column and leaves the block unspecified.
 //
-// Right-looking, two columns per step.  The block lives in registers for the whole
-// factorisation: thread (ty, tx) of a 16 x 16 grid owns entries (ty + 16 u, tx + 16 v),
-// an 8 x 8 sub-block.  Per step only the two pivot rows travel: the threads that own them
-// put them (as updated so far) into one of two LDS buffers, one barrier later every thread
-// reads the entries it needs, finishes the two rows for itself and subtracts their outer
-// products from its sub-block.  Rows up to the pivot rows are masked out of the update by
-// zero factors, so finished rows keep their values.
-// BT: sixteenths of 128 columns a workgroup carries beside the block (8: 128 columns, 4: 64).
-template <bool ROW, int BT>
-__global__ void __launch_bounds__(kThreads) cholesky_block_kernel(const BlockArgs a) {
-    __shared__ float pivot_rows[2][2][kRowFloats];   // [buffer][row j, row j + 1][column]
+// ROW: the workgroup also carries 64 columns to the right of the block, which take the same row
+// operations and so become U_jj^-T A_jr, the block row of the factor.  Every workgroup factors the block
+// itself (from the matrix, which nobody overwrites: the factor goes to `factor_out`), and the first one stores it.
+//
+// Right-looking over panels of 16 rows.  The block and the carried columns are 16 x 16 tiles (negated) in the
+// accumulators of four wavefronts, wavefront w owning tile columns 3 - w, 4 + w and, beside the block, w.  Per panel:
+//   1. the owners put the panel's tiles into LDS by columns;
+//   2. a lane takes a column of 16 values into registers, lanes 0 ... 15 of EVERY wavefront the diagonal tile's, the
+//      other lanes those of the wavefront's three tiles, and all 16 elimination steps run inside the wavefront: row j is
+//      scaled by 1 / sqrt(pivot), row i > j loses U[j][i] (a scalar, from lane i) times row j;
+//   3. the finished rows go back to LDS, and the tiles below lose U_r^T U_c on the matrix cores.  A 16 x 16 x 4
+//      accumulator holds rows 4 (lane / 16) + i of a column where the operands hold k = lane / 16, so product i takes
+//      k = 4 (lane / 16) + i and a tile is read as an operand exactly as it is held: one 16-byte LDS read.
+// Two barriers per 16 columns (one per two columns before, with every pivot row passed through LDS): what
+// bounds the kernel is the chain of 128 pivots.  One copy of the code serves all panels, since a
+// launch runs it once and instruction fetches would show.  A block with 768 columns beside it, called back to back: 25 us
+// (48 us a launch as a pair of columns per barrier); carrying the 64 columns costs 3 us of that.
+template <bool ROW>
+__global__ void __launch_bounds__(kThreads, 2) cholesky_block_kernel(const BlockArgs a) {
+    __shared__ __align__(16) float panel[2][kTiles + kWaves][kTile][kColumnFloats];   // [buffer][tile column][column][row]
     __shared__ int failed;
+    if (threadIdx.x == 0) failed = *a.status;
     const int n = a.size;
-    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-    if (threadIdx.x == 0) failed = *a.status != 0;   // an earlier block already failed: do nothing
-    float mine[kTile][kTile], beside[kTile][BT];
-    constexpr int kCarried = 16 * BT;
-    // ROW: workgroup b carries columns kCarried b ... kCarried (b + 1) - 1 of the block row; every workgroup
-    // factors the block itself (from the matrix, which nobody overwrites: the factor goes to
-    // `factor_out`), and the first one stores it.
-    const int beside_first_column = n + kCarried * blockIdx.x;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int column = lane & 15, quarter = lane >> 4;
+    const int left_column = kWaves - 1 - wave, right_column = wave + kWaves;
+    const int carried_first = kCarried * static_cast<int>(blockIdx.x) + kTile * wave;   // of this wavefront, counted from the block's end
+
+    // tiles of row r: tile column 3 - wave (r <= 3), tile column wave + 4, the carried ones
+    f32x4 left[kWaves], right[kTiles], beside[kTiles];
+    // Addresses are clamped into the block instead of guarded: a branch per load would wait for each of them in turn.
+    const uint32_t leading = static_cast<uint32_t>(a.leading), last = static_cast<uint32_t>(n - 1);
+    auto block_tile = [&](int r, int c) __attribute__((always_inline)) -> f32x4 {
+        f32x4 tile;
 #pragma unroll
-    for (int u = 0; u < kTile; ++u)
-#pragma unroll
-        for (int v = 0; v < kTile; ++v) {
-            const int row = ty + 16 * u, column = tx + 16 * v;
-            const bool inside = row < n && column < n && column >= row;
-            const float loaded = a.matrix[(inside ? row : 0) * a.leading + (inside ? column : 0)];
-            // Outside the block: an identity diagonal keeps every pivot of the padding at one.
-            mine[u][v] = inside ? loaded : (row == column ? 1.0f : 0.0f);
-            if (v < BT) {
-                beside[u][v] = 0.0f;
-                if constexpr (ROW) {
-                    const bool present = row < n && kCarried * static_cast<int>(blockIdx.x) + column < a.row_columns;
-                    const float carried = a.matrix[(present ? row : 0) * a.leading + (present ? beside_first_column + column : 0)];
-                    beside[u][v] = present ? carried : 0.0f;
-                }
-            }
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t first = r * kTile + 4 * quarter + i, second = c * kTile + column;
+            const uint32_t row = min(first, second), col = max(first, second);   // the upper triangle stands for both
+            tile[i] = a.matrix[min(row, last) * leading + min(col, last)];
         }
-    if (ty < 2) {
+        return tile;
+    };
+    const uint32_t carried_column = n + min(carried_first + column, a.row_columns - 1);
 #pragma unroll
-        for (int v = 0; v < kTile; ++v) {
-            pivot_rows[0][ty][tx + 16 * v] = mine[0][v];
-            if constexpr (ROW) {
-                if (v < BT) pivot_rows[0][ty][kBlock + tx + 16 * v] = beside[0][v];
+    for (int r = 0; r < kTiles; ++r) {
+        if (r < kWaves) left[r] = block_tile(r, left_column);   // (tiles below the diagonal: any numbers, never used)
+        right[r] = block_tile(r, right_column);
+        if constexpr (ROW) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                beside[r][i] = a.matrix[min(static_cast<uint32_t>(r * kTile + 4 * quarter + i), last) * leading + carried_column];
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < kTiles; ++r) {
+        // Outside the block: an identity diagonal keeps every pivot of the padding at one.
+        auto negated = [&](f32x4 &tile, int c) __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int row = r * kTile + 4 * quarter + i, col = c * kTile + column;
+                tile[i] = max(row, col) < n ? -tile[i] : (row == col ? -1.0f : 0.0f);
             }
+        };
+        if (r < kWaves) negated(left[r], left_column);
+        negated(right[r], right_column);
+        if constexpr (ROW) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) beside[r][i] = r * kTile + 4 * quarter + i < n ? -beside[r][i] : 0.0f;
         }
     }
     __syncthreads();
-    if (failed) return;
+    if (failed) return;   // an earlier block already did: do nothing
 
-    // All 128 columns run (the padding is an identity): no data-dependent exit other than a bad pivot.
-    bool good = sixteen_steps<0, ROW, BT>(a, mine, beside, pivot_rows, tx, ty);
-    good = good && sixteen_steps<1, ROW, BT>(a, mine, beside, pivot_rows, tx, ty);
-    good = good && sixteen_steps<2, ROW, BT>(a, mine, beside, pivot_rows, tx, ty);
-    good = good && sixteen_steps<3, ROW, BT>(a, mine, beside, pivot_rows, tx, ty);
-    good = good && sixteen_steps<4, ROW, BT>(a, mine, beside, pivot_rows, tx, ty);
-    good = good && sixteen_steps<5, ROW, BT>(a, mine, beside, pivot_rows, tx, ty);
-    good = good && sixteen_steps<6, ROW, BT>(a, mine, beside, pivot_rows, tx, ty);
-    good = good && sixteen_steps<7, ROW, BT>(a, mine, beside, pivot_rows, tx, ty);
-    if (!good) return;
     float *factor = ROW ? a.factor_out : a.matrix;
-    const long long factor_leading = ROW ? kBlock : a.leading;
+    const uint32_t factor_leading = ROW ? kBlock : leading;
+    const int panels = (n + kTile - 1) / kTile;
+#pragma unroll 1
+    for (int s = 0; s < panels; ++s) {
+        float (*tiles)[kTile][kColumnFloats] = panel[s & 1];
+        auto publish = [&](int tile_column, f32x4 tile) __attribute__((always_inline)) {
+            *reinterpret_cast<f32x4 *>(&tiles[tile_column][column][4 * quarter]) = -tile;
+        };
 #pragma unroll
-    for (int u = 0; u < kTile; ++u)
+        for (int r = 0; r < kTiles; ++r)
+            if (r == s) {
+                if (r < kWaves) publish(left_column, left[r]);
+                publish(right_column, right[r]);
+                if constexpr (ROW) publish(wave + kTiles, beside[r]);
+            }
+        __syncthreads();
+
+        // a column of the panel per lane
+        const int own = quarter == 1 ? left_column : wave + kWaves * (quarter - 1);   // tile column of lanes 16 ... 63
+        float *source = tiles[quarter == 0 ? s : own][column];
+        float value[kTile];
 #pragma unroll
-        for (int v = 0; v < kTile; ++v) {
-            const int row = ty + 16 * u, column = tx + 16 * v;
-            if (blockIdx.x == 0 && row < n && column < n) factor[row * factor_leading + column] = column >= row ? mine[u][v] : 0.0f;
-            if constexpr (ROW) {
-                if (v < BT && row < n && kCarried * static_cast<int>(blockIdx.x) + column < a.row_columns)
-                    a.matrix[row * a.leading + beside_first_column + column] = beside[u][v];
+        for (int i = 0; i < 4; ++i) {
+            const f32x4 four = reinterpret_cast<const f32x4 *>(source)[i];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) value[4 * i + k] = four[k];
+        }
+        uint32_t refused = 0;
+        auto reciprocal_root = [&](int j) __attribute__((always_inline)) -> float {
+            const float pivot = lane_value(value[j], j);
+            refused |= static_cast<uint32_t>(__float_as_int(pivot)) - 1u < 0x7f7fffffu ? 0u : 1u << j;   // positive and finite
+            return __builtin_amdgcn_rsqf(pivot);   // accurate to an ulp; an IEEE square root and division would double the chain
+        };
+        float reciprocal = reciprocal_root(0);
+#pragma unroll
+        for (int j = 0; j < kTile; ++j) {
+            value[j] *= reciprocal;
+            if (j + 1 < kTile) {   // the next pivot's chain first: the rest of this step hides its latency
+                value[j + 1] = __builtin_fmaf(-lane_value(value[j], j + 1), value[j], value[j + 1]);
+                reciprocal = reciprocal_root(j + 1);
+            }
+            float factors[kTile];
+#pragma unroll
+            for (int i = j + 2; i < kTile; ++i) factors[i] = lane_value(value[j], i);
+#pragma unroll
+            for (int i = j + 2; i < kTile; ++i) value[i] = __builtin_fmaf(-factors[i], value[j], value[i]);
+            // step by step: put off, as the compiler would have it, the updates of a row are one dependent chain
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (refused) {   // every wavefront of every workgroup comes to the same value
+            if (threadIdx.x == 0) *a.status = a.first_column + s * kTile + __builtin_ctz(refused) + 1;
+            return;
+        }
+        // (the diagonal tile stays as it is: another wavefront may still have to read it)
+        if (s + 1 < panels && quarter > 0 && own != s && (ROW || quarter < 3)) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                reinterpret_cast<f32x4 *>(source)[i] = f32x4{value[4 * i], value[4 * i + 1], value[4 * i + 2], value[4 * i + 3]};
+        }
+        // The finished rows: lanes 0 ... 15 of the diagonal tile's owner, and the other tiles from their columns' lanes.
+        if (blockIdx.x == 0 && (quarter == 0 ? s == left_column || s == right_column : quarter < 3 && own != s)) {
+            const int to = (quarter == 0 ? s : own) * kTile + column;
+            if (to < n) {
+#pragma unroll
+                for (int j = 0; j < kTile; ++j) {
+                    const int row = s * kTile + j;   // uniform
+                    if (row < n) factor[row * factor_leading + to] = to >= row ? value[j] : 0.0f;
+                }
             }
         }
+        if constexpr (ROW) {
+            if (quarter == 3 && carried_first + column < a.row_columns) {
+#pragma unroll
+                for (int j = 0; j < kTile; ++j) {
+                    const int row = s * kTile + j;
+                    if (row < n) a.matrix[row * leading + carried_column] = value[j];
+                }
+            }
+        }
+        if (s + 1 == panels) return;
+        __syncthreads();
+
+        auto operand = [&](int tile_column) __attribute__((always_inline)) -> f32x4 {
+            return *reinterpret_cast<const f32x4 *>(&tiles[tile_column][column][4 * quarter]);
+        };
+        const f32x4 u_left = operand(left_column), u_right = operand(right_column), u_beside = operand(ROW ? wave + kTiles : wave);
+        f32x4 rows[kTiles];
+#pragma unroll
+        for (int r = 1; r < kTiles; ++r) rows[r] = operand(r);
+#pragma unroll
+        for (int r = 1; r < kTiles; ++r) {
+            if (r <= s) continue;   // uniform
+            auto update = [&](f32x4 &tile, f32x4 u) __attribute__((always_inline)) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) tile = __builtin_amdgcn_mfma_f32_16x16x4f32(rows[r][i], u[i], tile, 0, 0, 0);
+            };
+            if constexpr (ROW) update(beside[r], u_beside);
+            if (r <= right_column) update(right[r], u_right);   // uniform
+            if (r < kWaves && r <= left_column) update(left[r], u_left);
+        }
+    }
 }
 
 }  // namespace
@@ -319,17 +316,14 @@ extern "C" int mk_cholesky_block(float *matrix, long long leading, int size, int
     MK_REQUIRE(size >= 1 && size <= kBlock, MK_ERR_UNSUPPORTED, "mk_cholesky_block: blocks of 1 to %d rows (got %d)", kBlock, size);
     MK_REQUIRE(row_columns >= 0 && leading >= static_cast<long long>(size) + row_columns && first_column >= 0, MK_ERR_INVALID,
                "mk_cholesky_block: rows overlap");
+    MK_REQUIRE(leading <= (1ll << 32) / kBlock, MK_ERR_INVALID, "mk_cholesky_block: a block's rows must lie within 2^32 floats");
     MK_REQUIRE(row_columns == 0 || factor_out, MK_ERR_INVALID,
                "mk_cholesky_block: a block row needs a separate place for the factor");
     BlockArgs a{matrix, leading, size, first_column, status, row_columns, factor_out};
-    // 64 columns per workgroup while that still fits one workgroup per CU (a step then costs a
-    // third less arithmetic); 128 beyond.
-    if (row_columns > 256 * 64)
-        hipLaunchKernelGGL((cholesky_block_kernel<true, 8>), dim3(mk_cdiv(row_columns, 128)), dim3(kThreads), 0, stream, a);
-    else if (row_columns > 0)
-        hipLaunchKernelGGL((cholesky_block_kernel<true, 4>), dim3(mk_cdiv(row_columns, 64)), dim3(kThreads), 0, stream, a);
+    if (row_columns > 0)
+        hipLaunchKernelGGL((cholesky_block_kernel<true>), dim3(mk_cdiv(row_columns, kCarried)), dim3(kThreads), 0, stream, a);
     else
-        hipLaunchKernelGGL((cholesky_block_kernel<false, 4>), dim3(1), dim3(kThreads), 0, stream, a);
+        hipLaunchKernelGGL((cholesky_block_kernel<false>), dim3(1), dim3(kThreads), 0, stream, a);
     MK_LAUNCH_CHECK("mk_cholesky_block");
     return MK_OK;
 }

@@ -321,3 +321,52 @@ def test_blocked_factorisation_reports_an_indefinite_matrix():
     quantizer = mk.gptq(mk.int(4, group=128))
     with pytest.raises(ValueError, match="positive definite"):
         quantizer(dev(np.zeros((8, width), dtype=np.float32)), mk.Ctx("layer", H=dev(hessian)))
+
+
+def block_factor(matrix, size, first=0):
+    """`mk_cholesky_block` on the first `size` rows of a matrix: (factor, block row, status)."""
+    from mlkit_amd import native
+
+    width = matrix.shape[0]
+    work = dev(matrix)
+    beside = width - size
+    factor = torch.zeros((128, 128), device="cuda")
+    status = torch.zeros((), dtype=torch.int32, device="cuda")
+    native.check(native.library().mk_cholesky_block(
+        work.data_ptr(), width, size, first, beside, factor.data_ptr() if beside else None, status.data_ptr(),
+        native.current_stream(work.device)))
+    out = host(work)
+    return (host(factor)[:size, :size] if beside else out[:size, :size]), out[:size, size:], int(status.item())
+
+
+@pytest.mark.parametrize("size,beside", [(1, 0), (15, 0), (16, 1), (17, 64), (64, 63), (100, 130), (113, 0), (127, 200), (128, 0),
+                                         (128, 1), (128, 65), (128, 700)])
+def test_a_factored_block_and_its_block_row(size, beside):
+    """Sizes at the edges of the 16-row panels and of the 64 columns a workgroup carries.  Normwise the factor of a
+    well-conditioned matrix is as good as a few fp32 roundings per pivot: 1e-5 of its norm leaves a factor of ten."""
+    rng = np.random.default_rng(size * 1000 + beside)
+    width = size + beside
+    inputs = rng.standard_normal((2 * width + 8, width))
+    matrix = (inputs.T @ inputs / inputs.shape[0] + 0.05 * np.eye(width)).astype(np.float32)
+    expected = np.linalg.cholesky(matrix[:size, :size].astype(np.float64)).T
+    factor, row, status = block_factor(matrix, size)
+    assert status == 0
+    assert np.linalg.norm(factor - expected) <= 1e-5 * np.linalg.norm(expected)
+    assert not np.tril(factor, -1).any()
+    if beside:
+        carried = np.linalg.solve(expected.T, matrix[:size, size:].astype(np.float64))
+        assert np.linalg.norm(row - carried) <= 1e-5 * np.linalg.norm(carried)
+
+
+@pytest.mark.parametrize("column", [0, 1, 15, 16, 47, 100, 126])
+@pytest.mark.parametrize("value", [-1.0, float("nan"), float("inf")])
+def test_a_factored_block_names_its_bad_pivot(column, value):
+    matrix = np.eye(130, dtype=np.float32) * 2
+    matrix[column, column] = value
+    assert block_factor(matrix, 128, first=256)[2] == 256 + column + 1
+
+
+@pytest.mark.parametrize("width,step", [(128, 1), (129, 1), (255, 1), (384, 8), (640, 1), (896, 1), (1000, 2), (1023, 1)])
+def test_blocked_factorisation_of_narrow_matrices(width, step):
+    """The same comparison as for wide matrices, from the narrowest one that is factored by blocks."""
+    test_blocked_factorisation_matches_the_float64_coefficients(width, step)
