@@ -69,7 +69,7 @@ extern "C" int mk_packed_matmul(const void *x, int x_dtype, const uint8_t *packe
     MatmulArgs a{};
     a.x = x; a.packed = packed; a.scales = static_cast<const uint16_t *>(scales); a.zeros = static_cast<const uint16_t *>(zeros);
     a.values = values; a.bias = bias; a.y = y;
-    a.samples = samples; a.rows = output_width; a.width = input_width; a.groups = mk_cdiv(input_width, group);
+    a.samples = samples; a.rows = output_width; a.width = input_width; a.groups = mk_cdiv(input_width, group); a.group = group;
     a.steps = mk_cdiv(input_width, mk_matmul::kStep);
     a.n_values = n_values; a.uniform = uniform; a.scale_bf16 = scale_dtype == MK_BF16; a.bias_dtype = bias_dtype;
     a.grid_min = grid_min; a.grid_step = grid_step;

@@ -45,7 +45,7 @@ struct MatmulArgs {
     const float *values;
     const void *bias;         // or null
     void *y;
-    int samples, rows, width, groups;
+    int samples, rows, width, groups, group;
     int steps;                // ceil(width / 128)
     int steps_per_group;      // SUB == 1: steps that share a scale
     uint32_t group_multiplier;   // step / steps_per_group = umulhi(step, multiplier) >> shift, where that is above one
@@ -180,6 +180,29 @@ struct Codes<kTable2, XT, CH> {
 
 __device__ __forceinline__ float table_value(const MatmulArgs &a, int code) {
     return a.uniform ? a.grid_min + static_cast<float>(code) * a.grid_step : a.values[code < a.n_values ? code : a.n_values - 1];
+}
+
+// An output by its definition, one product after the other, for sums that are not finite: an infinite activation times
+// operand and offset gives infinities of both signs where its product with the decoded weight has one.
+template <int FORMAT, int XT>
+__device__ __forceinline__ float plain_output(const MatmulArgs &a, int row, int sample, float bias) {
+    constexpr int kBits = Codes<FORMAT, XT, 32>::kBits;
+    const uint8_t *codes = a.packed + static_cast<size_t>(row) * (a.width / 8 * kBits);
+    const size_t x = static_cast<size_t>(sample) * a.width, side = static_cast<size_t>(row) * a.groups;
+    const int side_type = a.scale_bf16 ? MK_BF16 : MK_F16;
+    float sum = 0.0f;
+#pragma unroll 1
+    for (int k = 0; k < a.width; ++k) {
+        const int bit = k * kBits, byte = bit >> 3;
+        uint32_t code = codes[byte];
+        if ((bit & 7) + kBits > 8) code |= static_cast<uint32_t>(codes[byte + 1]) << 8;
+        code = (code >> (bit & 7)) & ((1u << kBits) - 1);
+        const int group = a.group >= a.width ? 0 : k / a.group;
+        float weight = table_value(a, static_cast<int>(code)) * mk_load_as_float(a.scales, side + group, side_type);
+        if (a.zeros) weight += mk_load_as_float(a.zeros, side + group, side_type);
+        sum = __builtin_fmaf(weight, mk_load_as_float(a.x, x + k, XT), sum);
+    }
+    return sum + bias;
 }
 
 // Dynamic LDS of a workgroup, in bytes; the sums of the wavefronts reuse the activations' stretch.
@@ -429,6 +452,10 @@ __global__ void __launch_bounds__(64 * kMaxWaves) packed_matmul_kernel(const Mat
         if (sample >= a.samples || row >= a.rows) continue;
         const size_t at = static_cast<size_t>(sample) * a.rows + row;
         const int valid = min(4, a.rows - row);
+        if (const float all = (value[0] + value[1]) + (value[2] + value[3]); __builtin_expect(all - all != 0.0f, 0)) {
+#pragma unroll 1
+            for (int i = 0; i < valid; ++i) value[i] = plain_output<FORMAT, XT>(a, row + i, sample, biases[local_row + i]);
+        }
         uint16_t *target = static_cast<uint16_t *>(a.y) + at;
         const mk_u32x2 packed = {pair_of<XT>(value[0], value[1]), pair_of<XT>(value[2], value[3])};
         if (a.whole_quads) *reinterpret_cast<mk_u32x2 *>(target) = packed;

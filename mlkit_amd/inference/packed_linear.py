@@ -247,7 +247,7 @@ class PackedLinear(nn.Module):
                 inputs = self._rotation(inputs)   # the general path: rotate, then as an unrotated layer
         if not fused:
             if (MAXIMUM_FUSED_ROWS < rows <= self.maximum_product_rows and not compiling and self._dense_weight is None
-                    and inputs.dtype in PRODUCT_DTYPES and not (inputs.requires_grad and torch.is_grad_enabled())):
+                    and inputs.dtype in PRODUCT_DTYPES and self._plain_call(inputs)):
                 product = self._product(inputs, rows)
                 if product is not None:
                     return product
@@ -326,6 +326,17 @@ class PackedLinear(nn.Module):
                 rotated = torch.empty((MAXIMUM_FUSED_ROWS, self.in_features), dtype=inputs.dtype, device=inputs.device)
                 bound = self._rotation_launch = (key, rotated, (order, power, basis, signs, scale), keep)
         return None if bound[1] is None else bound
+
+    def _plain_call(self, inputs: Tensor) -> bool:
+        """Whether a library call may stand for ``functional.linear``: nothing differentiates, batches, records or casts
+        what this call does, and the dense product would take these types and devices."""
+        bias = self._buffers["bias"]
+        return (type(inputs) is Tensor and inputs.device == self._buffers["packed"].device
+                and (bias is None or bias.dtype == inputs.dtype)
+                and not (inputs.requires_grad and torch.is_grad_enabled())
+                and not torch.is_autocast_enabled("cuda") and torch._C._get_tracing_state() is None
+                and torch._C._functorch.peek_interpreter_stack() is None   # vmap, functional gradients
+                and torch.autograd.forward_ad._current_level < 0 and torch._C._len_torch_dispatch_stack() == 0)
 
     def _product(self, inputs: Tensor, rows: int) -> Tensor | None:
         """More rows than a matvec on the codes; None when the library refuses the call (a buffer that was moved

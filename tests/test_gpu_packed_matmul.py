@@ -122,3 +122,45 @@ def test_packed_linear_on_both_sides_of_the_row_limit(samples):
     x.requires_grad_(True)
     packed(x).float().sum().backward()     # more than eight rows stay differentiable in the input
     assert torch.isfinite(x.grad).all()
+
+
+@pytest.mark.parametrize("name,asym", [("int4", True), ("int4", False), ("nf4", False), ("seven", False), ("int2", True), ("int8", True)])
+def test_infinite_activations_reach_the_outputs_as_in_a_dense_product(name, asym):
+    values, bits, integer = CODECS[name]
+    rng = np.random.default_rng(5)
+    layer = helpers.quantised_layer(helpers.normal_weight(37, 224, seed=2), values, bits=bits, group=64, integer=integer, asym=asym)
+    x = torch.from_numpy(rng.standard_normal((19, 224), dtype=F32)).to("cuda", torch.bfloat16)
+    x[3, 7], x[4, 100], x[5, 9] = float("inf"), float("-inf"), float("nan")
+    y = run(layer, x).double().cpu().numpy()
+    with np.errstate(invalid="ignore"):
+        expected = (x.double().cpu().numpy()[:, None, :] * layer["dense"].astype(np.float64)[None]).sum(-1)
+    np.testing.assert_array_equal(np.isnan(y), np.isnan(expected))
+    np.testing.assert_array_equal(np.isinf(y) * np.sign(y), np.isinf(expected) * np.sign(expected))
+
+
+def test_calls_that_are_recorded_batched_differentiated_or_cast_take_the_dense_product():
+    import torch.autograd.forward_ad as forward_ad
+
+    import mlkit_amd as mk
+
+    linear = torch.nn.Linear(256, 48, device="cuda", dtype=torch.float16)
+    layer = mk.PackedLinear(linear, mk.int(4, 128)(linear.weight.detach()))
+    x = torch.randn((17, 256), device="cuda", dtype=torch.float16)
+
+    def dense(inputs):
+        return torch.nn.functional.linear(inputs, layer.weight.to(inputs.dtype), layer.bias)
+
+    stacked = torch.stack([x, 2 * x])
+    assert torch.equal(torch.func.vmap(layer)(stacked), torch.func.vmap(dense)(stacked))
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert layer(x).dtype == torch.bfloat16
+    traced = torch.jit.trace(layer, (x,), check_trace=False)
+    torch.testing.assert_close(traced(3 * x), dense(3 * x))
+    with forward_ad.dual_level():
+        out = forward_ad.unpack_dual(layer(forward_ad.make_dual(x, torch.ones_like(x))))
+        torch.testing.assert_close(out.tangent, torch.nn.functional.linear(torch.ones_like(x), layer.weight))
+    wanted = x.clone().requires_grad_()
+    layer(wanted).sum().backward()
+    assert wanted.grad is not None
+    with pytest.raises(RuntimeError):
+        layer(x.bfloat16())   # a bias of another type: refused, as the dense product refuses it
