@@ -303,6 +303,20 @@ int mk_rotate_blocks(const void *source, int source_dtype, void *target, int tar
                      int order, int power, const float *basis, int transpose, const float *signs_before,
                      const float *signs_after, float scale, void *stream);
 
+/* target[:, c] = scale * H source[:, c] for every column c of a contiguous [rows, columns] matrix, in fp32; rows 1024,
+ * 2048 or 4096 (MK_ERR_UNSUPPORTED otherwise).  signs_before / signs_after: one float per row, or NULL.  Agrees with mk_fwht
+ * of the turned matrix to fp32 rounding (another order of stages), not bit for bit.
+ * Replaces: `rotate(w.T.contiguous()).T` of quantization/algorithms/incoherence.py:56-98. */
+int mk_fwht_columns(const void *source, int source_dtype, float *target, int rows, int columns,
+                    const float *signs_before, const float *signs_after, float scale, void *stream);
+
+/* target[c, r] = fp32(source[r, c]) of a contiguous [rows, columns] matrix. */
+int mk_transpose(const void *source, int source_dtype, float *target, int rows, int columns, void *stream);
+
+/* The +-1 vector of a seed: out[i] from a 32-bit hash of i + seed.
+ * Replaces: formats/composition.py:14-20 (deterministic_signs). */
+int mk_hash_signs(float *out, int width, unsigned int seed, void *stream);
+
 /* The rotation of mk_rotate_blocks for a few activation rows, on order * rows workgroups:
  * target[r, f', :] = scale * H_power( sum_f basis[f', f] * (source[r, f, :] * signs[f, :]) ),
  * the same transform with the mix applied before the Walsh-Hadamard stages (they commute),

@@ -43,7 +43,7 @@ def translation_units() -> list[tuple[str, pathlib.Path, list[str]]]:
     for code_format in MATMUL_FORMATS:
         units.append((f"packed_matmul_f{code_format}", CSRC / "packed_matmul_kernels.hip",
                       [f"-DMK_MATMUL_FORMAT={code_format}"]))
-    exact = {"packed_decode", "scalar_codec", "scalar_round", "error_feedback", "hadamard", "vector_feedback"}
+    exact = {"packed_decode", "scalar_codec", "scalar_round", "error_feedback", "hadamard", "vector_feedback", "column_transforms"}
     for source in sorted(CSRC.glob("*.hip")):
         if source.name in ("packed_matvec_bits.hip", "packed_matmul_kernels.hip"):
             continue

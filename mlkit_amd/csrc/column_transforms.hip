@@ -1,0 +1,245 @@
+// Transforms down the columns of a weight, and what goes with them: the Walsh-Hadamard transform of every column without
+// turning the matrix, turning a matrix (and converting it to FP32 on the way), and the signs of a seeded rotation.
+//
+// Covers quantization/algorithms/incoherence.py:56-98 and formats/composition.py:14-47 of the reference, which
+// rotate the output side of a weight as `rotate(w.T.contiguous()).T`.
+
+#include "mk_common.h"
+
+namespace {
+
+// ---- columns --------------------------------------------------------------------------------
+
+struct ColumnArgs {
+    const void *source;
+    float *target;
+    const float *signs_before, *signs_after;   // of the rows, or null
+    int columns, groups, groups_per_xcd;
+    float scale;
+};
+
+// The transform of GROUPS * VALUES rows.  Thread (c, g) first holds rows g + GROUPS k of column c, k = 0 ... VALUES - 1, and
+// does the stages over k in registers; through LDS it comes to hold VALUES / GROUPS of the k with all g, whose stages
+// follow.  A matrix is read once and written once.  The exchange takes two turns so that a workgroup's values fit LDS and
+// a thread its registers: in turn p a thread in half h of the groups puts half h ^ p of its k there and takes
+// what it needs of the groups' half h ^ p, into the registers that came free.
+//
+// Bound by HBM.  Neighbouring workgroups share 128-byte lines, so they are given to one XCD, whose L2 has
+// the line: workgroup b takes column group (b % 8) * groups_per_xcd + b / 8.
+//
+// fp32, 14336 columns of 1024 / 2048 / 4096 values: 21 / 41 / 141 us, against 63 + 63 us for torch's strided copies around
+// the row transform at 1024, 119 + 119 at 2048 and 255 + 255 at 4096.  4096 rows run at 3.3 TB/s: 144 registers keep a
+// second workgroup off the compute unit, and held to 128 the kernel spills (206 us); 16 columns a workgroup take 151 us.
+template <int COLUMNS, int GROUPS, int VALUES, int SOURCE>
+__global__ void __launch_bounds__(COLUMNS * GROUPS) fwht_columns_kernel(const ColumnArgs a) {
+    constexpr int kHeld = VALUES / GROUPS;         // the k of a thread behind the exchange
+    constexpr int kHalf = VALUES / 2, kHalfGroups = GROUPS / 2;
+    extern __shared__ float exchange[];
+    const int group = static_cast<int>(blockIdx.x & 7) * a.groups_per_xcd + static_cast<int>(blockIdx.x >> 3);
+    if (group >= a.groups) return;   // whole workgroups
+    const int local = threadIdx.x & (COLUMNS - 1), g = threadIdx.x / COLUMNS;
+    const int half = __builtin_amdgcn_readfirstlane(g / kHalfGroups);   // a wavefront's groups lie in one half
+    const int column = group * COLUMNS + local;
+    const bool inside = column < a.columns;
+    const size_t from = inside ? column : a.columns - 1;
+    float value[2][kHalf];   // [k / kHalf][k % kHalf]
+#pragma unroll
+    for (int k = 0; k < VALUES; ++k)
+        value[k / kHalf][k % kHalf] = mk_load_as_float(a.source, static_cast<size_t>(g + GROUPS * k) * a.columns + from, SOURCE);
+    if (a.signs_before) {   // uniform
+#pragma unroll
+        for (int k = 0; k < VALUES; ++k) value[k / kHalf][k % kHalf] *= a.signs_before[g + GROUPS * k];
+    }
+    auto butterfly = [](float &first, float &second) __attribute__((always_inline)) {
+        const float low = first, high = second;
+        first = low + high;
+        second = low - high;
+    };
+    auto turned_halves = [&]() __attribute__((always_inline)) {
+        if (half)
+#pragma unroll
+            for (int i = 0; i < kHalf; ++i) {
+                const float first = value[0][i];
+                value[0][i] = value[1][i];
+                value[1][i] = first;
+            }
+    };
+#pragma unroll
+    for (int stride = 1; stride < VALUES; stride *= 2)
+#pragma unroll
+        for (int k = 0; k < VALUES; ++k)
+            if ((k & stride) == 0) butterfly(value[k / kHalf][k % kHalf], value[(k + stride) / kHalf][(k + stride) % kHalf]);
+    // (a pad of a group's floats behind the k of one reader keeps the readers of a wavefront on different banks)
+    auto slot = [&](int k, int in_half) __attribute__((always_inline)) -> int {
+        return (k * kHalfGroups + k / kHeld + in_half) * COLUMNS + local;
+    };
+    turned_halves();
+#pragma unroll
+    for (int turn = 0; turn < 2; ++turn) {
+        if (turn) __syncthreads();   // the turn before has been read
+#pragma unroll
+        for (int i = 0; i < kHalf; ++i) exchange[slot((half ^ turn) * kHalf + i, g & (kHalfGroups - 1))] = value[turn][i];
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < kHeld; ++m)
+#pragma unroll
+            for (int j = 0; j < kHalfGroups; ++j) value[turn][m * kHalfGroups + j] = exchange[slot(g * kHeld + m, j)];
+    }
+    turned_halves();
+    // now [half of the groups][which of the thread's k, group within the half]
+#pragma unroll
+    for (int stride = 1; stride < kHalfGroups; stride *= 2)
+#pragma unroll
+        for (int i = 0; i < kHalf; ++i)
+            if ((i & stride) == 0) {
+                butterfly(value[0][i], value[0][i + stride]);
+                butterfly(value[1][i], value[1][i + stride]);
+            }
+#pragma unroll
+    for (int i = 0; i < kHalf; ++i) butterfly(value[0][i], value[1][i]);
+    if (!inside) return;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int i = 0; i < kHalf; ++i) {
+            const int row = (g * kHeld + i / kHalfGroups) * GROUPS + h * kHalfGroups + i % kHalfGroups;
+            float result = value[h][i] * a.scale;
+            if (a.signs_after) result *= a.signs_after[row];
+            a.target[static_cast<size_t>(row) * a.columns + column] = result;
+        }
+}
+
+template <int COLUMNS, int GROUPS, int VALUES, int SOURCE>
+void launch_columns(ColumnArgs a, hipStream_t stream) {
+    a.groups = mk_cdiv(a.columns, COLUMNS);
+    a.groups_per_xcd = mk_cdiv(a.groups, 8);
+    constexpr size_t lds = (VALUES * (GROUPS / 2) + GROUPS) * COLUMNS * sizeof(float);
+    static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void *>(&fwht_columns_kernel<COLUMNS, GROUPS, VALUES, SOURCE>),
+                                                          hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    static_cast<void>(allowed);   // a refusal shows in the launch
+    hipLaunchKernelGGL((fwht_columns_kernel<COLUMNS, GROUPS, VALUES, SOURCE>), dim3(8 * a.groups_per_xcd), dim3(COLUMNS * GROUPS), lds, stream, a);
+}
+
+template <int SOURCE>
+void launch_rows(const ColumnArgs &a, int rows, hipStream_t stream) {
+    if (rows == 1024) launch_columns<16, 32, 32, SOURCE>(a, stream);
+    else if (rows == 2048) launch_columns<16, 32, 64, SOURCE>(a, stream);
+    else launch_columns<8, 64, 64, SOURCE>(a, stream);
+}
+
+// ---- turning a matrix -----------------------------------------------------------------------
+
+struct TransposeArgs {
+    const void *source;
+    float *target;
+    int rows, columns;
+};
+
+// 64 x 64 tiles through LDS, fp32 4096 x 14336 in 98 us (4.8 TB/s; torch's strided copy 255), from bf16 in 84 (320 with its conversion); reads and writes both move whole 16-byte pieces along rows where the sizes allow it (VEC).
+template <int SOURCE, bool VEC>
+__global__ void __launch_bounds__(256) transpose_kernel(const TransposeArgs a) {
+    __shared__ float tile[64][65];
+    const int tx = (threadIdx.x & 15) * 4, ty = threadIdx.x >> 4;
+    const int row0 = blockIdx.y * 64, column0 = blockIdx.x * 64;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int local = ty + 16 * j, row = min(row0 + local, a.rows - 1);
+        const size_t base = static_cast<size_t>(row) * a.columns;
+        if constexpr (VEC) {
+            const size_t at = base + min(column0 + tx, a.columns - 4);   // past the edge: numbers that nobody writes out
+            if constexpr (SOURCE == MK_F32) {
+                const float4 four = *reinterpret_cast<const float4 *>(static_cast<const float *>(a.source) + at);
+                tile[local][tx] = four.x; tile[local][tx + 1] = four.y; tile[local][tx + 2] = four.z; tile[local][tx + 3] = four.w;
+            } else {
+                const uint2 four = *reinterpret_cast<const uint2 *>(static_cast<const uint16_t *>(a.source) + at);
+                const uint32_t word[2] = {four.x, four.y};
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const uint16_t raw = static_cast<uint16_t>(word[i / 2] >> (16 * (i & 1)));
+                    tile[local][tx + i] = SOURCE == MK_F16 ? static_cast<float>(__builtin_bit_cast(_Float16, raw)) : mk_bf16_to_float(raw);
+                }
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) tile[local][tx + i] = mk_load_as_float(a.source, base + min(column0 + tx + i, a.columns - 1), SOURCE);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int local = ty + 16 * j, column = column0 + local, row = row0 + tx;
+        if (column >= a.columns) continue;
+        float *to = a.target + static_cast<size_t>(column) * a.rows + row;
+        if constexpr (VEC) {
+            if (row < a.rows) *reinterpret_cast<float4 *>(to) = make_float4(tile[tx][local], tile[tx + 1][local], tile[tx + 2][local], tile[tx + 3][local]);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (row + i < a.rows) to[i] = tile[tx + i][local];
+        }
+    }
+}
+
+template <int SOURCE>
+void launch_transpose(const TransposeArgs &a, hipStream_t stream) {
+    const dim3 grid(mk_cdiv(a.columns, 64), mk_cdiv(a.rows, 64));
+    const bool whole = a.rows % 4 == 0 && a.columns % 4 == 0
+                       && ((reinterpret_cast<uintptr_t>(a.source) | reinterpret_cast<uintptr_t>(a.target)) & 15u) == 0;
+    if (whole) hipLaunchKernelGGL((transpose_kernel<SOURCE, true>), grid, dim3(256), 0, stream, a);
+    else hipLaunchKernelGGL((transpose_kernel<SOURCE, false>), grid, dim3(256), 0, stream, a);
+}
+
+// ---- signs ------------------------------------------------------------------------------------
+
+// The hash works on 32 bits: every step is masked to them.
+__global__ void __launch_bounds__(256) hash_signs_kernel(float *out, int width, uint32_t seed) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= width) return;
+    uint32_t v = static_cast<uint32_t>(i) + seed;
+    v = (v ^ (v >> 16)) * 0x45D9F3Bu;
+    v = (v ^ (v >> 16)) * 0x45D9F3Bu;
+    v ^= v >> 16;
+    out[i] = v & 1u ? 1.0f : -1.0f;
+}
+
+}  // namespace
+
+extern "C" int mk_fwht_columns(const void *source, int source_dtype, float *target, int rows, int columns,
+                               const float *signs_before, const float *signs_after, float scale, void *stream_) {
+    hipStream_t stream = static_cast<hipStream_t>(stream_);
+    MK_REQUIRE(rows == 1024 || rows == 2048 || rows == 4096, MK_ERR_UNSUPPORTED,
+               "mk_fwht_columns: columns of 1024, 2048 or 4096 values, not %d", rows);
+    MK_REQUIRE(columns >= 1, MK_ERR_INVALID, "mk_fwht_columns: sizes must be positive");
+    MK_REQUIRE(source && target, MK_ERR_INVALID, "mk_fwht_columns: null tensor pointer");
+    MK_REQUIRE(source != target, MK_ERR_INVALID, "mk_fwht_columns: source and target must not alias");
+    MK_REQUIRE(mk_dtype_valid(source_dtype), MK_ERR_INVALID, "mk_fwht_columns: unknown dtype code");
+    ColumnArgs a{source, target, signs_before, signs_after, columns, 0, 0, scale};
+    if (source_dtype == MK_F32) launch_rows<MK_F32>(a, rows, stream);
+    else if (source_dtype == MK_F16) launch_rows<MK_F16>(a, rows, stream);
+    else launch_rows<MK_BF16>(a, rows, stream);
+    MK_LAUNCH_CHECK("mk_fwht_columns");
+    return MK_OK;
+}
+
+extern "C" int mk_transpose(const void *source, int source_dtype, float *target, int rows, int columns, void *stream_) {
+    hipStream_t stream = static_cast<hipStream_t>(stream_);
+    MK_REQUIRE(rows >= 1 && columns >= 1, MK_ERR_INVALID, "mk_transpose: sizes must be positive");
+    MK_REQUIRE(mk_cdiv(rows, 64) <= 65535, MK_ERR_UNSUPPORTED, "mk_transpose: too many rows");
+    MK_REQUIRE(source && target, MK_ERR_INVALID, "mk_transpose: null tensor pointer");
+    MK_REQUIRE(source != target, MK_ERR_INVALID, "mk_transpose: source and target must not alias");
+    MK_REQUIRE(mk_dtype_valid(source_dtype), MK_ERR_INVALID, "mk_transpose: unknown dtype code");
+    TransposeArgs a{source, target, rows, columns};
+    if (source_dtype == MK_F32) launch_transpose<MK_F32>(a, stream);
+    else if (source_dtype == MK_F16) launch_transpose<MK_F16>(a, stream);
+    else launch_transpose<MK_BF16>(a, stream);
+    MK_LAUNCH_CHECK("mk_transpose");
+    return MK_OK;
+}
+
+extern "C" int mk_hash_signs(float *out, int width, unsigned int seed, void *stream_) {
+    hipStream_t stream = static_cast<hipStream_t>(stream_);
+    MK_REQUIRE(out && width >= 1, MK_ERR_INVALID, "mk_hash_signs: a buffer of at least one value is required");
+    hipLaunchKernelGGL(hash_signs_kernel, dim3(mk_cdiv(width, 256)), dim3(256), 0, stream, out, width, seed);
+    MK_LAUNCH_CHECK("mk_hash_signs");
+    return MK_OK;
+}

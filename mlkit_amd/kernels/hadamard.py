@@ -61,6 +61,34 @@ def transform(
     return output
 
 
+def transform_columns(matrix: Tensor, *, signs_before: Tensor | None = None, signs_after: Tensor | None = None) -> Tensor:
+    """The transform of every column of a contiguous matrix of 1024, 2048 or 4096 rows, in FP32; one sign per row."""
+    device = native.require_device(matrix, signs_before, signs_after)
+    if matrix.dim() != 2 or not matrix.is_contiguous():
+        raise ValueError("transform_columns requires a contiguous two-dimensional tensor")
+    rows, columns = matrix.shape
+    for signs in (signs_before, signs_after):
+        if signs is not None and (signs.dtype != torch.float32 or not signs.is_contiguous() or signs.numel() != rows):
+            raise ValueError("sign vectors must be contiguous FP32 with one entry per row")
+    output = torch.empty((rows, columns), dtype=torch.float32, device=device)
+    native.check(native.library().mk_fwht_columns(
+        matrix.data_ptr(), native.dtype_code(matrix), output.data_ptr(), rows, columns, native.pointer(signs_before),
+        native.pointer(signs_after), normaliser(rows), native.current_stream(device)))
+    return output
+
+
+def turned(matrix: Tensor) -> Tensor:
+    """The FP32 transpose of a contiguous matrix, as a contiguous tensor."""
+    device = native.require_device(matrix)
+    if matrix.dim() != 2 or not matrix.is_contiguous():
+        raise ValueError("turned requires a contiguous two-dimensional tensor")
+    rows, columns = matrix.shape
+    output = torch.empty((columns, rows), dtype=torch.float32, device=device)
+    native.check(native.library().mk_transpose(matrix.data_ptr(), native.dtype_code(matrix), output.data_ptr(), rows, columns,
+                                               native.current_stream(device)))
+    return output
+
+
 def mix_blocks(value: Tensor, basis: Tensor, *, transpose: bool, signs_after: Tensor | None = None) -> Tensor:
     """``out[..., f', p] = sum_f mix[f', f] * value[..., f, p]`` with ``mix = basis`` or ``basis.T``."""
     device = native.require_device(value, basis, signs_after)

@@ -132,6 +132,13 @@ def decode_vector_scaled(codes: Tensor, *, scales: Tensor, values: Tensor | None
 
 def deterministic_signs(width: int, seed: int, device: torch.device | str) -> Tensor:
     """Rademacher signs from an integer hash of ``index + seed``: identical on every device."""
+    if torch.device(device).type == "cuda" and width > 0:
+        from mlkit_amd import native
+
+        signs = torch.empty(width, dtype=torch.float32, device=device)
+        native.check(native.library().mk_hash_signs(signs.data_ptr(), width, seed & 0xFFFFFFFF,
+                                                    native.current_stream(signs.device)))
+        return signs
     v = (torch.arange(width, device=device, dtype=torch.int64) + seed) & 0xFFFFFFFF
     for _ in range(2):
         v = ((v ^ (v >> 16)) * 0x45D9F3B) & 0xFFFFFFFF
@@ -145,7 +152,7 @@ def decode_basis(codes: Tensor, *, inner_codec: str, shape: "tuple[int, int] | l
                  **parameters: Any) -> Tensor:
     """Codes of a matrix quantized in a rotated basis: the inner decoder's reconstruction is
     rotated back, input side (columns) first, then output side (rows)."""
-    from mlkit_amd.quantization.transforms import rotate
+    from mlkit_amd.quantization.transforms import rotate, rotate_columns
 
     inner = {key.removeprefix("inner_"): value for key, value in parameters.items()}
     restored = decoder(inner_codec)(codes, **inner)
@@ -154,7 +161,7 @@ def decode_basis(codes: Tensor, *, inner_codec: str, shape: "tuple[int, int] | l
         restored = rotate(restored, inverse=True, signs=signs)
     if left_seed is not None:
         signs = left_signs if left_signs is not None else deterministic_signs(shape[0], left_seed, codes.device)
-        restored = rotate(restored.T.contiguous(), inverse=True, signs=signs).T
+        restored = rotate_columns(restored, inverse=True, signs=signs)
     return restored
 
 

@@ -20,7 +20,7 @@ from torch import Tensor
 
 from mlkit_amd.quantization.codecs import compose, deterministic_signs, registered
 from mlkit_amd.quantization.core import Ctx, Q, Quantizer, as_q, layer_seed
-from mlkit_amd.quantization.transforms import rotate
+from mlkit_amd.quantization.transforms import rotate, rotate_columns
 
 SIDE_KINDS = (None, "rht")
 
@@ -38,7 +38,7 @@ class _Side:
 
     def along_rows(self, matrix: Tensor, back: bool = False) -> Tensor:
         """``(T diag(signs)) @ matrix`` (every column transformed), or its inverse."""
-        return self.along_columns(matrix.T, back).T
+        return rotate_columns(matrix, inverse=back, signs=self.signs)
 
     def conjugate(self, symmetric: Tensor) -> Tensor:
         """``(T S) M (T S)^T`` for a square matrix over this side's width."""
@@ -84,7 +84,8 @@ class Incoherent(Quantizer):
         output_side = _Side(rows, base_seed, w.device) if self.left else None
         input_side = _Side(columns, base_seed + 1, w.device) if self.right else None
 
-        in_basis = w.float()
+        # (16-bit weights on a HIP device are converted by the first transform)
+        in_basis = w.float() if output_side is None or not w.is_cuda or w.requires_grad else w
         if output_side is not None:
             in_basis = output_side.along_rows(in_basis)
         if input_side is not None:

@@ -177,6 +177,25 @@ def rotate(value: Tensor, *, inverse: bool = False, signs: Tensor | None = None,
     return mixed.reshape(value.shape).to(value.dtype)
 
 
+COLUMN_KERNEL_ROWS = frozenset({1024, 2048, 4096})   # columns that one workgroup transforms without turning the matrix
+
+
+def rotate_columns(matrix: Tensor, *, signs: Tensor, inverse: bool = False) -> Tensor:
+    """``rotate(matrix.T).T``: every column of a matrix transformed, FP32 on a HIP device.  Columns of 1024 to 4096 values
+    (powers of two) take one kernel; others are turned, rotated as rows and turned back, 16-bit ones converted on the way."""
+    if not (matrix.is_cuda and matrix.dim() == 2 and matrix.numel() and matrix.dtype in _KERNEL_DTYPES
+            and not (torch.is_grad_enabled() and (matrix.requires_grad or signs.requires_grad))
+            and matrix.shape[0] <= MAXIMUM_KERNEL_WIDTH):
+        return rotate(matrix.T.contiguous(), inverse=inverse, signs=signs).T
+    from mlkit_amd.kernels import hadamard as kernel
+
+    matrix = matrix.contiguous()
+    if matrix.shape[0] in COLUMN_KERNEL_ROWS:
+        signs = signs.to(device=matrix.device, dtype=torch.float32).contiguous()
+        return kernel.transform_columns(matrix, signs_before=None if inverse else signs, signs_after=signs if inverse else None)
+    return kernel.turned(rotate(kernel.turned(matrix), inverse=inverse, signs=signs))
+
+
 def _structured_on_host(value: Tensor, order: int, power: int, basis: Tensor | None, inverse: bool) -> Tensor:
     if basis is None:
         return hadamard(value)

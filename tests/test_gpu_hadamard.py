@@ -279,3 +279,45 @@ def test_known_answers_of_the_bases_on_the_device():
         np.testing.assert_allclose(out[:, :, 0], dct.T / np.sqrt(power), atol=1e-6)
     for case in known["signs"]:
         assert codecs.deterministic_signs(16, case["seed"], "cuda").tolist() == case["first"]
+
+
+@pytest.mark.parametrize("rows", [256, 640, 1024, 1216, 2048, 4096, 8192])
+@pytest.mark.parametrize("columns", [1, 7, 16, 129, 260])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_columns_are_transformed_as_the_rows_of_the_turned_matrix(rows, columns, dtype):
+    """`rotate_columns` (one kernel for 1024, 2048 and 4096 rows, a turned matrix otherwise), there and back, against the row
+    transform of the same fp32 numbers: log2(rows) additions in another order, each rounding 2^-24 of the norm."""
+    from mlkit_amd.quantization import transforms as device_transforms
+    from mlkit_amd.quantization.codecs import deterministic_signs
+
+    generator = torch.Generator(device="cuda").manual_seed(rows + columns)
+    matrix = torch.randn((rows, columns), device="cuda", generator=generator).to(dtype)
+    signs = deterministic_signs(rows, 5, matrix.device)
+    for inverse in (False, True):
+        out = device_transforms.rotate_columns(matrix, signs=signs, inverse=inverse)
+        expected = device_transforms.rotate(matrix.float().T.contiguous(), signs=signs, inverse=inverse).T
+        assert out.dtype == torch.float32 and out.shape == matrix.shape
+        assert (out - expected).norm() <= 16 * 2.0**-24 * expected.norm()
+    back = device_transforms.rotate_columns(device_transforms.rotate_columns(matrix, signs=signs), signs=signs, inverse=True)
+    assert (back - matrix.float()).norm() <= 64 * 2.0**-24 * matrix.float().norm()
+    view = torch.randn((columns, rows), device="cuda", generator=generator).T   # another order of strides
+    np.testing.assert_allclose(host(device_transforms.rotate_columns(view, signs=signs)),
+                               host(device_transforms.rotate_columns(view.contiguous(), signs=signs)), rtol=0, atol=0)
+
+
+@pytest.mark.parametrize("rows,columns", [(1, 1), (3, 70), (64, 64), (65, 4), (100, 132), (260, 68)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_turning_a_matrix(rows, columns, dtype):
+    from mlkit_amd.kernels import hadamard
+
+    matrix = torch.randn((rows, columns), device="cuda").to(dtype)
+    assert torch.equal(hadamard.turned(matrix), matrix.float().T.contiguous())
+    if rows > 1:   # a base that is not 16-byte aligned
+        assert torch.equal(hadamard.turned(matrix.reshape(-1)[columns:].view(rows - 1, columns)), matrix[1:].float().T.contiguous())
+
+
+@pytest.mark.parametrize("seed", [0, 1, 2**32 - 17, 2**40 + 3])
+def test_signs_of_a_seed_are_the_same_on_every_device(seed):
+    from mlkit_amd.quantization.codecs import deterministic_signs
+
+    assert torch.equal(deterministic_signs(1003, seed, "cuda").cpu(), deterministic_signs(1003, seed, "cpu"))
