@@ -381,6 +381,15 @@ int mk_feedback_block_update_staged(float *feedback, const float *deviations, co
                                     int width, int first_column, int chain_width, int chains, int column_begin,
                                     int column_end, void *stream);
 
+/* mk_feedback_sweep for a vector grid (codewords of `dimension` columns, or the E8P lattice, as in
+ * mk_feedback_round_vector_tile): tiles of at most 256 columns, scales without offsets.  encoded: [rows, width / dimension].
+ * deviations: NULL, or [width, rows] scratch.  Replaces: the host loop of quantization/algorithms/error_feedback.py:296-370. */
+int mk_feedback_vector_sweep(const float *original, float *feedback, float *output, int32_t *encoded,
+                             const float *coeff, float *scales, float *workspace, float *deviations,
+                             const float *codebook, int dimension, int codebook_size, int lattice, int rows, int width,
+                             int group, int refit, int block, float reciprocal, int scale_format, int deferred_tiles,
+                             void *stream);
+
 /* The whole natural-order error-feedback sweep of a layer with per-region absmax / minmax
  * scale fits, enqueued in one call: for every region of `refit` columns the pending
  * continuation (into workspace, [rows, refit] fp32; may be NULL when refit >= width), the

@@ -1340,34 +1340,35 @@ extern "C" int mk_feedback_block_update(float *feedback, const float *original, 
 // kernel launches and no host round trips: per region the pending-continuation solve into
 // `workspace`, the scale fit on those targets, then per tile the column sweep and the
 // (deferred, chained) trailing updates.
-extern "C" int mk_feedback_sweep(const float *original, float *feedback, float *output, uint8_t *encoded,
-                                 const float *coeff, float *scales, float *zeros, float *workspace,
-                                 float *deviations, const float *values, int n_values, int rows, int width,
-                                 int group, int refit,
-                                 int block, int integer_grid, float code_min, float code_max, int asym,
-                                 float reciprocal, float value_minimum, int scale_format, int deferred_tiles,
-                                 void *stream_) {
-    hipStream_t stream = static_cast<hipStream_t>(stream_);
-    MK_REQUIRE(original && feedback && output && encoded && coeff && scales && (!asym || zeros), MK_ERR_INVALID,
-               "mk_feedback_sweep: null tensor pointer");
-    MK_REQUIRE(rows >= 1 && width >= 1 && group >= 1 && block >= 1 && block <= 1024 && refit >= 1 && deferred_tiles >= 1,
-               MK_ERR_INVALID, "mk_feedback_sweep: sizes must be positive and tiles at most 1024 columns wide");
-    MK_REQUIRE(refit >= width || (refit <= 1024 && workspace), MK_ERR_INVALID,
-               "mk_feedback_sweep: regions of %d columns need a workspace and at most 1024 columns", refit);
-    if (integer_grid) {
-        MK_REQUIRE(code_max >= code_min && code_max - code_min <= 255.0f, MK_ERR_INVALID,
-                   "mk_feedback_sweep: integer grid must span at most 256 codes");
-    } else {
-        MK_REQUIRE(values && n_values >= 1 && n_values <= 256, MK_ERR_INVALID,
-                   "mk_feedback_sweep: a value table of 1..256 entries is required");
-    }
+namespace {
+
+// What the sweeps over scalar and vector grids have in common: per region the pending continuation and the fit of its
+// scales, then tile by tile the rounding and the trailing updates.
+struct RegionPlan {
+    const float *original;
+    float *feedback, *output;
+    const float *coeff;
+    float *scales, *zeros, *workspace, *deviations;
+    int rows, width, group, refit, block, asym;
+    float reciprocal, value_minimum;
+    int scale_format, deferred_tiles;
+};
+
+// `fits_itself(span, group)`: the rounding of such a region also solves and fits; `round_tile`: rounds one tile.
+template <typename FitsItself, typename RoundTile>
+int sweep_regions(const char *name, const RegionPlan &p, FitsItself fits_itself, RoundTile round_tile, hipStream_t stream) {
+    const float *original = p.original, *coeff = p.coeff;
+    float *feedback = p.feedback, *output = p.output, *scales = p.scales, *zeros = p.zeros, *workspace = p.workspace, *deviations = p.deviations;
+    const int rows = p.rows, width = p.width, group = p.group, refit = p.refit, block = p.block, asym = p.asym;
+    const int scale_format = p.scale_format, deferred_tiles = p.deferred_tiles;
+    const float reciprocal = p.reciprocal, value_minimum = p.value_minimum;
     const int region_width = refit < width ? refit : width;
     long long total_groups = 0;
     for (int start = 0; start < width; start += region_width) {
         const int span = width - start < region_width ? width - start : region_width;
         total_groups += mk_cdiv(span, group < span ? group : span);
     }
-    MK_REQUIRE(total_groups < (1ll << 31) / rows, MK_ERR_INVALID, "mk_feedback_sweep: too many scale groups");
+    MK_REQUIRE(total_groups < (1ll << 31) / rows, MK_ERR_INVALID, "%s: too many scale groups", name);
 
     struct Tile { int start, stop; };
     Tile deferred[64];
@@ -1405,8 +1406,7 @@ extern "C" int mk_feedback_sweep(const float *original, float *feedback, float *
         }
         float *region_scales = scales + group_offset;
         float *region_zeros = asym ? zeros + group_offset : nullptr;
-        const bool fused = region_fusable(span, block, fitted_group, integer_grid != 0, n_values) && scale_format >= 0 &&
-                           scale_format <= 4;
+        const bool fused = fits_itself(span, fitted_group);
         if (fused) {
             // fitted inside the sweep kernel below
         } else if (region_start == 0) {
@@ -1425,19 +1425,8 @@ extern "C" int mk_feedback_sweep(const float *original, float *feedback, float *
         }
         for (int tile_start = region_start; tile_start < region_stop; tile_start += block) {
             const int tile_stop = tile_start + block < region_stop ? tile_start + block : region_stop;
-            SweepArgs a{};
-            a.original = original; a.feedback = feedback; a.coeff = coeff; a.scales = region_scales;
-            a.zeros = region_zeros; a.values = values; a.output = output; a.encoded = encoded; a.rows = rows;
-            a.width = width; a.region_start = region_start; a.tile_start = tile_start;
-            a.tile_width = tile_stop - tile_start; a.group = fitted_group;
-            a.groups_per_row = static_cast<int>(total_groups); a.n_values = n_values;
-            a.code_min = code_min; a.code_max = code_max; a.deviation_t = deviations;
-            if (fused) {
-                a.fit_scales = region_scales; a.fit_zeros = region_zeros; a.solve_first = region_start != 0;
-                a.asym = asym; a.scale_format = scale_format; a.reciprocal = reciprocal; a.value_minimum = value_minimum;
-                launch_region(a, integer_grid != 0, stream);
-            } else if (integer_grid) launch_sweep<kModeInteger>(a, stream);
-            else launch_sweep<kModeCodebook>(a, stream);
+            if (int status = round_tile(region_start, tile_start, tile_stop, fitted_group, static_cast<int>(total_groups), region_scales, region_zeros, fused))
+                return status;
             if (tile_stop >= width) continue;
             if (tile_stop < limit)
                 if (int status = update(tile_start, tile_stop - tile_start, 1, tile_stop, limit)) return status;
@@ -1451,6 +1440,83 @@ extern "C" int mk_feedback_sweep(const float *original, float *feedback, float *
         }
         group_offset += region_groups;
     }
+    return MK_OK;
+}
+
+}  // namespace
+
+extern "C" int mk_feedback_sweep(const float *original, float *feedback, float *output, uint8_t *encoded,
+                                 const float *coeff, float *scales, float *zeros, float *workspace,
+                                 float *deviations, const float *values, int n_values, int rows, int width,
+                                 int group, int refit,
+                                 int block, int integer_grid, float code_min, float code_max, int asym,
+                                 float reciprocal, float value_minimum, int scale_format, int deferred_tiles,
+                                 void *stream_) {
+    hipStream_t stream = static_cast<hipStream_t>(stream_);
+    MK_REQUIRE(original && feedback && output && encoded && coeff && scales && (!asym || zeros), MK_ERR_INVALID,
+               "mk_feedback_sweep: null tensor pointer");
+    MK_REQUIRE(rows >= 1 && width >= 1 && group >= 1 && block >= 1 && block <= 1024 && refit >= 1 && deferred_tiles >= 1,
+               MK_ERR_INVALID, "mk_feedback_sweep: sizes must be positive and tiles at most 1024 columns wide");
+    MK_REQUIRE(refit >= width || (refit <= 1024 && workspace), MK_ERR_INVALID,
+               "mk_feedback_sweep: regions of %d columns need a workspace and at most 1024 columns", refit);
+    if (integer_grid) {
+        MK_REQUIRE(code_max >= code_min && code_max - code_min <= 255.0f, MK_ERR_INVALID,
+                   "mk_feedback_sweep: integer grid must span at most 256 codes");
+    } else {
+        MK_REQUIRE(values && n_values >= 1 && n_values <= 256, MK_ERR_INVALID,
+                   "mk_feedback_sweep: a value table of 1..256 entries is required");
+    }
+    const RegionPlan plan{original, feedback, output, coeff, scales, zeros, workspace, deviations, rows, width, group, refit, block,
+                          asym, reciprocal, value_minimum, scale_format, deferred_tiles};
+    const auto fits_itself = [&](int span, int fitted_group) {
+        return region_fusable(span, block, fitted_group, integer_grid != 0, n_values) && scale_format >= 0 && scale_format <= 4;
+    };
+    const auto round_tile = [&](int region_start, int tile_start, int tile_stop, int fitted_group, int total_groups,
+                                float *region_scales, float *region_zeros, bool fused) -> int {
+        SweepArgs a{};
+        a.original = original; a.feedback = feedback; a.coeff = coeff; a.scales = region_scales;
+        a.zeros = region_zeros; a.values = values; a.output = output; a.encoded = encoded; a.rows = rows;
+        a.width = width; a.region_start = region_start; a.tile_start = tile_start;
+        a.tile_width = tile_stop - tile_start; a.group = fitted_group;
+        a.groups_per_row = total_groups; a.n_values = n_values;
+        a.code_min = code_min; a.code_max = code_max; a.deviation_t = deviations;
+        if (fused) {
+            a.fit_scales = region_scales; a.fit_zeros = region_zeros; a.solve_first = region_start != 0;
+            a.asym = asym; a.scale_format = scale_format; a.reciprocal = reciprocal; a.value_minimum = value_minimum;
+            launch_region(a, integer_grid != 0, stream);
+        } else if (integer_grid) launch_sweep<kModeInteger>(a, stream);
+        else launch_sweep<kModeCodebook>(a, stream);
+        return MK_OK;
+    };
+    if (int status = sweep_regions("mk_feedback_sweep", plan, fits_itself, round_tile, stream)) return status;
     MK_LAUNCH_CHECK("mk_feedback_sweep");
+    return MK_OK;
+}
+
+extern "C" int mk_feedback_vector_sweep(const float *original, float *feedback, float *output, int32_t *encoded,
+                                        const float *coeff, float *scales, float *workspace, float *deviations,
+                                        const float *codebook, int dimension, int codebook_size, int lattice, int rows, int width,
+                                        int group, int refit, int block, float reciprocal, int scale_format,
+                                        int deferred_tiles, void *stream_) {
+    hipStream_t stream = static_cast<hipStream_t>(stream_);
+    MK_REQUIRE(original && feedback && output && encoded && coeff && scales && codebook, MK_ERR_INVALID,
+               "mk_feedback_vector_sweep: null tensor pointer");
+    MK_REQUIRE(rows >= 1 && width >= 1 && group >= 1 && block >= 1 && block <= 256 && refit >= 1 && deferred_tiles >= 1,
+               MK_ERR_INVALID, "mk_feedback_vector_sweep: sizes must be positive and tiles at most 256 columns wide");
+    MK_REQUIRE(refit >= width || (refit <= 1024 && workspace), MK_ERR_INVALID,
+               "mk_feedback_vector_sweep: regions of %d columns need a workspace and at most 1024 columns", refit);
+    MK_REQUIRE(dimension >= 1 && width % dimension == 0 && block % dimension == 0 && (refit >= width || refit % dimension == 0),
+               MK_ERR_INVALID, "mk_feedback_vector_sweep: rows, regions and tiles must hold whole codewords");
+    const RegionPlan plan{original, feedback, output, coeff, scales, nullptr, workspace, deviations, rows, width, group, refit, block,
+                          0, reciprocal, 0.0f, scale_format, deferred_tiles};
+    const auto fits_itself = [](int, int) { return false; };
+    const auto round_tile = [&](int region_start, int tile_start, int tile_stop, int fitted_group, int total_groups,
+                                float *region_scales, float *, bool) -> int {
+        return mk_round_vector_tile(original, feedback, coeff, region_scales, codebook, output, deviations, encoded, rows, width,
+                                    region_start, tile_start, tile_stop - tile_start, fitted_group, total_groups, dimension,
+                                    codebook_size, lattice, stream);
+    };
+    if (int status = sweep_regions("mk_feedback_vector_sweep", plan, fits_itself, round_tile, stream)) return status;
+    MK_LAUNCH_CHECK("mk_feedback_vector_sweep");
     return MK_OK;
 }

@@ -39,6 +39,11 @@ static inline int mk_gcd(int a, int b) {
 int mk_fit_scales_strided(const float *value, long long row_stride, float *scales, float *zeros,
                           long long out_row_stride, int rows, int span, int group, int asym, float reciprocal,
                           float value_minimum, int scale_format, int store_zero, hipStream_t stream);
+// vector_feedback.hip: one tile of the error-feedback sweep over a vector grid.
+int mk_round_vector_tile(const float *original, const float *feedback, const float *coeff, const float *scales,
+                         const float *codebook, float *output, float *deviation_t, int32_t *encoded, int rows, int width,
+                         int region_start, int tile_start, int tile_width, int group, int groups_per_row, int dimension,
+                         int codebook_size, int lattice, hipStream_t stream);
 
 #ifdef __HIPCC__
 

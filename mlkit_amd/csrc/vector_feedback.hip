@@ -78,108 +78,101 @@ __device__ __forceinline__ float lane_value(float value, int lane) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, value), lane));
 }
 
-// This lane's four magnitude patterns (pattern lane + 64 j) and their squared norms.
+// This lane's four magnitude patterns (pattern lane + 64 j), their squared norms and, in bit 31, the parity of their sums.
 struct LanePatterns {
     float value[kPatternsPerLane][8];
     float norm[kPatternsPerLane];
+    uint32_t parity[kPatternsPerLane];
 };
 
 // `patterns`: the 256 x 8 table in LDS.
 __device__ __forceinline__ void load_patterns(LanePatterns &p, const float *patterns, int lane) {
 #pragma unroll
     for (int j = 0; j < kPatternsPerLane; ++j) {
-        float norm = 0.0f;
+        float norm = 0.0f, total = 0.0f;   // (a sum of half-integers: exact)
 #pragma unroll
         for (int d = 0; d < 8; ++d) {
             const float value = patterns[(lane + 64 * j) * 8 + d];
             p.value[j][d] = value;
+            total += value;
             norm = __fadd_rn(norm, __fmul_rn(value, value));
         }
         p.norm[j] = norm;
+        p.parity[j] = static_cast<uint32_t>(static_cast<int>(total)) << 31;
     }
 }
 
 // Code of the E8P point nearest to v, and the point itself (all lanes hold the same v and
-// receive the same answer).  Per coset every lane scores its four patterns -- the flip of the
+// receive the same answer).  For either coset every lane scores its four patterns -- the flip of the
 // cheapest coordinate priced in when the pattern's parity disagrees with the signs of v -- the
-// wavefront agrees on the winner, and only then are the winner's parity correction and its
-// first cheapest coordinate worked out, from its row of the table in LDS.
+// wavefront agrees on the winner of both (index 256 coset + pattern, so that the -1/4 coset stays on a tie),
+// and only then are the winner's parity correction and its first cheapest coordinate worked out, from its row of
+// the table in LDS.
 __device__ __forceinline__ int nearest_lattice_code(const float (&v)[8], const LanePatterns &p, const float *patterns,
                                                     int lane, float (&point)[8]) {
-    float best_cost = __builtin_inff();
-    int best_code = 0;
-    {   // Code 0 (pattern 0, no sign bits, the +1/4 coset): the answer when no cost compares below infinity (NaN).
-        float total = 0.0f;
-#pragma unroll
-        for (int d = 0; d < 8; ++d) total += patterns[d];
-        const int parity = static_cast<int>(total) & 1;
-#pragma unroll
-        for (int d = 0; d < 8; ++d) point[d] = __fadd_rn((d == 7 && parity) ? -patterns[d] : patterns[d], 0.25f);
-    }
+    float cost = __builtin_inff();
+    int winner = 0;
 #pragma unroll
     for (int coset = 0; coset < 2; ++coset) {
         const float shift = coset == 0 ? -0.25f : 0.25f;
-        float absolute[8];
-        int negatives = 0, sign_bits = 0;
-        float squares = 0.0f;
+        float absolute[8], squares = 0.0f;
+        uint32_t signs = 0;   // bit 31: the parity of the negative coordinates
 #pragma unroll
         for (int d = 0; d < 8; ++d) {
             const float centered = __fsub_rn(v[d], shift);
             absolute[d] = __builtin_fabsf(centered);
-            const int negative = centered < 0.0f ? 1 : 0;
-            negatives += negative;
-            if (d < 7) sign_bits |= negative << d;
+            signs ^= __float_as_uint(centered);   // (a difference of unequal numbers is not -0, of equal ones +0)
             squares = __fadd_rn(squares, __fmul_rn(centered, centered));
         }
-        const int sign_parity = negatives & 1;
-        float cost = __builtin_inff();
-        int pattern = 0;
 #pragma unroll
         for (int j = 0; j < kPatternsPerLane; ++j) {
-            float dots = 0.0f, cheapest = __builtin_inff(), total = 0.0f;
+            float dots = 0.0f, cheapest = __builtin_inff();
 #pragma unroll
             for (int d = 0; d < 8; ++d) {
                 const float product = __fmul_rn(absolute[d], p.value[j][d]);
                 dots = __fadd_rn(dots, product);
                 cheapest = __builtin_fminf(cheapest, product);
-                total += p.value[j][d];  // a sum of half-integers: exact, and constant per lane
             }
-            const int mismatch = (static_cast<int>(total) & 1) != sign_parity ? 1 : 0;
+            const bool mismatch = static_cast<int>(signs ^ p.parity[j]) < 0;
             float candidate = __fsub_rn(__fadd_rn(squares, p.norm[j]), __fmul_rn(2.0f, dots));
-            candidate = __fadd_rn(candidate, __fmul_rn(__fmul_rn(4.0f, cheapest), static_cast<float>(mismatch)));
-            if (candidate < cost) {  // ascending pattern index within the lane
+            candidate = __fadd_rn(candidate, mismatch ? __fmul_rn(4.0f, cheapest) : 0.0f);
+            if (candidate < cost) {  // ascending index within the lane
                 cost = candidate;
-                pattern = lane + 64 * j;
-            }
-        }
-        wave_best(cost, pattern, lane);
-        if (cost < best_cost) {  // uniform; the -1/4 coset stays on a tie
-            float row[8], total = 0.0f, cheapest = __builtin_inff();
-            int axis = 0;
-#pragma unroll
-            for (int d = 0; d < 8; ++d) {
-                row[d] = patterns[pattern * 8 + d];
-                total += row[d];
-                const float product = __fmul_rn(absolute[d], row[d]);
-                if (product < cheapest) {  // the first minimum
-                    cheapest = product;
-                    axis = d;
-                }
-            }
-            const int parity = static_cast<int>(total) & 1;
-            const int flipped = (parity != sign_parity && axis < 7) ? (1 << axis) : 0;
-            const int signs = sign_bits ^ flipped;
-            best_cost = cost;
-            best_code = pattern * 128 + signs + (coset == 0 ? 32768 : 0);
-            const int eighth = (__builtin_popcount(signs) + parity) & 1;
-#pragma unroll
-            for (int d = 0; d < 8; ++d) {
-                const int negative = d < 7 ? (signs >> d) & 1 : eighth;
-                point[d] = __fadd_rn(negative ? -row[d] : row[d], shift);
+                winner = 256 * coset + lane + 64 * j;
             }
         }
     }
-    return best_code;
+    wave_best(cost, winner, lane);
+    // no cost compares below infinity (NaN): pattern 0, no sign bits, the +1/4 coset
+    const bool found = cost < __builtin_inff();
+    const int pattern = found ? winner & 255 : 0;
+    const float shift = found && winner < 256 ? -0.25f : 0.25f;
+    float row[8], total = 0.0f, cheapest = __builtin_inff();
+    int axis = 0, negatives = 0, sign_bits = 0;
+#pragma unroll
+    for (int d = 0; d < 8; ++d) {
+        row[d] = patterns[pattern * 8 + d];
+        total += row[d];
+        const float centered = __fsub_rn(v[d], shift);
+        const int negative = centered < 0.0f ? 1 : 0;
+        negatives += negative;
+        if (d < 7) sign_bits |= negative << d;
+        const float product = __fmul_rn(__builtin_fabsf(centered), row[d]);
+        if (product < cheapest) {  // the first minimum
+            cheapest = product;
+            axis = d;
+        }
+    }
+    const int parity = static_cast<int>(total) & 1;
+    const int flipped = (parity != (negatives & 1) && axis < 7) ? (1 << axis) : 0;
+    const int signs = found ? sign_bits ^ flipped : 0;
+    const int eighth = (__builtin_popcount(signs) + parity) & 1;
+#pragma unroll
+    for (int d = 0; d < 8; ++d) {
+        const int negative = d < 7 ? (signs >> d) & 1 : eighth;
+        point[d] = __fadd_rn(negative ? -row[d] : row[d], shift);
+    }
+    return found ? pattern * 128 + signs + (winner < 256 ? 32768 : 0) : 0;
 }
 
 // Index of the nearest of `count` codewords of DIM floats (lowest index on ties).
@@ -250,6 +243,7 @@ __global__ void __launch_bounds__(256) vector_nearest_kernel(const NearestArgs a
 struct VectorTileArgs {
     const float *original, *feedback, *coeff, *scales, *codebook;
     float *output;
+    float *deviation_t;   // null, or [width, rows]: original - output, for the trailing updates
     int32_t *encoded;
     int rows, width, region_start, tile_start, tile_width, group, groups_per_row, codebook_size;
 };
@@ -319,11 +313,14 @@ __global__ void __launch_bounds__(64 * kWaveRows) round_vector_tile_kernel(const
             request_rows<DIM>(ahead, a.coeff, a.width, a.tile_start, a.tile_width, local + DIM, lane);
 
         const float scale = block_element<DIM>(scale_at, local, 0);  // a block lies inside one scale group
-        float weight[DIM], normalized[DIM];
+        float weight[DIM], normalized[DIM], quotients[kPerLane];
+        // every lane divides its own columns: four divisions for a block's two lanes, not one per column
+#pragma unroll
+        for (int s = 0; s < kPerLane; ++s) quotients[s] = __fdiv_rn(__fadd_rn(weights[s], corrections[s]), scale_at[s]);
 #pragma unroll
         for (int d = 0; d < DIM; ++d) {
             weight[d] = block_element<DIM>(weights, local, d);
-            normalized[d] = __fdiv_rn(__fadd_rn(weight[d], block_element<DIM>(corrections, local, d)), scale);
+            normalized[d] = block_element<DIM>(quotients, local, d);
         }
         int code;
         float word[DIM];
@@ -366,7 +363,10 @@ __global__ void __launch_bounds__(64 * kWaveRows) round_vector_tile_kernel(const
 #pragma unroll
     for (int s = 0; s < kPerLane; ++s) {
         const int column = kPerLane * lane + s;
-        if (column < a.tile_width) a.output[row_base + a.tile_start + column] = restored[s];
+        if (column < a.tile_width) {
+            a.output[row_base + a.tile_start + column] = restored[s];
+            if (a.deviation_t) a.deviation_t[static_cast<size_t>(a.tile_start + column) * a.rows + row] = __fsub_rn(weights[s], restored[s]);
+        }
     }
     const int blocks = a.tile_width / DIM;
     int32_t *codes = a.encoded + static_cast<size_t>(row) * (a.width / DIM) + a.tile_start / DIM;
@@ -412,12 +412,11 @@ extern "C" int mk_vector_nearest(const float *vectors, long long count, int dime
     return MK_OK;
 }
 
-extern "C" int mk_feedback_round_vector_tile(const float *original, const float *feedback, const float *coeff,
-                                             const float *scales, const float *codebook, float *output,
-                                             int32_t *encoded, int rows, int width, int region_start,
-                                             int tile_start, int tile_width, int group, int groups_per_row,
-                                             int dimension, int codebook_size, int lattice, void *stream_) {
-    hipStream_t stream = static_cast<hipStream_t>(stream_);
+// Shared with the sweep over all regions, whose scales lie `groups_per_row` apart and whose deviations are kept.
+int mk_round_vector_tile(const float *original, const float *feedback, const float *coeff, const float *scales,
+                         const float *codebook, float *output, float *deviation_t, int32_t *encoded, int rows, int width,
+                         int region_start, int tile_start, int tile_width, int group, int groups_per_row, int dimension,
+                         int codebook_size, int lattice, hipStream_t stream) {
     MK_REQUIRE(original && feedback && coeff && scales && codebook && output && encoded, MK_ERR_INVALID,
                "mk_feedback_round_vector_tile: null tensor pointer");
     MK_REQUIRE(rows >= 1 && width >= 1 && group >= 1 && codebook_size >= 1, MK_ERR_INVALID,
@@ -434,7 +433,7 @@ extern "C" int mk_feedback_round_vector_tile(const float *original, const float 
                MK_ERR_INVALID, "mk_feedback_round_vector_tile: rows, tiles and scale groups must hold whole codewords");
     MK_REQUIRE(!lattice || (dimension == 8 && codebook_size == 65536), MK_ERR_INVALID,
                "mk_feedback_round_vector_tile: the lattice search needs the 65536-point table of 8 coordinates");
-    VectorTileArgs a{original, feedback, coeff, scales, codebook, output, encoded, rows, width, region_start, tile_start,
+    VectorTileArgs a{original, feedback, coeff, scales, codebook, output, deviation_t, encoded, rows, width, region_start, tile_start,
                      tile_width, group, groups_per_row, codebook_size};
     const dim3 grid(mk_cdiv(rows, kWaveRows)), block(64 * kWaveRows);
     const bool staged_codebook = !lattice && fits_in_lds(codebook_size, dimension);
@@ -451,4 +450,14 @@ extern "C" int mk_feedback_round_vector_tile(const float *original, const float 
 #undef MK_TILE
     MK_LAUNCH_CHECK("mk_feedback_round_vector_tile");
     return MK_OK;
+}
+
+extern "C" int mk_feedback_round_vector_tile(const float *original, const float *feedback, const float *coeff,
+                                             const float *scales, const float *codebook, float *output,
+                                             int32_t *encoded, int rows, int width, int region_start,
+                                             int tile_start, int tile_width, int group, int groups_per_row,
+                                             int dimension, int codebook_size, int lattice, void *stream) {
+    return mk_round_vector_tile(original, feedback, coeff, scales, codebook, output, nullptr, encoded, rows, width, region_start,
+                                tile_start, tile_width, group, groups_per_row, dimension, codebook_size, lattice,
+                                static_cast<hipStream_t>(stream));
 }

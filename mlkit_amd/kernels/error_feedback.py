@@ -183,6 +183,51 @@ def sweep(
     return scales, zeros
 
 
+def vector_sweep(
+    original: Tensor,
+    feedback: Tensor,
+    output: Tensor,
+    encoded: Tensor,
+    coefficients: Tensor,
+    *,
+    codebook: Tensor,
+    dimension: int,
+    codebook_size: int,
+    lattice: bool,
+    group: int,
+    refit: int,
+    block: int,
+    reciprocal: float,
+    scale_format: str,
+    deferred_tiles: int = 4,
+) -> Tensor:
+    """The whole natural-order sweep over a vector grid in one call; returns the regions' scales side by side."""
+    device = native.require_device(original, feedback, output, encoded, coefficients, codebook)
+    rows, width = original.shape
+    _check("original", original)
+    _check("feedback", feedback, (rows, width))
+    _check("output", output, (rows, width))
+    _check("coefficients", coefficients, (width, width))
+    _check("codebook", codebook, (codebook_size + (256 if lattice else 0), dimension))
+    if encoded.dtype != torch.int32 or tuple(encoded.shape) != (rows, width // dimension) or not encoded.is_contiguous():
+        raise ValueError("encoded must be a contiguous int32 tensor with one code per block of columns")
+    region = min(refit, width)
+    groups = 0
+    for start in range(0, width, region):
+        span = min(region, width - start)
+        groups += -(-span // min(group, span))
+    scales = torch.empty((rows, groups), device=device, dtype=torch.float32)
+    workspace = torch.empty((rows, region), device=device, dtype=torch.float32) if region < width else None
+    # column-major deviations, read by the trailing updates that take whole tiles of 128 rows
+    deviations = torch.empty((width, rows), device=device, dtype=torch.float32) if rows % 128 == 0 and width % 4 == 0 else None
+    native.check(native.library().mk_feedback_vector_sweep(
+        original.data_ptr(), feedback.data_ptr(), output.data_ptr(), encoded.data_ptr(), coefficients.data_ptr(),
+        scales.data_ptr(), native.pointer(workspace), native.pointer(deviations), codebook.data_ptr(), dimension,
+        codebook_size, int(lattice), rows, width, group, refit, block, float(reciprocal),
+        native.SCALE_FORMAT_CODES[scale_format], deferred_tiles, native.current_stream(device)))
+    return scales
+
+
 MAXIMUM_VECTOR_TILE_WIDTH = 256
 
 

@@ -485,6 +485,46 @@ class ErrorFeedback(Quantizer):
         collected.count(inner.grid.bits * rows * width + side_bits)
         return True
 
+    def _whole_vector_sweep(self, original: Tensor, feedback: Tensor, output: Tensor, coefficients: Tensor,
+                            collected: "_Collected", ctx: Ctx) -> bool:
+        """The same for a vector grid with range-fitted scales whose dimension is the step."""
+        from mlkit_amd.quantization.scaled import SCALE_FORMAT_BITS, Scaled
+
+        inner = self.inner
+        rows, width = original.shape
+        refit = width if self.refit is None else self.refit
+        if not (type(inner) is Scaled and self.backend != "torch" and inner.scale == "absmax"
+                and isinstance(inner.scale_fmt, str) and inner.scale_fmt in SCALE_FORMAT_BITS
+                and inner.grid.values is not None and inner.grid.dim == self.step and self.step in FUSED_VECTOR_DIMENSIONS
+                and inner.grid.values.shape[0] <= FUSED_VECTOR_CODEBOOK_LIMIT
+                and self.block_size <= MAXIMUM_FUSED_VECTOR_TILE and (refit >= width or refit <= MAXIMUM_FUSED_TILE)):
+            return False
+        dimension, codebook_size = inner.grid.dim, inner.grid.values.shape[0]
+        group = width if inner.group is None else inner.group
+        regions = [min(refit, width - start) for start in range(0, width, refit)]
+        if any(min(group, span) % dimension for span in regions):
+            return False   # the fit of that region raises
+        from mlkit_amd.kernels import error_feedback as kernel
+        from mlkit_amd.quantization.lattice import device_table
+
+        lattice = inner.grid.name == "e8p"
+        if not lattice:
+            inner.count_codebook(ctx)
+        codebook = device_table(original.device) if lattice else inner.values_on(original.device)
+        encoded = torch.empty((rows, width // dimension), dtype=torch.int32, device=original.device)
+        scales = kernel.vector_sweep(
+            original, feedback, output, encoded, coefficients, codebook=codebook, dimension=dimension,
+            codebook_size=codebook_size, lattice=lattice, group=group, refit=refit, block=self.block_size,
+            reciprocal=inner._magnitude_reciprocal, scale_format=inner.scale_fmt, deferred_tiles=DEFERRED_TILES)
+        if not bool(torch.isfinite(scales).all()):
+            raise ValueError("scaled requires a finite floating-point weight matrix")
+        collected.codes = encoded
+        collected.shared = {"values": None if lattice else codebook, "group": min(group, regions[0]), "dim": dimension}
+        collected.metadata = {"code_bits": inner.grid.bits, "scale_fmt": inner.scale_fmt, "trainable": ["scales"]}
+        collected.scales = [scales]
+        collected.count(inner.grid.bits * rows * width / dimension + scales.numel() * SCALE_FORMAT_BITS[inner.scale_fmt])
+        return True
+
     @staticmethod
     def _pending_continuation(feedback: Tensor, coefficients: Tensor, start: int, stop: int) -> Tensor:
         """The adjustment the region's columns would take if nothing more were rounded:
@@ -551,7 +591,9 @@ class ErrorFeedback(Quantizer):
         # one pass when the super-block ends (or when a region needs those columns).  Every
         # column still receives the tiles' sums one by one in tile order, so nothing changes
         # in the result.
-        fused = self._whole_sweep(original, feedback, output, coefficients, collected) if on_device else False
+        fused = on_device and (self._whole_sweep(original, feedback, output, coefficients, collected)
+                               or (permutation is None
+                                   and self._whole_vector_sweep(original, feedback, output, coefficients, collected, ctx)))
         if fused:
             return collected.result(output, permutation, refit_width, ctx)
         deferred: list[tuple[int, int]] = []

@@ -210,6 +210,13 @@ class Scaled(Quantizer):
             best = torch.minimum(best, error)
         return chosen
 
+    def count_codebook(self, ctx: Ctx) -> None:
+        """The codebook of a vector grid is side information, paid for once."""
+        counted = ctx.cache.setdefault("_mlkit_vector_codebooks", set())
+        if id(self.grid) not in counted:
+            ctx.add_bits(self.grid.values.numel() * self.grid.values.element_size() * 8)
+            counted.add(id(self.grid))
+
     def fit(self, w: Tensor, ctx: Ctx) -> FittedRounder:
         if w.ndim != 2 or not w.is_floating_point():
             raise ValueError("scaled requires a finite floating-point weight matrix")
@@ -220,10 +227,7 @@ class Scaled(Quantizer):
             raise ValueError("group width must be divisible by the vector grid dimension")
         lattice = self.grid.name == "e8p"
         if dimension > 1 and codebook is not None and not lattice:
-            counted = ctx.cache.setdefault("_mlkit_vector_codebooks", set())
-            if id(self.grid) not in counted:  # the codebook is side information, paid for once
-                ctx.add_bits(codebook.numel() * codebook.element_size() * 8)
-                counted.add(id(self.grid))
+            self.count_codebook(ctx)
         weight = w.float()
         table = None if codebook is None or dimension != 1 else self.values_on(w.device)
         on_kernels = self._kernel_path(weight, table)

@@ -367,3 +367,36 @@ def test_vector_codecs_survive_a_checkpoint_and_stay_dense_under_optimize(tmp_pa
     calibrated_model = mk.quantize(build(), mk.ldlq(mk.scaled(mk.grid.e8p(), group=None), step=8),
                                    calib=[torch.randn(32, 64) for _ in range(4)])
     assert calibrated_model.quantized["0"].codec == "vector_feedback"
+
+
+@pytest.mark.parametrize("rows,width,refit,group,block", [
+    (128, 512, 128, 128, 128),     # whole tiles: the updates read the kept deviations
+    (256, 1040, 128, 64, 128),     # a ragged last region
+    (5, 384, None, 32, 128),       # one region
+    (130, 768, 256, 256, 64),      # rows that fill no tile, several tiles to a region
+    (384, 640, 96, 200, 32),       # a group wider than its region
+])
+@pytest.mark.parametrize("name", ["e8p", "vector"])
+def test_whole_vector_sweep_equals_the_region_by_region_loop(name, rows, width, refit, group, block, monkeypatch):
+    import mlkit_amd as mk
+
+    generator = torch.Generator().manual_seed(rows + width)
+    grid = mk.grid.e8p() if name == "e8p" else mk.grid.vector(torch.randn((64, 8), generator=generator))
+    weight = (torch.randn((rows, width), generator=generator) * 0.02).cuda()
+    inputs = torch.randn((2 * width, width), generator=generator).cuda()
+    hessian = inputs.T @ inputs / inputs.shape[0]
+    quantizer = mk.ldlq(mk.scaled(grid, group=group), step=8, refit=refit, block_size=block)
+    contexts = [Ctx("layer", H=hessian) for _ in range(2)]
+    whole = quantizer(weight, contexts[0])
+    monkeypatch.setattr(type(quantizer), "_whole_vector_sweep", lambda *arguments: False)
+    steps = quantizer(weight, contexts[1])
+    assert torch.equal(whole.codes, steps.codes)
+    assert torch.equal(whole.params["scales"], steps.params["scales"])
+    assert torch.equal(whole.w, steps.w)
+    assert (whole.bits, whole.metadata, contexts[0].additional_bits) == (steps.bits, steps.metadata, contexts[1].additional_bits)
+    assert {key: value for key, value in whole.params.items() if not torch.is_tensor(value)} == \
+        {key: value for key, value in steps.params.items() if not torch.is_tensor(value)}
+    weight[rows // 2, width - 1] = float("inf")
+    with pytest.raises(ValueError, match="finite"):
+        monkeypatch.undo()
+        quantizer(weight, Ctx("layer", H=hessian))
