@@ -289,6 +289,10 @@ int mk_basis_mix(const float *source, float *target, const float *basis, long lo
 int mk_cholesky_block(float *matrix, long long leading, int size, int first_column, int row_columns,
                       float *factor_out, int *status, void *stream);
 
+/* The same with another order of additions (two columns per step; slower). */
+int mk_cholesky_block_pairs(float *matrix, long long leading, int size, int first_column, int row_columns,
+                            float *factor_out, int *status, void *stream);
+
 /* The blocked transform of a width order * power (power a power of two) in one launch:
  * every row [order, power] of `source` is multiplied by signs_before (NULL or
  * [order * power] floats), each block goes through the Walsh-Hadamard stages of mk_fwht

@@ -16,6 +16,8 @@
 
 #include "mk_common.h"
 
+#include <type_traits>
+
 namespace {
 
 constexpr int kBlock = 128;
@@ -224,6 +226,206 @@ __global__ void __launch_bounds__(kThreads, 2) cholesky_block_kernel(const Block
     }
 }
 
+// ---- the same, two columns per step ------------------------------------------------------------
+//
+// The order of additions that the coefficients of vector grids are worked out in.  Kept for them although it takes twice as
+// long (48 against 25 us with 768 columns beside the block): a code that a last bit of a coefficient turns takes the rest of
+// its row along when it stands for eight weights, and conversions stay what they were, bit for bit.
+
+constexpr int kSub = kBlock / 16;
+constexpr int kRowFloats = 2 * kBlock;   // a published row: the block's columns, then the columns carried beside it
+
+// Columns 16 SIXTEEN ... 16 SIXTEEN + 15 of the factorisation below, two per step (their rows
+// sit in register row SIXTEEN of their owners).  False after a pivot that is not positive and
+// finite, which every thread sees in the same step.
+//
+// A step takes rows j and j + 1 as the updates of columns < j left them (`pivot_rows`), and
+// every thread derives what it needs of the two finished rows itself:
+//   U[j][k]     = A[j][k] / sqrt(A[j][j])
+//   U[j+1][k]   = (A[j+1][k] - U[j][j+1] U[j][k]) / sqrt(A[j+1][j+1] - U[j][j+1]^2)
+// and subtracts both outer products from its sub-block: one LDS round trip and one barrier
+// per two columns.
+//
+// ROW: the workgroup also carries 128 columns to the right of the block (`beside`), which take
+// the same row operations and so become U_jj^-T A_jr, the block row of the factor.
+template <int SIXTEEN, bool ROW, int BT>
+__device__ __forceinline__ bool sixteen_steps(const BlockArgs &a, float (&mine)[kSub][kSub], float (&beside)[kSub][BT],
+                                              float (&pivot_rows)[2][2][kRowFloats], int tx, int ty) {
+#pragma unroll 1
+    for (int lane = 0; lane < 16; lane += 2) {
+        const int j = 16 * SIXTEEN + lane;
+        const float *first = pivot_rows[(j >> 1) & 1][0], *second = pivot_rows[(j >> 1) & 1][1];
+        const float pivot = first[j];
+        if (!(pivot > 0.0f) || !(pivot - pivot == 0.0f)) {
+            if (threadIdx.x == 0) *a.status = a.first_column + j + 1;
+            return false;
+        }
+        // (one v_rsq_f32, accurate to an ulp; the IEEE square root and division were a fifth of a step's chain)
+        const float reciprocal = __builtin_amdgcn_rsqf(pivot);
+        const float link = first[j + 1] * reciprocal;                 // U[j][j+1]
+        const float next_pivot = second[j + 1] - link * link;
+        if (!(next_pivot > 0.0f) || !(next_pivot - next_pivot == 0.0f)) {
+            if (threadIdx.x == 0) *a.status = a.first_column + j + 2;
+            return false;
+        }
+        const float next_reciprocal = __builtin_amdgcn_rsqf(next_pivot);
+        // Register rows below SIXTEEN hold only rows <= j (finished); register columns below
+        // SIXTEEN only columns < j, which for the rows still changing lie below the diagonal
+        // (never read): neither takes part, so a step costs 2 (8 - SIXTEEN)^2 multiply-adds.
+        float rows_first[kSub], rows_second[kSub], columns_first[kSub], columns_second[kSub];
+#pragma unroll
+        for (int u = SIXTEEN; u < kSub; ++u) {
+            const int i = ty + 16 * u, k = tx + 16 * u;
+            const float upper = first[i] * reciprocal;                                   // U[j][i]
+            const float lower = (second[i] - link * upper) * next_reciprocal;            // U[j+1][i]
+            rows_first[u] = i > j + 1 ? upper : 0.0f;   // zero keeps rows <= j + 1 as they are
+            rows_second[u] = i > j + 1 ? lower : 0.0f;
+            columns_first[u] = first[k] * reciprocal;                                    // U[j][k]
+            columns_second[u] = (second[k] - link * columns_first[u]) * next_reciprocal; // U[j+1][k]
+        }
+        float beside_first[BT], beside_second[BT];
+        if constexpr (ROW) {
+#pragma unroll
+            for (int v = 0; v < BT; ++v) {
+                const int c = kBlock + tx + 16 * v;
+                beside_first[v] = first[c] * reciprocal;
+                beside_second[v] = (second[c] - link * beside_first[v]) * next_reciprocal;
+            }
+        }
+        // The two rows' owners keep the finished rows.
+        if (ty == lane) {
+#pragma unroll
+            for (int v = SIXTEEN; v < kSub; ++v) mine[SIXTEEN][v] = columns_first[v];
+            if constexpr (ROW) {
+#pragma unroll
+                for (int v = 0; v < BT; ++v) beside[SIXTEEN][v] = beside_first[v];
+            }
+        }
+        if (ty == lane + 1) {
+#pragma unroll
+            for (int v = SIXTEEN; v < kSub; ++v) mine[SIXTEEN][v] = columns_second[v];
+            if constexpr (ROW) {
+#pragma unroll
+                for (int v = 0; v < BT; ++v) beside[SIXTEEN][v] = beside_second[v];
+            }
+        }
+#pragma unroll
+        for (int u = SIXTEEN; u < kSub; ++u) {
+#pragma unroll
+            for (int v = SIXTEEN; v < kSub; ++v)
+                mine[u][v] -= rows_first[u] * columns_first[v] + rows_second[u] * columns_second[v];
+            if constexpr (ROW) {
+#pragma unroll
+                for (int v = 0; v < BT; ++v)
+                    beside[u][v] -= rows_first[u] * beside_first[v] + rows_second[u] * beside_second[v];
+            }
+        }
+        // Rows j + 2 and j + 3 have all their updates now: their owners publish them.
+        float (*next)[kRowFloats] = pivot_rows[((j >> 1) + 1) & 1];
+        if (lane < 14) {
+            if (ty == lane + 2 || ty == lane + 3) {
+#pragma unroll
+                for (int v = SIXTEEN; v < kSub; ++v) next[ty - lane - 2][tx + 16 * v] = mine[SIXTEEN][v];   // columns < j are not read
+                if constexpr (ROW) {
+#pragma unroll
+                    for (int v = 0; v < BT; ++v) next[ty - lane - 2][kBlock + tx + 16 * v] = beside[SIXTEEN][v];
+                }
+            }
+        } else if constexpr (SIXTEEN + 1 < kSub) {
+            if (ty < 2) {
+#pragma unroll
+                for (int v = SIXTEEN + 1; v < kSub; ++v) next[ty][tx + 16 * v] = mine[SIXTEEN + 1][v];
+                if constexpr (ROW) {
+#pragma unroll
+                    for (int v = 0; v < BT; ++v) next[ty][kBlock + tx + 16 * v] = beside[SIXTEEN + 1][v];
+                }
+            }
+        }
+        __syncthreads();
+    }
+    return true;
+}
+
+// In: the upper triangle of a symmetric positive definite block.  Out: U with block = U^T U
+// in the upper triangle, zeros below it.  A pivot that is not positive (or not finite)
+// records its column and leaves the block unspecified.
+//
+// Right-looking, two columns per step.  The block lives in registers for the whole
+// factorisation: thread (ty, tx) of a 16 x 16 grid owns entries (ty + 16 u, tx + 16 v),
+// an 8 x 8 sub-block.  Per step only the two pivot rows travel: the threads that own them
+// put them (as updated so far) into one of two LDS buffers, one barrier later every thread
+// reads the entries it needs, finishes the two rows for itself and subtracts their outer
+// products from its sub-block.  Rows up to the pivot rows are masked out of the update by
+// zero factors, so finished rows keep their values.
+// BT: sixteenths of 128 columns a workgroup carries beside the block (8: 128 columns, 4: 64).
+template <bool ROW, int BT>
+__global__ void __launch_bounds__(kThreads) cholesky_pairs_kernel(const BlockArgs a) {
+    __shared__ float pivot_rows[2][2][kRowFloats];   // [buffer][row j, row j + 1][column]
+    __shared__ int failed;
+    const int n = a.size;
+    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
+    if (threadIdx.x == 0) failed = *a.status != 0;   // an earlier block already failed: do nothing
+    float mine[kSub][kSub], beside[kSub][BT];
+    constexpr int kBeside = 16 * BT;
+    // ROW: workgroup b carries columns kBeside b ... kBeside (b + 1) - 1 of the block row; every workgroup
+    // factors the block itself (from the matrix, which nobody overwrites: the factor goes to
+    // `factor_out`), and the first one stores it.
+    const int beside_first_column = n + kBeside * blockIdx.x;
+#pragma unroll
+    for (int u = 0; u < kSub; ++u)
+#pragma unroll
+        for (int v = 0; v < kSub; ++v) {
+            const int row = ty + 16 * u, column = tx + 16 * v;
+            const bool inside = row < n && column < n && column >= row;
+            const float loaded = a.matrix[(inside ? row : 0) * a.leading + (inside ? column : 0)];
+            // Outside the block: an identity diagonal keeps every pivot of the padding at one.
+            mine[u][v] = inside ? loaded : (row == column ? 1.0f : 0.0f);
+            if (v < BT) {
+                beside[u][v] = 0.0f;
+                if constexpr (ROW) {
+                    const bool present = row < n && kBeside * static_cast<int>(blockIdx.x) + column < a.row_columns;
+                    const float carried = a.matrix[(present ? row : 0) * a.leading + (present ? beside_first_column + column : 0)];
+                    beside[u][v] = present ? carried : 0.0f;
+                }
+            }
+        }
+    if (ty < 2) {
+#pragma unroll
+        for (int v = 0; v < kSub; ++v) {
+            pivot_rows[0][ty][tx + 16 * v] = mine[0][v];
+            if constexpr (ROW) {
+                if (v < BT) pivot_rows[0][ty][kBlock + tx + 16 * v] = beside[0][v];
+            }
+        }
+    }
+    __syncthreads();
+    if (failed) return;
+
+    // All 128 columns run (the padding is an identity): no data-dependent exit other than a bad pivot.
+    bool good = sixteen_steps<0, ROW, BT>(a, mine, beside, pivot_rows, tx, ty);
+    good = good && sixteen_steps<1, ROW, BT>(a, mine, beside, pivot_rows, tx, ty);
+    good = good && sixteen_steps<2, ROW, BT>(a, mine, beside, pivot_rows, tx, ty);
+    good = good && sixteen_steps<3, ROW, BT>(a, mine, beside, pivot_rows, tx, ty);
+    good = good && sixteen_steps<4, ROW, BT>(a, mine, beside, pivot_rows, tx, ty);
+    good = good && sixteen_steps<5, ROW, BT>(a, mine, beside, pivot_rows, tx, ty);
+    good = good && sixteen_steps<6, ROW, BT>(a, mine, beside, pivot_rows, tx, ty);
+    good = good && sixteen_steps<7, ROW, BT>(a, mine, beside, pivot_rows, tx, ty);
+    if (!good) return;
+    float *factor = ROW ? a.factor_out : a.matrix;
+    const long long factor_leading = ROW ? kBlock : a.leading;
+#pragma unroll
+    for (int u = 0; u < kSub; ++u)
+#pragma unroll
+        for (int v = 0; v < kSub; ++v) {
+            const int row = ty + 16 * u, column = tx + 16 * v;
+            if (blockIdx.x == 0 && row < n && column < n) factor[row * factor_leading + column] = column >= row ? mine[u][v] : 0.0f;
+            if constexpr (ROW) {
+                if (v < BT && row < n && kBeside * static_cast<int>(blockIdx.x) + column < a.row_columns)
+                    a.matrix[row * a.leading + beside_first_column + column] = beside[u][v];
+            }
+        }
+}
+
 }  // namespace
 
 // ---- the matrix that goes into the factorisation, and the coefficients that come out ---------
@@ -309,9 +511,10 @@ extern "C" int mk_unit_upper_from_factor(const float *factor, float *out, int wi
     return MK_OK;
 }
 
-extern "C" int mk_cholesky_block(float *matrix, long long leading, int size, int first_column, int row_columns,
-                                 float *factor_out, int *status, void *stream_) {
-    hipStream_t stream = static_cast<hipStream_t>(stream_);
+namespace {
+
+int check_block(const float *matrix, long long leading, int size, int first_column, int row_columns, const float *factor_out,
+                const int *status) {
     MK_REQUIRE(matrix && status, MK_ERR_INVALID, "mk_cholesky_block: null pointer");
     MK_REQUIRE(size >= 1 && size <= kBlock, MK_ERR_UNSUPPORTED, "mk_cholesky_block: blocks of 1 to %d rows (got %d)", kBlock, size);
     MK_REQUIRE(row_columns >= 0 && leading >= static_cast<long long>(size) + row_columns && first_column >= 0, MK_ERR_INVALID,
@@ -319,11 +522,37 @@ extern "C" int mk_cholesky_block(float *matrix, long long leading, int size, int
     MK_REQUIRE(leading <= (1ll << 32) / kBlock, MK_ERR_INVALID, "mk_cholesky_block: a block's rows must lie within 2^32 floats");
     MK_REQUIRE(row_columns == 0 || factor_out, MK_ERR_INVALID,
                "mk_cholesky_block: a block row needs a separate place for the factor");
+    return MK_OK;
+}
+
+}  // namespace
+
+extern "C" int mk_cholesky_block(float *matrix, long long leading, int size, int first_column, int row_columns,
+                                 float *factor_out, int *status, void *stream_) {
+    hipStream_t stream = static_cast<hipStream_t>(stream_);
+    if (int refused = check_block(matrix, leading, size, first_column, row_columns, factor_out, status)) return refused;
     BlockArgs a{matrix, leading, size, first_column, status, row_columns, factor_out};
     if (row_columns > 0)
         hipLaunchKernelGGL((cholesky_block_kernel<true>), dim3(mk_cdiv(row_columns, kCarried)), dim3(kThreads), 0, stream, a);
     else
         hipLaunchKernelGGL((cholesky_block_kernel<false>), dim3(1), dim3(kThreads), 0, stream, a);
     MK_LAUNCH_CHECK("mk_cholesky_block");
+    return MK_OK;
+}
+
+extern "C" int mk_cholesky_block_pairs(float *matrix, long long leading, int size, int first_column, int row_columns,
+                                 float *factor_out, int *status, void *stream_) {
+    hipStream_t stream = static_cast<hipStream_t>(stream_);
+    if (int refused = check_block(matrix, leading, size, first_column, row_columns, factor_out, status)) return refused;
+    BlockArgs a{matrix, leading, size, first_column, status, row_columns, factor_out};
+    // 64 columns per workgroup while that still fits one workgroup per CU (a step then costs a
+    // third less arithmetic); 128 beyond.
+    if (row_columns > 256 * 64)
+        hipLaunchKernelGGL((cholesky_pairs_kernel<true, 8>), dim3(mk_cdiv(row_columns, 128)), dim3(kThreads), 0, stream, a);
+    else if (row_columns > 0)
+        hipLaunchKernelGGL((cholesky_pairs_kernel<true, 4>), dim3(mk_cdiv(row_columns, 64)), dim3(kThreads), 0, stream, a);
+    else
+        hipLaunchKernelGGL((cholesky_pairs_kernel<false, 4>), dim3(1), dim3(kThreads), 0, stream, a);
+    MK_LAUNCH_CHECK("mk_cholesky_block_pairs");
     return MK_OK;
 }

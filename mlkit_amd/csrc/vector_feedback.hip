@@ -14,8 +14,8 @@
 // lane l holding columns l, l + 64, ...: weights, corrections, scales on the way in,
 // reconstructions and codes on the way out (read and written with coalesced accesses before
 // and after the block loop).  A block's values are read out of them with wavefront-uniform
-// lane reads.  Inside the loop the only memory traffic is the coefficient rows of the NEXT
-// block, requested before the search of the current one so that their latency hides behind it.
+// lane reads.  Inside the loop the only memory traffic is the block's coefficient rows,
+// requested before its search so that their latency hides behind it.
 // An E8P point is rebuilt from its pattern, sign bits and coset instead of being fetched from
 // the 2 MiB table.
 //
@@ -246,6 +246,7 @@ struct VectorTileArgs {
     float *deviation_t;   // null, or [width, rows]: original - output, for the trailing updates
     int32_t *encoded;
     int rows, width, region_start, tile_start, tile_width, group, groups_per_row, codebook_size;
+    int whole_quads;   // a lane's four coefficients of a row are one aligned load
 };
 
 // A tile of up to 256 columns in a wavefront's registers: lane l holds columns 4 l .. 4 l + 3 in
@@ -264,18 +265,25 @@ __device__ __forceinline__ float block_element(const float (&values)[kPerLane], 
     }
 }
 
-// Coefficient rows of the block at `local` for the lane's columns behind that block (zero elsewhere).
+// Coefficient rows of the block at `local` for the lane's columns.  Columns that are not behind the block (or past the
+// tile) receive numbers too: nothing reads the corrections of a rounded column again.
 template <int DIM>
-__device__ __forceinline__ void request_rows(float (&rows)[DIM][kPerLane], const float *coeff, int width,
-                                             int tile_start, int tile_width, int local, int lane) {
+__device__ __forceinline__ void request_rows(float (&rows)[DIM][kPerLane], const VectorTileArgs &a, int local, int lane) {
+    const float *first = a.coeff + static_cast<size_t>(a.tile_start + local) * a.width + a.tile_start;
+    if (a.whole_quads) {   // uniform
+        const int column = min(kPerLane * lane, a.tile_width - kPerLane);
 #pragma unroll
-    for (int d = 0; d < DIM; ++d)
-#pragma unroll
-        for (int s = 0; s < kPerLane; ++s) {
-            const int column = kPerLane * lane + s;
-            const bool later = column >= local + DIM && column < tile_width;
-            rows[d][s] = later ? coeff[static_cast<size_t>(tile_start + local + d) * width + tile_start + column] : 0.0f;
+        for (int d = 0; d < DIM; ++d) {
+            const float4 four = *reinterpret_cast<const float4 *>(first + static_cast<size_t>(d) * a.width + column);
+            rows[d][0] = four.x; rows[d][1] = four.y; rows[d][2] = four.z; rows[d][3] = four.w;
         }
+    } else {
+#pragma unroll
+        for (int d = 0; d < DIM; ++d)
+#pragma unroll
+            for (int s = 0; s < kPerLane; ++s)
+                rows[d][s] = first[static_cast<size_t>(d) * a.width + min(kPerLane * lane + s, a.tile_width - 1)];
+    }
 }
 
 template <int DIM, bool LATTICE, bool STAGED>
@@ -301,16 +309,10 @@ __global__ void __launch_bounds__(64 * kWaveRows) round_vector_tile_kernel(const
         scale_at[s] = a.scales[static_cast<size_t>(row) * a.groups_per_row + group];
         restored[s] = 0.0f;
     }
-    float ahead[DIM][kPerLane];
-    request_rows<DIM>(ahead, a.coeff, a.width, a.tile_start, a.tile_width, 0, lane);
     for (int local = 0; local < a.tile_width; local += DIM) {
         float along[DIM][kPerLane];
-#pragma unroll
-        for (int d = 0; d < DIM; ++d)
-#pragma unroll
-            for (int s = 0; s < kPerLane; ++s) along[d][s] = ahead[d][s];
-        if (local + DIM < a.tile_width)  // uniform
-            request_rows<DIM>(ahead, a.coeff, a.width, a.tile_start, a.tile_width, local + DIM, lane);
+        request_rows<DIM>(along, a, local, lane);   // on their way during the search
+        __builtin_amdgcn_sched_barrier(0);
 
         const float scale = block_element<DIM>(scale_at, local, 0);  // a block lies inside one scale group
         float weight[DIM], normalized[DIM], quotients[kPerLane];
@@ -357,7 +359,7 @@ __global__ void __launch_bounds__(64 * kWaveRows) round_vector_tile_kernel(const
             float pushed = __fmul_rn(deviation[0], along[0][s]);
 #pragma unroll
             for (int d = 1; d < DIM; ++d) pushed = __fadd_rn(pushed, __fmul_rn(deviation[d], along[d][s]));
-            corrections[s] = __fadd_rn(corrections[s], pushed);  // columns that are not later hold zeros in `along`
+            corrections[s] = __fadd_rn(corrections[s], pushed);
         }
     }
 #pragma unroll
@@ -434,7 +436,8 @@ int mk_round_vector_tile(const float *original, const float *feedback, const flo
     MK_REQUIRE(!lattice || (dimension == 8 && codebook_size == 65536), MK_ERR_INVALID,
                "mk_feedback_round_vector_tile: the lattice search needs the 65536-point table of 8 coordinates");
     VectorTileArgs a{original, feedback, coeff, scales, codebook, output, deviation_t, encoded, rows, width, region_start, tile_start,
-                     tile_width, group, groups_per_row, codebook_size};
+                     tile_width, group, groups_per_row, codebook_size,
+                     width % 4 == 0 && tile_start % 4 == 0 && tile_width % 4 == 0 && (reinterpret_cast<uintptr_t>(coeff) & 15u) == 0};
     const dim3 grid(mk_cdiv(rows, kWaveRows)), block(64 * kWaveRows);
     const bool staged_codebook = !lattice && fits_in_lds(codebook_size, dimension);
     const size_t lds = lattice ? kPatternFloats * sizeof(float)

@@ -39,13 +39,16 @@ DEFERRED_TILES = 4  # tiles whose far-column updates are applied in one pass on 
 # coefficients of 128 / 256 / 512 / 896 columns 0.12 / 0.15 / 0.25 / 0.42 ms against 0.26 / 0.65 / 1.34 / 2.47 with the library,
 # relative error against 64 bits 2.2e-7 / 2.9e-7 / 3.7e-7 / 3.7e-7 against 2.3e-7 / 3.5e-7 / 4.4e-7 / 4.2e-7.
 BLOCKED_FACTORIZATION_WIDTH = 128
+# Steps of several columns (vector grids) keep the arithmetic their conversions have had -- the library below this width and the
+# two-column block kernel from it on: a code for eight weights that the last bit of a coefficient turns takes its row along.
+STEPPED_FACTORIZATION_WIDTH = 1024
 FACTORIZATION_BLOCK = 128           # one workgroup factors a diagonal block of this size
 FACTORIZATION_PANEL = 1024          # rank of the trailing updates of the whole matrix
 TRAILING_BAND = 1024                # rows per product of a trailing update (only the upper triangle is needed)
 LOOK_AHEAD_WIDTH = 8192             # from here on the far part of a trailing update runs on a second stream
 
 
-def _factor_in_place(matrix: Tensor, status: Tensor, factored: Tensor) -> None:
+def _factor_in_place(matrix: Tensor, status: Tensor, factored: Tensor, pairs: bool = False) -> None:
     """``matrix = U^T U`` for a symmetric positive definite FP32 matrix on a HIP device, factored
     in place (``status``: an int32 device scalar holding zero; ``factored``: scratch for the
     diagonal blocks, ``[ceil(width / 128), 128, 128]``).
@@ -69,12 +72,14 @@ def _factor_in_place(matrix: Tensor, status: Tensor, factored: Tensor) -> None:
 
     ``status`` stays zero, or becomes one plus the first column whose pivot is not positive (as
     ``torch.linalg.cholesky_ex`` reports it).  Nothing here allocates device memory or reads
-    anything back, so the whole sequence can be captured in a HIP graph."""
+    anything back, so the whole sequence can be captured in a HIP graph.
+
+    ``pairs``: blocks take two columns per step (``mk_cholesky_block_pairs``)."""
     from mlkit_amd import native
 
     width = matrix.shape[0]
     device = matrix.device
-    library = native.library()
+    factor_block = native.library().mk_cholesky_block_pairs if pairs else native.library().mk_cholesky_block
     main = torch.cuda.current_stream(device)
     look_ahead = width >= LOOK_AHEAD_WIDTH   # narrower: the event traffic costs more than it hides
     side = torch.cuda.Stream(device) if look_ahead else None    # far rows of a panel's update
@@ -110,8 +115,8 @@ def _factor_in_place(matrix: Tensor, status: Tensor, factored: Tensor) -> None:
             # `factored`, since every workgroup of that launch reads the block itself
             beside = width - stop
             slot = factored[start // FACTORIZATION_BLOCK]
-            native.check(library.mk_cholesky_block(matrix[start, start:].data_ptr(), width, stop - start, start, beside,
-                                                   slot.data_ptr() if beside else None, status.data_ptr(), raw_stream))
+            native.check(factor_block(matrix[start, start:].data_ptr(), width, stop - start, start, beside,
+                                      slot.data_ptr() if beside else None, status.data_ptr(), raw_stream))
         # the diagonal block's lower triangle holds leftovers of the products above
         matrix[panel_start:panel_stop, panel_start:panel_stop].triu_()
         if panel_stop == width:
@@ -152,7 +157,8 @@ class _FactorGraph:
     launches cost more to issue from Python than to run, and they are the same for every matrix
     of that width.  The graph owns the buffer it factors in."""
 
-    def __init__(self, width: int, device: torch.device) -> None:
+    def __init__(self, width: int, device: torch.device, pairs: bool) -> None:
+        self.pairs = pairs
         self.matrix = torch.empty((width, width), dtype=torch.float32, device=device)
         self.status = torch.zeros((), dtype=torch.int32, device=device)
         self.factored = _factor_scratch(width, device)
@@ -179,7 +185,7 @@ class _FactorGraph:
         graph.capture_begin()
         try:
             self.status.zero_()   # a fill kernel
-            _factor_in_place(self.matrix, self.status, self.factored)
+            _factor_in_place(self.matrix, self.status, self.factored, self.pairs)
         finally:
             graph.capture_end()
         return graph
@@ -192,7 +198,7 @@ class _FactorGraph:
 
 FACTOR_GRAPHS = True        # capture the factorisation of a width the second time it is asked for
 FACTOR_GRAPH_LIMIT = 2      # graphs (and their width x width buffers) kept per process
-_factor_graphs: dict[tuple[int, int], "_FactorGraph | None"] = {}
+_factor_graphs: dict[tuple, "_FactorGraph | None"] = {}   # by device and width
 
 
 def clear_factor_graphs() -> None:
@@ -202,25 +208,25 @@ def clear_factor_graphs() -> None:
     _factor_graphs.clear()
 
 
-def _blocked_upper_factor(fill: Callable[[Tensor], None], width: int, device: torch.device) -> tuple[Tensor, Tensor]:
+def _blocked_upper_factor(fill: Callable[[Tensor], None], width: int, device: torch.device, pairs: bool) -> tuple[Tensor, Tensor]:
     """``(U, status)`` with ``U^T U`` = the matrix that ``fill(target)`` writes into a
     ``[width, width]`` FP32 tensor.  The first matrix of a width is factored launch by launch
     (which also warms every kernel up); from the second on the captured graph of that width
     runs.  The result may live in the graph's own buffer: it is valid until the next call."""
-    key = (torch.cuda.current_device() if device.index is None else device.index, width)
+    key = (torch.cuda.current_device() if device.index is None else device.index, width) + (("pairs",) if pairs else ())
     if FACTOR_GRAPHS and key in _factor_graphs and not torch.cuda.is_current_stream_capturing():
         graph = _factor_graphs[key]
         if graph is None:
             while sum(entry is not None for entry in _factor_graphs.values()) >= FACTOR_GRAPH_LIMIT:
                 oldest = next(k for k, entry in _factor_graphs.items() if entry is not None)
                 del _factor_graphs[oldest]
-            graph = _factor_graphs[key] = _FactorGraph(width, device)
+            graph = _factor_graphs[key] = _FactorGraph(width, device, pairs)
         return graph(fill)
     _factor_graphs.setdefault(key, None)   # seen once
     matrix = torch.empty((width, width), dtype=torch.float32, device=device)
     fill(matrix)
     status = torch.zeros((), dtype=torch.int32, device=device)
-    _factor_in_place(matrix, status, _factor_scratch(width, device))
+    _factor_in_place(matrix, status, _factor_scratch(width, device), pairs)
     return matrix, status
 
 
@@ -236,7 +242,7 @@ def feedback_coefficients(hessian: Tensor, step: int, *, damp: float = 0.01,
     reversed back, is the upper factor ``R``.
     """
     width = hessian.shape[0]
-    if width >= BLOCKED_FACTORIZATION_WIDTH and hessian.is_cuda and hessian.dtype == torch.float32:
+    if width >= (BLOCKED_FACTORIZATION_WIDTH if step == 1 else STEPPED_FACTORIZATION_WIDTH) and hessian.is_cuda and hessian.dtype == torch.float32:
         return _coefficients_on_kernels(hessian, step, damp, permutation)
     if permutation is None:
         flipped = hessian.flip(0, 1)
@@ -256,7 +262,7 @@ def feedback_coefficients(hessian: Tensor, step: int, *, damp: float = 0.01,
 
 
 def _coefficients_on_kernels(hessian: Tensor, step: int, damp: float, permutation: Tensor | None) -> tuple[Tensor, int]:
-    """The same on a HIP device for matrices of 128 columns and more: one pass writes the
+    """The same on a HIP device for matrices of 128 columns and more (1024 for steps of several): one pass writes the
     reversed, damped matrix where it is factored (``mk_hessian_reversed``), the blocked
     factorisation runs, and for ``step == 1`` one pass turns the factor into the coefficients
     (``mk_unit_upper_from_factor``)."""
@@ -274,7 +280,7 @@ def _coefficients_on_kernels(hessian: Tensor, step: int, damp: float, permutatio
         native.check(library.mk_hessian_reversed(source.data_ptr(), target.data_ptr(), width, native.pointer(order),
                                                  addend.data_ptr(), native.current_stream(device)))
 
-    factor, status = _blocked_upper_factor(fill, width, device)
+    factor, status = _blocked_upper_factor(fill, width, device, pairs=step > 1)
     if step == 1 and int(status.item()) == 0:
         coefficients = torch.empty_like(factor)
         native.check(library.mk_unit_upper_from_factor(factor.data_ptr(), coefficients.data_ptr(), width,
