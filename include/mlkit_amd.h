@@ -74,6 +74,22 @@ int mk_packed_matmul(const void *x, int x_dtype, const uint8_t *packed, const vo
                      int input_width, int group, int bits, int uniform, float grid_min,
                      float grid_step, void *stream);
 
+/* What a packed layer's calls have in common; the fields are the arguments of mk_packed_matvec of the same names.  The
+ * caller keeps it (and the memory it points to) for as long as it calls; nothing of it is retained. */
+typedef struct mk_packed_layer {
+    const uint8_t *packed;
+    const void *scales;
+    const float *values;
+    const void *zeros;
+    const void *bias;
+    int scale_dtype, n_values, bias_dtype, output_width, input_width, group, bits, uniform;
+    float grid_min, grid_step;
+} mk_packed_layer;
+
+/* mk_packed_matvec and mk_packed_matmul with those arguments in one place (a call from Python costs by the argument). */
+int mk_packed_layer_matvec(const mk_packed_layer *layer, const void *x, int x_dtype, void *y, int samples, void *stream);
+int mk_packed_layer_matmul(const mk_packed_layer *layer, const void *x, int x_dtype, void *y, int samples, void *stream);
+
 /* mk_packed_matvec for `count` (1..8) weight matrices of one input width and one codec in a
  * single call: y[i] = x[i] @ dequant(packed[i])^T (+ bias[i]) for every i, each with
  * output_widths[i] rows.  The activation pointers may all be the same (sibling projections

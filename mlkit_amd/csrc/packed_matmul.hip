@@ -109,3 +109,10 @@ extern "C" int mk_packed_matmul(const void *x, int x_dtype, const uint8_t *packe
     MK_LAUNCH_CHECK("mk_packed_matmul");
     return MK_OK;
 }
+
+extern "C" int mk_packed_layer_matmul(const mk_packed_layer *layer, const void *x, int x_dtype, void *y, int samples, void *stream) {
+    MK_REQUIRE(layer, MK_ERR_INVALID, "mk_packed_layer_matmul: null layer");
+    const mk_packed_layer &l = *layer;
+    return mk_packed_matmul(x, x_dtype, l.packed, l.scales, l.scale_dtype, l.values, l.n_values, l.zeros, l.bias, l.bias_dtype, y, samples,
+                            l.output_width, l.input_width, l.group, l.bits, l.uniform, l.grid_min, l.grid_step, stream);
+}

@@ -391,3 +391,10 @@ extern "C" int mk_packed_matvec_group(const void *const *x, int x_dtype, int cou
     }
     return MK_OK;
 }
+
+extern "C" int mk_packed_layer_matvec(const mk_packed_layer *layer, const void *x, int x_dtype, void *y, int samples, void *stream) {
+    MK_REQUIRE(layer, MK_ERR_INVALID, "mk_packed_layer_matvec: null layer");
+    const mk_packed_layer &l = *layer;
+    return mk_packed_matvec(x, x_dtype, l.packed, l.scales, l.scale_dtype, l.values, l.n_values, l.zeros, l.bias, l.bias_dtype, y, samples,
+                            l.output_width, l.input_width, l.group, l.bits, l.uniform, l.grid_min, l.grid_step, stream);
+}

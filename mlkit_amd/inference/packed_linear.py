@@ -19,6 +19,7 @@ How a call is served here:
 """
 
 import copy
+import ctypes
 from collections.abc import Callable
 from dataclasses import dataclass
 
@@ -254,6 +255,11 @@ class PackedLinear(nn.Module):
             return functional.linear(inputs, self.weight.to(inputs.dtype), self.bias)
         if inputs.requires_grad and torch.is_grad_enabled():
             raise RuntimeError("packed CUDA inference does not support autograd")
+        if not compiling and (rotate_here or self._siblings is None):
+            # the plain launch: no views around it, each costs as much as the output's allocation
+            output = inputs.new_empty(inputs.shape[:-1] + (self.out_features,))
+            self._matvec(inputs if inputs.is_contiguous() else inputs.contiguous(), output, rows, rotate_here)
+            return output
         flat = inputs.reshape(rows, self.in_features)
         if not flat.is_contiguous():
             flat = flat.contiguous()
@@ -261,11 +267,8 @@ class PackedLinear(nn.Module):
             output = packed_matvec_op(flat, self.packed, self.scales, self.values, self.zeros, self.bias,
                                       self.out_features, self.group, self.code_bits, self.uniform_grid,
                                       self.grid_minimum, self.grid_step)
-        elif self._siblings is not None and not rotate_here:
-            output = self._siblings.output_for(self, inputs, flat)
         else:
-            output = inputs.new_empty((rows, self.out_features))
-            self._matvec(flat, output, rows, rotate_here)
+            output = self._siblings.output_for(self, inputs, flat)
         return output.view(inputs.shape[:-1] + (self.out_features,))
 
     # -- grouped launches with sibling layers ------------------------------------------------
@@ -296,12 +299,14 @@ class PackedLinear(nn.Module):
                scales.dtype, None if bias is None else bias.dtype)
         launch = self._launch
         if launch is None or launch[0] != key:
+            scale_code, bias_code = native.dtype_code(scales), 0 if bias is None else native.dtype_code(bias)
+            constants = (self.out_features, self.in_features, self.group, self.code_bits, int(self.uniform_grid),
+                         self.grid_minimum, self.grid_step)
+            layer = native.PackedLayer(*key[:5], scale_code, values.numel(), bias_code, *constants)
             launch = self._launch = (
                 key,
-                (key[0], key[1], native.dtype_code(scales), key[2], values.numel(), native.pointer(zeros),
-                 native.pointer(bias), 0 if bias is None else native.dtype_code(bias)),
-                (self.out_features, self.in_features, self.group, self.code_bits, int(self.uniform_grid),
-                 self.grid_minimum, self.grid_step),
+                (key[0], key[1], scale_code, key[2], values.numel(), native.pointer(zeros), native.pointer(bias), bias_code),
+                constants, ctypes.addressof(layer), layer,
             )
         return launch
 
@@ -341,22 +346,21 @@ class PackedLinear(nn.Module):
     def _product(self, inputs: Tensor, rows: int) -> Tensor | None:
         """More rows than a matvec on the codes; None when the library refuses the call (a buffer that was moved
         to an unaligned address, say): the caller decodes the weight then."""
-        flat = inputs.reshape(rows, self.in_features)
-        if not flat.is_contiguous():
-            flat = flat.contiguous()
-        output = inputs.new_empty((rows, self.out_features))
-        _, tensors, constants = self._bound_arguments()
-        status = native.library().mk_packed_matmul(flat.data_ptr(), native.DTYPE_CODES[flat.dtype], *tensors, output.data_ptr(),
-                                                   rows, *constants, native.current_stream(flat.device))
+        if not inputs.is_contiguous():
+            inputs = inputs.contiguous()
+        output = inputs.new_empty(inputs.shape[:-1] + (self.out_features,))
+        status = native.library().mk_packed_layer_matmul(
+            self._bound_arguments()[3], inputs.data_ptr(), native.DTYPE_CODES[inputs.dtype], output.data_ptr(), rows,
+            native.current_stream(inputs.device))
         if status == native.MK_ERR_UNSUPPORTED:
             return None
         if status:
             native.check(status)
-        return output.view(inputs.shape[:-1] + (self.out_features,))
+        return output
 
     def _matvec(self, inputs: Tensor, output: Tensor, rows: int, rotate: bool = False) -> None:
         """One call into the C ABI on the current stream."""
-        _, tensors, constants = self._bound_arguments()
+        _, tensors, constants, layer, _ = self._bound_arguments()
         stream = native.current_stream(inputs.device)
         code = native.DTYPE_CODES[inputs.dtype]
         if rotate:
@@ -365,8 +369,7 @@ class PackedLinear(nn.Module):
                 inputs.data_ptr(), code, rotated.data_ptr(), *rotation, *tensors, output.data_ptr(), rows, *constants,
                 stream)
         else:
-            status = native.library().mk_packed_matvec(inputs.data_ptr(), code, *tensors, output.data_ptr(), rows,
-                                                       *constants, stream)
+            status = native.library().mk_packed_layer_matvec(layer, inputs.data_ptr(), code, output.data_ptr(), rows, stream)
         if status:
             native.check(status)
 

@@ -27,6 +27,14 @@ _c_int, _c_float, _c_void_p, _c_longlong = ctypes.c_int, ctypes.c_float, ctypes.
 
 SCALE_FORMAT_CODES = {"fp32": 0, "fp16": 1, "bf16": 2, "fp8": 3, "e8m0": 4}
 
+class PackedLayer(ctypes.Structure):
+    """``mk_packed_layer``."""
+
+    _fields_ = [(name, _c_void_p) for name in ("packed", "scales", "values", "zeros", "bias")] + [
+        (name, _c_int) for name in ("scale_dtype", "n_values", "bias_dtype", "output_width", "input_width", "group", "bits",
+                                    "uniform")] + [("grid_min", _c_float), ("grid_step", _c_float)]
+
+
 # name -> (restype, argtypes); mirrors include/mlkit_amd.h declaration by declaration.
 SIGNATURES: dict[str, tuple[Any, list[Any]]] = {
     "mk_version": (ctypes.c_char_p, []),
@@ -40,6 +48,8 @@ SIGNATURES: dict[str, tuple[Any, list[Any]]] = {
     "mk_fwht_columns": (_c_int, [_c_void_p, _c_int, _c_void_p, _c_int, _c_int, _c_void_p, _c_void_p, _c_float, _c_void_p]),
     "mk_transpose": (_c_int, [_c_void_p, _c_int, _c_void_p, _c_int, _c_int, _c_void_p]),
     "mk_hash_signs": (_c_int, [_c_void_p, _c_int, ctypes.c_uint, _c_void_p]),
+    "mk_packed_layer_matvec": (_c_int, [_c_void_p, _c_void_p, _c_int, _c_void_p, _c_int, _c_void_p]),
+    "mk_packed_layer_matmul": (_c_int, [_c_void_p, _c_void_p, _c_int, _c_void_p, _c_int, _c_void_p]),
     "mk_packed_matmul": (_c_int, [
         _c_void_p, _c_int, _c_void_p, _c_void_p, _c_int, _c_void_p, _c_int, _c_void_p,
         _c_void_p, _c_int, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
