@@ -11,8 +11,10 @@
 // 4096 x 14336 fp16 to INT4 g128 with offsets: 43 us = 4.1 TB/s (a device copy: 5.1), against 163 us for the
 // conversion to FP32, the range fit and the encoding as passes of their own (53 + 58 + 52).
 // A search is bound by the vector ALUs: 21 candidates, each a quotient and a rounding per weight.  4096 x 4096 on
-// seven values, g64: 236 us, against 496 us with an IEEE division and a bisection of the table per candidate and
-// weight; here tables of at most eight values are compared with thresholds kept in registers.
+// seven values, g64: 128 us, against 496 us with an IEEE division and a bisection of the table per candidate and
+// weight, and 236 us with thresholds kept in registers and the exact error of every candidate; groups of 64 columns and
+// more on integers or at most eight values now work out an estimate for each candidate (7 instructions a weight where the
+// values lie symmetrically about zero) and the exact error only where the estimate leaves the choice open.
 
 #include "scalar_codec_impl.h"
 
@@ -125,6 +127,16 @@ __global__ void __launch_bounds__(kThreads) round_groups_kernel(const RoundArgs 
         } else {
             while ((1 << steps) < a.n_values) ++steps;
         }
+    }
+    // Searched scales, teams of eight: a first pass over the candidates with a cheaper error (see `prune`).
+    constexpr bool kPruned = SEARCH && TEAM == 8 && ROUNDING != kTable;
+    __shared__ float estimate[kPruned ? kTeams : 1][64 + 1];
+    bool symmetric = ROUNDING == kFewValues;   // uniform
+    float magnitude[kFew / 2];                 // then: the values from zero up
+    if constexpr (kPruned && ROUNDING == kFewValues) {
+        for (int k = 0; k < a.n_values; ++k) symmetric = symmetric && table[k] == -table[a.n_values - 1 - k];
+#pragma unroll
+        for (int k = 0; k < kFew / 2; ++k) magnitude[k] = table[min(a.n_values / 2 + k, a.n_values - 1)];
     }
     bool ordinary_fractions = true;
     if constexpr (SEARCH) {
@@ -286,8 +298,95 @@ __global__ void __launch_bounds__(kThreads) round_groups_kernel(const RoundArgs 
                     best = fminf(best, error);
                 }
             };
+            // The candidates whose error can be the least, from a first pass with contracted arithmetic: the distance to
+            // the nearest multiple of the scale, or to the nearest scaled value, without the correctly rounded quotient.
+            // Against the error of `error_of` a distance d of a value x may be off by a few 2^-24 (|x| + |d|), so a sum by
+            // less than 2^-20 sqrt(E X) + 2^-40 X + 2^-18 E, X the sum of x^2; the margin below is at least four times that on
+            // either side.  What remains, one or two candidates as a rule, goes through `error_of` in order.
+            auto prune = [&](auto symmetric_) __attribute__((always_inline)) {
+                constexpr bool kSymmetric = decltype(symmetric_)::value;
+                auto over_team = [&](float sum) __attribute__((always_inline)) -> float {
+                    sum += mk_matvec::lane_exchange<0>(sum, threadIdx.x & 63);
+                    sum += mk_matvec::lane_exchange<1>(sum, threadIdx.x & 63);
+                    return sum + mk_matvec::lane_exchange<2>(sum, threadIdx.x & 63);
+                };
+                auto estimated = [&](float s) __attribute__((always_inline)) -> float {
+                    float sum[2] = {0.0f, 0.0f};
+                    const float inverse = __builtin_amdgcn_rcpf(s);
+                    float scaled[kFew];
+                    if constexpr (ROUNDING == kFewValues) {
+#pragma unroll
+                        for (int k = 0; k < (kSymmetric ? kFew / 2 : kFew); ++k) scaled[k] = (kSymmetric ? magnitude[k] : few_value[k]) * s;
+                    }
+#pragma unroll
+                    for (int t = 0; t < TRIPS; ++t)
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) {
+                            const float x = sample[t][i];
+                            float distance;
+                            if constexpr (ROUNDING == kInteger) {
+                                distance = __builtin_fmaf(-nearest_grid_integer(x * inverse, a.minimum, a.maximum), s, x);
+                            } else {
+                                const float from = kSymmetric ? fabsf(x) : x;
+                                distance = fabsf(from - scaled[0]);
+#pragma unroll
+                                for (int k = 1; k < (kSymmetric ? kFew / 2 : kFew); ++k) distance = fminf(distance, fabsf(from - scaled[k]));
+                            }
+                            sum[i & 1] = __builtin_fmaf(distance, distance, sum[i & 1]);
+                        }
+                    return over_team(sum[0] + sum[1]);
+                };
+                float *const estimates = estimate[threadIdx.x / TEAM];
+                const float base_scale = scale, of_base = estimated(base_scale);
+                float least = of_base;
+                for (int c = 0; c < a.n_fractions; ++c) {
+                    const float error = estimated(mk_rounded_scale(__fmul_rn(base_scale, fraction[c]), a.format));
+                    if (lane_in_team == 0) estimates[c] = error;
+                    least = fminf(least, error);
+                }
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                float squares = 0.0f;
+#pragma unroll
+                for (int t = 0; t < TRIPS; ++t)
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) squares = __builtin_fmaf(sample[t][i], sample[t][i], squares);
+                squares = over_team(squares);
+                const float bound = least + (0x1p-14f * least + (0x1p-17f * sqrtf(least * squares) + 0x1p-36f * squares));
+                unsigned long long open = 0;
+                for (int c = 0; c < a.n_fractions; ++c) open |= static_cast<unsigned long long>(estimates[c] <= bound) << c;
+                float best = __builtin_inff();
+                if (__any(of_base <= bound)) {
+                    const float error = error_of(base_scale, std::integral_constant<bool, false>{});
+                    best = of_base <= bound ? error : best;
+                }
+                while (__any(open != 0)) {   // at most n_fractions turns: each clears a bit of every team that has one
+                    const float candidate = mk_rounded_scale(__fmul_rn(base_scale, fraction[open ? __builtin_ctzll(open) : 0]), a.format);
+                    const float error = error_of(candidate, std::integral_constant<bool, false>{});
+                    if (open && error < best) {
+                        best = error;
+                        scale = candidate;
+                    }
+                    open &= open - 1;
+                }
+                __builtin_amdgcn_wave_barrier();   // the estimates have been read
+            };
+            // (2^40: no square or product of the first pass leaves the normal range)
+            const bool moderate = kPruned && all_whole && __all(base_scale > 0x1p-40f && base_scale < 0x1p40f && ordinary_fractions);
+            if constexpr (kPruned) {
+                if (moderate) {
+                    if constexpr (ROUNDING == kFewValues) {
+                        if (symmetric) prune(std::integral_constant<bool, true>{});
+                        else prune(std::integral_constant<bool, false>{});
+                    } else {
+                        prune(std::integral_constant<bool, false>{});
+                    }
+                }
+            }
             // candidates are fractions of the base (or the smallest value of the storage format)
-            if (all_whole && __all(base_scale > 0x1p-90f && base_scale < 0x1p90f && ordinary_fractions))
+            if (moderate) {
+            } else if (all_whole && __all(base_scale > 0x1p-90f && base_scale < 0x1p90f && ordinary_fractions))
                 search(std::integral_constant<bool, false>{});
             else
                 search(std::integral_constant<bool, true>{});

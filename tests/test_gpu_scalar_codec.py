@@ -282,3 +282,36 @@ def test_rounding_in_one_pass_reports_non_finite_weights(bad):
     weight[39, 199] = bad
     with pytest.raises(ValueError, match="finite"):
         mk.int(4, 64)(weight)
+
+
+@pytest.mark.parametrize("values,integer", [(SEVEN, False), (REPEATED, False), (INT3, True), (INT4, True),
+                                            (np.array([-1.5, -0.5, 0.5, 1.5], dtype=F32), False),
+                                            (np.array([0.25, 1.0], dtype=F32), False)])
+@pytest.mark.parametrize("group", [64, 128, 256])
+@pytest.mark.parametrize("asym", [False, True])
+def test_a_search_over_estimated_errors_chooses_as_the_full_search(values, integer, group, asym):
+    """Groups of 64 columns and more are searched among candidates whose estimated error can be the least: the same scales,
+    bit for bit, as an exact error for every candidate, on ordinary weights, on groups of zeros, of one value, on the grid
+    itself (errors of zero and ties among candidates) and next to rounding boundaries."""
+    from mlkit_amd.kernels import scalar_encode
+
+    rows, width = 300, 1024
+    weight = torch.from_numpy(helpers.normal_weight(rows, width, seed=group, student_t=True))
+    weight[3] = 0
+    weight[4] = 0.25
+    weight[5:40] = torch.from_numpy(values)[torch.randint(len(values), (35, width), generator=torch.Generator().manual_seed(1))] * 0.125
+    weight[40:80] = (weight[40:80] * 64).round() / 128
+    weight[80:90] *= 1e-4
+    weight[90:100, ::7] *= 1e3
+    weight = weight.half().cuda()
+    table, fractions = dev(values), dev(FRACTIONS)
+    minimum = float(values.min())
+    reciprocal = float(scaling.f32_reciprocal(float(values.max() - values.min()) if asym else float(np.abs(values).max())))
+    codes, scales, zeros, _ = scalar_encode.round_matrix(
+        weight, table, fractions, group, asym=asym, integer=integer, minimum=minimum, maximum=float(values.max()),
+        reciprocal=reciprocal, scale_format="fp16")
+    base, offset = scalar_encode.fit_scales(weight.float(), group, asym=asym, reciprocal=reciprocal, value_minimum=minimum,
+                                            scale_format="fp16", store_zero=False)
+    expected = scalar_encode.search_scales(weight.float(), base, offset, table, fractions, group, None, "fp16", integer=integer,
+                                           minimum=minimum, maximum=float(values.max()))
+    assert torch.equal(scales, expected)
