@@ -61,7 +61,10 @@ __device__ __forceinline__ float lane_value(float x, int lane) {
 //      scaled by 1 / sqrt(pivot), row i > j loses U[j][i] (a scalar, from lane i) times row j;
 //   3. the finished rows go back to LDS, and the tiles below lose U_r^T U_c on the matrix cores.  A 16 x 16 x 4
 //      accumulator holds rows 4 (lane / 16) + i of a column where the operands hold k = lane / 16, so product i takes
-//      k = 4 (lane / 16) + i and a tile is read as an operand exactly as it is held: one 16-byte LDS read.
+//      k = 4 (lane / 16) + i and a tile is read as an operand exactly as it is held: one 16-byte LDS read.  A panel's sixteen
+//      products are summed first and subtracted in one addition, so an entry is rounded at most 7 + 15 times on its way (128
+//      times in a running accumulator, which left the coefficients of 1024 columns 4.1e-7 from 64 bits; now 2.6e-7, 3.3e-7
+//      with the two-column kernel below).
 // Two barriers per 16 columns (one per two columns before, with every pivot row passed through LDS): what
 // bounds the kernel is the chain of 128 pivots.  One copy of the code serves all panels, since a
 // launch runs it once and instruction fetches would show.  A block with 768 columns beside it, called back to back: 25 us
@@ -215,13 +218,17 @@ __global__ void __launch_bounds__(kThreads, 2) cholesky_block_kernel(const Block
 #pragma unroll
         for (int r = 1; r < kTiles; ++r) {
             if (r <= s) continue;   // uniform
-            auto update = [&](f32x4 &tile, f32x4 u) __attribute__((always_inline)) {
+            auto products = [&](f32x4 u) __attribute__((always_inline)) -> f32x4 {
+                f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-                for (int i = 0; i < 4; ++i) tile = __builtin_amdgcn_mfma_f32_16x16x4f32(rows[r][i], u[i], tile, 0, 0, 0);
+                for (int i = 0; i < 4; ++i) sum = __builtin_amdgcn_mfma_f32_16x16x4f32(rows[r][i], u[i], sum, 0, 0, 0);
+                return sum;
             };
-            if constexpr (ROW) update(beside[r], u_beside);
-            if (r <= right_column) update(right[r], u_right);   // uniform
-            if (r < kWaves && r <= left_column) update(left[r], u_left);
+            // (on tiles below the diagonal too, whose numbers nothing reads: skipping those puts a branch, and a full wait for
+            // the products, in front of every addition)
+            if (r < kWaves) left[r] += products(u_left);
+            right[r] += products(u_right);
+            if constexpr (ROW) beside[r] += products(u_beside);
         }
     }
 }

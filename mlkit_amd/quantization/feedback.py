@@ -37,7 +37,8 @@ DEFERRED_TILES = 4  # tiles whose far-column updates are applied in one pass on 
 
 # Narrower matrices (less than one block) go to the library factorisation.  From here on blocks are faster and no less exact:
 # coefficients of 128 / 256 / 512 / 896 columns 0.12 / 0.15 / 0.25 / 0.42 ms against 0.26 / 0.65 / 1.34 / 2.47 with the library,
-# relative error against 64 bits 2.2e-7 / 2.9e-7 / 3.7e-7 / 3.7e-7 against 2.3e-7 / 3.5e-7 / 4.4e-7 / 4.2e-7.
+# relative error against 64 bits at 128 / 384 / 640 / 896 columns 1.3e-7 / 1.8e-7 / 2.5e-7 / 3.0e-7 against 2.5e-7 / 4.0e-7 /
+# 4.3e-7 / 4.4e-7.
 BLOCKED_FACTORIZATION_WIDTH = 128
 # Steps of several columns (vector grids) keep the arithmetic their conversions have had -- the library below this width and the
 # two-column block kernel from it on: a code for eight weights that the last bit of a coefficient turns takes its row along.

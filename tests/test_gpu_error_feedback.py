@@ -323,7 +323,7 @@ def test_blocked_factorisation_reports_an_indefinite_matrix():
         quantizer(dev(np.zeros((8, width), dtype=np.float32)), mk.Ctx("layer", H=dev(hessian)))
 
 
-def block_factor(matrix, size, first=0):
+def block_factor(matrix, size, first=0, entry="mk_cholesky_block"):
     """`mk_cholesky_block` on the first `size` rows of a matrix: (factor, block row, status)."""
     from mlkit_amd import native
 
@@ -332,7 +332,7 @@ def block_factor(matrix, size, first=0):
     beside = width - size
     factor = torch.zeros((128, 128), device="cuda")
     status = torch.zeros((), dtype=torch.int32, device="cuda")
-    native.check(native.library().mk_cholesky_block(
+    native.check(getattr(native.library(), entry)(
         work.data_ptr(), width, size, first, beside, factor.data_ptr() if beside else None, status.data_ptr(),
         native.current_stream(work.device)))
     out = host(work)
@@ -356,6 +356,28 @@ def test_a_factored_block_and_its_block_row(size, beside):
     if beside:
         carried = np.linalg.solve(expected.T, matrix[:size, size:].astype(np.float64))
         assert np.linalg.norm(row - carried) <= 1e-5 * np.linalg.norm(carried)
+
+
+@pytest.mark.parametrize("beside", [0, 200])
+def test_a_factored_block_is_as_close_to_64_bits_as_the_two_column_kernel(beside):
+    """Entries are subtracted from in panels of sixteen products, not product by product: summed over eight matrices the
+    distance to the float64 factor is no larger than that of the kernel which subtracts two products at a time."""
+    error = {"mk_cholesky_block": 0.0, "mk_cholesky_block_pairs": 0.0}
+    for seed in range(8):
+        rng = np.random.default_rng(seed)
+        width = 128 + beside
+        inputs = rng.standard_normal((2 * width, width))
+        matrix = (inputs.T @ inputs / inputs.shape[0]).astype(np.float32)
+        matrix += 0.01 * np.eye(width, dtype=np.float32)
+        exact = np.linalg.cholesky(matrix[:128, :128].astype(np.float64)).T
+        for entry in error:
+            factor, row, status = block_factor(matrix, 128, entry=entry)
+            assert status == 0
+            error[entry] += np.linalg.norm(factor - exact) / np.linalg.norm(exact)
+            if beside:
+                carried = np.linalg.solve(exact.T, matrix[:128, 128:].astype(np.float64))
+                error[entry] += np.linalg.norm(row - carried) / np.linalg.norm(carried)
+    assert error["mk_cholesky_block"] <= error["mk_cholesky_block_pairs"], error
 
 
 @pytest.mark.parametrize("column", [0, 1, 15, 16, 47, 100, 126])
