@@ -324,8 +324,8 @@ int mk_rotate_blocks(const void *source, int source_dtype, void *target, int tar
                      const float *signs_after, float scale, void *stream);
 
 /* target[:, c] = scale * H source[:, c] for every column c of a contiguous [rows, columns] matrix, in fp32; rows 1024,
- * 2048 or 4096 (MK_ERR_UNSUPPORTED otherwise).  signs_before / signs_after: one float per row, or NULL.  Agrees with mk_fwht
- * of the turned matrix to fp32 rounding (another order of stages), not bit for bit.
+ * 2048 or 4096 (MK_ERR_UNSUPPORTED otherwise).  signs_before / signs_after: one float per row, or NULL.  Equals mk_fwht
+ * of the turned fp32 matrix bit for bit (the same order of stages).
  * Replaces: `rotate(w.T.contiguous()).T` of quantization/algorithms/incoherence.py:56-98. */
 int mk_fwht_columns(const void *source, int source_dtype, float *target, int rows, int columns,
                     const float *signs_before, const float *signs_after, float scale, void *stream);

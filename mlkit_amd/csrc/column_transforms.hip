@@ -18,23 +18,31 @@ struct ColumnArgs {
     float scale;
 };
 
-// The transform of GROUPS * VALUES rows.  Thread (c, g) first holds rows g + GROUPS k of column c, k = 0 ... VALUES - 1, and
+template <int COLUMNS, int GROUPS, int VALUES>
+constexpr int kExchangeFloats = (VALUES * (GROUPS / 2) + GROUPS) * COLUMNS;   // half of a workgroup's values, padded
+
+// The transform of GROUPS * VALUES rows.  Thread (c, g) first holds rows VALUES g + k of column c, k = 0 ... VALUES - 1, and
 // does the stages over k in registers; through LDS it comes to hold VALUES / GROUPS of the k with all g, whose stages
-// follow.  A matrix is read once and written once.  The exchange takes two turns so that a workgroup's values fit LDS and
+// follow: ascending strides, as in the transform of rows, so that both give the same bits.  A matrix is read once and
+// written once.  The exchange takes two turns so that a workgroup's values fit LDS and
 // a thread its registers: in turn p a thread in half h of the groups puts half h ^ p of its k there and takes
 // what it needs of the groups' half h ^ p, into the registers that came free.
 //
-// Bound by HBM.  Neighbouring workgroups share 128-byte lines, so they are given to one XCD, whose L2 has
+// Up to 2048 rows bound by HBM.  Neighbouring workgroups share 128-byte lines, so they are given to one XCD, whose L2 has
 // the line: workgroup b takes column group (b % 8) * groups_per_xcd + b / 8.
 //
-// fp32, 14336 columns of 1024 / 2048 / 4096 values: 21 / 41 / 141 us, against 63 + 63 us for torch's strided copies around
-// the row transform at 1024, 119 + 119 at 2048 and 255 + 255 at 4096.  4096 rows run at 3.3 TB/s: 144 registers keep a
-// second workgroup off the compute unit, and held to 128 the kernel spills (206 us); 16 columns a workgroup take 151 us.
+// 14336 columns of 1024 / 2048 / 4096 fp32 values, signs before or behind: 20 / 40 / 145 us (from bf16 17 / 33 / 146), against
+// 63 + 63 us for torch's strided copies around the row transform at 1024, 119 + 119 at 2048 and 255 + 255 at 4096.  4096 rows
+// run at 3.2 TB/s, bound by latency: 144 registers keep a second workgroup off the compute unit, and held to 128 the kernel
+// spills (206 us); 16 columns a workgroup take 151 us.  With the signs behind read from memory as they are needed 25 / 47 /
+// 177 us; multiplied in a pass of their own 22 / 43 / 147.
 template <int COLUMNS, int GROUPS, int VALUES, int SOURCE>
 __global__ void __launch_bounds__(COLUMNS * GROUPS) fwht_columns_kernel(const ColumnArgs a) {
     constexpr int kHeld = VALUES / GROUPS;         // the k of a thread behind the exchange
     constexpr int kHalf = VALUES / 2, kHalfGroups = GROUPS / 2;
-    extern __shared__ float exchange[];
+    constexpr int kSignStride = GROUPS + 4;        // signs of one k, its groups side by side
+    extern __shared__ __align__(16) float exchange[];
+    float *const signs = exchange + kExchangeFloats<COLUMNS, GROUPS, VALUES>;
     const int group = static_cast<int>(blockIdx.x & 7) * a.groups_per_xcd + static_cast<int>(blockIdx.x >> 3);
     if (group >= a.groups) return;   // whole workgroups
     const int local = threadIdx.x & (COLUMNS - 1), g = threadIdx.x / COLUMNS;
@@ -45,10 +53,14 @@ __global__ void __launch_bounds__(COLUMNS * GROUPS) fwht_columns_kernel(const Co
     float value[2][kHalf];   // [k / kHalf][k % kHalf]
 #pragma unroll
     for (int k = 0; k < VALUES; ++k)
-        value[k / kHalf][k % kHalf] = mk_load_as_float(a.source, static_cast<size_t>(g + GROUPS * k) * a.columns + from, SOURCE);
+        value[k / kHalf][k % kHalf] = mk_load_as_float(a.source, static_cast<size_t>(g * VALUES + k) * a.columns + from, SOURCE);
+    if (a.signs_after) {   // uniform; a thread's rows lie VALUES apart, their signs are turned to lie side by side
+        for (int row = threadIdx.x; row < GROUPS * VALUES; row += COLUMNS * GROUPS)
+            signs[(row % VALUES) * kSignStride + row / VALUES] = a.signs_after[row];   // (read behind the exchange's barriers)
+    }
     if (a.signs_before) {   // uniform
 #pragma unroll
-        for (int k = 0; k < VALUES; ++k) value[k / kHalf][k % kHalf] *= a.signs_before[g + GROUPS * k];
+        for (int k = 0; k < VALUES; ++k) value[k / kHalf][k % kHalf] *= a.signs_before[g * VALUES + k];
     }
     auto butterfly = [](float &first, float &second) __attribute__((always_inline)) {
         const float low = first, high = second;
@@ -101,11 +113,14 @@ __global__ void __launch_bounds__(COLUMNS * GROUPS) fwht_columns_kernel(const Co
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int i = 0; i < kHalf; ++i) {
-            const int row = (g * kHeld + i / kHalfGroups) * GROUPS + h * kHalfGroups + i % kHalfGroups;
-            float result = value[h][i] * a.scale;
-            if (a.signs_after) result *= a.signs_after[row];
-            a.target[static_cast<size_t>(row) * a.columns + column] = result;
+        for (int i = 0; i < kHalf; i += 4) {
+            const int k = g * kHeld + i / kHalfGroups, of = h * kHalfGroups + i % kHalfGroups;   // of ... of + 3: four groups of one k
+            float4 sign = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
+            if (a.signs_after) sign = *reinterpret_cast<const float4 *>(signs + k * kSignStride + of);
+            const float along[4] = {sign.x, sign.y, sign.z, sign.w};
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                a.target[static_cast<size_t>((of + j) * VALUES + k) * a.columns + column] = value[h][i + j] * a.scale * along[j];
         }
 }
 
@@ -113,7 +128,7 @@ template <int COLUMNS, int GROUPS, int VALUES, int SOURCE>
 void launch_columns(ColumnArgs a, hipStream_t stream) {
     a.groups = mk_cdiv(a.columns, COLUMNS);
     a.groups_per_xcd = mk_cdiv(a.groups, 8);
-    constexpr size_t lds = (VALUES * (GROUPS / 2) + GROUPS) * COLUMNS * sizeof(float);
+    constexpr size_t lds = (kExchangeFloats<COLUMNS, GROUPS, VALUES> + VALUES * (GROUPS + 4)) * sizeof(float);
     static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void *>(&fwht_columns_kernel<COLUMNS, GROUPS, VALUES, SOURCE>),
                                                           hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     static_cast<void>(allowed);   // a refusal shows in the launch

@@ -305,6 +305,20 @@ def test_columns_are_transformed_as_the_rows_of_the_turned_matrix(rows, columns,
                                host(device_transforms.rotate_columns(view.contiguous(), signs=signs)), rtol=0, atol=0)
 
 
+@pytest.mark.parametrize("rows", [640, 1024, 2048, 4096])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_columns_and_rows_run_their_stages_in_one_order(rows, dtype):
+    """The transform of columns rounds exactly as that of the turned matrix: ascending strides, signs and scale alike."""
+    from mlkit_amd.quantization import transforms as device_transforms
+    from mlkit_amd.quantization.codecs import deterministic_signs
+
+    matrix = torch.randn((rows, 131), device="cuda").to(dtype)
+    signs = deterministic_signs(rows, 9, matrix.device)
+    for inverse in (False, True):
+        expected = device_transforms.rotate(matrix.float().T.contiguous(), signs=signs, inverse=inverse).T
+        assert torch.equal(device_transforms.rotate_columns(matrix, signs=signs, inverse=inverse), expected)
+
+
 @pytest.mark.parametrize("rows,columns", [(1, 1), (3, 70), (64, 64), (65, 4), (100, 132), (260, 68)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 def test_turning_a_matrix(rows, columns, dtype):
