@@ -138,6 +138,56 @@ def test_infinite_activations_reach_the_outputs_as_in_a_dense_product(name, asym
     np.testing.assert_array_equal(np.isinf(y) * np.sign(y), np.isinf(expected) * np.sign(expected))
 
 
+@pytest.mark.parametrize("name,group,asym", [("int4", 128, True), ("nf4", 64, False), ("int3", 1184, True), ("int2", 64, False), ("int8", 128, False)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_outputs_by_their_definition_on_rows_of_several_pieces(name, group, asym, dtype):
+    """Rows that are neither a whole number of 512 columns nor of tiles: infinities of one sign and of both in different
+    pieces, a NaN in the last one, and finite activations whose products with operand and offset overflow although the
+    outputs do not."""
+    values, bits, integer = CODECS[name]
+    layer = helpers.quantised_layer(helpers.normal_weight(37, 1184, seed=3), values, bits=bits, group=group, integer=integer, asym=asym)
+    x = helpers.activations(21, 1184, seed=2, dtype=torch.float32)
+    if dtype == torch.bfloat16:
+        x[1] *= 1e36   # 128 columns times operands of 128 pass 2^128
+    x = x.to(dtype)
+    x[3, 1183], x[4, 0], x[4, 600], x[5, 511], x[6, 1183], x[20, 512] = (float(v) for v in ("inf", "inf", "-inf", "-inf", "nan", "inf"))
+    y = run(layer, x.cuda()).double().cpu().numpy()
+    with np.errstate(invalid="ignore"):
+        expected = (x.double().numpy()[:, None, :] * layer["dense"].astype(np.float64)[None]).sum(-1)
+    np.testing.assert_array_equal(np.isnan(y), np.isnan(expected))
+    np.testing.assert_array_equal(np.isinf(y) * np.sign(y), np.isinf(expected) * np.sign(expected))
+    for sample in (0, 1, 2, 7, 19):
+        error = np.abs(y[sample] - expected[sample]).max() / np.abs(expected[sample]).max()
+        assert error <= RANGE_TOLERANCE[dtype], (sample, error)
+
+
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_an_activation_that_is_not_finite_does_not_make_a_call_a_slow_one(value):
+    """One such row (a padded token behind a masked softmax) among 32: a few more microseconds, no other order of magnitude."""
+    import mlkit_amd as mk
+
+    linear = torch.nn.Linear(14336, 4096, bias=False, device="cuda", dtype=torch.bfloat16)
+    layer = mk.PackedLinear(linear, mk.int(4, 128, asym=True)(linear.weight.detach()))
+    finite = torch.randn((32, 14336), device="cuda", dtype=torch.bfloat16)
+    other = finite.clone()
+    other[3, 100] = value
+
+    def microseconds(x):
+        best = float("inf")
+        with torch.no_grad():
+            layer(x)
+            for _ in range(10):
+                start, stop = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+                start.record()
+                layer(x)
+                stop.record()
+                stop.synchronize()
+                best = min(best, 1e3 * start.elapsed_time(stop))
+        return best
+
+    assert microseconds(other) <= 10 * microseconds(finite)
+
+
 def test_calls_that_are_recorded_batched_differentiated_or_cast_take_the_dense_product():
     import torch.autograd.forward_ad as forward_ad
 
