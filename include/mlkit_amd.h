@@ -66,7 +66,8 @@ int mk_packed_matvec(const void *x, int x_dtype, const uint8_t *packed, const vo
  *   input_width           a multiple of 32; x and packed 16-byte aligned
  *   group                 64, a multiple of 128, or at least input_width
  * MK_ERR_UNSUPPORTED otherwise (nothing was launched): decode the weight and multiply.
- * Codes are exact operands and scales multiply fp32 sums, so no weight is rounded to x's type.
+ * Operands are exact on uniform grids; a table value that x's type does not hold is split into two operands, to 2^-17 of it
+ * (bf16) or 2^-23 (fp16).  Scales multiply fp32 sums, so no weight is rounded to x's type.
  * Replaces: the decode and dense product of inference/packed_linear.py:110-154. */
 int mk_packed_matmul(const void *x, int x_dtype, const uint8_t *packed, const void *scales,
                      int scale_dtype, const float *values, int n_values, const void *zeros,
@@ -84,6 +85,8 @@ typedef struct mk_packed_layer {
     const void *bias;
     int scale_dtype, n_values, bias_dtype, output_width, input_width, group, bits, uniform;
     float grid_min, grid_step;
+    int values_held;   /* not 0: fp16 and bf16 hold every table value times some power of two, so that one operand will do.
+                        * Results stay right where that is not so, at a hundred times the time. */
 } mk_packed_layer;
 
 /* mk_packed_matvec and mk_packed_matmul with those arguments in one place (a call from Python costs by the argument). */

@@ -5,6 +5,8 @@
 
 #include "packed_matmul_impl.h"
 
+#include <cmath>
+
 using mk_matmul::MatmulArgs;
 using mk_matmul::MatmulPlan;
 
@@ -41,12 +43,23 @@ MatmulPlan plan_for(int samples, int rows) {
     return plan;
 }
 
-}  // namespace
+// Whether fp16 and bf16 hold every value of a grid, in the range the kernel brings them to.
+bool grid_held(float minimum, float step, int codes) {
+    float largest = 0.0f;
+    for (int code = 0; code < codes; ++code) largest = std::fmax(largest, std::fabs(std::fmaf(static_cast<float>(code), step, minimum)));
+    if (!(largest > 0.0f) || !std::isfinite(largest)) return false;
+    int exponent;
+    std::frexp(largest, &exponent);
+    for (int code = 0; code < codes; ++code) {
+        const float units = std::ldexp(std::fmaf(static_cast<float>(code), step, minimum), 8 - exponent);   // 2^7 ... 2^8 and below
+        if (units != std::rint(units)) return false;   // eight bits from the largest value's first on: both types have them
+    }
+    return true;
+}
 
-extern "C" int mk_packed_matmul(const void *x, int x_dtype, const uint8_t *packed, const void *scales, int scale_dtype,
-                                const float *values, int n_values, const void *zeros, const void *bias, int bias_dtype,
-                                void *y, int samples, int output_width, int input_width, int group, int bits,
-                                int uniform, float grid_min, float grid_step, void *stream_) {
+int matmul(const void *x, int x_dtype, const uint8_t *packed, const void *scales, int scale_dtype, const float *values, int n_values,
+           const void *zeros, const void *bias, int bias_dtype, void *y, int samples, int output_width, int input_width, int group,
+           int bits, int uniform, float grid_min, float grid_step, int values_held, void *stream_) {
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     MK_REQUIRE(x && packed && scales && y, MK_ERR_INVALID, "mk_packed_matmul: null tensor pointer");
     MK_REQUIRE(samples >= 1 && output_width >= 1 && input_width >= 1 && group >= 1, MK_ERR_INVALID,
@@ -79,6 +92,7 @@ extern "C" int mk_packed_matmul(const void *x, int x_dtype, const uint8_t *packe
     a.need_sums = zeros != nullptr || format == mk_matmul::kUniform4 || format == mk_matmul::kUniform8;
 
     MatmulPlan plan = plan_for(samples, output_width);
+    plan.split = bits != 8 && format != mk_matmul::kUniform4 && !(uniform ? grid_held(grid_min, grid_step, 1 << bits) : values_held != 0);
     plan.sub = whole_row || group % 128 == 0 ? 1 : 2;
     a.steps_per_group = whole_row ? a.steps : group / 128 > 0 ? group / 128 : 1;
     if (a.steps_per_group > 1) {   // exact for the steps of any row: below 2^31
@@ -89,10 +103,11 @@ extern "C" int mk_packed_matmul(const void *x, int x_dtype, const uint8_t *packe
     }
     a.whole_quads = output_width % 4 == 0 && (reinterpret_cast<uintptr_t>(y) & 7u) == 0;
     if (plan.waves > a.steps) plan.waves = a.steps;
+    const size_t table = (bits == 2 ? 2048 : bits == 3 ? 256 : format == mk_matmul::kTable4 ? 1024 : 0) * (plan.split ? 2 : 1);
     auto lds = [&] {
         const size_t stage = static_cast<size_t>(plan.waves) * plan.sample_tiles * 4096;
         const size_t sums = static_cast<size_t>(plan.waves) * plan.row_tiles * plan.sample_tiles * 1024;
-        return (stage > sums ? stage : sums) + 2048 + (64 + static_cast<size_t>(a.groups) * 64 * (a.need_sums ? 2 : 1)) * plan.row_tiles;
+        return (stage > sums ? stage : sums) + table + (64 + static_cast<size_t>(a.groups) * 64 * (a.need_sums ? 2 : 1)) * plan.row_tiles;
     };
     while (lds() > 160 * 1024 && plan.row_tiles > 1) plan.row_tiles = plan.sample_tiles > 1 ? (plan.sample_tiles = plan.row_tiles = 1) : plan.row_tiles / 2;
     while (lds() > 160 * 1024 && plan.waves > 1) plan.waves /= 2;
@@ -110,9 +125,19 @@ extern "C" int mk_packed_matmul(const void *x, int x_dtype, const uint8_t *packe
     return MK_OK;
 }
 
+}  // namespace
+
+extern "C" int mk_packed_matmul(const void *x, int x_dtype, const uint8_t *packed, const void *scales, int scale_dtype,
+                                const float *values, int n_values, const void *zeros, const void *bias, int bias_dtype,
+                                void *y, int samples, int output_width, int input_width, int group, int bits,
+                                int uniform, float grid_min, float grid_step, void *stream) {
+    return matmul(x, x_dtype, packed, scales, scale_dtype, values, n_values, zeros, bias, bias_dtype, y, samples, output_width,
+                  input_width, group, bits, uniform, grid_min, grid_step, 0, stream);
+}
+
 extern "C" int mk_packed_layer_matmul(const mk_packed_layer *layer, const void *x, int x_dtype, void *y, int samples, void *stream) {
     MK_REQUIRE(layer, MK_ERR_INVALID, "mk_packed_layer_matmul: null layer");
     const mk_packed_layer &l = *layer;
-    return mk_packed_matmul(x, x_dtype, l.packed, l.scales, l.scale_dtype, l.values, l.n_values, l.zeros, l.bias, l.bias_dtype, y, samples,
-                            l.output_width, l.input_width, l.group, l.bits, l.uniform, l.grid_min, l.grid_step, stream);
+    return matmul(x, x_dtype, l.packed, l.scales, l.scale_dtype, l.values, l.n_values, l.zeros, l.bias, l.bias_dtype, y, samples,
+                  l.output_width, l.input_width, l.group, l.bits, l.uniform, l.grid_min, l.grid_step, l.values_held, stream);
 }

@@ -1,7 +1,7 @@
 // Packed weight x several rows of activations on the matrix cores of gfx950: kernel template.
 //
 // y[m, n] = sum_k dequant(code[n, k]) * x[m, k] (+ bias[n]) for nine rows of x and more; fp16 or bf16 x, codes of 2, 3,
-// 4 or 8 bits, fp16 or bf16 scales, scale groups of 32 or 64 columns, of a multiple of 128, or of the whole row.
+// 4 or 8 bits, fp16 or bf16 scales, scale groups of 64 columns, of a multiple of 128, or of the whole row.
 //
 // Codes go straight from HBM to the matrix cores.  v_mfma_f32_16x16x32 takes a 16 x 32 piece of the weight as eight
 // values per lane; lane (n, q) loads the quarter of row n's scale group that the instructions of the group give to
@@ -9,7 +9,15 @@
 // numbers of x's type (arithmetic for uniform 4- and 8-bit grids, an LDS table of several values per lookup
 // otherwise); the group's products are summed first and scaled in fp32 afterwards:
 //     y += s * sum(operand * x) + b * sum(x),   b = s * (grid minimum - operand of code 0) + zero,
-// with sum(x) from a multiplication by ones where b is not zero.  Nothing is rounded between code and fp32 sum.
+// with sum(x) from a multiplication by ones where b is not zero.
+//
+// Table values that x's type cannot hold (NF4, fitted codebooks) are two operands (SPLIT), the value rounded and what the
+// rounding left of it: all weights of one code share its error, which adds up over x with a mean where errors of single weights
+// cancel (NF4, 14336 columns of relu(normal) x: 3.1e-2 of y in bf16 and 2.1e-3 in fp16 with the rounded value alone, 2.8e-3
+// and 3.4e-4 with a decoded weight rounded as a whole, 1.7e-3 and 2.1e-4 -- the rounding of y -- with both).  A table is
+// multiplied by a power of two that puts its largest value at 2^14, the scales by the inverse, so that in fp16 neither part
+// runs out of range: the two hold a value to 2^-23 of it, or 2^-39 of the largest; in bf16 to 2^-17 of it.  Without SPLIT every
+// wavefront makes sure that x's type holds its table; outputs over one that it does not hold come from plain_outputs.
 //
 // A workgroup owns 16 * RT rows of the weight and 16 * MT rows of x; its wavefronts take the row's steps of 128 columns
 // in turn, so a step's activations are read by one wavefront only.  They pass through a stretch of LDS of its own (no
@@ -76,6 +84,7 @@ __device__ __forceinline__ uint32_t pair_of(float low, float high) {
 }
 
 // What a format is made of: the dwords a lane holds of CH consecutive codes, and the operand of codes 8 j ... 8 j + 7.
+// Behind the kTableWords dwords of a table of values there are as many of what their rounding left (SPLIT).
 template <int FORMAT, int XT, int CH>
 struct Codes;
 
@@ -182,7 +191,7 @@ __device__ __forceinline__ float table_value(const MatmulArgs &a, int code) {
     return a.uniform ? a.grid_min + static_cast<float>(code) * a.grid_step : a.values[code < a.n_values ? code : a.n_values - 1];
 }
 
-// Outputs of a tile by their definition, for sums that are not finite: an infinite activation times operand and offset gives
+// Outputs of a tile by their definition, for sums that are not finite (and for tables, see above): an infinite activation times operand and offset gives
 // infinities of both signs where its product with the decoded weight has one.  Lane (c, q) of the wavefront holds the
 // sums of rows row + 4 q ... + 3 with sample `sample` + c; `open`: the lanes whose four are wanted.
 //
@@ -276,15 +285,15 @@ __device__ __forceinline__ void plain_outputs(const MatmulArgs &a, unsigned long
 }
 
 // Dynamic LDS of a workgroup, in bytes; the sums of the wavefronts reuse the activations' stretch.
-template <int FORMAT, int RT, int MT>
+template <int FORMAT, int RT, int MT, bool SPLIT>
 constexpr size_t lds_bytes(int waves, int scale_groups, bool sums_needed) {
-    constexpr int table = Codes<FORMAT, MK_F16, 32>::kTableWords * 4;
+    constexpr int table = Codes<FORMAT, MK_F16, 32>::kTableWords * (SPLIT ? 8 : 4);
     const size_t stage = static_cast<size_t>(waves) * MT * 16 * 256;
     const size_t sums = static_cast<size_t>(waves) * RT * MT * 1024;
     return (stage > sums ? stage : sums) + table + 64 * RT + static_cast<size_t>(scale_groups) * 16 * RT * 4 * (sums_needed ? 2 : 1);
 }
 
-template <int FORMAT, int XT, int RT, int MT, int SUB, bool SUMS>
+template <int FORMAT, int XT, int RT, int MT, int SUB, bool SUMS, bool SPLIT>
 __global__ void __launch_bounds__(64 * kMaxWaves) packed_matmul_kernel(const MatmulArgs a) {
     constexpr int kChunk = 32 / SUB;          // codes of a lane per scale group
     constexpr int kProducts = kChunk / 8;     // matrix instructions per scale group
@@ -301,7 +310,7 @@ __global__ void __launch_bounds__(64 * kMaxWaves) packed_matmul_kernel(const Mat
     const size_t stage_bytes = static_cast<size_t>(waves) * MT * 16 * 256, sum_bytes = static_cast<size_t>(waves) * RT * MT * 1024;
     mk_u32x4 *stage = lds + wave * (MT * 16 * 16);
     uint32_t *table = reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(lds) + (stage_bytes > sum_bytes ? stage_bytes : sum_bytes));
-    float *biases = reinterpret_cast<float *>(table + C::kTableWords);
+    float *biases = reinterpret_cast<float *>(table + (SPLIT ? 2 : 1) * C::kTableWords);
     float *scales = biases + kRows;
 
     // -- loads of a step: the codes of this lane's rows, the pieces of activations this lane passes on ---------------
@@ -378,12 +387,31 @@ __global__ void __launch_bounds__(64 * kMaxWaves) packed_matmul_kernel(const Mat
     load_codes(raw, wave);
 
     // -- tables and scales into LDS, once ---------------------------------------------------------------------------
-    for (int i = threadIdx.x; i < C::kTableWords; i += blockDim.x) {
-        if constexpr (FORMAT == kTable4) table[i] = pair_of<XT>(table_value(a, i & 15), table_value(a, i >> 4));
-        else if constexpr (FORMAT == kTable3) table[i] = pair_of<XT>(table_value(a, i & 7), table_value(a, i >> 3));
-        else if constexpr (FORMAT == kTable2) {
-            const int codes = (i >> 1) >> (4 * (i & 1));
-            table[i] = pair_of<XT>(table_value(a, codes & 3), table_value(a, (codes >> 2) & 3));
+    bool held = true;            // uniform: x's type holds the table, or there is a second operand
+    float table_inverse = 1.0f;  // the inverse of the table's power of two, for the scales
+    if constexpr (C::kTableWords > 0) {
+        constexpr int kCodes = 1 << C::kBits;
+        float largest = 0.0f;
+#pragma unroll
+        for (int code = 0; code < kCodes; ++code) largest = fmaxf(largest, fabsf(table_value(a, code)));
+        int exponent = (__float_as_int(largest) >> 23) - (127 + 14);
+        exponent = largest > 0.0f && largest < __builtin_inff() ? min(max(exponent, -100), 100) : 0;
+        table_inverse = __int_as_float((127 + exponent) << 23);
+        const float factor = __int_as_float((127 - exponent) << 23);
+        auto rounded = [&](float value) __attribute__((always_inline)) -> float {
+            if constexpr (XT == MK_F16) return static_cast<float>(static_cast<_Float16>(value));
+            else return static_cast<float>(static_cast<__bf16>(value));
+        };
+        if constexpr (!SPLIT) {
+            const float own = table_value(a, lane % kCodes) * factor;
+            held = __all(rounded(own) == own);
+        }
+        for (int i = threadIdx.x; i < C::kTableWords; i += blockDim.x) {
+            const int codes = FORMAT == kTable2 ? (i >> 1) >> (4 * (i & 1)) : i;
+            const float low = table_value(a, codes & (kCodes - 1)) * factor;
+            const float high = table_value(a, (codes >> C::kBits) & (kCodes - 1)) * factor;
+            table[i] = pair_of<XT>(low, high);
+            if constexpr (SPLIT) table[C::kTableWords + i] = pair_of<XT>(low - rounded(low), high - rounded(high));
         }
     }
     float *offsets = scales + a.groups * kRows;
@@ -414,7 +442,7 @@ __global__ void __launch_bounds__(64 * kMaxWaves) packed_matmul_kernel(const Mat
             for (int i = 0; i < kBatch; ++i) {
                 const int slot = min(first + i * per_row, a.groups - 1) * kRows + local_row;
                 const float scale = side_value(stored[i]);
-                scales[slot] = kArithmetic ? scale * a.grid_step : scale;
+                scales[slot] = kArithmetic ? scale * a.grid_step : scale * table_inverse;
                 if constexpr (SUMS) {
                     const float offset = side_value(zero[i] & zero_mask);
                     offsets[slot] = kArithmetic ? __builtin_fmaf(scale, a.grid_min - C::kOffset * a.grid_step, offset) : offset;
@@ -459,6 +487,11 @@ __global__ void __launch_bounds__(64 * kMaxWaves) packed_matmul_kernel(const Mat
 #pragma unroll
                     for (int mt = 0; mt < MT; ++mt)
                         product[rt][mt] = mfma<XT>(weights, activations[mt], j == 0 ? none : product[rt][mt]);
+                    if constexpr (SPLIT) {
+                        const mk_u32x4 rest = format.operand(raw[rt][sub], j, table + C::kTableWords, shift);
+#pragma unroll
+                        for (int mt = 0; mt < MT; ++mt) product[rt][mt] = mfma<XT>(rest, activations[mt], product[rt][mt]);
+                    }
                 }
             }
             int group = step * SUB + sub;
@@ -521,7 +554,7 @@ __global__ void __launch_bounds__(64 * kMaxWaves) packed_matmul_kernel(const Mat
         for (int w = 0; w < waves; ++w) value += sums[w * RT * MT * 64 + item];
         const bool inside = sample < a.samples && row < a.rows;
         const float all = (value[0] + value[1]) + (value[2] + value[3]);
-        if (const unsigned long long open = __ballot(inside && all - all != 0.0f); __builtin_expect(open != 0, 0))   // (whole wavefronts take a turn)
+        if (const unsigned long long open = __ballot(inside && (!held || all - all != 0.0f)); __builtin_expect(open != 0, 0))   // (whole wavefronts take a turn)
             plain_outputs<FORMAT, XT>(a, open, first_row + rt * 16, first_sample + mt * 16, biases + rt * 16, value, lane);
         if (!inside) continue;
         const size_t at = static_cast<size_t>(sample) * a.rows + row;
@@ -539,6 +572,7 @@ __global__ void __launch_bounds__(64 * kMaxWaves) packed_matmul_kernel(const Mat
 // How a launch is cut.
 struct MatmulPlan {
     int row_tiles, sample_tiles, waves, sub;   // RT, MT, wavefronts per workgroup, SUB
+    bool split;                                // SPLIT
 };
 
 }  // namespace mk_matmul

@@ -5,10 +5,10 @@ using namespace mk_matmul;
 
 namespace {
 
-template <int FORMAT, int XT, int RT, int MT, int SUB, bool SUMS>
+template <int FORMAT, int XT, int RT, int MT, int SUB, bool SUMS, bool SPLIT>
 int launch(const MatmulArgs &a, const MatmulPlan &plan, hipStream_t stream) {
-    const size_t lds = lds_bytes<FORMAT, RT, MT>(plan.waves, a.groups, SUMS);
-    auto *kernel = &packed_matmul_kernel<FORMAT, XT, RT, MT, SUB, SUMS>;
+    const size_t lds = lds_bytes<FORMAT, RT, MT, SPLIT>(plan.waves, a.groups, SUMS);
+    auto *kernel = &packed_matmul_kernel<FORMAT, XT, RT, MT, SUB, SUMS, SPLIT>;
     static std::atomic<size_t> allowed{64 * 1024};   // raised once per kernel when a launch needs more
     if (lds > allowed.load(std::memory_order_relaxed)) {
         const hipError_t status = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
@@ -21,28 +21,36 @@ int launch(const MatmulArgs &a, const MatmulPlan &plan, hipStream_t stream) {
     return MK_OK;
 }
 
-template <int FORMAT, int XT, int SUB, bool SUMS>
+template <int FORMAT, int XT, int SUB, bool SUMS, bool SPLIT>
 int with_tiles(const MatmulArgs &a, const MatmulPlan &plan, hipStream_t stream) {
     switch (plan.sample_tiles * 8 + plan.row_tiles) {
-        case 1 * 8 + 1: return launch<FORMAT, XT, 1, 1, SUB, SUMS>(a, plan, stream);
-        case 1 * 8 + 2: return launch<FORMAT, XT, 2, 1, SUB, SUMS>(a, plan, stream);
-        case 1 * 8 + 4: return launch<FORMAT, XT, 4, 1, SUB, SUMS>(a, plan, stream);
-        case 2 * 8 + 2: return launch<FORMAT, XT, 2, 2, SUB, SUMS>(a, plan, stream);
-        case 2 * 8 + 4: return launch<FORMAT, XT, 4, 2, SUB, SUMS>(a, plan, stream);
-        default: return launch<FORMAT, XT, 2, 4, SUB, SUMS>(a, plan, stream);
+        case 1 * 8 + 1: return launch<FORMAT, XT, 1, 1, SUB, SUMS, SPLIT>(a, plan, stream);
+        case 1 * 8 + 2: return launch<FORMAT, XT, 2, 1, SUB, SUMS, SPLIT>(a, plan, stream);
+        case 1 * 8 + 4: return launch<FORMAT, XT, 4, 1, SUB, SUMS, SPLIT>(a, plan, stream);
+        case 2 * 8 + 2: return launch<FORMAT, XT, 2, 2, SUB, SUMS, SPLIT>(a, plan, stream);
+        case 2 * 8 + 4: return launch<FORMAT, XT, 4, 2, SUB, SUMS, SPLIT>(a, plan, stream);
+        default: return launch<FORMAT, XT, 2, 4, SUB, SUMS, SPLIT>(a, plan, stream);
     }
 }
 
-template <int FORMAT, int XT>
+template <int FORMAT, int XT, bool SPLIT>
 int with_groups(const MatmulArgs &a, const MatmulPlan &plan, hipStream_t stream) {
     if constexpr (FORMAT != kUniform4 && FORMAT != kUniform8) {   // (those two are compiled with sums only)
         if (!a.need_sums) {
-            if (plan.sub == 2) return with_tiles<FORMAT, XT, 2, false>(a, plan, stream);
-            return with_tiles<FORMAT, XT, 1, false>(a, plan, stream);
+            if (plan.sub == 2) return with_tiles<FORMAT, XT, 2, false, SPLIT>(a, plan, stream);
+            return with_tiles<FORMAT, XT, 1, false, SPLIT>(a, plan, stream);
         }
     }
-    if (plan.sub == 2) return with_tiles<FORMAT, XT, 2, true>(a, plan, stream);
-    return with_tiles<FORMAT, XT, 1, true>(a, plan, stream);
+    if (plan.sub == 2) return with_tiles<FORMAT, XT, 2, true, SPLIT>(a, plan, stream);
+    return with_tiles<FORMAT, XT, 1, true, SPLIT>(a, plan, stream);
+}
+
+template <int FORMAT, int XT>
+int with_operands(const MatmulArgs &a, const MatmulPlan &plan, hipStream_t stream) {
+    if constexpr (FORMAT != kUniform4 && FORMAT != kUniform8) {   // (their operands are exact)
+        if (plan.split) return with_groups<FORMAT, XT, true>(a, plan, stream);
+    }
+    return with_groups<FORMAT, XT, false>(a, plan, stream);
 }
 
 }  // namespace
@@ -50,6 +58,6 @@ int with_groups(const MatmulArgs &a, const MatmulPlan &plan, hipStream_t stream)
 #define MK_PASTE_(a, b) a##b
 #define MK_PASTE(a, b) MK_PASTE_(a, b)
 int MK_PASTE(mk_matmul_launch_, MK_MATMUL_FORMAT)(const MatmulArgs &a, const MatmulPlan &plan, int x_dtype, hipStream_t stream) {
-    if (x_dtype == MK_F16) return with_groups<MK_MATMUL_FORMAT, MK_F16>(a, plan, stream);
-    return with_groups<MK_MATMUL_FORMAT, MK_BF16>(a, plan, stream);
+    if (x_dtype == MK_F16) return with_operands<MK_MATMUL_FORMAT, MK_F16>(a, plan, stream);
+    return with_operands<MK_MATMUL_FORMAT, MK_BF16>(a, plan, stream);
 }

@@ -20,6 +20,7 @@ How a call is served here:
 
 import copy
 import ctypes
+import math
 from collections.abc import Callable
 from dataclasses import dataclass
 
@@ -37,10 +38,11 @@ from mlkit_amd.quantization.core import Q
 SCALE_STORAGE_DTYPES = {"fp16": torch.float16, "bf16": torch.bfloat16}
 MAXIMUM_FUSED_ROWS = 8
 # Rows up to which multiplying the codes beats decoding the weight for a library product (us, 4096 x 14336 / 14336 x 4096
-# INT4 at 128 rows 38 / 44 against 90 / 60, NF4 54 / 52 against 85 / 55; at 192 rows NF4 and INT8 14336 x 4096 lose, 74
-# and 80 against 62 and 65).  Layers of at most 2^24 weights gain up to 256 rows (4096 x 4096: INT4 23 against 35, INT8 29
-# against 34), where the decode and the product are two short launches.
-MAXIMUM_PRODUCT_ROWS, MAXIMUM_PRODUCT_ROWS_SMALL, SMALL_WEIGHTS = 128, 256, 1 << 24
+# INT4 at 128 rows 38 / 45 against 90 / 59; at 192 rows INT8 14336 x 4096 loses, 80 against 65).  Tables that take two operands
+# a value (NF4, fitted codebooks) win up to 64 rows: NF4 at 64 rows 39 / 34 against 63 / 53, at 96 rows 72 / 58 against 76 / 53.
+# Layers of at most 2^24 weights gain up to 256 rows (4096 x 4096: INT4 23 against 35, INT8 29 against 34, NF4 32 against 35;
+# 2048 x 2048 at 192 rows NF4 16.1 against 17.1), where the decode and the product are two short launches.
+MAXIMUM_PRODUCT_ROWS, MAXIMUM_PRODUCT_ROWS_SPLIT, MAXIMUM_PRODUCT_ROWS_SMALL, SMALL_WEIGHTS = 128, 64, 256, 1 << 24
 PRODUCT_DTYPES = frozenset({torch.float16, torch.bfloat16})
 _LAUNCH_BUFFERS = frozenset({"packed", "scales", "values", "zeros", "bias"})
 
@@ -90,6 +92,16 @@ class _Grid:
         return _Grid(bool(torch.allclose(gaps, gaps[0].expand_as(gaps))), float(table[0]), float(gaps[0]))
 
 
+def _values_held(values: Tensor) -> bool:
+    """Whether fp16 and bf16 hold every value exactly once a power of two has brought the largest to 2^14."""
+    table = values.detach().double().cpu()
+    largest = float(table.abs().max()) if table.numel() else 0.0
+    if not 0 < largest < math.inf:
+        return False
+    table = torch.ldexp(table, torch.tensor(15 - math.frexp(largest)[1]))
+    return all(torch.equal(table.to(dtype).double(), table) for dtype in PRODUCT_DTYPES)
+
+
 class PackedLinear(nn.Module):
     """Exact scalar-grid codes of one to eight bits with fused decode for short inputs.
 
@@ -103,6 +115,7 @@ class PackedLinear(nn.Module):
     zeros: Tensor | None
     bias: Tensor | None
     _dense_weight: Tensor | None
+    values_held = False   # (layers pickled without it)
 
     def __init__(self, original: nn.Linear, quantized: Q, *, cache_dense: bool = False,
                  overflow: Tensor | None = None) -> None:
@@ -140,6 +153,7 @@ class PackedLinear(nn.Module):
         self.register_buffer("_dense_weight", None, persistent=False)
         grid = _Grid.of(parameters["values"])
         self.uniform_grid, self.grid_minimum, self.grid_step = grid.uniform, grid.minimum, grid.step
+        self.values_held = _values_held(parameters["values"])
         self.layout: PackedLayout | None = layout_for(self.code_bits, self.in_features, self.group)
         self.maximum_fused_rows = MAXIMUM_FUSED_ROWS if self.layout is not None else 0
         self.maximum_product_rows = self._product_rows()
@@ -158,7 +172,10 @@ class PackedLinear(nn.Module):
                  and self.scales.dtype in (torch.float16, torch.bfloat16) and self.packed.data_ptr() % 16 == 0)
         if not taken:
             return 0
-        return MAXIMUM_PRODUCT_ROWS_SMALL if width * self.out_features <= SMALL_WEIGHTS else MAXIMUM_PRODUCT_ROWS
+        if width * self.out_features <= SMALL_WEIGHTS:
+            return MAXIMUM_PRODUCT_ROWS_SMALL
+        on_table = bits in (2, 3) or not self.uniform_grid
+        return MAXIMUM_PRODUCT_ROWS_SPLIT if on_table and not self.values_held else MAXIMUM_PRODUCT_ROWS
 
     # -- online input rotation ---------------------------------------------------------------
 
@@ -302,7 +319,7 @@ class PackedLinear(nn.Module):
             scale_code, bias_code = native.dtype_code(scales), 0 if bias is None else native.dtype_code(bias)
             constants = (self.out_features, self.in_features, self.group, self.code_bits, int(self.uniform_grid),
                          self.grid_minimum, self.grid_step)
-            layer = native.PackedLayer(*key[:5], scale_code, values.numel(), bias_code, *constants)
+            layer = native.PackedLayer(*key[:5], scale_code, values.numel(), bias_code, *constants, int(self.values_held))
             launch = self._launch = (
                 key,
                 (key[0], key[1], scale_code, key[2], values.numel(), native.pointer(zeros), native.pointer(bias), bias_code),

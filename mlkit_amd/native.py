@@ -32,7 +32,7 @@ class PackedLayer(ctypes.Structure):
 
     _fields_ = [(name, _c_void_p) for name in ("packed", "scales", "values", "zeros", "bias")] + [
         (name, _c_int) for name in ("scale_dtype", "n_values", "bias_dtype", "output_width", "input_width", "group", "bits",
-                                    "uniform")] + [("grid_min", _c_float), ("grid_step", _c_float)]
+                                    "uniform")] + [("grid_min", _c_float), ("grid_step", _c_float), ("values_held", _c_int)]
 
 
 # name -> (restype, argtypes); mirrors include/mlkit_amd.h declaration by declaration.

@@ -18,7 +18,7 @@ SEVEN = np.array([-1, -0.5, -0.25, 0, 0.25, 0.5, 1], dtype=F32)
 CODECS = {"int4": (INT4, 4, True), "nf4": (scaling.NF4_VALUES, 4, False), "seven": (SEVEN, 3, False),
           "int3": (scaling.int_values(3), 3, True), "int2": (scaling.int_values(2), 2, True),
           "int8": (scaling.int_values(8), 8, True)}
-# An output is rounded once to x's type (2^-12 / 2^-9 of it); table values are rounded to that type too.
+# An output is rounded once to x's type (2^-12 / 2^-9 of it).
 RANGE_TOLERANCE = {torch.float16: 1e-3, torch.bfloat16: 8e-3}
 
 
@@ -93,6 +93,52 @@ def test_bf16_scales_and_activations_with_a_common_offset():
     for dtype in (torch.float16, torch.bfloat16):
         x = (helpers.activations(20, 1024, seed=1, dtype=torch.float32) + 3).to(dtype).cuda()
         check(run(layer, x, scale_dtype=torch.bfloat16), layer, x)
+
+
+WIDE = np.array([-1, -0.3, -0.11, -0.03, -0.011, -0.003, -0.0011, 0, 0.0007, 0.0023, 0.007, 0.023, 0.07, 0.23, 0.7, 1], dtype=F32)
+FITTED3 = np.array([-1, -0.61, -0.33, -0.1, 0.1, 0.33, 0.61, 0.97], dtype=F32)
+
+
+@pytest.mark.parametrize("values,bits,group,asym", [
+    (scaling.NF4_VALUES, 4, 64, False), (scaling.NF4_VALUES, 4, 128, True), (WIDE, 4, 128, False),
+    (scaling.NF4_VALUES * F32(2.0e-6), 4, 64, False), (scaling.NF4_VALUES * F32(3.0e6), 4, 2048, False),   # past fp16's range
+    (FITTED3, 3, 64, False), (FITTED3, 3, 128, True), (np.array([-1, -0.31, 0.31, 1], dtype=F32), 2, 64, False),
+])
+@pytest.mark.parametrize("samples", [9, 40])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_activations_with_a_mean_on_values_their_type_does_not_hold(values, bits, group, asym, samples, dtype):
+    """Weights of one code share the error of its value, which activations of one sign add up: with both parts of a value
+    (2^-17 of it and better) nothing but the rounding of an output remains, half a unit of at most 2^-8 / 2^-11 of it; an
+    eighth of that is left for the sums."""
+    layer = helpers.quantised_layer(helpers.normal_weight(64, 4096, seed=bits), values, bits=bits, group=group, integer=False, asym=asym)
+    x = torch.relu(helpers.activations(samples, 4096, seed=samples, dtype=torch.float32)).to(dtype).cuda()
+    y = run(layer, x).double().cpu().numpy()
+    expected = x.double().cpu().numpy() @ layer["dense"].astype(np.float64).T
+    half_unit = 2.0**-9 if dtype == torch.bfloat16 else 2.0**-12
+    assert np.linalg.norm(y - expected) <= 1.125 * half_unit * np.linalg.norm(expected)
+
+
+@pytest.mark.parametrize("name,held", [("nf4", False), ("seven", True), ("int3", True), ("int2", True)])
+def test_a_wrong_statement_about_a_table_costs_time_and_not_digits(name, held):
+    """`values_held` chooses the kernel with one operand a value; over a table that needs two, it works its outputs out
+    by their definition."""
+    import mlkit_amd as mk
+
+    values, bits, _ = CODECS[name]
+    linear = torch.nn.Linear(640, 70, bias=False, device="cuda", dtype=torch.bfloat16)
+    layer = mk.PackedLinear(linear, mk.scaled(mk.grid.values(values.tolist(), bits=bits), group=64)(linear.weight.detach()))
+    assert layer.values_held is held
+    x = torch.relu(torch.randn((33, 640), device="cuda")).bfloat16()
+    dense = torch.empty((70, 640), device="cuda")
+    layer.storage_dtype = torch.float32
+    dense.copy_(layer.weight)
+    expected = (x.double() @ dense.double().T)
+    for stated in (True, False):
+        layer.values_held = stated
+        layer._launch = None
+        with torch.no_grad():
+            y = layer._product(x, 33)
+        assert (y.double() - expected).norm() <= 1.125 * 2.0**-9 * expected.norm()
 
 
 def test_refuses_what_it_does_not_take():
