@@ -16,8 +16,9 @@ codewords, the E8P lattice) with ``step`` equal to their dimension run the same 
 """
 
 import math
+import threading
 from collections.abc import Callable
-from typing import Any
+from typing import Any, TypeVar
 
 import torch
 from torch import Tensor
@@ -153,13 +154,19 @@ def _factor_scratch(width: int, device: torch.device) -> Tensor:
                        device=device)
 
 
+_Read = TypeVar("_Read")
+
+
 class _FactorGraph:
     """The launches of ``_factor_in_place`` for one width, captured once: several hundred small
     launches cost more to issue from Python than to run, and they are the same for every matrix
-    of that width.  The graph owns the buffer it factors in."""
+    of that width.  The graph owns the buffer it factors in, and one caller at a time has it: from the
+    matrix it fills in to the launches that read the factor.  Callers on other streams wait for those."""
 
     def __init__(self, width: int, device: torch.device, pairs: bool) -> None:
-        self.pairs = pairs
+        self.pairs, self.device = pairs, device
+        self.lock = threading.Lock()
+        self.read: torch.cuda.Event | None = None   # behind the last caller's reads of the factor
         self.matrix = torch.empty((width, width), dtype=torch.float32, device=device)
         self.status = torch.zeros((), dtype=torch.int32, device=device)
         self.factored = _factor_scratch(width, device)
@@ -183,7 +190,7 @@ class _FactorGraph:
 
     def _captured(self) -> "torch.cuda.CUDAGraph":
         graph = torch.cuda.CUDAGraph()
-        graph.capture_begin()
+        graph.capture_begin(capture_error_mode="thread_local")   # (other threads may go on allocating)
         try:
             self.status.zero_()   # a fill kernel
             _factor_in_place(self.matrix, self.status, self.factored, self.pairs)
@@ -191,46 +198,65 @@ class _FactorGraph:
             graph.capture_end()
         return graph
 
-    def __call__(self, fill: Callable[[Tensor], None]) -> tuple[Tensor, Tensor]:
-        fill(self.matrix)
-        self.graph.replay()
-        return self.matrix, self.status
+    def __call__(self, fill: Callable[[Tensor], None], read: "Callable[[Tensor, int], _Read]") -> "_Read":
+        with self.lock:
+            stream = torch.cuda.current_stream(self.device)
+            if self.read is not None:
+                stream.wait_event(self.read)
+            fill(self.matrix)
+            self.graph.replay()
+            try:
+                return read(self.matrix, int(self.status.item()))
+            finally:
+                self.matrix.record_stream(stream)   # (a graph may be dropped while its factor is being read)
+                self.read = stream.record_event()
 
 
 FACTOR_GRAPHS = True        # capture the factorisation of a width the second time it is asked for
+FACTOR_GRAPH_WIDTH = 1024   # from here on: 896 columns take 414 us from a graph, 420 launch by launch
 FACTOR_GRAPH_LIMIT = 2      # graphs (and their width x width buffers) kept per process
 _factor_graphs: dict[tuple, "_FactorGraph | None"] = {}   # by device and width
+_factor_graphs_lock = threading.Lock()
 
 
 def clear_factor_graphs() -> None:
     """Drop the captured factorisations and their buffers (up to FACTOR_GRAPH_LIMIT graphs, each holding a
     width x width fp32 matrix plus scratch: about 0.5 GB at 11008 columns).  ``mk.quantize`` calls this at
     the end of a pass; callers that drive ``mk.gptq`` layer by layer themselves call it when they are done."""
-    _factor_graphs.clear()
+    with _factor_graphs_lock:
+        _factor_graphs.clear()
 
 
-def _blocked_upper_factor(fill: Callable[[Tensor], None], width: int, device: torch.device, pairs: bool) -> tuple[Tensor, Tensor]:
-    """``(U, status)`` with ``U^T U`` = the matrix that ``fill(target)`` writes into a
-    ``[width, width]`` FP32 tensor.  The first matrix of a width is factored launch by launch
-    (which also warms every kernel up); from the second on the captured graph of that width
-    runs.  The result may live in the graph's own buffer: it is valid until the next call."""
+def _factor_graph(width: int, device: torch.device, pairs: bool) -> "_FactorGraph | None":
+    """The captured factorisation of a width, from the second matrix on (the first one warms every kernel up)."""
+    if not FACTOR_GRAPHS or width < FACTOR_GRAPH_WIDTH or torch.cuda.is_current_stream_capturing():
+        return None
     key = (torch.cuda.current_device() if device.index is None else device.index, width) + (("pairs",) if pairs else ())
-    if FACTOR_GRAPHS and key in _factor_graphs and not torch.cuda.is_current_stream_capturing():
+    with _factor_graphs_lock:
+        if key not in _factor_graphs:
+            _factor_graphs[key] = None   # seen once
+            return None
         graph = _factor_graphs[key]
         if graph is None:
             while sum(entry is not None for entry in _factor_graphs.values()) >= FACTOR_GRAPH_LIMIT:
                 oldest = next(k for k, entry in _factor_graphs.items() if entry is not None)
                 del _factor_graphs[oldest]
             graph = _factor_graphs[key] = _FactorGraph(width, device, pairs)
-        return graph(fill)
-    _factor_graphs.setdefault(key, None)   # seen once
+        return graph
+
+
+def _with_upper_factor(fill: Callable[[Tensor], None], read: "Callable[[Tensor, int], _Read]", width: int,
+                       device: torch.device, pairs: bool) -> "_Read":
+    """``read(U, status)`` with ``U^T U`` = the matrix that ``fill(target)`` writes into a ``[width, width]`` FP32
+    tensor.  The factor may live in a graph's own buffer: it is ``read``'s only until that returns."""
+    graph = _factor_graph(width, device, pairs)
+    if graph is not None:
+        return graph(fill, read)
     matrix = torch.empty((width, width), dtype=torch.float32, device=device)
     fill(matrix)
     status = torch.zeros((), dtype=torch.int32, device=device)
     _factor_in_place(matrix, status, _factor_scratch(width, device), pairs)
-    return matrix, status
-
-
+    return read(matrix, int(status.item()))
 
 
 def feedback_coefficients(hessian: Tensor, step: int, *, damp: float = 0.01,
@@ -259,7 +285,7 @@ def feedback_coefficients(hessian: Tensor, step: int, *, damp: float = 0.01,
         lower = factor.T
     else:
         lower, status = torch.linalg.cholesky_ex(flipped)
-    return _coefficients_of(lower, status, step)
+    return _coefficients_of(lower, int(status.item()), step)
 
 
 def _coefficients_on_kernels(hessian: Tensor, step: int, damp: float, permutation: Tensor | None) -> tuple[Tensor, int]:
@@ -281,20 +307,22 @@ def _coefficients_on_kernels(hessian: Tensor, step: int, damp: float, permutatio
         native.check(library.mk_hessian_reversed(source.data_ptr(), target.data_ptr(), width, native.pointer(order),
                                                  addend.data_ptr(), native.current_stream(device)))
 
-    factor, status = _blocked_upper_factor(fill, width, device, pairs=step > 1)
-    if step == 1 and int(status.item()) == 0:
+    def read(factor: Tensor, status: int) -> tuple[Tensor, int]:
+        if step != 1 or status != 0:
+            return _coefficients_of(factor.T, status, step)
         coefficients = torch.empty_like(factor)
         native.check(library.mk_unit_upper_from_factor(factor.data_ptr(), coefficients.data_ptr(), width,
                                                        native.current_stream(device)))
         return coefficients, 0
-    return _coefficients_of(factor.T, status, step)
+
+    return _with_upper_factor(fill, read, width, device, pairs=step > 1)
 
 
-def _coefficients_of(lower: Tensor, status: Tensor, step: int) -> tuple[Tensor, int]:
+def _coefficients_of(lower: Tensor, status: int, step: int) -> tuple[Tensor, int]:
     """``R blockdiag(R)^-1`` from the lower factor of the index-reversed matrix."""
     width = lower.shape[0]
-    if int(status.item()) != 0:
-        return lower.clone(), int(status.item())
+    if status != 0:
+        return lower.clone(), status
     if step == 1:
         lower = lower / lower.diagonal().clone()
         return lower.flip(0, 1).contiguous(), 0

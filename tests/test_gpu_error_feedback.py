@@ -308,6 +308,48 @@ def test_captured_factorisation_equals_the_launch_by_launch_one(look_ahead, monk
         feedback.clear_factor_graphs()
 
 
+@pytest.mark.parametrize("width,step", [(384, 1), (1152, 1), (1152, 8)])
+def test_coefficients_from_several_threads(width, step):
+    """Threads with streams of their own and matrices of one width, with another width in between (which may drop the
+    width's graph): everyone receives the coefficients that one thread alone works out, bit for bit."""
+    import threading
+
+    import mlkit_amd as mk
+    from mlkit_amd.quantization import feedback
+
+    generator = torch.Generator(device="cuda").manual_seed(width + step)
+
+    def hessian_of(columns):
+        inputs = torch.randn((2 * columns, columns), device="cuda", generator=generator)
+        return inputs.T @ inputs / inputs.shape[0]
+
+    matrices = [[hessian_of(width), hessian_of(width), hessian_of(width + 128)] for _ in range(3)]
+    expected = [[mk.feedback_coefficients(matrix.clone(), step)[0] for matrix in some] for some in matrices]
+    torch.cuda.synchronize()
+    feedback.clear_factor_graphs()
+    wrong, failures = [], []
+
+    def work(index):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                for turn in range(6):
+                    for matrix, right in zip(matrices[index], expected[index]):
+                        result, status = mk.feedback_coefficients(matrix.clone(), step)
+                        torch.cuda.current_stream().synchronize()
+                        if status != 0 or not torch.equal(result.triu(step), right.triu(step)):
+                            wrong.append((index, turn, matrix.shape[0]))
+        except Exception as error:   # reported by the main thread
+            failures.append(repr(error))
+
+    threads = [threading.Thread(target=work, args=(index,)) for index in range(3)]
+    for thread in threads:
+        thread.start()
+    for thread in threads:
+        thread.join(timeout=60)
+    feedback.clear_factor_graphs()
+    assert not failures and not wrong, (failures, wrong)
+
+
 def test_blocked_factorisation_reports_an_indefinite_matrix():
     import mlkit_amd as mk
 

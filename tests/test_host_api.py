@@ -441,3 +441,42 @@ def test_copies_of_an_online_rotation_prepare_their_own_plans():
     for other in (copy.deepcopy(rotation), pickle.loads(pickle.dumps(rotation))):
         assert (other.seed, other.block) == (5, 2048) and not other._plans
         assert torch.equal(other(value), expected)
+
+
+def test_a_captured_factorisation_serves_one_caller_at_a_time(monkeypatch):
+    """Reading the status lets other threads run: none of them may fill the graph's matrix before the factor in it has been
+    read, and each caller's stream waits for the reads of the one before."""
+    import threading
+    import time
+    from types import SimpleNamespace
+
+    from mlkit_amd.quantization import feedback
+
+    waited, recorded = [], []
+
+    def record():
+        recorded.append(object())
+        return recorded[-1]
+
+    def status():
+        time.sleep(0.005)
+        return 0
+
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: SimpleNamespace(wait_event=waited.append, record_event=record))
+    graph = feedback._FactorGraph.__new__(feedback._FactorGraph)
+    graph.lock, graph.read, graph.device = threading.Lock(), None, None
+    graph.matrix = SimpleNamespace(holder=None, record_stream=lambda stream: None)
+    graph.graph, graph.status = SimpleNamespace(replay=lambda: None), SimpleNamespace(item=status)
+    seen = []
+
+    def caller(name):
+        for _ in range(5):
+            seen.append((name, graph(lambda matrix: setattr(matrix, "holder", name), lambda matrix, failed: matrix.holder)))
+
+    threads = [threading.Thread(target=caller, args=(name,)) for name in "abc"]
+    for thread in threads:
+        thread.start()
+    for thread in threads:
+        thread.join()
+    assert len(seen) == 15 and all(name == held for name, held in seen)
+    assert waited == recorded[:-1]
