@@ -264,7 +264,7 @@ class PackedLinear(nn.Module):
             else:
                 inputs = self._rotation(inputs)   # the general path: rotate, then as an unrotated layer
         if not fused:
-            if (MAXIMUM_FUSED_ROWS < rows <= self.maximum_product_rows and not compiling and self._dense_weight is None
+            if (MAXIMUM_FUSED_ROWS < rows <= self.maximum_product_rows and not compiling and not self.cache_dense
                     and inputs.dtype in PRODUCT_DTYPES and self._plain_call(inputs)):
                 product = self._product(inputs, rows)
                 if product is not None:

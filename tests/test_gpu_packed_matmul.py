@@ -260,3 +260,23 @@ def test_calls_that_are_recorded_batched_differentiated_or_cast_take_the_dense_p
     assert wanted.grad is not None
     with pytest.raises(RuntimeError):
         layer(x.bfloat16())   # a bias of another type: refused, as the dense product refuses it
+
+
+@pytest.mark.parametrize("cache_dense", [False, True])
+def test_a_call_does_not_depend_on_the_calls_before_it(cache_dense):
+    """A cached dense weight is asked for once and for all: from the first call of more than eight rows on it is there and
+    used; without it, a longer call or a look at the weight changes nothing."""
+    import mlkit_amd as mk
+
+    linear = torch.nn.Linear(512, 320, device="cuda", dtype=torch.bfloat16)
+    quantized = mk.int(4, 128, asym=True)(linear.weight.detach())
+    layer = mk.PackedLinear(linear, quantized, cache_dense=cache_dense)
+    x, longer = torch.randn((32, 512), device="cuda").bfloat16(), torch.randn((300, 512), device="cuda").bfloat16()
+    with torch.no_grad():
+        first = layer(x)
+        assert (layer._dense_weight is not None) is cache_dense
+        if cache_dense:
+            assert torch.equal(first, torch.nn.functional.linear(x, layer.weight, layer.bias))
+        layer(longer)
+        layer.weight
+        assert torch.equal(layer(x), first)
