@@ -115,7 +115,9 @@ class PackedLinear(nn.Module):
     zeros: Tensor | None
     bias: Tensor | None
     _dense_weight: Tensor | None
-    values_held = False   # (layers pickled without it)
+    # (of layers pickled without them: the dense product serves more than eight rows)
+    values_held = False
+    maximum_product_rows = 0
 
     def __init__(self, original: nn.Linear, quantized: Q, *, cache_dense: bool = False,
                  overflow: Tensor | None = None) -> None:

@@ -280,3 +280,18 @@ def test_a_call_does_not_depend_on_the_calls_before_it(cache_dense):
         layer(longer)
         layer.weight
         assert torch.equal(layer(x), first)
+
+
+def test_a_layer_pickled_before_the_product_existed():
+    import mlkit_amd as mk
+
+    linear = torch.nn.Linear(512, 320, device="cuda", dtype=torch.bfloat16)
+    layer = mk.PackedLinear(linear, mk.nf4(64)(linear.weight.detach()))
+    state = layer.__getstate__()
+    del state["maximum_product_rows"], state["values_held"]
+    older = mk.PackedLinear.__new__(mk.PackedLinear)
+    older.__setstate__(state)
+    for rows in (3, 20):
+        x = torch.randn((rows, 512), device="cuda").bfloat16()
+        with torch.no_grad():
+            assert torch.allclose(older(x).float(), layer(x).float(), rtol=2e-2, atol=2e-2)
