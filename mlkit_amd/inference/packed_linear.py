@@ -27,6 +27,7 @@ from dataclasses import dataclass
 import torch
 import torch.nn.functional as functional
 from torch import Tensor, nn
+from torch.utils._device import DeviceContext
 
 from mlkit_amd import native
 from mlkit_amd.kernels.packed_linear import (MAXIMUM_CODE_BITS, GroupLaunch, PackedLayout, decode, layout_for,
@@ -45,6 +46,19 @@ MAXIMUM_FUSED_ROWS = 8
 MAXIMUM_PRODUCT_ROWS, MAXIMUM_PRODUCT_ROWS_SPLIT, MAXIMUM_PRODUCT_ROWS_SMALL, SMALL_WEIGHTS = 128, 64, 256, 1 << 24
 PRODUCT_DTYPES = frozenset({torch.float16, torch.bfloat16})
 _LAUNCH_BUFFERS = frozenset({"packed", "scales", "values", "zeros", "bias"})
+
+
+def _unobserved() -> bool:
+    """Whether no tracing, function transform, forward-mode level or dispatch / function mode would see a torch call made
+    here.  (A default device is a function mode too, but one that only looks at factory functions.)"""
+    try:
+        return (torch._C._get_tracing_state() is None
+                and torch._C._functorch.peek_interpreter_stack() is None   # vmap, functional gradients
+                and torch.autograd.forward_ad._current_level < 0 and torch._C._len_torch_dispatch_stack() == 0
+                and (torch._C._len_torch_function_stack() == 0
+                     or all(type(mode) is DeviceContext for mode in torch.overrides._get_current_function_mode_stack())))
+    except AttributeError:   # a torch that keeps one of these elsewhere: let torch make the call
+        return False
 
 
 def preserve_input_processing(original: nn.Module, replacement: nn.Module) -> None:
@@ -352,15 +366,13 @@ class PackedLinear(nn.Module):
         return None if bound[1] is None else bound
 
     def _plain_call(self, inputs: Tensor) -> bool:
-        """Whether a library call may stand for ``functional.linear``: nothing differentiates, batches, records or casts
-        what this call does, and the dense product would take these types and devices."""
+        """Whether a library call may stand for ``functional.linear``: nothing differentiates, batches, records, watches or
+        casts what this call does, and the dense product would take these types and devices."""
         bias = self._buffers["bias"]
         return (type(inputs) is Tensor and inputs.device == self._buffers["packed"].device
                 and (bias is None or bias.dtype == inputs.dtype)
                 and not (inputs.requires_grad and torch.is_grad_enabled())
-                and not torch.is_autocast_enabled("cuda") and torch._C._get_tracing_state() is None
-                and torch._C._functorch.peek_interpreter_stack() is None   # vmap, functional gradients
-                and torch.autograd.forward_ad._current_level < 0 and torch._C._len_torch_dispatch_stack() == 0)
+                and not torch.is_autocast_enabled("cuda") and _unobserved())
 
     def _product(self, inputs: Tensor, rows: int) -> Tensor | None:
         """More rows than a matvec on the codes; None when the library refuses the call (a buffer that was moved

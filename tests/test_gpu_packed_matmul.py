@@ -295,3 +295,29 @@ def test_a_layer_pickled_before_the_product_existed():
         x = torch.randn((rows, 512), device="cuda").bfloat16()
         with torch.no_grad():
             assert torch.allclose(older(x).float(), layer(x).float(), rtol=2e-2, atol=2e-2)
+
+
+def test_a_function_mode_sees_the_dense_product():
+    """A mode that watches torch calls (a counter of operations, say) is shown `linear`, as before there was a product on
+    the codes; a default device watches nothing and changes nothing."""
+    from torch.overrides import TorchFunctionMode
+
+    import mlkit_amd as mk
+
+    class Watch(TorchFunctionMode):
+        def __torch_function__(self, function, types, args=(), kwargs=None):
+            seen.append(function)
+            return function(*args, **(kwargs or {}))
+
+    linear = torch.nn.Linear(512, 320, device="cuda", dtype=torch.bfloat16)
+    layer = mk.PackedLinear(linear, mk.int(4, 128)(linear.weight.detach()))
+    x = torch.randn((32, 512), device="cuda").bfloat16()
+    seen = []
+    with torch.no_grad():
+        on_codes = layer(x)
+        with Watch():
+            watched = layer(x)
+        assert torch.nn.functional.linear in seen or torch._C._nn.linear in seen
+        assert torch.equal(watched, torch.nn.functional.linear(x, layer.weight, layer.bias))
+        with torch.device("cuda"):
+            assert torch.equal(layer(x), on_codes)
