@@ -380,8 +380,9 @@ class PackedLinear(nn.Module):
         if not inputs.is_contiguous():
             inputs = inputs.contiguous()
         output = inputs.new_empty(inputs.shape[:-1] + (self.out_features,))
+        launch = self._bound_arguments()   # (held during the call: another thread may bind anew)
         status = native.library().mk_packed_layer_matmul(
-            self._bound_arguments()[3], inputs.data_ptr(), native.DTYPE_CODES[inputs.dtype], output.data_ptr(), rows,
+            launch[3], inputs.data_ptr(), native.DTYPE_CODES[inputs.dtype], output.data_ptr(), rows,
             native.current_stream(inputs.device))
         if status == native.MK_ERR_UNSUPPORTED:
             return None
@@ -391,7 +392,8 @@ class PackedLinear(nn.Module):
 
     def _matvec(self, inputs: Tensor, output: Tensor, rows: int, rotate: bool = False) -> None:
         """One call into the C ABI on the current stream."""
-        _, tensors, constants, layer, _ = self._bound_arguments()
+        launch = self._bound_arguments()   # (held during the call: another thread may bind anew)
+        tensors, constants, layer = launch[1:4]
         stream = native.current_stream(inputs.device)
         code = native.DTYPE_CODES[inputs.dtype]
         if rotate:

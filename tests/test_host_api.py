@@ -480,3 +480,37 @@ def test_a_captured_factorisation_serves_one_caller_at_a_time(monkeypatch):
         thread.join()
     assert len(seen) == 15 and all(name == held for name, held in seen)
     assert waited == recorded[:-1]
+
+
+def test_a_packed_call_holds_its_bound_arguments(monkeypatch):
+    """The library reads a structure whose address the call passes: it stays alive until the call returns, also when
+    another thread drops the layer's binding meanwhile."""
+    import gc
+    import weakref
+    from types import SimpleNamespace
+
+    from mlkit_amd import native
+    from mlkit_amd.inference.packed_linear import PackedLinear
+
+    layer = PackedLinear.__new__(PackedLinear)
+    torch.nn.Module.__init__(layer)
+    for name, value in (("packed", torch.zeros(64, dtype=torch.uint8)), ("scales", torch.ones(4, 1, dtype=torch.float16)),
+                        ("values", torch.arange(16.0)), ("zeros", None), ("bias", None)):
+        layer.register_buffer(name, value)
+    layer.out_features, layer.in_features, layer.group, layer.code_bits = 4, 32, 32, 4
+    layer.uniform_grid, layer.grid_minimum, layer.grid_step, layer._launch = True, 0.0, 1.0, None
+    alive = []
+
+    def called(*arguments):
+        structure = weakref.ref(layer._launch[4])
+        layer._launch = None
+        gc.collect()
+        alive.append(structure() is not None)
+        return 0
+
+    monkeypatch.setattr(native, "library", lambda: SimpleNamespace(mk_packed_layer_matmul=called, mk_packed_layer_matvec=called))
+    monkeypatch.setattr(native, "current_stream", lambda device: 0)
+    x = torch.zeros((12, 32), dtype=torch.float16)
+    layer._product(x, 12)
+    layer._matvec(x[:2], torch.empty((2, 4), dtype=torch.float16), 2)
+    assert alive == [True, True]
