@@ -152,7 +152,7 @@ def decode_basis(codes: Tensor, *, inner_codec: str, shape: "tuple[int, int] | l
                  **parameters: Any) -> Tensor:
     """Codes of a matrix quantized in a rotated basis: the inner decoder's reconstruction is
     rotated back, input side (columns) first, then output side (rows)."""
-    from mlkit_amd.quantization.transforms import rotate, rotate_columns
+    from mlkit_amd.quantization.transforms import rotate, rotate_columns_in_type
 
     inner = {key.removeprefix("inner_"): value for key, value in parameters.items()}
     restored = decoder(inner_codec)(codes, **inner)
@@ -161,7 +161,7 @@ def decode_basis(codes: Tensor, *, inner_codec: str, shape: "tuple[int, int] | l
         restored = rotate(restored, inverse=True, signs=signs)
     if left_seed is not None:
         signs = left_signs if left_signs is not None else deterministic_signs(shape[0], left_seed, codes.device)
-        restored = rotate_columns(restored, inverse=True, signs=signs)
+        restored = rotate_columns_in_type(restored, inverse=True, signs=signs)
     return restored
 
 

@@ -20,7 +20,7 @@ from torch import Tensor
 
 from mlkit_amd.quantization.codecs import compose, deterministic_signs, registered
 from mlkit_amd.quantization.core import Ctx, Q, Quantizer, as_q, layer_seed
-from mlkit_amd.quantization.transforms import rotate, rotate_columns
+from mlkit_amd.quantization.transforms import columns_on_kernel, rotate, rotate_columns, rotate_columns_in_type
 
 SIDE_KINDS = (None, "rht")
 
@@ -38,7 +38,7 @@ class _Side:
 
     def along_rows(self, matrix: Tensor, back: bool = False) -> Tensor:
         """``(T diag(signs)) @ matrix`` (every column transformed), or its inverse."""
-        return rotate_columns(matrix, inverse=back, signs=self.signs)
+        return rotate_columns_in_type(matrix, inverse=back, signs=self.signs)
 
     def conjugate(self, symmetric: Tensor) -> Tensor:
         """``(T S) M (T S)^T`` for a square matrix over this side's width."""
@@ -84,10 +84,12 @@ class Incoherent(Quantizer):
         output_side = _Side(rows, base_seed, w.device) if self.left else None
         input_side = _Side(columns, base_seed + 1, w.device) if self.right else None
 
-        # (16-bit weights on a HIP device are converted by the first transform)
-        in_basis = w.float() if output_side is None or not w.is_cuda or w.requires_grad else w
-        if output_side is not None:
-            in_basis = output_side.along_rows(in_basis)
+        if output_side is None:
+            in_basis = w.float()
+        elif columns_on_kernel(w, output_side.signs):   # (16-bit weights are converted by the transform)
+            in_basis = rotate_columns(w, signs=output_side.signs)
+        else:
+            in_basis = output_side.along_rows(w.float())
         if input_side is not None:
             in_basis = input_side.along_columns(in_basis)
         inner_ctx = ctx.replace() if input_side is None else ctx.derive(_statistics_in(input_side, ctx, w.device))

@@ -180,12 +180,17 @@ def rotate(value: Tensor, *, inverse: bool = False, signs: Tensor | None = None,
 COLUMN_KERNEL_ROWS = frozenset({1024, 2048, 4096})   # columns that one workgroup transforms without turning the matrix
 
 
+def columns_on_kernel(matrix: Tensor, signs: Tensor) -> bool:
+    """Whether ``rotate_columns`` transforms this matrix in kernels, from its own type to FP32."""
+    return (matrix.is_cuda and matrix.dim() == 2 and matrix.numel() > 0 and matrix.dtype in _KERNEL_DTYPES
+            and not (torch.is_grad_enabled() and (matrix.requires_grad or signs.requires_grad))
+            and matrix.shape[0] <= MAXIMUM_KERNEL_WIDTH)
+
+
 def rotate_columns(matrix: Tensor, *, signs: Tensor, inverse: bool = False) -> Tensor:
     """``rotate(matrix.T).T``: every column of a matrix transformed, FP32 on a HIP device.  Columns of 1024 to 4096 values
     (powers of two) take one kernel; others are turned, rotated as rows and turned back, 16-bit ones converted on the way."""
-    if not (matrix.is_cuda and matrix.dim() == 2 and matrix.numel() and matrix.dtype in _KERNEL_DTYPES
-            and not (torch.is_grad_enabled() and (matrix.requires_grad or signs.requires_grad))
-            and matrix.shape[0] <= MAXIMUM_KERNEL_WIDTH):
+    if not columns_on_kernel(matrix, signs):
         return rotate(matrix.T.contiguous(), inverse=inverse, signs=signs).T
     from mlkit_amd.kernels import hadamard as kernel
 
@@ -194,6 +199,16 @@ def rotate_columns(matrix: Tensor, *, signs: Tensor, inverse: bool = False) -> T
         signs = signs.to(device=matrix.device, dtype=torch.float32).contiguous()
         return kernel.transform_columns(matrix, signs_before=None if inverse else signs, signs_after=signs if inverse else None)
     return kernel.turned(rotate(kernel.turned(matrix), inverse=inverse, signs=signs))
+
+
+def rotate_columns_in_type(matrix: Tensor, *, signs: Tensor, inverse: bool = False) -> Tensor:
+    """The same with the result ``rotate(matrix.T).T`` has for a 16-bit matrix: one of its type where the row kernels take
+    its columns, and whatever the stages in tensor operations make of it where they do not."""
+    if matrix.dtype not in (torch.float16, torch.bfloat16) or not columns_on_kernel(matrix, signs):
+        return rotate_columns(matrix, signs=signs, inverse=inverse)
+    if transform_factor(matrix.shape[0])[0] > MAXIMUM_KERNEL_ORDER:
+        return rotate(matrix.T.contiguous(), inverse=inverse, signs=signs).T
+    return rotate_columns(matrix, signs=signs, inverse=inverse).to(matrix.dtype)
 
 
 def _structured_on_host(value: Tensor, order: int, power: int, basis: Tensor | None, inverse: bool) -> Tensor:

@@ -319,6 +319,32 @@ def test_columns_and_rows_run_their_stages_in_one_order(rows, dtype):
         assert torch.equal(device_transforms.rotate_columns(matrix, signs=signs, inverse=inverse), expected)
 
 
+@pytest.mark.parametrize("rows", [64, 1024, 4099, 33000])   # 33000: past the row kernels, in tensor operations
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32, torch.float64])
+def test_a_rotated_basis_is_entered_in_fp32(rows, dtype):
+    """Whatever type a weight has, the inner quantizer sees the rotation of its fp32 numbers, and a reconstruction that
+    comes back in 16 bits leaves the basis as the turned matrix would."""
+    import mlkit_amd as mk
+    from mlkit_amd.quantization import transforms as device_transforms
+    from mlkit_amd.quantization.codecs import deterministic_signs
+    from mlkit_amd.quantization.core import layer_seed
+
+    weight = torch.randn((rows, 24), device="cuda").to(dtype)
+    entered = []
+
+    def inner(value, ctx):
+        entered.append(value)
+        return mk.Q(value.half(), bits=1)
+
+    ctx = mk.Ctx("layer", device="cuda")
+    left = mk.incoherent(inner, right=None)(weight, ctx).w
+    signs = deterministic_signs(rows, layer_seed("layer", ctx._seed) % 2**32, weight.device)
+    expected = device_transforms.rotate(weight.float().T.contiguous(), signs=signs).T
+    assert entered[0].dtype == torch.float32 and torch.equal(entered[0], expected)
+    back = device_transforms.rotate(expected.half().T.contiguous(), inverse=True, signs=signs).T
+    assert left.dtype == back.dtype and torch.equal(left, back)
+
+
 @pytest.mark.parametrize("rows,columns", [(1, 1), (3, 70), (64, 64), (65, 4), (100, 132), (260, 68)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 def test_turning_a_matrix(rows, columns, dtype):
