@@ -147,7 +147,7 @@ void launch_rows(const ColumnArgs &a, int rows, hipStream_t stream) {
 struct TransposeArgs {
     const void *source;
     float *target;
-    int rows, columns;
+    int rows, columns, tiles_across;
 };
 
 // 64 x 64 tiles through LDS, fp32 4096 x 14336 in 98 us (4.8 TB/s; torch's strided copy 255), from bf16 in 84 (320 with its conversion); reads and writes both move whole 16-byte pieces along rows where the sizes allow it (VEC).
@@ -155,7 +155,7 @@ template <int SOURCE, bool VEC>
 __global__ void __launch_bounds__(256) transpose_kernel(const TransposeArgs a) {
     __shared__ float tile[64][65];
     const int tx = (threadIdx.x & 15) * 4, ty = threadIdx.x >> 4;
-    const int row0 = blockIdx.y * 64, column0 = blockIdx.x * 64;
+    const int row_tile = blockIdx.x / a.tiles_across, row0 = row_tile * 64, column0 = (blockIdx.x - row_tile * a.tiles_across) * 64;   // uniform
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const int local = ty + 16 * j, row = min(row0 + local, a.rows - 1);
@@ -197,7 +197,7 @@ __global__ void __launch_bounds__(256) transpose_kernel(const TransposeArgs a) {
 
 template <int SOURCE>
 void launch_transpose(const TransposeArgs &a, hipStream_t stream) {
-    const dim3 grid(mk_cdiv(a.columns, 64), mk_cdiv(a.rows, 64));
+    const dim3 grid(static_cast<unsigned>(a.tiles_across) * mk_cdiv(a.rows, 64));
     const bool whole = a.rows % 4 == 0 && a.columns % 4 == 0
                        && ((reinterpret_cast<uintptr_t>(a.source) | reinterpret_cast<uintptr_t>(a.target)) & 15u) == 0;
     if (whole) hipLaunchKernelGGL((transpose_kernel<SOURCE, true>), grid, dim3(256), 0, stream, a);
@@ -239,11 +239,11 @@ extern "C" int mk_fwht_columns(const void *source, int source_dtype, float *targ
 extern "C" int mk_transpose(const void *source, int source_dtype, float *target, int rows, int columns, void *stream_) {
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     MK_REQUIRE(rows >= 1 && columns >= 1, MK_ERR_INVALID, "mk_transpose: sizes must be positive");
-    MK_REQUIRE(mk_cdiv(rows, 64) <= 65535, MK_ERR_UNSUPPORTED, "mk_transpose: too many rows");
+    MK_REQUIRE((rows + 63ll) / 64 * ((columns + 63ll) / 64) < (1ll << 24), MK_ERR_UNSUPPORTED, "mk_transpose: too many tiles");
     MK_REQUIRE(source && target, MK_ERR_INVALID, "mk_transpose: null tensor pointer");
     MK_REQUIRE(source != target, MK_ERR_INVALID, "mk_transpose: source and target must not alias");
     MK_REQUIRE(mk_dtype_valid(source_dtype), MK_ERR_INVALID, "mk_transpose: unknown dtype code");
-    TransposeArgs a{source, target, rows, columns};
+    TransposeArgs a{source, target, rows, columns, mk_cdiv(columns, 64)};
     if (source_dtype == MK_F32) launch_transpose<MK_F32>(a, stream);
     else if (source_dtype == MK_F16) launch_transpose<MK_F16>(a, stream);
     else launch_transpose<MK_BF16>(a, stream);

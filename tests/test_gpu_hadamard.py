@@ -319,6 +319,17 @@ def test_columns_and_rows_run_their_stages_in_one_order(rows, dtype):
         assert torch.equal(device_transforms.rotate_columns(matrix, signs=signs, inverse=inverse), expected)
 
 
+@pytest.mark.parametrize("rows", [2, 3])
+def test_columns_of_a_very_wide_matrix(rows):
+    """More columns than a launch has workgroups in its second dimension (65535 tiles of 64)."""
+    from mlkit_amd.quantization import transforms as device_transforms
+
+    matrix = torch.randn((rows, 64 * 65536 + 1), device="cuda").half()
+    signs = torch.tensor([1.0, -1.0, 1.0][:rows], device="cuda")
+    expected = device_transforms.rotate(matrix.float().T.contiguous(), signs=signs).T
+    assert torch.equal(device_transforms.rotate_columns(matrix, signs=signs), expected)
+
+
 @pytest.mark.parametrize("rows", [64, 1024, 4099, 33000])   # 33000: past the row kernels, in tensor operations
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32, torch.float64])
 def test_a_rotated_basis_is_entered_in_fp32(rows, dtype):
