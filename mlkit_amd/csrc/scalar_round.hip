@@ -353,7 +353,8 @@ __global__ void __launch_bounds__(kThreads) round_groups_kernel(const RoundArgs 
 #pragma unroll
                     for (int i = 0; i < 8; ++i) squares = __builtin_fmaf(sample[t][i], sample[t][i], squares);
                 squares = over_team(squares);
-                const float bound = least + (0x1p-14f * least + (0x1p-17f * sqrtf(least * squares) + 0x1p-36f * squares));
+                // (two roots: the product of the sums leaves the normal range for scales below 2^-32 or so)
+                const float bound = least + (0x1p-14f * least + (0x1p-17f * (sqrtf(least) * sqrtf(squares)) + 0x1p-36f * squares));
                 unsigned long long open = 0;
                 for (int c = 0; c < a.n_fractions; ++c) open |= static_cast<unsigned long long>(estimates[c] <= bound) << c;
                 float best = __builtin_inff();
@@ -372,7 +373,7 @@ __global__ void __launch_bounds__(kThreads) round_groups_kernel(const RoundArgs 
                 }
                 __builtin_amdgcn_wave_barrier();   // the estimates have been read
             };
-            // (2^40: no square or product of the first pass leaves the normal range)
+            // (2^40: no square of the first pass leaves the normal range, nor 2^-36 of a sum of them)
             const bool moderate = kPruned && all_whole && __all(base_scale > 0x1p-40f && base_scale < 0x1p40f && ordinary_fractions);
             if constexpr (kPruned) {
                 if (moderate) {

@@ -284,6 +284,26 @@ def test_rounding_in_one_pass_reports_non_finite_weights(bad):
         mk.int(4, 64)(weight)
 
 
+@pytest.mark.parametrize("power", [-38, -33, 30, 38])
+@pytest.mark.parametrize("bits", [3, 8])
+def test_a_search_at_the_edges_of_the_estimates_range(power, bits):
+    """Scales of 2^-40 and 2^38 and so on, where a product of two sums of squares would leave the normal range: the scales
+    of the full search, bit for bit."""
+    from mlkit_amd.kernels import scalar_encode
+
+    values = scaling.int_values(bits)
+    weight = torch.from_numpy(helpers.normal_weight(512, 1024, seed=bits, scale=1.0)).cuda() * 2.0**power
+    weight[:64] = (weight[:64] * 2.0**-power * 64).round() / 128 * 2.0**power
+    options = dict(integer=True, minimum=float(values.min()), maximum=float(values.max()))
+    reciprocal = float(scaling.f32_reciprocal(float(np.abs(values).max())))
+    _, scales, _, _ = scalar_encode.round_matrix(weight, dev(values), dev(FRACTIONS), 64, asym=False, reciprocal=reciprocal,
+                                                 scale_format="fp32", **options)
+    fitted, _ = scalar_encode.fit_scales(weight, 64, asym=False, reciprocal=reciprocal, value_minimum=options["minimum"],
+                                         scale_format="fp32", store_zero=False)
+    expected = scalar_encode.search_scales(weight, fitted, None, dev(values), dev(FRACTIONS), 64, None, "fp32", **options)
+    assert torch.equal(scales, expected)
+
+
 @pytest.mark.parametrize("values,integer", [(SEVEN, False), (REPEATED, False), (INT3, True), (INT4, True),
                                             (np.array([-1.5, -0.5, 0.5, 1.5], dtype=F32), False),
                                             (np.array([0.25, 1.0], dtype=F32), False)])
