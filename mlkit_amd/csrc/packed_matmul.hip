@@ -43,6 +43,20 @@ MatmulPlan plan_for(int samples, int rows) {
     return plan;
 }
 
+// The next smaller tiles, where the scales of a plan's rows do not fit LDS (8192 x 28672 INT4 with offsets, 64 rows of x: 114 us
+// with 2 x 2 tiles, 209 straight to 1 x 1).  Where they fit but keep a second workgroup of 2 x 4 tiles off the compute unit
+// smaller tiles lose all the same (14336 x 4096 in groups of 64, 64 rows: 34 us, 48 with 2 x 2).
+void step_down(MatmulPlan &plan, int steps) {
+    if (plan.sample_tiles == 4) {
+        plan.sample_tiles = 2;
+        plan.waves = steps < mk_matmul::kMaxWaves ? steps : mk_matmul::kMaxWaves;
+    } else if (plan.row_tiles == 4 || plan.sample_tiles == 1) {
+        plan.row_tiles /= 2;
+    } else {
+        plan.sample_tiles = 1;
+    }
+}
+
 // Whether fp16 and bf16 hold every value of a grid, in the range the kernel brings them to.
 bool grid_held(float minimum, float step, int codes) {
     float largest = 0.0f;
@@ -109,7 +123,7 @@ int matmul(const void *x, int x_dtype, const uint8_t *packed, const void *scales
         const size_t sums = static_cast<size_t>(plan.waves) * plan.row_tiles * plan.sample_tiles * 1024;
         return (stage > sums ? stage : sums) + table + (64 + static_cast<size_t>(a.groups) * 64 * (a.need_sums ? 2 : 1)) * plan.row_tiles;
     };
-    while (lds() > 160 * 1024 && plan.row_tiles > 1) plan.row_tiles = plan.sample_tiles > 1 ? (plan.sample_tiles = plan.row_tiles = 1) : plan.row_tiles / 2;
+    while (lds() > 160 * 1024 && plan.row_tiles > 1) step_down(plan, a.steps);
     while (lds() > 160 * 1024 && plan.waves > 1) plan.waves /= 2;
     MK_REQUIRE(lds() <= 160 * 1024, MK_ERR_UNSUPPORTED, "mk_packed_matmul: the scales of 16 rows do not fit a compute unit");
     int status;
