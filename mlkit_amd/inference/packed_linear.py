@@ -38,12 +38,22 @@ from mlkit_amd.quantization.core import Q
 
 SCALE_STORAGE_DTYPES = {"fp16": torch.float16, "bf16": torch.bfloat16}
 MAXIMUM_FUSED_ROWS = 8
-# Rows up to which multiplying the codes beats decoding the weight for a library product (us, 4096 x 14336 / 14336 x 4096
-# INT4 at 128 rows 38 / 45 against 90 / 59; at 192 rows INT8 14336 x 4096 loses, 80 against 65).  Tables that take two operands
-# a value (NF4, fitted codebooks) win up to 64 rows: NF4 at 64 rows 39 / 34 against 63 / 53, at 96 rows 72 / 58 against 76 / 53.
-# Layers of at most 2^24 weights gain up to 256 rows (4096 x 4096: INT4 23 against 35, INT8 29 against 34, NF4 32 against 35;
-# 2048 x 2048 at 192 rows NF4 16.1 against 17.1), where the decode and the product are two short launches.
-MAXIMUM_PRODUCT_ROWS, MAXIMUM_PRODUCT_ROWS_SPLIT, MAXIMUM_PRODUCT_ROWS_SMALL, SMALL_WEIGHTS = 128, 64, 256, 1 << 24
+# Rows of x up to which multiplying the codes beats decoding the weight for a library product, us against us:
+# * 64 on any layer (151936 x 896 INT4 / INT8 / NF4 82 / 98 / 103 against 140 / 144 / 134, 28672 x 8192 101 / 126 / 137 against
+#   218 / 237 / 219), and no more with tables that take two operands a value (NF4 4096 x 14336 / 14336 x 4096 at 96 rows 72 / 58
+#   against 76 / 53), on tall layers of shorter rows (96 rows, 22016 x 5120 INT8 107 against 96, 151936 x 896 INT4 146 against 144) or
+#   in groups of 64 from 8192 rows of weight on (96 rows, 9353 x 9984 INT4 99 against 87, 8192 x 8192 57 against 65); 32 with
+#   two operands and offsets (NF4 9353 x 9984 at 48 rows 106 against 81);
+# * 128 elsewhere (4096 x 14336 / 14336 x 4096 INT4 38 / 45 against 90 / 59, INT8 55 / 57 against 91 / 59, 28672 x 8192 217
+#   against 235; at 192 rows INT8 14336 x 4096 loses, 80 against 65);
+# * 256 on layers of at most 2^24 weights (4096 x 4096 INT4 24 against 35, 12288 x 1024 25 against 34), where the decode and the
+#   product are two short launches; 192 with bytes or two operands a value (2239 x 4992 NF4 at 256 rows 41 against 34, 9765 x 896
+#   INT8 31 against 30); 128 on tall ones (24832 x 512 INT4 / INT8 / NF4 22 / 25 / 29 against 32 / 30 / 31, at 256 rows INT8 42
+#   against 33).
+MAXIMUM_PRODUCT_ROWS = 128
+MAXIMUM_PRODUCT_ROWS_TALL, TALL_LAYER, LONG_ROW, TALL_IN_SHORT_GROUPS = 64, 16384, 8192, 8192
+MAXIMUM_PRODUCT_ROWS_HEAVIEST = 32
+MAXIMUM_PRODUCT_ROWS_SMALL, MAXIMUM_PRODUCT_ROWS_SMALL_HEAVY, SMALL_WEIGHTS, SMALL_HEIGHT = 256, 192, 1 << 24, 12288
 PRODUCT_DTYPES = frozenset({torch.float16, torch.bfloat16})
 _LAUNCH_BUFFERS = frozenset({"packed", "scales", "values", "zeros", "bias"})
 
@@ -188,10 +198,18 @@ class PackedLinear(nn.Module):
                  and self.scales.dtype in (torch.float16, torch.bfloat16) and self.packed.data_ptr() % 16 == 0)
         if not taken:
             return 0
-        if width * self.out_features <= SMALL_WEIGHTS:
-            return MAXIMUM_PRODUCT_ROWS_SMALL
-        on_table = bits in (2, 3) or not self.uniform_grid
-        return MAXIMUM_PRODUCT_ROWS_SPLIT if on_table and not self.values_held else MAXIMUM_PRODUCT_ROWS
+        height = self.out_features
+        two_operands = (bits in (2, 3) or not self.uniform_grid) and not self.values_held
+        if width * height <= SMALL_WEIGHTS:
+            if height > SMALL_HEIGHT:
+                return MAXIMUM_PRODUCT_ROWS
+            return MAXIMUM_PRODUCT_ROWS_SMALL_HEAVY if two_operands or bits == 8 else MAXIMUM_PRODUCT_ROWS_SMALL
+        if two_operands and self.zeros is not None:
+            return MAXIMUM_PRODUCT_ROWS_HEAVIEST
+        if (two_operands or (height > TALL_LAYER and width < LONG_ROW)
+                or (group == 64 and height > TALL_IN_SHORT_GROUPS)):
+            return MAXIMUM_PRODUCT_ROWS_TALL
+        return MAXIMUM_PRODUCT_ROWS
 
     # -- online input rotation ---------------------------------------------------------------
 

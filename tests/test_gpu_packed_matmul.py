@@ -321,3 +321,46 @@ def test_a_function_mode_sees_the_dense_product():
         assert torch.equal(watched, torch.nn.functional.linear(x, layer.weight, layer.bias))
         with torch.device("cuda"):
             assert torch.equal(layer(x), on_codes)
+
+
+@pytest.mark.parametrize("rows,width,quantizer,limit", [
+    (320, 512, "int4", 256), (320, 512, "nf4", 192), (320, 512, "int8", 192), (12800, 512, "int4", 128),   # up to 2^24 weights
+    (4100, 4128, "int4", 128), (4100, 4128, "nf4", 64), (17000, 1024, "int4", 64), (2048, 8224, "seven", 128),
+])
+def test_which_calls_reach_the_product(rows, width, quantizer, limit):
+    """Exactly the calls of 9 rows to the layer's limit are multiplied on their codes, and agree with the dense product."""
+    import mlkit_amd as mk
+
+    quantizers = {"int4": mk.int(4, 128), "nf4": mk.nf4(64), "int8": mk.int(8, 128), "seven": mk.scaled(mk.grid.values(SEVEN.tolist(), bits=3), group=64)}
+    linear = torch.nn.Linear(width, rows, device="cuda", dtype=torch.float16)
+    layer = mk.PackedLinear(linear, quantizers[quantizer](linear.weight.detach()))
+    made = []
+    product = layer._product
+    layer._product = lambda inputs, samples: made.append(samples) or product(inputs, samples)
+    for samples in (8, 9, limit, limit + 1):
+        x = torch.randn((samples, width), device="cuda").half()
+        with torch.no_grad():
+            y = layer(x)
+        expected = torch.nn.functional.linear(x.float(), layer.weight.float(), layer.bias.float())
+        assert ((y.float() - expected).norm() / expected.norm()).item() < 2e-3
+    assert made == [9, limit]
+
+
+def test_calls_the_library_refuses_take_the_dense_product():
+    """Activations that start off 16 bytes, and scales that were cast to fp32 after the layer was built."""
+    import mlkit_amd as mk
+
+    linear = torch.nn.Linear(512, 320, device="cuda", dtype=torch.float16)
+    layer = mk.PackedLinear(linear, mk.int(4, 128)(linear.weight.detach()))
+    x = torch.randn(20 * 512 + 1, device="cuda").half()[1:].view(20, 512)
+    with torch.no_grad():
+        assert layer._product(x, 20) is None
+        assert torch.equal(layer(x), torch.nn.functional.linear(x, layer.weight, layer.bias))
+        aligned = x.clone()
+        expected = layer(aligned).float()
+        layer.float()
+        assert layer.scales.dtype == torch.float32
+        torch.testing.assert_close(layer(aligned.float()), expected, rtol=2e-3, atol=2e-3)
+        layer.bias = layer.bias.half()
+        assert layer._product(aligned, 20) is None
+        torch.testing.assert_close(layer(aligned).float(), expected, rtol=2e-3, atol=4e-3)
