@@ -342,7 +342,7 @@ class Scaled(Quantizer):
         if flag.item():
             raise ValueError("scaled requires a finite floating-point weight matrix")
         side_bits = scales.numel() * SCALE_FORMAT_BITS[self.scale_fmt] * (2 if zero is not None else 1)
-        return Q(bits=self.grid.bits * w.numel() + side_bits, codes=codes, decode=decode_scaled, codec="scaled",
+        return Q(bits=float(self.grid.bits * w.numel() + side_bits), codes=codes, decode=decode_scaled, codec="scaled",
                  metadata={"code_bits": self.grid.bits, "scale_fmt": self.scale_fmt,
                            "trainable": ["scales"] + (["zero"] if zero is not None else [])},
                  params={"scales": scales, "values": table, "group": group, "offset": 0, "zero": zero})

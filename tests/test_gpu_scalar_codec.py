@@ -274,6 +274,17 @@ def test_rounding_in_one_pass_matches_oracle(rows, width, group, values, integer
     np.testing.assert_array_equal(host(codes), expected["codes"])
 
 
+@pytest.mark.parametrize("asym", [False, True])
+def test_rounding_in_one_pass_describes_its_result_as_the_steps_do(asym):
+    import mlkit_amd as mk
+
+    weight, quantizer = torch.randn(40, 200, device="cuda").half(), mk.int(4, 64, asym=asym)
+    whole = quantizer(weight)
+    steps = quantizer.fit(weight, mk.Ctx(device="cuda"))(weight, slice(None))
+    assert type(whole.bits) is type(steps.bits) and whole.bits == steps.bits
+    assert whole.metadata == steps.metadata and whole.codec == steps.codec and list(whole.params) == list(steps.params)
+
+
 @pytest.mark.parametrize("bad", [float("inf"), float("nan")])
 def test_rounding_in_one_pass_reports_non_finite_weights(bad):
     import mlkit_amd as mk
