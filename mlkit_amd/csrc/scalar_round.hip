@@ -114,11 +114,18 @@ __global__ void __launch_bounds__(kThreads) round_groups_kernel(const RoundArgs 
     __shared__ float fraction[64];
     float few_threshold[kFew - 1], few_value[kFew];
     int steps = 0;
+    // Quotients up to which the thresholds say what nearest_entry() does.  Past the last entry that one takes the entry
+    // below it once both distances round to one number (or the two are equal), which 2^21 of their distance keep well away.
+    float limit = __builtin_inff();
+    auto uniform = [](float x) __attribute__((always_inline)) -> float {   // in a scalar register
+        return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x)));
+    };
     if constexpr (ROUNDING != kInteger) {
         stage_table(table, a.values, a.n_values);
         for (int k = threadIdx.x; k < a.n_values; k += kThreads)
             threshold[k] = k + 1 < a.n_values ? upper_threshold(table, k) : __builtin_inff();
         __syncthreads();
+        if (a.n_values > 1) limit = uniform(table[a.n_values - 1] + (table[a.n_values - 1] - table[a.n_values - 2]) * 0x1p21f);
         if constexpr (ROUNDING == kFewValues) {
 #pragma unroll
             for (int k = 0; k < kFew - 1; ++k) few_threshold[k] = k < a.n_values ? threshold[k] : __builtin_inff();
@@ -139,10 +146,15 @@ __global__ void __launch_bounds__(kThreads) round_groups_kernel(const RoundArgs 
         for (int k = 0; k < kFew / 2; ++k) magnitude[k] = table[min(a.n_values / 2 + k, a.n_values - 1)];
     }
     bool ordinary_fractions = true;
+    float least_fraction = 1.0f;
     if constexpr (SEARCH) {
         for (int i = threadIdx.x; i < a.n_fractions; i += kThreads) fraction[i] = a.fractions[i];
         __syncthreads();
-        for (int i = 0; i < a.n_fractions; ++i) ordinary_fractions = ordinary_fractions && fraction[i] > 0x1p-10f && fraction[i] < 0x1p10f;
+        for (int i = 0; i < a.n_fractions; ++i) {
+            ordinary_fractions = ordinary_fractions && fraction[i] > 0x1p-10f && fraction[i] < 0x1p10f;
+            least_fraction = fminf(least_fraction, fraction[i]);
+        }
+        least_fraction = uniform(least_fraction);
     }
     const int lane_in_team = threadIdx.x % TEAM;
 
@@ -161,6 +173,11 @@ __global__ void __launch_bounds__(kThreads) round_groups_kernel(const RoundArgs 
             }
             return code;
         }
+    };
+    // The same for any quotient (see `limit`).
+    auto below_the_last = [&](float x) __attribute__((always_inline)) -> bool {
+        const float last = table[a.n_values - 1], before = table[max(a.n_values - 2, 0)];
+        return x > last && a.n_values > 1 && fabsf(__fsub_rn(x, before)) <= fabsf(__fsub_rn(x, last));
     };
     auto value_of = [&](float x) __attribute__((always_inline)) -> float {
         if constexpr (ROUNDING == kInteger) {
@@ -262,7 +279,7 @@ __global__ void __launch_bounds__(kThreads) round_groups_kernel(const RoundArgs 
                 for (int i = 0; i < 8; ++i) sample[t][i] = __fsub_rn(sample[t][i], zero);
         }
         if constexpr (SEARCH) {
-            // `careful`: some lane's divisor is extreme, or some lane has columns past the row
+            // `careful`: some lane's divisor or quotients are extreme, or some lane has columns past the row
             auto error_of = [&](float s, auto careful_) __attribute__((always_inline)) -> float {
                 constexpr bool kCareful = decltype(careful_)::value;
                 const float inverse = __fdiv_rn(1.0f, s);
@@ -277,7 +294,9 @@ __global__ void __launch_bounds__(kThreads) round_groups_kernel(const RoundArgs 
                         float q;
                         if constexpr (kCareful) q = __fdiv_rn(x, s);
                         else q = corrected_quotient(x, s, inverse);
-                        float difference = __fsub_rn(__fmul_rn(value_of(q), s), x);
+                        float nearest = value_of(q);
+                        if constexpr (kCareful && ROUNDING != kInteger) nearest = below_the_last(q) ? table[max(a.n_values - 2, 0)] : nearest;
+                        float difference = __fsub_rn(__fmul_rn(nearest, s), x);
                         if constexpr (kCareful) difference = start + t * kSpan + i < a.width ? difference : 0.0f;
                         partial[i] = __fadd_rn(partial[i], __fmul_rn(difference, difference));
                     }
@@ -374,7 +393,9 @@ __global__ void __launch_bounds__(kThreads) round_groups_kernel(const RoundArgs 
                 __builtin_amdgcn_wave_barrier();   // the estimates have been read
             };
             // (2^40: no square of the first pass leaves the normal range, nor 2^-36 of a sum of them)
-            const bool moderate = kPruned && all_whole && __all(base_scale > 0x1p-40f && base_scale < 0x1p40f && ordinary_fractions);
+            const float smallest_scale = fminf(base_scale, mk_rounded_scale(__fmul_rn(base_scale, least_fraction), a.format));
+            const bool within = all_whole && ordinary_fractions && __all((a.asym ? high - zero : high) <= limit * smallest_scale);
+            const bool moderate = kPruned && within && __all(base_scale > 0x1p-40f && base_scale < 0x1p40f);
             if constexpr (kPruned) {
                 if (moderate) {
                     if constexpr (ROUNDING == kFewValues) {
@@ -387,7 +408,7 @@ __global__ void __launch_bounds__(kThreads) round_groups_kernel(const RoundArgs 
             }
             // candidates are fractions of the base (or the smallest value of the storage format)
             if (moderate) {
-            } else if (all_whole && __all(base_scale > 0x1p-90f && base_scale < 0x1p90f && ordinary_fractions))
+            } else if (within && __all(base_scale > 0x1p-90f && base_scale < 0x1p90f))
                 search(std::integral_constant<bool, false>{});
             else
                 search(std::integral_constant<bool, true>{});
@@ -419,11 +440,12 @@ __global__ void __launch_bounds__(kThreads) round_groups_kernel(const RoundArgs 
                         packed[t][i / 4] = __builtin_amdgcn_cvt_pk_u8_f32(
                             __fsub_rn(nearest_grid_integer(q, a.minimum, a.maximum), a.minimum), i % 4, packed[t][i / 4]);
                     else
-                        packed[t][i / 4] |= static_cast<uint32_t>(code_of(q)) << (8 * (i % 4));
+                        packed[t][i / 4] |= static_cast<uint32_t>(decltype(careful_)::value && below_the_last(q) ? a.n_values - 2 : code_of(q)) << (8 * (i % 4));
                 }
             }
         };
-        if (__all(scale > 0x1p-100f && scale < 0x1p100f)) encode(std::integral_constant<bool, false>{});
+        if (__all(scale > 0x1p-100f && scale < 0x1p100f && (a.asym ? high - zero : high) <= limit * scale))
+            encode(std::integral_constant<bool, false>{});
         else encode(std::integral_constant<bool, true>{});
         if (wanted >= a.total_groups) continue;
         if (lane_in_team == 0) {

@@ -274,6 +274,40 @@ def test_rounding_in_one_pass_matches_oracle(rows, width, group, values, integer
     np.testing.assert_array_equal(host(codes), expected["codes"])
 
 
+@pytest.mark.parametrize("values", [SEVEN, TABLE9, np.array([-1, 0, 1, 1], dtype=F32), np.array([-2, -1, -1], dtype=F32),
+                                    np.array([0.5], dtype=F32), np.array([0, 1, np.nextafter(F32(1), F32(2))], dtype=F32)])
+@pytest.mark.parametrize("scale,asym,fmt", [("absmax", False, "fp16"), ("absmax", True, "fp8"), ("mse", False, "fp8"), ("mse", True, "fp16")])
+@pytest.mark.parametrize("group", [32, 64])
+def test_rounding_in_one_pass_past_the_last_entry(values, scale, asym, fmt, group):
+    """Weights far beyond what the scales' format reaches, and tables whose last entry repeats or nearly does: past the
+    last entry the entry below it is taken when both distances round to one number, as the separate steps have it."""
+    import mlkit_amd as mk
+    from mlkit_amd.kernels import scalar_encode
+
+    if asym and values.max() == values.min():
+        pytest.skip("an offset needs two values")
+    weight = torch.from_numpy(helpers.normal_weight(24, 256, seed=group, scale=1.0)).cuda()
+    weight *= torch.logspace(-3, 24, 24, device="cuda")[:, None]
+    minimum, maximum = float(values.min()), float(values.max())
+    reciprocal = float(scaling.f32_reciprocal(maximum - minimum if asym else float(np.abs(values).max())))
+    fractions = dev(FRACTIONS) if scale == "mse" else None
+    codes, scales, zeros, flag = scalar_encode.round_matrix(weight, dev(values), fractions, group, asym=asym, integer=False,
+                                                            minimum=minimum, maximum=maximum, reciprocal=reciprocal, scale_format=fmt)
+    assert flag.item() == 0
+    expected, offset = scalar_encode.fit_scales(weight, group, asym=asym, reciprocal=reciprocal, value_minimum=minimum,
+                                                scale_format=fmt, store_zero=scale == "absmax")
+    if scale == "mse":
+        expected = scalar_encode.search_scales(weight, expected, offset, dev(values), fractions, group, None, fmt, integer=False,
+                                               minimum=minimum, maximum=maximum)
+        if asym:
+            offset = mk.quantization.scaled.store_scale(offset.abs().clamp_min(1e-12), fmt)[0] * offset.sign()
+    assert torch.equal(scales, expected) and (zeros is None) is not asym
+    if asym:
+        assert torch.equal(zeros, offset)
+    assert torch.equal(codes, scalar_encode.encode(weight, expected, offset, dev(values), group, None, integer=False,
+                                                   minimum=minimum, maximum=maximum))
+
+
 @pytest.mark.parametrize("asym", [False, True])
 def test_rounding_in_one_pass_describes_its_result_as_the_steps_do(asym):
     import mlkit_amd as mk
