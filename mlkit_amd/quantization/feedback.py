@@ -190,7 +190,7 @@ class _FactorGraph:
 
     def _captured(self) -> "torch.cuda.CUDAGraph":
         graph = torch.cuda.CUDAGraph()
-        graph.capture_begin(capture_error_mode="thread_local")   # (other threads may go on allocating)
+        graph.capture_begin()
         try:
             self.status.zero_()   # a fill kernel
             _factor_in_place(self.matrix, self.status, self.factored, self.pairs)
@@ -213,7 +213,7 @@ class _FactorGraph:
 
 
 FACTOR_GRAPHS = True        # capture the factorisation of a width the second time it is asked for
-FACTOR_GRAPH_WIDTH = 1024   # from here on: 896 columns take 414 us from a graph, 420 launch by launch
+FACTOR_GRAPH_WIDTH = 1024   # from here on (a conversion of 4864 x 896 takes 876 us with a graph of its own, 910 without)
 FACTOR_GRAPH_LIMIT = 2      # graphs (and their width x width buffers) kept per process
 _factor_graphs: dict[tuple, "_FactorGraph | None"] = {}   # by device and width
 _factor_graphs_lock = threading.Lock()
@@ -228,8 +228,11 @@ def clear_factor_graphs() -> None:
 
 
 def _factor_graph(width: int, device: torch.device, pairs: bool) -> "_FactorGraph | None":
-    """The captured factorisation of a width, from the second matrix on (the first one warms every kernel up)."""
-    if not FACTOR_GRAPHS or width < FACTOR_GRAPH_WIDTH or torch.cuda.is_current_stream_capturing():
+    """The captured factorisation of a width, from the second matrix on (the first one warms every kernel up).  The main
+    thread's alone: the library's handles belong to a thread, so that the first matrix warms up the one it runs on, and a
+    capture must not run beside other threads' first calls.  Those threads launch one by one, in buffers of their own."""
+    if (not FACTOR_GRAPHS or width < FACTOR_GRAPH_WIDTH or threading.current_thread() is not threading.main_thread()
+            or torch.cuda.is_current_stream_capturing()):
         return None
     key = (torch.cuda.current_device() if device.index is None else device.index, width) + (("pairs",) if pairs else ())
     with _factor_graphs_lock:

@@ -514,3 +514,30 @@ def test_a_packed_call_holds_its_bound_arguments(monkeypatch):
     layer._product(x, 12)
     layer._matvec(x[:2], torch.empty((2, 4), dtype=torch.float16), 2)
     assert alive == [True, True]
+
+
+def test_only_the_main_thread_captures_factorisations(monkeypatch):
+    import threading
+
+    from mlkit_amd.quantization import feedback
+
+    made = []
+    monkeypatch.setattr(feedback, "_FactorGraph", lambda *arguments: made.append(threading.current_thread()) or object())
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    device = torch.device("cuda", 0)
+    feedback.clear_factor_graphs()
+
+    def ask(width):
+        return [feedback._factor_graph(width, device, False) for _ in range(3)]
+
+    got = []
+    threads = [threading.Thread(target=lambda: got.extend(ask(2048))) for _ in range(3)]
+    for thread in threads:
+        thread.start()
+    for thread in threads:
+        thread.join()
+    assert got == [None] * 9 and not made
+    assert ask(1023) == [None] * 3
+    captured = ask(2048)
+    assert captured[0] is None and captured[1] is captured[2] is not None and len(made) == 1
+    feedback.clear_factor_graphs()
