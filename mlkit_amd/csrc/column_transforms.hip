@@ -150,7 +150,8 @@ struct TransposeArgs {
     int rows, columns, tiles_across;
 };
 
-// 64 x 64 tiles through LDS, fp32 4096 x 14336 in 98 us (4.8 TB/s; torch's strided copy 255), from bf16 in 84 (320 with its conversion); reads and writes both move whole 16-byte pieces along rows where the sizes allow it (VEC).
+// 64 x 64 tiles through LDS, fp32 4096 x 14336 in 100 us (4.7 TB/s; torch's strided copy 255), from bf16 in 77 (320 with its
+// conversion); reads and writes both move whole 16-byte pieces along rows where the sizes allow it (VEC).
 template <int SOURCE, bool VEC>
 __global__ void __launch_bounds__(256) transpose_kernel(const TransposeArgs a) {
     __shared__ float tile[64][65];

@@ -11,7 +11,7 @@
 // 4096 x 14336 fp16 to INT4 g128 with offsets: 43 us = 4.1 TB/s (a device copy: 5.1), against 163 us for the
 // conversion to FP32, the range fit and the encoding as passes of their own (53 + 58 + 52).
 // A search is bound by the vector ALUs: 21 candidates, each a quotient and a rounding per weight.  4096 x 4096 on
-// seven values, g64: 128 us, against 496 us with an IEEE division and a bisection of the table per candidate and
+// seven values, g64: 131 us, against 496 us with an IEEE division and a bisection of the table per candidate and
 // weight, and 236 us with thresholds kept in registers and the exact error of every candidate; groups of 64 columns and
 // more on integers or at most eight values now work out an estimate for each candidate (7 instructions a weight where the
 // values lie symmetrically about zero) and the exact error only where the estimate leaves the choice open.
