@@ -346,6 +346,21 @@ def test_which_calls_reach_the_product(rows, width, quantizer, limit):
     assert made == [9, limit]
 
 
+def test_bytes_on_a_fractional_grid_take_the_dense_product():
+    """255 steps of a rounded length do not end on the last value: the error is one for all weights, so such layers stay
+    with the decoded weight, whose own rounding hides part of it."""
+    import mlkit_amd as mk
+
+    linear = torch.nn.Linear(512, 64, bias=False, device="cuda", dtype=torch.float16)
+    x = torch.relu(torch.randn((16, 512), device="cuda")).half()
+    for values, taken in ((torch.linspace(-0.7, 1.1, 256), False), (torch.arange(-128.0, 128.0), True)):
+        layer = mk.PackedLinear(linear, mk.scaled(mk.grid.values(values.tolist(), bits=8), group=None)(linear.weight.detach()))
+        assert layer.uniform_grid and (layer.maximum_product_rows > 0) is taken
+        if not taken:
+            with torch.no_grad():
+                assert torch.equal(layer(x), torch.nn.functional.linear(x, layer.weight))
+
+
 def test_calls_the_library_refuses_take_the_dense_product():
     """Activations that start off 16 bytes, and scales that were cast to fp32 after the layer was built."""
     import mlkit_amd as mk
