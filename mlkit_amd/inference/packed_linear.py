@@ -193,8 +193,8 @@ class PackedLinear(nn.Module):
     def _product_rows(self) -> int:
         """Rows up to which ``mk_packed_matmul`` serves this layer; zero when it does not take the layer."""
         width, group, bits = self.in_features, self.group, self.code_bits
-        # (Bytes on a fractional grid: 255 steps leave the last value 6e-6 off, which a rounded weight hides in part: 3.1e-4 of
-        # y against 2.7e-4 in fp16 on activations of one sign.  Fifteen steps do not show.)
+        # Bytes on a fractional grid: 255 steps leave the last value 6e-6 off, which a rounded weight hides in part (3.1e-4 of y
+        # against 2.7e-4 in fp16 on activations of one sign).  Fifteen steps do not show.
         codes = bits in (2, 3, 4) or (bits == 8 and self.uniform_grid and float(self.grid_step).is_integer()
                                       and float(self.grid_minimum).is_integer())
         taken = (self.layout is not None and codes and width % 32 == 0
