@@ -56,6 +56,11 @@ __device__ __forceinline__ void rows_to_lds(const float *source, float *target) 
     __builtin_amdgcn_global_load_lds(source, target, 16, 0, 0);
 }
 
+// The same with 4 bytes per lane (sources that start on any float).
+__device__ __forceinline__ void floats_to_lds(const float *source, float *target) {
+    __builtin_amdgcn_global_load_lds(source, target, 4, 0, 0);
+}
+
 // Waits until this wavefront's vector memory loads, LDS transfers included, are complete.
 __device__ __forceinline__ void wait_for_loads() {
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0), other counters untouched
@@ -955,12 +960,17 @@ __global__ void __launch_bounds__(kUpdateThreads, 2) block_update_kernel(const U
 }
 
 // The same update with the deviations read from the column-major buffer the sweep kernel
-// fills, for launches made of whole tiles only (rows and updated columns in multiples of
-// 128, chains in multiples of 32 columns): the left operand loads and lands in LDS as whole
-// float4s along the rows (no subtraction, no transposing stores), nothing is masked, and
-// every address that does not depend on k is computed once.
+// fills, for chains in multiples of 32 columns: both operands go from global memory straight
+// into LDS (no subtraction, no transposing stores) and every address that does not depend on k is
+// computed once.  Rows and columns beyond the matrix are read from its last ones and not written.
+//
+// VEC: rows of both operands start on 16-byte boundaries and move in 16-byte pieces; otherwise in
+// single floats (four times the instructions, which the matrix products hide).  Bound by the fp32 matrix cores.  All
+// updates of a sweep of 1000 x 2777 / 704 x 1384 / 3001 x 8184, whose tiles are not whole: 0.25 / 0.08 / 2.59 ms (107 TFLOP/s
+// in the wide ones of the last), against 1.21 / 0.39 / 4.08 with the kernel above.
 constexpr int kDeviationStride = kTileRows;  // floats per k row in LDS
 
+template <bool VEC>
 __global__ void __launch_bounds__(kUpdateThreads, 2) block_update_from_deviations_kernel(const UpdateArgs a) {
     // Two buffers per operand, each a variable of its own: the compiler then sees that the
     // transfer into one buffer cannot touch the buffer being read, and does not wait for it.
@@ -979,21 +989,32 @@ __global__ void __launch_bounds__(kUpdateThreads, 2) block_update_from_deviation
     const int wave_row = (wave >> 1) * 64, wave_column = (wave & 1) * 64;
     const int chunks_per_chain = a.chain_width / kDepthChunk;
     const int steps = a.chains * chunks_per_chain;
+    const bool inside = row0 + kTileRows <= a.rows && column0 + kTileColumns <= a.column_end;   // uniform
 
     // Operands go from global memory straight into LDS: one wavefront instruction moves two
     // consecutive k rows of a tile (2 x 128 floats = 64 lanes x 16 bytes, lane l's bytes at
-    // 16 l from the wavefront-uniform LDS address). Per chunk a wavefront moves k rows
+    // 16 l from the wavefront-uniform LDS address), or half of one. Per chunk a wavefront moves k rows
     // 8 wave ... 8 wave + 7 of both tiles.
-    const uint32_t left_lane = static_cast<uint32_t>(lane >> 5) * a.rows + (lane & 31) * 4;
-    const uint32_t right_lane = static_cast<uint32_t>(lane >> 5) * a.width + (lane & 31) * 4;
-    const float *left_tile = a.deviation_t + row0;     // + k * rows
-    const float *right_tile = a.coeff + column0;       // + k * width
+    constexpr int kPiece = VEC ? 4 : 1, kPieceLanes = VEC ? 32 : 64, kHalves = VEC ? 1 : 2;
+    uint32_t left_lane[kHalves], right_lane[kHalves];
+#pragma unroll
+    for (int half = 0; half < kHalves; ++half) {
+        const int along = half * 64 + (lane & (kPieceLanes - 1)) * kPiece;
+        left_lane[half] = (VEC ? static_cast<uint32_t>(lane >> 5) * a.rows : 0u) + min(row0 + along, a.rows - kPiece);
+        right_lane[half] = (VEC ? static_cast<uint32_t>(lane >> 5) * a.width : 0u) + min(column0 + along, a.width - kPiece);
+    }
+    const float *left_tile = a.deviation_t;     // + k * rows
+    const float *right_tile = a.coeff;          // + k * width
 
     // This lane's cell of every 32 x 32 MFMA tile: rows (lane / 32) * 4 + ..., column lane % 32.
     const uint32_t cell_lane = static_cast<uint32_t>((lane >> 5) * 4) * a.width + (lane & 31);
     float *quarter = a.feedback + static_cast<size_t>(row0 + wave_row) * a.width + column0 + wave_column;
     auto cell = [&](int mi, int ni, int r) __attribute__((always_inline)) -> float * {
         return quarter + static_cast<size_t>(mi * 32 + (r >> 2) * 8 + (r & 3)) * a.width + ni * 32 + cell_lane;
+    };
+    const int rows_left = a.rows - row0 - wave_row - (lane >> 5) * 4, columns_left = a.column_end - column0 - wave_column - (lane & 31);
+    auto present = [&](int mi, int ni, int r) __attribute__((always_inline)) -> bool {
+        return mi * 32 + (r >> 2) * 8 + (r & 3) < rows_left && ni * 32 < columns_left;
     };
     // feedback's own values: one 32 x 32 quarter is requested in each of the first four steps,
     // behind that step's operand loads, so that no step waits for the whole tile.
@@ -1004,18 +1025,22 @@ __global__ void __launch_bounds__(kUpdateThreads, 2) block_update_from_deviation
         const size_t k_base = static_cast<size_t>(a.first_column + chain * a.chain_width + chunk * kDepthChunk + wave * 8);
         const float *left = left_tile + k_base * a.rows;
         const float *right = right_tile + k_base * a.width;
+        if constexpr (VEC) {
 #pragma unroll
-        for (int pair = 0; pair < 4; ++pair) {
-            const float *left_source = left + static_cast<size_t>(2 * pair) * a.rows + left_lane;
-            const float *right_source = right + static_cast<size_t>(2 * pair) * a.width + right_lane;
-            const int k = wave * 8 + 2 * pair;
-            if constexpr (odd.value) {
-                rows_to_lds(left_source, &deviation_odd[k][0]);
-                rows_to_lds(right_source, &coefficient_odd[k][0]);
-            } else {
-                rows_to_lds(left_source, &deviation_even[k][0]);
-                rows_to_lds(right_source, &coefficient_even[k][0]);
+            for (int pair = 0; pair < 4; ++pair) {
+                const int k = wave * 8 + 2 * pair;
+                rows_to_lds(left + static_cast<size_t>(2 * pair) * a.rows + left_lane[0], odd.value ? &deviation_odd[k][0] : &deviation_even[k][0]);
+                rows_to_lds(right + static_cast<size_t>(2 * pair) * a.width + right_lane[0], odd.value ? &coefficient_odd[k][0] : &coefficient_even[k][0]);
             }
+        } else {
+#pragma unroll
+            for (int one = 0; one < 8; ++one)
+#pragma unroll
+                for (int half = 0; half < kHalves; ++half) {
+                    const int k = wave * 8 + one, at = half * 64;
+                    floats_to_lds(left + static_cast<size_t>(one) * a.rows + left_lane[half], odd.value ? &deviation_odd[k][at] : &deviation_even[k][at]);
+                    floats_to_lds(right + static_cast<size_t>(one) * a.width + right_lane[half], odd.value ? &coefficient_odd[k][at] : &coefficient_even[k][at]);
+                }
         }
     };
     // A wavefront's own transfers have landed once its vector memory counter reads zero; the
@@ -1044,9 +1069,14 @@ __global__ void __launch_bounds__(kUpdateThreads, 2) block_update_from_deviation
         const bool more = step + 1 < steps;
         if (more) fetch(step + 1, std::bool_constant<!odd.value>{});
         if constexpr (quarter.value >= 0) {
+            constexpr int mi = quarter.value >> 1, ni = quarter.value & 1;
+            if (inside) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r)
-                totals[quarter.value >> 1][quarter.value & 1][r] = *cell(quarter.value >> 1, quarter.value & 1, r);
+                for (int r = 0; r < 16; ++r) totals[mi][ni][r] = *cell(mi, ni, r);
+            } else {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) totals[mi][ni][r] = present(mi, ni, r) ? *cell(mi, ni, r) : 0.0f;
+            }
         }
         const float *left_rows = (odd.value ? &deviation_odd[0][0] : &deviation_even[0][0]) + left_read;
         const float *right_rows = (odd.value ? &coefficient_odd[0][0] : &coefficient_even[0][0]) + right_read;
@@ -1098,7 +1128,8 @@ __global__ void __launch_bounds__(kUpdateThreads, 2) block_update_from_deviation
 #pragma unroll
         for (int ni = 0; ni < 2; ++ni)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) *cell(mi, ni, r) = totals[mi][ni][r];
+            for (int r = 0; r < 16; ++r)
+                if (inside || present(mi, ni, r)) *cell(mi, ni, r) = totals[mi][ni][r];
 }
 
 // Chains of exactly 128 columns on 64 x 64 tiles.  Two uses: the update of a super-block's own
@@ -1115,6 +1146,7 @@ constexpr int kSmallTile = 64;
 
 constexpr int kSmallDepth = 64;  // k rows per step: half a chain, two LDS buffers of 2 x 16 KB
 
+template <bool VEC>
 __global__ void __launch_bounds__(kUpdateThreads) block_update_small_tile_kernel(const UpdateArgs a) {
     __shared__ __attribute__((aligned(16))) float deviation_even[kSmallDepth][kSmallTile];     // [k][row]
     __shared__ __attribute__((aligned(16))) float deviation_odd[kSmallDepth][kSmallTile];
@@ -1129,21 +1161,33 @@ __global__ void __launch_bounds__(kUpdateThreads) block_update_small_tile_kernel
     const int column0 = a.column_begin + (large - large_row * a.column_tiles) * kTileColumns + (quarter & 1) * kSmallTile;
     const int wave_row = (wave >> 1) * 32, wave_column = (wave & 1) * 32;
 
+    if (row0 >= a.rows || column0 >= a.column_end) return;   // a quarter outside the matrix (uniform)
+    const bool inside = row0 + kSmallTile <= a.rows && column0 + kSmallTile <= a.column_end;   // uniform
+
     // One instruction moves four k rows of a tile (4 x 64 floats; lane l's 16 bytes land at
-    // 16 l from the uniform LDS address); per step a wavefront moves k rows 16 wave ... 16 wave + 15.
-    const uint32_t left_lane = static_cast<uint32_t>(lane >> 4) * a.rows + (lane & 15) * 4;
-    const uint32_t right_lane = static_cast<uint32_t>(lane >> 4) * a.width + (lane & 15) * 4;
+    // 16 l from the uniform LDS address), or one; per step a wavefront moves k rows 16 wave ... 16 wave + 15.
+    constexpr int kPiece = VEC ? 4 : 1, kPieceLanes = VEC ? 16 : 64, kRowsAtOnce = VEC ? 4 : 1;
+    const int along = (lane & (kPieceLanes - 1)) * kPiece;
+    const uint32_t left_lane = (VEC ? static_cast<uint32_t>(lane >> 4) * a.rows : 0u) + min(row0 + along, a.rows - kPiece);
+    const uint32_t right_lane = (VEC ? static_cast<uint32_t>(lane >> 4) * a.width : 0u) + min(column0 + along, a.width - kPiece);
     auto fetch = [&](int step, auto odd) __attribute__((always_inline)) {
         const size_t k_base = static_cast<size_t>(a.first_column + step * kSmallDepth + wave * 16);  // chains are adjacent
-        const float *left = a.deviation_t + row0 + k_base * a.rows;
-        const float *right = a.coeff + column0 + k_base * a.width;
+        const float *left = a.deviation_t + k_base * a.rows;
+        const float *right = a.coeff + k_base * a.width;
 #pragma unroll
-        for (int four = 0; four < 4; ++four) {
-            const int k = wave * 16 + 4 * four;
-            rows_to_lds(left + static_cast<size_t>(4 * four) * a.rows + left_lane,
-                        odd.value ? &deviation_odd[k][0] : &deviation_even[k][0]);
-            rows_to_lds(right + static_cast<size_t>(4 * four) * a.width + right_lane,
-                        odd.value ? &coefficient_odd[k][0] : &coefficient_even[k][0]);
+        for (int one = 0; one < 16; one += kRowsAtOnce) {
+            const int k = wave * 16 + one;
+            float *left_target = odd.value ? &deviation_odd[k][0] : &deviation_even[k][0];
+            float *right_target = odd.value ? &coefficient_odd[k][0] : &coefficient_even[k][0];
+            const float *left_source = left + static_cast<size_t>(one) * a.rows + left_lane;
+            const float *right_source = right + static_cast<size_t>(one) * a.width + right_lane;
+            if constexpr (VEC) {
+                rows_to_lds(left_source, left_target);
+                rows_to_lds(right_source, right_target);
+            } else {
+                floats_to_lds(left_source, left_target);
+                floats_to_lds(right_source, right_target);
+            }
         }
     };
     const int steps = a.chains * (kWholeChain / kSmallDepth);
@@ -1151,9 +1195,15 @@ __global__ void __launch_bounds__(kUpdateThreads) block_update_small_tile_kernel
 
     // This lane's cells of the 32 x 32 tile: rows (lane / 32) * 4 + ..., column lane % 32.
     float *cells = a.feedback + static_cast<size_t>(row0 + wave_row + (lane >> 5) * 4) * a.width + column0 + wave_column + (lane & 31);
+    const int rows_left = column0 + wave_column + (lane & 31) < a.column_end ? a.rows - row0 - wave_row - (lane >> 5) * 4 : 0;
     mk_f32x16 totals, sums;
+    if (inside) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) totals[r] = cells[static_cast<size_t>((r >> 2) * 8 + (r & 3)) * a.width];
+        for (int r = 0; r < 16; ++r) totals[r] = cells[static_cast<size_t>((r >> 2) * 8 + (r & 3)) * a.width];
+    } else {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) totals[r] = (r >> 2) * 8 + (r & 3) < rows_left ? cells[static_cast<size_t>((r >> 2) * 8 + (r & 3)) * a.width] : 0.0f;
+    }
 
     const uint32_t left_read = (lane >> 5) * kSmallTile + wave_row + (lane & 31);
     const uint32_t right_read = (lane >> 5) * kSmallTile + wave_column + (lane & 31);
@@ -1182,7 +1232,8 @@ __global__ void __launch_bounds__(kUpdateThreads) block_update_small_tile_kernel
         advance(step + 1, std::true_type{});
     }
 #pragma unroll
-    for (int r = 0; r < 16; ++r) cells[static_cast<size_t>((r >> 2) * 8 + (r & 3)) * a.width] = totals[r];
+    for (int r = 0; r < 16; ++r)
+        if (inside || (r >> 2) * 8 + (r & 3) < rows_left) cells[static_cast<size_t>((r >> 2) * 8 + (r & 3)) * a.width] = totals[r];
 }
 
 // Workgroup slots of block_update_from_deviations_kernel on the whole GPU (two per CU).
@@ -1196,25 +1247,32 @@ int launch_update(UpdateArgs a, hipStream_t stream) {
     const auto aligned = [](const void *pointer) { return (reinterpret_cast<uintptr_t>(pointer) & 15u) == 0; };
     const bool vec = a.width % 4 == 0 && a.first_column % 4 == 0 && a.chain_width % 4 == 0 && a.column_begin % 4 == 0 &&
                      aligned(a.original) && aligned(a.output) && aligned(a.coeff);
-    // The deviation buffer path handles whole tiles only.
-    const bool staged = a.deviation_t && aligned(a.deviation_t) && aligned(a.coeff) && a.rows % kTileRows == 0 &&
-                        a.width % 4 == 0 && a.column_begin % 4 == 0 &&
-                        (a.column_end - a.column_begin) % kTileColumns == 0 && a.chain_width % kDepthChunk == 0 &&
-                        a.chain_width / kDepthChunk >= 4;   // the first chain spans the four steps that read feedback
+    // The kernels that read the deviation buffer; chains of at least the four steps in which the first one reads feedback.
+    const bool staged = a.deviation_t && a.chain_width % kDepthChunk == 0 && a.chain_width / kDepthChunk >= 4;
+    // (rows of both operands in 16-byte pieces)
+    const bool pieces = aligned(a.deviation_t) && aligned(a.coeff) && a.rows % 4 == 0 && a.width % 4 == 0 && a.column_begin % 4 == 0;
+    const auto launch_large = [&](unsigned count) {
+        if (pieces) hipLaunchKernelGGL((block_update_from_deviations_kernel<true>), dim3(count), dim3(kUpdateThreads), 0, stream, a);
+        else hipLaunchKernelGGL((block_update_from_deviations_kernel<false>), dim3(count), dim3(kUpdateThreads), 0, stream, a);
+    };
+    const auto launch_small = [&](unsigned count) {
+        if (pieces) hipLaunchKernelGGL((block_update_small_tile_kernel<true>), dim3(count * 4), dim3(kUpdateThreads), 0, stream, a);
+        else hipLaunchKernelGGL((block_update_small_tile_kernel<false>), dim3(count * 4), dim3(kUpdateThreads), 0, stream, a);
+    };
     // (launches that leave most of the GPU idle with 128 x 128 tiles)
     const unsigned tiles = grid.x * grid.y;
     if (staged && a.chains == 1 && a.chain_width == kWholeChain && tiles <= 128) {
-        hipLaunchKernelGGL(block_update_small_tile_kernel, dim3(tiles * 4), dim3(kUpdateThreads), 0, stream, a);
+        launch_small(tiles);
     } else if (staged) {
         // Whole rounds of workgroup slots on 128 x 128 tiles; a last round that would fill at most
         // half of the slots runs as quarter tiles instead (chains of 128 columns only).
         const unsigned tail = tiles % kUpdateSlots;
         const bool split = a.chain_width == kWholeChain && tail > 0 && tail <= kUpdateSlots / 2;
         const unsigned whole = split ? tiles - tail : tiles;
-        if (whole) hipLaunchKernelGGL(block_update_from_deviations_kernel, dim3(whole), dim3(kUpdateThreads), 0, stream, a);
+        if (whole) launch_large(whole);
         if (split) {
             a.tile_first = static_cast<int>(whole);
-            hipLaunchKernelGGL(block_update_small_tile_kernel, dim3(tail * 4), dim3(kUpdateThreads), 0, stream, a);
+            launch_small(tail);
         }
     } else if (vec)
         hipLaunchKernelGGL((block_update_kernel<true>), grid, dim3(kUpdateThreads), 0, stream, a);

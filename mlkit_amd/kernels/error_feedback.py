@@ -169,8 +169,7 @@ def sweep(
     scales = torch.empty((rows, groups), device=device, dtype=torch.float32)
     zeros = torch.empty_like(scales) if asym else None
     workspace = torch.empty((rows, region), device=device, dtype=torch.float32) if region < width else None
-    # column-major deviations of finished columns: what the trailing updates multiply
-    deviations = torch.empty((width, rows), device=device, dtype=torch.float32) if rows % 4 == 0 and width % 4 == 0 else None
+    deviations = _kept_deviations(rows, width, block, device)
     values = values.to(torch.float32).contiguous()
     native.check(native.library().mk_feedback_sweep(
         original.data_ptr(), feedback.data_ptr(), output.data_ptr(), encoded.data_ptr(), coefficients.data_ptr(),
@@ -181,6 +180,14 @@ def sweep(
         native.current_stream(device),
     ))
     return scales, zeros
+
+
+def _kept_deviations(rows: int, width: int, block: int, device: torch.device) -> Tensor | None:
+    """Room for the column-major deviations of finished columns, which the trailing updates multiply: those after tiles of
+    128 columns or more in whole chunks of 32 (shorter ones work them out again from weights and reconstruction)."""
+    if width <= block or block < 128 or block % 32:
+        return None
+    return torch.empty((width, rows), device=device, dtype=torch.float32)
 
 
 def vector_sweep(
@@ -218,8 +225,7 @@ def vector_sweep(
         groups += -(-span // min(group, span))
     scales = torch.empty((rows, groups), device=device, dtype=torch.float32)
     workspace = torch.empty((rows, region), device=device, dtype=torch.float32) if region < width else None
-    # column-major deviations, read by the trailing updates that take whole tiles of 128 rows
-    deviations = torch.empty((width, rows), device=device, dtype=torch.float32) if rows % 128 == 0 and width % 4 == 0 else None
+    deviations = _kept_deviations(rows, width, block, device)
     native.check(native.library().mk_feedback_vector_sweep(
         original.data_ptr(), feedback.data_ptr(), output.data_ptr(), encoded.data_ptr(), coefficients.data_ptr(),
         scales.data_ptr(), native.pointer(workspace), native.pointer(deviations), codebook.data_ptr(), dimension,

@@ -212,6 +212,31 @@ def test_update_from_kept_deviations_equals_the_recomputing_update(rows, width, 
     assert torch.equal(updated[:, :begin], feedback[:, :begin])
 
 
+@pytest.mark.parametrize("rows,width", [(1, 260), (3, 389), (63, 516), (130, 641), (129, 1157), (260, 1284), (517, 2049), (1029, 3076)])
+def test_sweep_with_kept_deviations_equals_the_one_without(rows, width):
+    """Rows and columns that fill no whole tile, on 16-byte boundaries and off them: the kernels that read the kept
+    deviations (64 x 64 and 128 x 128 tiles) against the one that works them out again, bit for bit."""
+    from mlkit_amd import native
+
+    generator = torch.Generator(device="cuda").manual_seed(rows * width)
+    weight = torch.randn((rows, width), device="cuda", generator=generator) * 0.02
+    coeff = (torch.randn((width, width), device="cuda", generator=generator) * 0.05).triu(1) + torch.eye(width, device="cuda")
+    values = torch.arange(-8.0, 8.0, device="cuda")
+    groups, results = -(-width // 128), []
+    for kept in (False, True):
+        feedback, output = torch.zeros_like(weight), torch.empty_like(weight)
+        encoded = torch.empty((rows, width), dtype=torch.uint8, device="cuda")
+        scales, workspace = torch.empty((rows, groups), device="cuda"), torch.empty((rows, 128), device="cuda")
+        deviations = torch.full((width, rows), float("nan"), device="cuda") if kept else None
+        native.check(native.library().mk_feedback_sweep(
+            weight.data_ptr(), feedback.data_ptr(), output.data_ptr(), encoded.data_ptr(), coeff.data_ptr(), scales.data_ptr(), None,
+            workspace.data_ptr(), native.pointer(deviations), values.data_ptr(), 16, rows, width, 128, 128, 128, 1, -8.0, 7.0, 0,
+            0.125, -8.0, native.SCALE_FORMAT_CODES["fp16"], 4, native.current_stream(weight.device)))
+        results.append((encoded, output, scales, feedback))
+    for one, other in zip(*results):
+        assert torch.equal(one, other)
+
+
 @pytest.mark.parametrize("width,step", [(1024, 1), (1100, 1), (1536, 8), (2304, 1)])
 def test_blocked_factorisation_matches_the_float64_coefficients(width, step):
     """`feedback_coefficients` on the device factors matrices of 1024 columns and more block by
