@@ -312,6 +312,18 @@ int mk_cholesky_block(float *matrix, long long leading, int size, int first_colu
 int mk_cholesky_block_pairs(float *matrix, long long leading, int size, int first_column, int row_columns,
                             float *factor_out, int *status, void *stream);
 
+/* The products of the blocked factorisation, in place on its [width, width] fp32 matrix whose rows k_first ... k_stop - 1
+ * hold the finished factor U:  matrix[r][c] -= sum over those k of U[k][r] U[k][c].
+ * mk_factor_block_rows: at most 128 rows r from row_first on, every column c >= row_first; k_stop - k_first a multiple of
+ * 128.  one_chain != 0: each sum is one chain of additions over ascending k, otherwise four that are added up.
+ * mk_factor_trailing: any number of rows, the columns c >= r (values below the diagonal are left or changed); k_stop -
+ * k_first a multiple of 64.  leave_room != 0: the launch leaves every compute unit room for kernels on another stream.
+ * Replaces: part of torch.linalg.cholesky_ex, quantization/algorithms/error_feedback.py:37-83. */
+int mk_factor_block_rows(float *matrix, int width, int k_first, int k_stop, int row_first, int row_stop, int one_chain,
+                         void *stream);
+int mk_factor_trailing(float *matrix, int width, int k_first, int k_stop, int row_first, int row_stop, int leave_room,
+                       void *stream);
+
 /* The blocked transform of a width order * power (power a power of two) in one launch:
  * every row [order, power] of `source` is multiplied by signs_before (NULL or
  * [order * power] floats), each block goes through the Walsh-Hadamard stages of mk_fwht
@@ -442,7 +454,7 @@ int mk_hessian_reversed(const float *source, float *target, int width, const lon
                         const float *addend, void *stream);
 
 /* Unit upper-triangular coefficients from the upper Cholesky factor U of the reversed matrix:
- * out[a][b] = U[w-1-b][w-1-a] / U[w-1-b][w-1-b] (true division).  [width, width] fp32, distinct.
+ * out[a][b] = U[w-1-b][w-1-a] / U[w-1-b][w-1-b] (true division), zero below the diagonal.  [width, width] fp32, distinct.
  * Replaces: quantization/algorithms/error_feedback.py:72-75 for step == 1 (division of the
  * lower factor's columns by its diagonal, flip back, contiguous copy). */
 int mk_unit_upper_from_factor(const float *factor, float *out, int width, void *stream);

@@ -35,15 +35,15 @@ struct BlockArgs {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
+__device__ __forceinline__ float lane_value(float x, int lane) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), lane));
+}
+
 constexpr int kTile = 16;                       // rows and columns of a tile
 constexpr int kTiles = kBlock / kTile;          // tile columns of the block
 constexpr int kWaves = kThreads / 64;
 constexpr int kCarried = kWaves * kTile;        // columns a workgroup carries beside the block
 constexpr int kColumnFloats = kTile + 4;        // a tile column in LDS (16-byte aligned, banks spread)
-
-__device__ __forceinline__ float lane_value(float x, int lane) {
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), lane));
-}
 
 // In: the upper triangle of a symmetric positive definite block.  Out: U with block = U^T U
 // in the upper triangle, zeros below it.  A pivot that is not positive (or not finite)
@@ -53,96 +53,171 @@ __device__ __forceinline__ float lane_value(float x, int lane) {
 // operations and so become U_jj^-T A_jr, the block row of the factor.  Every workgroup factors the block
 // itself (from the matrix, which nobody overwrites: the factor goes to `factor_out`), and the first one stores it.
 //
-// Right-looking over panels of 16 rows.  The block and the carried columns are 16 x 16 tiles (negated) in the
-// accumulators of four wavefronts, wavefront w owning tile columns 3 - w, 4 + w and, beside the block, w.  Per panel:
-//   1. the owners put the panel's tiles into LDS by columns;
-//   2. a lane takes a column of 16 values into registers, lanes 0 ... 15 of EVERY wavefront the diagonal tile's, the
-//      other lanes those of the wavefront's three tiles, and all 16 elimination steps run inside the wavefront: row j is
-//      scaled by 1 / sqrt(pivot), row i > j loses U[j][i] (a scalar, from lane i) times row j;
-//   3. the finished rows go back to LDS, and the tiles below lose U_r^T U_c on the matrix cores.  A 16 x 16 x 4
-//      accumulator holds rows 4 (lane / 16) + i of a column where the operands hold k = lane / 16, so product i takes
-//      k = 4 (lane / 16) + i and a tile is read as an operand exactly as it is held: one 16-byte LDS read.  A panel's sixteen
-//      products are summed first and subtracted in one addition, so an entry is rounded at most 7 + 15 times on its way (128
-//      times in a running accumulator, which left the coefficients of 1024 columns 4.1e-7 from 64 bits; now 2.6e-7, 3.3e-7
-//      with the two-column kernel below).
-// Two barriers per 16 columns (one per two columns before, with every pivot row passed through LDS): what
-// bounds the kernel is the chain of 128 pivots.  One copy of the code serves all panels, since a
-// launch runs it once and instruction fetches would show.  A block with 768 columns beside it, called back to back: 25 us
-// (48 us a launch as a pair of columns per barrier); carrying the 64 columns costs 3 us of that.
+// Right-looking over panels of 16 rows, by two sets of four wavefronts.  The second set holds the block and the carried
+// columns as 16 x 16 tiles (negated) in its accumulators, wavefront w of it tile columns 3 - w, 4 + w and, beside the block, w;
+// the first eliminates, its wavefront w the columns of the same tiles.  Per panel:
+//   1. the tiles' owners put the panel's row of tiles into LDS by columns; barrier;
+//   2. a lane of the first set takes a column of 16 values into registers, lanes 0 ... 15 of EVERY wavefront the diagonal
+//      tile's, the other lanes those of the wavefront's three tiles, and all 16 elimination steps run inside the wavefront: row
+//      j is scaled by 1 / sqrt(pivot), row i > j loses U[j][i] (a scalar, from lane i) times row j.  Finished rows go back to
+//      LDS four at a time; barrier;
+//   3. the next row of tiles loses U_r^T U_c on the matrix cores and goes out as in 1; barrier.  The other rows, and the
+//      finished rows' way to memory, follow beside the next elimination.
+// A 16 x 16 x 4 accumulator holds rows 4 (lane / 16) + i of a column where the operands hold k = lane / 16, so product i takes
+// k = 4 (lane / 16) + i and a tile is read as an operand exactly as it is held: one 16-byte LDS read.  A panel's sixteen
+// products are summed first and subtracted in one addition, so an entry is rounded at most 7 + 15 times on its way (128
+// times in a running accumulator, which left the coefficients of 1024 columns 4.1e-7 from 64 bits; now 2.6e-7, 3.3e-7
+// with the two-column kernel below).
+//
+// What bounds the kernel is the chain of 128 pivots: a panel takes about 4000 cycles, 1550 of them elimination (up to 2700
+// while the other set's products share the SIMD), 700 the products it waits for.  One copy of the code serves all panels, since
+// a launch runs it once and instruction fetches would show.  A block with 768 columns beside it, called back to back: 17.9 us;
+// with one set of four wavefronts doing all of it in turn 24.9 (2200 cycles a panel went into the stores alone, and as many
+// into products that nobody waited for yet).  The rows' factors as row broadcasts instead of scalars, with the diagonal tile
+// in all lanes: 26.8 (the broadcasts do not become part of the multiply-adds).  A pair of columns per barrier: 48.
 template <bool ROW>
-__global__ void __launch_bounds__(kThreads, 2) cholesky_block_kernel(const BlockArgs a) {
+__global__ void __launch_bounds__(2 * kThreads, 2) cholesky_block_kernel(const BlockArgs a) {
+    __builtin_amdgcn_s_setprio(3);   // in front of a trailing update that runs beside it
     __shared__ __align__(16) float panel[2][kTiles + kWaves][kTile][kColumnFloats];   // [buffer][tile column][column][row]
-    __shared__ int failed;
-    if (threadIdx.x == 0) failed = *a.status;
+    // (in the padding: 30720 bytes of LDS go beside two workgroups of a trailing update, one word more does not)
+    int &failed = reinterpret_cast<int &>(panel[1][0][0][kTile]), &stopped = reinterpret_cast<int &>(panel[1][0][0][kTile + 1]);
+    if (threadIdx.x == 0) failed = *a.status, stopped = 0;
     const int n = a.size;
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & (kWaves - 1));
+    const bool eliminating = __builtin_amdgcn_readfirstlane(threadIdx.x / kThreads) == 0;
     const int column = lane & 15, quarter = lane >> 4;
     const int left_column = kWaves - 1 - wave, right_column = wave + kWaves;
     const int carried_first = kCarried * static_cast<int>(blockIdx.x) + kTile * wave;   // of this wavefront, counted from the block's end
-
-    // tiles of row r: tile column 3 - wave (r <= 3), tile column wave + 4, the carried ones
-    f32x4 left[kWaves], right[kTiles], beside[kTiles];
     // Addresses are clamped into the block instead of guarded: a branch per load would wait for each of them in turn.
     const uint32_t leading = static_cast<uint32_t>(a.leading), last = static_cast<uint32_t>(n - 1);
-    auto block_tile = [&](int r, int c) __attribute__((always_inline)) -> f32x4 {
-        f32x4 tile;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint32_t first = r * kTile + 4 * quarter + i, second = c * kTile + column;
-            const uint32_t row = min(first, second), col = max(first, second);   // the upper triangle stands for both
-            tile[i] = a.matrix[min(row, last) * leading + min(col, last)];
-        }
-        return tile;
-    };
     const uint32_t carried_column = n + min(carried_first + column, a.row_columns - 1);
-#pragma unroll
-    for (int r = 0; r < kTiles; ++r) {
-        if (r < kWaves) left[r] = block_tile(r, left_column);   // (tiles below the diagonal: any numbers, never used)
-        right[r] = block_tile(r, right_column);
-        if constexpr (ROW) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                beside[r][i] = a.matrix[min(static_cast<uint32_t>(r * kTile + 4 * quarter + i), last) * leading + carried_column];
-        }
-    }
-#pragma unroll
-    for (int r = 0; r < kTiles; ++r) {
-        // Outside the block: an identity diagonal keeps every pivot of the padding at one.
-        auto negated = [&](f32x4 &tile, int c) __attribute__((always_inline)) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int row = r * kTile + 4 * quarter + i, col = c * kTile + column;
-                tile[i] = max(row, col) < n ? -tile[i] : (row == col ? -1.0f : 0.0f);
-            }
-        };
-        if (r < kWaves) negated(left[r], left_column);
-        negated(right[r], right_column);
-        if constexpr (ROW) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) beside[r][i] = r * kTile + 4 * quarter + i < n ? -beside[r][i] : 0.0f;
-        }
-    }
-    __syncthreads();
-    if (failed) return;   // an earlier block already did: do nothing
-
+    const int panels = (n + kTile - 1) / kTile;
     float *factor = ROW ? a.factor_out : a.matrix;
     const uint32_t factor_leading = ROW ? kBlock : leading;
-    const int panels = (n + kTile - 1) / kTile;
+
+    if (!eliminating) {   // uniform
+        // tiles of row r: tile column 3 - wave (r <= 3), tile column wave + 4, the carried ones
+        f32x4 left[kWaves], right[kTiles], beside[kTiles];
+        auto block_tile = [&](int r, int c) __attribute__((always_inline)) -> f32x4 {
+            f32x4 tile;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t first = r * kTile + 4 * quarter + i, second = c * kTile + column;
+                const uint32_t row = min(first, second), col = max(first, second);   // the upper triangle stands for both
+                tile[i] = a.matrix[min(row, last) * leading + min(col, last)];
+            }
+            return tile;
+        };
+#pragma unroll
+        for (int r = 0; r < kTiles; ++r) {
+            if (r < kWaves) left[r] = block_tile(r, left_column);   // (tiles below the diagonal: any numbers, never used)
+            right[r] = block_tile(r, right_column);
+            if constexpr (ROW) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    beside[r][i] = a.matrix[min(static_cast<uint32_t>(r * kTile + 4 * quarter + i), last) * leading + carried_column];
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < kTiles; ++r) {
+            // Outside the block: an identity diagonal keeps every pivot of the padding at one.
+            auto negated = [&](f32x4 &tile, int c) __attribute__((always_inline)) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int row = r * kTile + 4 * quarter + i, col = c * kTile + column;
+                    tile[i] = max(row, col) < n ? -tile[i] : (row == col ? -1.0f : 0.0f);
+                }
+            };
+            if (r < kWaves) negated(left[r], left_column);
+            negated(right[r], right_column);
+            if constexpr (ROW) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) beside[r][i] = r * kTile + 4 * quarter + i < n ? -beside[r][i] : 0.0f;
+            }
+        }
+        auto publish = [&](int r) __attribute__((always_inline)) {   // row r of the wavefront's tiles, by columns
+            float (*tiles)[kTile][kColumnFloats] = panel[r & 1];
+            auto put = [&](int tile_column, f32x4 tile) __attribute__((always_inline)) {
+                *reinterpret_cast<f32x4 *>(&tiles[tile_column][column][4 * quarter]) = -tile;
+            };
+            if (r < kWaves) put(left_column, left[r]);
+            put(right_column, right[r]);
+            if constexpr (ROW) put(wave + kTiles, beside[r]);
+        };
+        publish(0);
+        __syncthreads();
+        if (failed) return;   // an earlier block already did: do nothing
+#pragma unroll 1
+        for (int s = 0; s + 1 < panels; ++s) {
+            __builtin_amdgcn_s_setprio(3);   // the other wavefronts wait
+            __syncthreads();   // the finished rows of panel s are there
+            if (stopped) return;
+            float (*tiles)[kTile][kColumnFloats] = panel[s & 1];
+            auto operand = [&](int tile_column) __attribute__((always_inline)) -> f32x4 {
+                return *reinterpret_cast<const f32x4 *>(&tiles[tile_column][column][4 * quarter]);
+            };
+            // what the next elimination waits for: tile row s + 1
+            const f32x4 next = operand(s + 1), u_left = operand(left_column), u_right = operand(right_column), u_beside = operand(ROW ? wave + kTiles : wave);
+            f32x4 from_left = {}, from_right = {}, from_beside = {};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                from_left = __builtin_amdgcn_mfma_f32_16x16x4f32(next[i], u_left[i], from_left, 0, 0, 0);
+                from_right = __builtin_amdgcn_mfma_f32_16x16x4f32(next[i], u_right[i], from_right, 0, 0, 0);
+                if constexpr (ROW) from_beside = __builtin_amdgcn_mfma_f32_16x16x4f32(next[i], u_beside[i], from_beside, 0, 0, 0);
+            }
+#pragma unroll
+            for (int r = 1; r < kTiles; ++r)
+                if (r == s + 1) {   // uniform
+                    if (r < kWaves) left[r] += from_left;
+                    right[r] += from_right;
+                    if constexpr (ROW) beside[r] += from_beside;
+                    publish(r);
+                }
+            __syncthreads();
+            // Beside that elimination: what panel s takes from the rows behind, and its finished rows to memory.
+            __builtin_amdgcn_s_setprio(2);
+#pragma unroll
+            for (int r = 2; r < kTiles; ++r) {
+                if (r <= s + 1) continue;   // uniform, as all the conditions here
+                const f32x4 row_operand = operand(r);
+                auto products = [&](f32x4 u) __attribute__((always_inline)) -> f32x4 {
+                    f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) sum = __builtin_amdgcn_mfma_f32_16x16x4f32(row_operand[i], u[i], sum, 0, 0, 0);
+                    return sum;
+                };
+                if (r < kWaves && r <= left_column) left[r] += products(u_left);   // (tiles below the diagonal are not needed)
+                if (r <= right_column) right[r] += products(u_right);
+                if constexpr (ROW) beside[r] += products(u_beside);
+            }
+            const int row = s * kTile + 4 * quarter;   // of this lane's first value
+            if (blockIdx.x == 0) {   // uniform
+                auto store = [&](int tile_column, f32x4 tile) __attribute__((always_inline)) {
+                    const int to = tile_column * kTile + column;
+                    if (tile_column == s) tile = operand(s);   // (finished behind the barrier)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        if (row + i < n && to < n) factor[(row + i) * factor_leading + to] = to >= row + i ? tile[i] : 0.0f;
+                };
+                store(left_column, u_left);
+                store(right_column, u_right);
+            }
+            if constexpr (ROW) {
+                if (carried_first + column < a.row_columns) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        if (row + i < n) a.matrix[(row + i) * leading + carried_column] = u_beside[i];
+                }
+            }
+        }
+        return;
+    }
+
+    __syncthreads();
+    if (failed) return;
 #pragma unroll 1
     for (int s = 0; s < panels; ++s) {
         float (*tiles)[kTile][kColumnFloats] = panel[s & 1];
-        auto publish = [&](int tile_column, f32x4 tile) __attribute__((always_inline)) {
-            *reinterpret_cast<f32x4 *>(&tiles[tile_column][column][4 * quarter]) = -tile;
-        };
-#pragma unroll
-        for (int r = 0; r < kTiles; ++r)
-            if (r == s) {
-                if (r < kWaves) publish(left_column, left[r]);
-                publish(right_column, right[r]);
-                if constexpr (ROW) publish(wave + kTiles, beside[r]);
-            }
-        __syncthreads();
-
         // a column of the panel per lane
         const int own = quarter == 1 ? left_column : wave + kWaves * (quarter - 1);   // tile column of lanes 16 ... 63
         float *source = tiles[quarter == 0 ? s : own][column];
@@ -153,11 +228,15 @@ __global__ void __launch_bounds__(kThreads, 2) cholesky_block_kernel(const Block
 #pragma unroll
             for (int k = 0; k < 4; ++k) value[4 * i + k] = four[k];
         }
-        uint32_t refused = 0;
+        auto keep = [&](int first, int stop) __attribute__((always_inline)) {   // finished rows, four at a time
+#pragma unroll
+            for (int i = first; i < stop; ++i)
+                reinterpret_cast<f32x4 *>(source)[i] = f32x4{value[4 * i], value[4 * i + 1], value[4 * i + 2], value[4 * i + 3]};
+        };
+        float pivot = 1.0f;   // of this lane's column
         auto reciprocal_root = [&](int j) __attribute__((always_inline)) -> float {
-            const float pivot = lane_value(value[j], j);
-            refused |= static_cast<uint32_t>(__float_as_int(pivot)) - 1u < 0x7f7fffffu ? 0u : 1u << j;   // positive and finite
-            return __builtin_amdgcn_rsqf(pivot);   // accurate to an ulp; an IEEE square root and division would double the chain
+            pivot = lane == j ? value[j] : pivot;
+            return __builtin_amdgcn_rsqf(lane_value(value[j], j));   // accurate to an ulp; an IEEE square root and division would double the chain
         };
         float reciprocal = reciprocal_root(0);
 #pragma unroll
@@ -172,20 +251,26 @@ __global__ void __launch_bounds__(kThreads, 2) cholesky_block_kernel(const Block
             for (int i = j + 2; i < kTile; ++i) factors[i] = lane_value(value[j], i);
 #pragma unroll
             for (int i = j + 2; i < kTile; ++i) value[i] = __builtin_fmaf(-factors[i], value[j], value[i]);
+            // (the diagonal tile later: another wavefront may still have to read it as it was)
+            if ((j & 3) == 3 && quarter > 0 && own != s && (ROW || quarter < 3)) keep(j / 4, j / 4 + 1);
             // step by step: put off, as the compiler would have it, the updates of a row are one dependent chain
             __builtin_amdgcn_sched_barrier(0);
         }
-        if (refused) {   // every wavefront of every workgroup comes to the same value
+        const uint64_t accepted = __builtin_amdgcn_ballot_w64(static_cast<uint32_t>(__float_as_int(pivot)) - 1u < 0x7f7fffffu);   // positive and finite
+        const uint32_t refused = ~static_cast<uint32_t>(accepted) & 0xffffu;
+        if (refused) {   // every eliminating wavefront of every workgroup comes to the same value
             if (threadIdx.x == 0) *a.status = a.first_column + s * kTile + __builtin_ctz(refused) + 1;
+            stopped = 1;
+            if (s + 1 < panels) __syncthreads();   // the others read it behind this barrier
             return;
         }
-        // (the diagonal tile stays as it is: another wavefront may still have to read it)
-        if (s + 1 < panels && quarter > 0 && own != s && (ROW || quarter < 3)) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                reinterpret_cast<f32x4 *>(source)[i] = f32x4{value[4 * i], value[4 * i + 1], value[4 * i + 2], value[4 * i + 3]};
+        if (s + 1 < panels) {
+            __syncthreads();
+            if (quarter == 0 && wave == 0) keep(0, 4);
+            __syncthreads();   // the next panel's rows are there
+            continue;
         }
-        // The finished rows: lanes 0 ... 15 of the diagonal tile's owner, and the other tiles from their columns' lanes.
+        // The last panel's rows: lanes 0 ... 15 of the diagonal tile's owner, and the other tiles from their columns' lanes.
         if (blockIdx.x == 0 && (quarter == 0 ? s == left_column || s == right_column : quarter < 3 && own != s)) {
             const int to = (quarter == 0 ? s : own) * kTile + column;
             if (to < n) {
@@ -204,31 +289,6 @@ __global__ void __launch_bounds__(kThreads, 2) cholesky_block_kernel(const Block
                     if (row < n) a.matrix[row * leading + carried_column] = value[j];
                 }
             }
-        }
-        if (s + 1 == panels) return;
-        __syncthreads();
-
-        auto operand = [&](int tile_column) __attribute__((always_inline)) -> f32x4 {
-            return *reinterpret_cast<const f32x4 *>(&tiles[tile_column][column][4 * quarter]);
-        };
-        const f32x4 u_left = operand(left_column), u_right = operand(right_column), u_beside = operand(ROW ? wave + kTiles : wave);
-        f32x4 rows[kTiles];
-#pragma unroll
-        for (int r = 1; r < kTiles; ++r) rows[r] = operand(r);
-#pragma unroll
-        for (int r = 1; r < kTiles; ++r) {
-            if (r <= s) continue;   // uniform
-            auto products = [&](f32x4 u) __attribute__((always_inline)) -> f32x4 {
-                f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-                for (int i = 0; i < 4; ++i) sum = __builtin_amdgcn_mfma_f32_16x16x4f32(rows[r][i], u[i], sum, 0, 0, 0);
-                return sum;
-            };
-            // (on tiles below the diagonal too, whose numbers nothing reads: skipping those puts a branch, and a full wait for
-            // the products, in front of every addition)
-            if (r < kWaves) left[r] += products(u_left);
-            right[r] += products(u_right);
-            if constexpr (ROW) beside[r] += products(u_beside);
         }
     }
 }
@@ -472,20 +532,25 @@ __global__ void __launch_bounds__(256) reversed_matrix_kernel(const ReverseArgs 
     }
 }
 
-// out[a][b] = U[w-1-b][w-1-a] / U[w-1-b][w-1-b]: the factor transposed, every column divided by
-// its diagonal entry, both index orders reversed; 32 x 32 tiles turned in LDS so that reads and
-// writes both run along rows.
+// out[a][b] = U[w-1-b][w-1-a] / U[w-1-b][w-1-b] on and above the diagonal, zero below it: the factor transposed, every
+// column divided by its diagonal entry, both index orders reversed; 32 x 32 tiles turned in LDS so that reads and writes both
+// run along rows.  Tiles below the diagonal are not read.
 __global__ void __launch_bounds__(256) unit_upper_kernel(const float *factor, float *out, int width) {
     __shared__ float tile[32][33];
     const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;   // 8 rows of 32 threads
     const int r0 = blockIdx.y * 32, c0 = blockIdx.x * 32;
+    if (blockIdx.x >= blockIdx.y) {   // uniform
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int r = r0 + ty + 8 * j, c = c0 + tx;
-        const bool inside = r < width && c < width;
-        const float value = factor[static_cast<size_t>(inside ? r : 0) * width + (inside ? c : 0)];
-        const float pivot = factor[static_cast<size_t>(inside ? r : 0) * (width + 1)];
-        tile[ty + 8 * j][tx] = inside ? __fdiv_rn(value, pivot) : 0.0f;
+        for (int j = 0; j < 4; ++j) {
+            const int r = r0 + ty + 8 * j, c = c0 + tx;
+            const bool inside = r < width && c < width && r <= c;
+            const float value = factor[static_cast<size_t>(inside ? r : 0) * width + (inside ? c : 0)];
+            const float pivot = factor[static_cast<size_t>(inside ? r : 0) * (width + 1)];
+            tile[ty + 8 * j][tx] = inside ? __fdiv_rn(value, pivot) : 0.0f;
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) tile[ty + 8 * j][tx] = 0.0f;
     }
     __syncthreads();
 #pragma unroll
@@ -540,9 +605,9 @@ extern "C" int mk_cholesky_block(float *matrix, long long leading, int size, int
     if (int refused = check_block(matrix, leading, size, first_column, row_columns, factor_out, status)) return refused;
     BlockArgs a{matrix, leading, size, first_column, status, row_columns, factor_out};
     if (row_columns > 0)
-        hipLaunchKernelGGL((cholesky_block_kernel<true>), dim3(mk_cdiv(row_columns, kCarried)), dim3(kThreads), 0, stream, a);
+        hipLaunchKernelGGL((cholesky_block_kernel<true>), dim3(mk_cdiv(row_columns, kCarried)), dim3(2 * kThreads), 0, stream, a);
     else
-        hipLaunchKernelGGL((cholesky_block_kernel<false>), dim3(1), dim3(kThreads), 0, stream, a);
+        hipLaunchKernelGGL((cholesky_block_kernel<false>), dim3(1), dim3(2 * kThreads), 0, stream, a);
     MK_LAUNCH_CHECK("mk_cholesky_block");
     return MK_OK;
 }

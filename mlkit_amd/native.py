@@ -110,6 +110,8 @@ SIGNATURES: dict[str, tuple[Any, list[Any]]] = {
     ]),
     "mk_cholesky_block": (_c_int, [_c_void_p, _c_longlong, _c_int, _c_int, _c_int, _c_void_p, _c_void_p, _c_void_p]),
     "mk_cholesky_block_pairs": (_c_int, [_c_void_p, _c_longlong, _c_int, _c_int, _c_int, _c_void_p, _c_void_p, _c_void_p]),
+    "mk_factor_block_rows": (_c_int, [_c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p]),
+    "mk_factor_trailing": (_c_int, [_c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p]),
     "mk_rotate_blocks": (_c_int, [
         _c_void_p, _c_int, _c_void_p, _c_int, _c_longlong, _c_int, _c_int, _c_void_p, _c_int, _c_void_p,
         _c_void_p, _c_float, _c_void_p,

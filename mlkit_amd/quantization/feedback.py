@@ -37,17 +37,22 @@ DEFERRED_TILES = 4  # tiles whose far-column updates are applied in one pass on 
 
 
 # Narrower matrices (less than one block) go to the library factorisation.  From here on blocks are faster and no less exact:
-# coefficients of 128 / 256 / 512 / 896 columns 0.12 / 0.15 / 0.25 / 0.42 ms against 0.26 / 0.65 / 1.34 / 2.47 with the library,
-# relative error against 64 bits at 128 / 384 / 640 / 896 columns 1.3e-7 / 1.8e-7 / 2.5e-7 / 3.0e-7 against 2.5e-7 / 4.0e-7 /
-# 4.3e-7 / 4.4e-7.
+# coefficients of 384 / 896 columns 0.15 / 0.25 ms against 1.1 / 2.5 with the library, relative error against 64 bits
+# 1.5e-7 / 1.9e-7 against 4.0e-7 / 4.4e-7.
 BLOCKED_FACTORIZATION_WIDTH = 128
 # Steps of several columns (vector grids) keep the arithmetic their conversions have had -- the library below this width and the
 # two-column block kernel from it on: a code for eight weights that the last bit of a coefficient turns takes its row along.
 STEPPED_FACTORIZATION_WIDTH = 1024
 FACTORIZATION_BLOCK = 128           # one workgroup factors a diagonal block of this size
-FACTORIZATION_PANEL = 1024          # rank of the trailing updates of the whole matrix
-TRAILING_BAND = 1024                # rows per product of a trailing update (only the upper triangle is needed)
-LOOK_AHEAD_WIDTH = 8192             # from here on the far part of a trailing update runs on a second stream
+# Rank of the trailing updates of the whole matrix: a small one keeps the chain of block kernels and products short, a large one
+# reads and writes the matrix less often.  Panels of 256 / 512 / 1024: 4096 columns 1046 / 1063 us, 6000 1913 / 1956, 8184
+# 3447 / 3392 / 3663, 11008 6585 / 6174 / 6731.
+FACTORIZATION_PANEL = 256
+WIDE_FACTORIZATION_WIDTH = 7168     # from here on panels of twice that
+STEPPED_FACTORIZATION_PANEL = 1024  # the same for steps of several columns
+# Columns left behind a panel: from here on the far part of its update runs on a second stream (11008 / 8184 columns 6174 /
+# 3392 us, 6601 / 3578 without; with fewer left the events cost what the second stream hides).
+LOOK_AHEAD_WIDTH = 3072
 
 
 def _factor_in_place(matrix: Tensor, status: Tensor, factored: Tensor, pairs: bool = False) -> None:
@@ -55,17 +60,12 @@ def _factor_in_place(matrix: Tensor, status: Tensor, factored: Tensor, pairs: bo
     in place (``status``: an int32 device scalar holding zero; ``factored``: scratch for the
     diagonal blocks, ``[ceil(width / 128), 128, 128]``).
 
-    Two levels of blocking.  Panels of 1024 columns update the rest of the matrix, right-looking (a
-    rank-1024 product reads and writes the trailing matrix an eighth as often as rank-128 ones
-    would).  Inside a panel 128-column blocks are factored left-looking: a block's rows first take
-    the updates of all earlier blocks of the panel in one product, then ``mk_cholesky_block``
-    factors the diagonal block and carries the rest of its rows, to the last column, through the
-    same elimination, which makes them the factor's block row; no triangular solve is left.  (The
-    chain block kernel -> product -> block kernel is what bounds the run time; right-looking blocks
-    with the far rows of each update on a stream of their own made it 7 % longer: every block then
-    waited for two products.)  The factored diagonal blocks themselves are needed by nobody before
-    the end (updates read block rows only): they wait in ``factored`` and go into the matrix in one
-    copy.
+    Two levels of blocking.  Panels of 256 columns update the rest of the matrix, right-looking (``mk_factor_trailing``).
+    Inside a panel 128-column blocks are factored left-looking: a block's rows first take the updates of all earlier blocks of
+    the panel in one product (``mk_factor_block_rows``), then ``mk_cholesky_block`` factors the diagonal block and carries the
+    rest of its rows, to the last column, through the same elimination, which makes them the factor's block row; no triangular
+    solve is left.  The factored diagonal blocks themselves are needed by nobody before the end (updates read block rows only):
+    they wait in ``factored`` and go into the matrix in one copy.
 
     Look-ahead between panels: only the band of rows the next panel consists of is updated on the
     current stream; the rest runs on a second stream while the next panel is factored.  Events fix
@@ -81,28 +81,20 @@ def _factor_in_place(matrix: Tensor, status: Tensor, factored: Tensor, pairs: bo
 
     width = matrix.shape[0]
     device = matrix.device
-    factor_block = native.library().mk_cholesky_block_pairs if pairs else native.library().mk_cholesky_block
+    library = native.library()
+    factor_block = library.mk_cholesky_block_pairs if pairs else library.mk_cholesky_block
     main = torch.cuda.current_stream(device)
-    look_ahead = width >= LOOK_AHEAD_WIDTH   # narrower: the event traffic costs more than it hides
-    side = torch.cuda.Stream(device) if look_ahead else None    # far rows of a panel's update
+    panel = STEPPED_FACTORIZATION_PANEL if pairs else FACTORIZATION_PANEL * (2 if width >= WIDE_FACTORIZATION_WIDTH else 1)
+    side = torch.cuda.Stream(device) if width >= LOOK_AHEAD_WIDTH + panel else None   # far rows of a panel's update
 
-    def subtract_outer_product(start: int, stop: int, first_row: int, last_row: int, limit: int, after_first_band=None):
-        """A[r, c] -= sum_k U[k, r] U[k, c] for k in start:stop, rows first_row:last_row, columns from
-        the row band's first column to ``limit``: bands of rows, so that little below the diagonal
-        is computed (what is, is never read).  ``after_first_band`` (a stream): returns an event
-        recorded on it behind the first band."""
-        event = None
-        for band_start in range(first_row, last_row, TRAILING_BAND):
-            band_stop = min(last_row, band_start + TRAILING_BAND)
-            matrix[band_start:band_stop, band_start:limit].addmm_(
-                matrix[start:stop, band_start:band_stop].T, matrix[start:stop, band_start:limit], alpha=-1.0)
-            if after_first_band is not None and event is None:
-                event = after_first_band.record_event()
-        return event
+    def update_rows(start: int, stop: int, first_row: int, last_row: int, stream: int, leave_room: bool = False) -> None:
+        """A[r, c] -= sum_k U[k, r] U[k, c] for k in start:stop, rows first_row:last_row, columns from the row on."""
+        if first_row < last_row:
+            native.check(library.mk_factor_trailing(matrix.data_ptr(), width, start, stop, first_row, last_row, int(leave_room), stream))
 
     side_done = band_done = None
-    for panel_start in range(0, width, FACTORIZATION_PANEL):
-        panel_stop = min(width, panel_start + FACTORIZATION_PANEL)
+    for panel_start in range(0, width, panel):
+        panel_stop = min(width, panel_start + panel)
         raw_stream = native.current_stream(device)
         for start in range(panel_start, panel_stop, FACTORIZATION_BLOCK):
             stop = min(panel_stop, start + FACTORIZATION_BLOCK)
@@ -110,8 +102,8 @@ def _factor_in_place(matrix: Tensor, status: Tensor, factored: Tensor, pairs: bo
                 # the block's rows take the updates of every earlier block of the panel at once: one
                 # product of rank start - panel_start, over all columns to the right (what a triangular
                 # solve with the panel's whole diagonal block would otherwise do for them)
-                matrix[start:stop, start:width].addmm_(matrix[panel_start:start, start:stop].T,
-                                                       matrix[panel_start:start, start:width], alpha=-1.0)
+                native.check(library.mk_factor_block_rows(matrix.data_ptr(), width, panel_start, start, start, stop, int(pairs),
+                                                          raw_stream))
             # the block kernel also carries the rest of rows start:stop, to the matrix's last column,
             # through the elimination (their block row of the factor); the factored block goes to
             # `factored`, since every workgroup of that launch reads the block itself
@@ -119,26 +111,32 @@ def _factor_in_place(matrix: Tensor, status: Tensor, factored: Tensor, pairs: bo
             slot = factored[start // FACTORIZATION_BLOCK]
             native.check(factor_block(matrix[start, start:].data_ptr(), width, stop - start, start, beside,
                                       slot.data_ptr() if beside else None, status.data_ptr(), raw_stream))
-        # the diagonal block's lower triangle holds leftovers of the products above
-        matrix[panel_start:panel_stop, panel_start:panel_stop].triu_()
+        if pairs:   # the diagonal block's lower triangle holds leftovers of the products above
+            matrix[panel_start:panel_stop, panel_start:panel_stop].triu_()
         if panel_stop == width:
             break
-        if not look_ahead:
-            subtract_outer_product(panel_start, panel_stop, panel_stop, width, width)
+        if width - panel_stop < LOOK_AHEAD_WIDTH:   # too little left for what the events cost
+            if side_done is not None:
+                main.wait_event(side_done)
+                side_done = None
+            update_rows(panel_start, panel_stop, panel_stop, width, raw_stream)
             continue
+        assert side is not None
         row_ready = main.record_event()
         # the rows of the next panel: here, after the second stream's earlier update of them (its
         # first band: the stream works through the bands from the top, and through the panels in
         # order, so that band being done means every earlier update of these rows is)
-        next_panel_stop = min(width, panel_stop + FACTORIZATION_PANEL)
+        next_panel_stop = min(width, panel_stop + panel)
         if band_done is not None:
             main.wait_event(band_done)
-        subtract_outer_product(panel_start, panel_stop, panel_stop, next_panel_stop, width)
+        update_rows(panel_start, panel_stop, panel_stop, next_panel_stop, raw_stream)
         if next_panel_stop < width:
             side.wait_event(row_ready)
-            with torch.cuda.stream(side):
-                band_done = subtract_outer_product(panel_start, panel_stop, next_panel_stop, width, width, after_first_band=side)
-                side_done = side.record_event()
+            band_stop = min(width, next_panel_stop + panel)
+            update_rows(panel_start, panel_stop, next_panel_stop, band_stop, side.cuda_stream, True)
+            band_done = side.record_event()
+            update_rows(panel_start, panel_stop, band_stop, width, side.cuda_stream, True)
+            side_done = side.record_event()
     if side_done is not None:
         main.wait_event(side_done)
     # the factored diagonal blocks (all but a last block that has no columns beside it, factored in place)

@@ -455,6 +455,46 @@ def test_a_factored_block_names_its_bad_pivot(column, value):
     assert block_factor(matrix, 128, first=256)[2] == 256 + column + 1
 
 
+@pytest.mark.parametrize("width,k_first,k_stop,row_first,row_stop", [
+    (200, 0, 128, 128, 200), (129, 0, 128, 128, 129), (517, 128, 384, 384, 512), (1000, 0, 256, 256, 384), (4300, 0, 128, 128, 256)])
+@pytest.mark.parametrize("one_chain", [0, 1])
+def test_products_of_a_block_of_rows(width, k_first, k_stop, row_first, row_stop, one_chain):
+    """`mk_factor_block_rows`: rows and columns that fill no tile, both tile widths; every sum within its rounding bound of 64
+    bits ((k + 1) half ulps of the magnitudes added), everything else untouched."""
+    check_products("mk_factor_block_rows", width, k_first, k_stop, row_first, row_stop, one_chain, triangular=False)
+
+
+@pytest.mark.parametrize("width,k_first,k_stop,row_first,row_stop", [
+    (130, 0, 64, 64, 130), (321, 64, 128, 128, 321), (600, 0, 256, 256, 600), (700, 0, 128, 128, 300), (1031, 512, 768, 768, 1031),
+    (5700, 0, 64, 64, 5700), (5701, 0, 64, 64, 5701)])
+@pytest.mark.parametrize("leave_room", [0, 1])
+def test_products_behind_a_panel(width, k_first, k_stop, row_first, row_stop, leave_room):
+    """`mk_factor_trailing`: both tile sizes, on 16-byte boundaries and off them, all rows behind the panel and a band of them."""
+    check_products("mk_factor_trailing", width, k_first, k_stop, row_first, row_stop, leave_room, triangular=True)
+
+
+def check_products(entry, width, k_first, k_stop, row_first, row_stop, option, triangular):
+    from mlkit_amd import native
+
+    generator = torch.Generator(device="cuda").manual_seed(width + k_stop)
+    matrix = torch.randn((width, width), device="cuda", generator=generator)
+    result = matrix.clone()
+    native.check(getattr(native.library(), entry)(result.data_ptr(), width, k_first, k_stop, row_first, row_stop, option,
+                                                  native.current_stream(matrix.device)))
+    finished = matrix[k_first:k_stop].double()
+    rows = finished[:, row_first:row_stop]
+    expected = matrix[row_first:row_stop].double() - rows.T @ finished
+    bound = (k_stop - k_first + 1) * 2.0**-24 * (matrix[row_first:row_stop].abs().double() + rows.abs().T @ finished.abs())
+    column, row = torch.arange(width, device="cuda"), torch.arange(row_first, row_stop, device="cuda")[:, None]
+    changed = column >= (row if triangular else torch.full_like(row, row_first))
+    got = result[row_first:row_stop]
+    assert ((got.double() - expected).abs() <= bound)[changed].all()
+    if triangular:   # tiles below the diagonal are skipped; what lies below it inside a diagonal tile may change
+        changed = column >= row_first + (row - row_first) // 128 * 128
+    assert torch.equal(got[~changed], matrix[row_first:row_stop][~changed])
+    assert torch.equal(result[:row_first], matrix[:row_first]) and torch.equal(result[row_stop:], matrix[row_stop:])
+
+
 @pytest.mark.parametrize("width,step", [(128, 1), (129, 1), (255, 1), (384, 8), (640, 1), (896, 1), (1000, 2), (1023, 1)])
 def test_blocked_factorisation_of_narrow_matrices(width, step):
     """The same comparison as for wide matrices, from the narrowest one that is factored by blocks."""
