@@ -291,6 +291,11 @@ int mk_fwht(const void *source, int source_dtype, void *target, int target_dtype
 int mk_basis_mix(const float *source, float *target, const float *basis, long long rows, int order,
                  int power, int transpose, const float *signs_after, void *stream);
 
+/* The same for larger bases (order up to 8192) of blocks of a power of two of at least four values; source, target and
+ * signs_after 16-byte aligned. */
+int mk_basis_product(const float *source, float *target, const float *basis, long long rows, int order, int power,
+                     int transpose, const float *signs_after, void *stream);
+
 /* Diagonal-block step of a blocked Cholesky factorisation: the upper triangle of the
  * symmetric positive definite size x size block at `matrix` (row-major, `leading` floats per
  * row, size <= 128) yields U with block = U^T U.  With row_columns == 0 (one workgroup) U

@@ -609,6 +609,9 @@ struct MixArgs {
 // (dynamically indexed registers would live in scratch memory); consecutive lanes take
 // consecutive p, and the basis entries are wavefront-uniform scalar loads.
 constexpr int kMaxOrder = 256;
+// A wavefront's registers hold the basis; the kernel of basis_products.hip beyond (5120 x 2816 as 20 blocks: 44 us here, 54
+// there; 2816 x 5120 as 44 blocks 114 us with two register tiles, 44 there).
+constexpr int kMaxRegisterOrder = 32;
 
 __global__ void __launch_bounds__(256) basis_mix_kernel(const MixArgs a) {
     extern __shared__ float columns_tile[];  // [order][blockDim.x]
@@ -632,29 +635,25 @@ __global__ void __launch_bounds__(256) basis_mix_kernel(const MixArgs a) {
     }
 }
 
-// The same product on the fp32 matrix cores for bases of up to 96 rows.  One wavefront
-// owns 32 adjacent columns p of one row r: the basis (zero-padded to TILES x 32 rows) is
+// The same product on the fp32 matrix cores for bases of up to 32 rows.  One wavefront
+// owns 32 adjacent columns p of one row r: the basis (zero-padded to 32 rows) is
 // the left operand, kept in registers; the right operand comes straight from global memory,
 // lanes 0..31 reading 32 adjacent p of block f and lanes 32..63 of block f + 1, so no LDS is
 // involved.  v_mfma_f32_32x32x2_f32 accumulates over ascending f from zero, which equals
 // the fused multiply-add chain of basis_mix_kernel bit for bit.
-template <int TILES>
 __global__ void __launch_bounds__(256) basis_mix_mfma_kernel(const MixArgs a) {
-    constexpr int kMaxPairs = TILES * 16;  // k-pairs of a basis padded to TILES * 32
+    constexpr int kMaxPairs = kMaxRegisterOrder / 2;
     const int lane = threadIdx.x & 63;
     const int half = lane >> 5, within = lane & 31;
     const int pairs = (a.order + 1) >> 1;
-    // left[t][q]: mix[32 t + within][2 q + half]
-    float left[TILES][kMaxPairs];
+    float left[kMaxPairs];   // mix[within][2 q + half]
 #pragma unroll
-    for (int t = 0; t < TILES; ++t)
-#pragma unroll
-        for (int q = 0; q < kMaxPairs; ++q) {
-            const int out = 32 * t + within, in = 2 * q + half;
-            const bool inside = out < a.order && in < a.order;
-            const int index = a.transpose ? in * a.order + out : out * a.order + in;
-            left[t][q] = inside ? a.basis[inside ? index : 0] : 0.0f;
-        }
+    for (int q = 0; q < kMaxPairs; ++q) {
+        const int in = 2 * q + half;
+        const bool inside = within < a.order && in < a.order;
+        const int index = a.transpose ? in * a.order + within : within * a.order + in;
+        left[q] = inside ? a.basis[inside ? index : 0] : 0.0f;
+    }
     const int tiles_per_row = (a.power + 31) >> 5;
     const long long total = a.rows * tiles_per_row;
     const long long first = static_cast<long long>(blockIdx.x) * (blockDim.x >> 6) + (threadIdx.x >> 6);
@@ -672,33 +671,29 @@ __global__ void __launch_bounds__(256) basis_mix_mfma_kernel(const MixArgs a) {
             const float loaded = a.source[base + static_cast<size_t>(inside ? in : 0) * a.power];
             right[q] = inside ? loaded : 0.0f;
         }
+        mk_mix16 sums;
 #pragma unroll
-        for (int t = 0; t < TILES; ++t) {
-            mk_mix16 sums;
+        for (int r = 0; r < 16; ++r) sums[r] = 0.0f;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) sums[r] = 0.0f;
+        for (int q = 0; q < kMaxPairs; ++q)
+            if (q < pairs) sums = __builtin_amdgcn_mfma_f32_32x32x2f32(left[q], right[q], sums, 0, 0, 0);
 #pragma unroll
-            for (int q = 0; q < kMaxPairs; ++q)
-                if (q < pairs) sums = __builtin_amdgcn_mfma_f32_32x32x2f32(left[t][q], right[q], sums, 0, 0, 0);
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int out = 32 * t + (r >> 2) * 8 + half * 4 + (r & 3);
-                if (out < a.order && column_ok) {
-                    float value = sums[r];
-                    if (a.signs_after) value *= a.signs_after[out * a.power + p];
-                    a.target[base + static_cast<size_t>(out) * a.power] = value;
-                }
+        for (int r = 0; r < 16; ++r) {
+            const int out = (r >> 2) * 8 + half * 4 + (r & 3);
+            if (out < a.order && column_ok) {
+                float value = sums[r];
+                if (a.signs_after) value *= a.signs_after[out * a.power + p];
+                a.target[base + static_cast<size_t>(out) * a.power] = value;
             }
         }
     }
 }
 
-template <int TILES>
 void launch_mix_mfma(const MixArgs &a, hipStream_t stream) {
     const long long tiles = a.rows * ((a.power + 31) / 32);
     long long blocks = (tiles + 3) / 4;
     if (blocks > 256 * 16) blocks = 256 * 16;
-    hipLaunchKernelGGL((basis_mix_mfma_kernel<TILES>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, a);
+    hipLaunchKernelGGL(basis_mix_mfma_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, a);
 }
 
 }  // namespace
@@ -792,13 +787,17 @@ extern "C" int mk_basis_mix(const float *source, float *target, const float *bas
     if (rows == 0) return MK_OK;
     MK_REQUIRE(source && target && basis, MK_ERR_INVALID, "mk_basis_mix: null tensor pointer");
     MK_REQUIRE(source != target, MK_ERR_INVALID, "mk_basis_mix: source and target must not alias");
+    const auto aligned = [](const void *pointer) { return (reinterpret_cast<uintptr_t>(pointer) & 15u) == 0; };
+    if (order > kMaxRegisterOrder && power >= 4 && (power & (power - 1)) == 0 && aligned(source) && aligned(target) && aligned(signs_after)) {
+        int log_power = 0;
+        while ((1 << log_power) < power) ++log_power;
+        if (int status = mk_basis_product_launch(source, target, basis, rows, order, log_power, transpose, signs_after, stream)) return status;
+        MK_LAUNCH_CHECK("mk_basis_mix");
+        return MK_OK;
+    }
     MixArgs a{source, target, basis, signs_after, rows, order, power, transpose};
-    if (order <= 32) {
-        launch_mix_mfma<1>(a, stream);
-    } else if (order <= 64) {
-        launch_mix_mfma<2>(a, stream);
-    } else if (order <= 96) {
-        launch_mix_mfma<3>(a, stream);
+    if (order <= kMaxRegisterOrder) {
+        launch_mix_mfma(a, stream);
     } else {
         // One LDS column of `order` floats per thread: fewer threads for larger bases (64 KB).
         const int threads = order <= 128 ? 128 : 64;

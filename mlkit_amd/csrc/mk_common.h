@@ -39,6 +39,9 @@ static inline int mk_gcd(int a, int b) {
 int mk_fit_scales_strided(const float *value, long long row_stride, float *scales, float *zeros,
                           long long out_row_stride, int rows, int span, int group, int asym, float reciprocal,
                           float value_minimum, int scale_format, int store_zero, hipStream_t stream);
+// basis_products.hip: the product for large bases; blocks of 2^log_power >= 4 values, 16-byte aligned tensors.
+int mk_basis_product_launch(const float *source, float *target, const float *basis, long long rows, int order, int log_power, int transpose,
+                            const float *signs_after, hipStream_t stream);
 // vector_feedback.hip: one tile of the error-feedback sweep over a vector grid.
 int mk_round_vector_tile(const float *original, const float *feedback, const float *coeff, const float *scales,
                          const float *codebook, float *output, float *deviation_t, int32_t *encoded, int rows, int width,

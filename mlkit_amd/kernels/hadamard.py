@@ -89,6 +89,9 @@ def turned(matrix: Tensor) -> Tensor:
     return output
 
 
+LARGE_ORDER = 256   # of mk_basis_mix
+
+
 def mix_blocks(value: Tensor, basis: Tensor, *, transpose: bool, signs_after: Tensor | None = None) -> Tensor:
     """``out[..., f', p] = sum_f mix[f', f] * value[..., f, p]`` with ``mix = basis`` or ``basis.T``."""
     device = native.require_device(value, basis, signs_after)
@@ -99,7 +102,13 @@ def mix_blocks(value: Tensor, basis: Tensor, *, transpose: bool, signs_after: Te
         raise ValueError("basis must be a contiguous FP32 [order, order] matrix")
     output = torch.empty_like(value)
     rows = value.numel() // (order * power)
-    native.check(native.library().mk_basis_mix(
+    if order > LARGE_ORDER and power >= 4 and value.data_ptr() % 16 == 0:
+        product = native.library().mk_basis_product
+        if signs_after is not None and signs_after.data_ptr() % 16:
+            signs_after = signs_after.clone()
+    else:
+        product = native.library().mk_basis_mix
+    native.check(product(
         value.data_ptr(), output.data_ptr(), basis.data_ptr(), rows, order, power, int(transpose),
         native.pointer(signs_after), native.current_stream(device),
     ))

@@ -122,6 +122,9 @@ SIGNATURES: dict[str, tuple[Any, list[Any]]] = {
     "mk_basis_mix": (_c_int, [
         _c_void_p, _c_void_p, _c_void_p, _c_longlong, _c_int, _c_int, _c_int, _c_void_p, _c_void_p,
     ]),
+    "mk_basis_product": (_c_int, [
+        _c_void_p, _c_void_p, _c_void_p, _c_longlong, _c_int, _c_int, _c_int, _c_void_p, _c_void_p,
+    ]),
     "mk_feedback_round_tile": (_c_int, [
         _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_void_p,
         _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float,

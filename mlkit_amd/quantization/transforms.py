@@ -17,7 +17,12 @@ from torch import Tensor
 
 _KERNEL_DTYPES = {torch.float32, torch.float16, torch.bfloat16}
 MAXIMUM_KERNEL_WIDTH = 32768
-MAXIMUM_KERNEL_ORDER = 256
+MAXIMUM_KERNEL_ORDER = 8192               # of mk_basis_product
+MAXIMUM_KERNEL_ORDER_SHORT_BLOCKS = 256   # of mk_basis_mix, which alone takes blocks of one or two values
+
+
+def _order_on_kernel(order: int, power: int) -> bool:
+    return order <= (MAXIMUM_KERNEL_ORDER if power >= 4 else MAXIMUM_KERNEL_ORDER_SHORT_BLOCKS)
 
 
 def _on_kernel(value: Tensor) -> bool:
@@ -147,14 +152,17 @@ def rotate(value: Tensor, *, inverse: bool = False, signs: Tensor | None = None,
     if block is not None:
         return _rotate_blocks_separately(value, block, inverse, signs)
     order, power, basis = transform_factor(value.shape[-1])
-    if not (_on_kernel(value) and power <= MAXIMUM_KERNEL_WIDTH and order <= MAXIMUM_KERNEL_ORDER):
+    if not (_on_kernel(value) and power <= MAXIMUM_KERNEL_WIDTH and _order_on_kernel(order, power)):
         if signs is not None and not inverse:
             value = value * signs
         out = _structured_on_host(value, order, power, basis, inverse)
         return out * signs if signs is not None and inverse else out
     from mlkit_amd.kernels import hadamard as kernel
 
+    result_dtype = value.dtype
     if signs is not None:
+        if order > MAXIMUM_KERNEL_ORDER_SHORT_BLOCKS:   # (as in tensor operations, which such bases took: FP32 signs make FP32 of 16 bits)
+            result_dtype = torch.promote_types(value.dtype, signs.dtype)
         signs = signs.to(device=value.device, dtype=torch.float32).contiguous()
     before, after = (None, signs) if inverse else (signs, None)
     value = value.contiguous()
@@ -174,7 +182,7 @@ def rotate(value: Tensor, *, inverse: bool = False, signs: Tensor | None = None,
     staged = torch.empty(blocks.shape, device=value.device, dtype=torch.float32)
     kernel.transform(blocks, signs_before=before, out=staged)
     mixed = kernel.mix_blocks(staged, _basis_on(value.shape[-1], value.device), transpose=inverse, signs_after=after)
-    return mixed.reshape(value.shape).to(value.dtype)
+    return mixed.reshape(value.shape).to(result_dtype)
 
 
 COLUMN_KERNEL_ROWS = frozenset({1024, 2048, 4096})   # columns that one workgroup transforms without turning the matrix
@@ -206,7 +214,7 @@ def rotate_columns_in_type(matrix: Tensor, *, signs: Tensor, inverse: bool = Fal
     its columns, and whatever the stages in tensor operations make of it where they do not."""
     if matrix.dtype not in (torch.float16, torch.bfloat16) or not columns_on_kernel(matrix, signs):
         return rotate_columns(matrix, signs=signs, inverse=inverse)
-    if transform_factor(matrix.shape[0])[0] > MAXIMUM_KERNEL_ORDER:
+    if not _order_on_kernel(*transform_factor(matrix.shape[0])[:2]):
         return rotate(matrix.T.contiguous(), inverse=inverse, signs=signs).T
     return rotate_columns(matrix, signs=signs, inverse=inverse).to(matrix.dtype)
 

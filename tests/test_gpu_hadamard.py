@@ -356,6 +356,54 @@ def test_a_rotated_basis_is_entered_in_fp32(rows, dtype):
     assert left.dtype == back.dtype and torch.equal(left, back)
 
 
+@pytest.mark.parametrize("rows,order,power", [
+    (1, 33, 4), (3, 43, 64), (70, 64, 128), (5, 65, 512), (130, 97, 8), (33, 129, 4), (1, 380, 16), (700, 204, 32), (9, 1040, 8),
+    (2100, 60, 16)])
+@pytest.mark.parametrize("transpose", [False, True])
+def test_mixing_with_large_bases(rows, order, power, transpose):
+    """More than 32 blocks: small and large tiles, blocks shorter and longer than a tile, edges in all three directions.  Every
+    sum within its rounding bound of 64 bits ((order + 1) half ulps of the magnitudes added)."""
+    from mlkit_amd.kernels import hadamard
+
+    generator = torch.Generator(device="cuda").manual_seed(rows + order)
+    value = torch.randn((rows, order, power), device="cuda", generator=generator)
+    basis = torch.randn((order, order), device="cuda", generator=generator)
+    signs = (torch.rand(order * power + 1, device="cuda", generator=generator) < 0.5).float()[1:] * 2 - 1   # off 16 bytes
+    mix = (basis.T if transpose else basis).double()
+    expected = torch.matmul(mix, value.double())
+    bound = (order + 1) * 2.0**-24 * torch.matmul(mix.abs(), value.double().abs())
+    for given in (None, signs, signs.clone()):
+        out = hadamard.mix_blocks(value, basis, transpose=transpose, signs_after=given)
+        exact = expected if given is None else expected * given.double().reshape(order, power)
+        assert ((out.double() - exact).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("width", [736, 1472, 4992, 6080])   # bases of 368, 368, 312 and 380 rows, blocks of 2, 4, 16 and 16
+@pytest.mark.parametrize("rows", [1, 19, 300])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_rotations_with_bases_of_more_than_256_rows(width, rows, dtype):
+    """There and back against 64 bits, with fp32 signs and without any.  fp32 results: rounding of width additions at most; 16
+    bits: of the result."""
+    from mlkit_amd.quantization import transforms as device_transforms
+    from mlkit_amd.quantization.codecs import deterministic_signs
+
+    order, power, basis = device_transforms.transform_factor(width)
+    value = torch.randn((rows, width), device="cuda").to(dtype)
+    signs = deterministic_signs(width, 3, value.device)
+    hadamard = device_transforms.hadamard(torch.eye(power, dtype=torch.float64)).cuda()
+    whole = torch.kron(basis.double().cuda(), hadamard)
+    step = {torch.float32: width * 2.0**-24, torch.float16: 2.0**-10, torch.bfloat16: 2.0**-7}
+    for inverse in (False, True):
+        for given in (signs, None):
+            out = device_transforms.rotate(value, inverse=inverse, signs=given)
+            flips = 1 if given is None else given
+            expected = (value.double() @ whole) * flips if inverse else (value.double() * flips) @ whole.T
+            assert out.dtype == (dtype if given is None else torch.float32)   # as the same operations on tensors have it
+            # (blocks of two values go through tensor operations, which round 16-bit ones on the way: width 736)
+            allowed = step[dtype] if power < 4 else step[out.dtype]
+            assert (out.double() - expected).norm() <= allowed * expected.norm()
+
+
 @pytest.mark.parametrize("rows,columns", [(1, 1), (3, 70), (64, 64), (65, 4), (100, 132), (260, 68)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 def test_turning_a_matrix(rows, columns, dtype):
