@@ -1,5 +1,4 @@
-// Packed scalar-codec matrix-vector product: planning, the word-at-a-time kernel for
-// layouts the chunked kernel does not take, and the C entry points.
+// Packed scalar-codec matrix-vector product: planning and the C entry points.
 //
 // Replaces the reference's `matrix_vector` wrapper and direct launch
 // (kernels/packed_linear.py:181-226, inference/packed_linear.py:181-245 in
@@ -22,75 +21,15 @@ using mk_matvec::kChunkCodes;
 using mk_matvec::kMaxTableEntries;
 using mk_matvec::MatvecArgs;
 using mk_matvec::Plan;
+using mk_matvec::WordArgs;
+
+constexpr int kChunkedSamples = 4;                   // the chunked kernel's (plan_chunked)
+constexpr long long kChunkedWeights = 1ll << 25;
 
 int next_pow2(int v) {
     int p = 1;
     while (p < v) p <<= 1;
     return p;
-}
-
-// ---------------------------------------------------------------------------------
-// Word-at-a-time kernel for every layout the chunked kernel does not take: one
-// wavefront per row, lanes stride over packing words assembled from bytes.
-// ---------------------------------------------------------------------------------
-struct WordArgs {
-    const void *x;
-    const uint8_t *packed;
-    const void *scales;
-    const void *zeros;
-    const float *values;
-    const void *bias;
-    void *y;
-    int samples, rows, width, group, groups;
-    int first_row;  // rows [first_row, rows) are multiplied
-    int x_dtype, scale_dtype, bias_dtype;
-    int bits, bytes_per_word, codes_per_word, uniform;
-    float grid_min, grid_step;
-};
-
-__global__ void packed_matvec_words_kernel(const WordArgs a) {
-    const int lane = threadIdx.x & 63;
-    const int row = a.first_row + blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-    const int sample_base = blockIdx.y * 8;
-    if (row >= a.rows) return;
-    const int row_words = a.width / a.codes_per_word;
-    const uint8_t *row_ptr = a.packed + static_cast<size_t>(row) * row_words * a.bytes_per_word;
-    const uint64_t mask = (1ull << a.bits) - 1ull;
-    float acc[8];
-#pragma unroll
-    for (int m = 0; m < 8; ++m) acc[m] = 0.0f;
-    for (int word = lane; word < row_words; word += 64) {
-        uint64_t bits = 0;
-        for (int b = 0; b < a.bytes_per_word; ++b)
-            bits |= static_cast<uint64_t>(row_ptr[static_cast<size_t>(word) * a.bytes_per_word + b]) << (8 * b);
-        for (int i = 0; i < a.codes_per_word; ++i) {
-            const int k = word * a.codes_per_word + i;
-            const uint32_t code = static_cast<uint32_t>((bits >> (i * a.bits)) & mask);
-            const size_t slot = static_cast<size_t>(row) * a.groups + k / a.group;
-            float weight = a.uniform ? a.grid_min + static_cast<float>(code) * a.grid_step
-                                     : a.values[code];
-            weight *= mk_load_as_float(a.scales, slot, a.scale_dtype);
-            if (a.zeros) weight += mk_load_as_float(a.zeros, slot, a.scale_dtype);
-#pragma unroll
-            for (int m = 0; m < 8; ++m) {
-                const int sample = sample_base + m;
-                if (sample < a.samples)
-                    acc[m] = __builtin_fmaf(
-                        weight, mk_load_as_float(a.x, static_cast<size_t>(sample) * a.width + k, a.x_dtype),
-                        acc[m]);
-            }
-        }
-    }
-#pragma unroll
-    for (int m = 0; m < 8; ++m) {
-        const float total = mk_segment_sum<64>(acc[m]);
-        const int sample = sample_base + m;
-        if (lane == 0 && sample < a.samples) {
-            float result = total;
-            if (a.bias) result += mk_load_as_float(a.bias, row, a.bias_dtype);
-            mk_store_from_float(a.y, static_cast<size_t>(sample) * a.rows + row, a.x_dtype, result);
-        }
-    }
 }
 
 // Dynamic LDS of one workgroup: value table, fp32 scale (and zero) tile, per-wave row sums.
@@ -101,7 +40,7 @@ size_t lds_bytes_for(const Plan &p, int groups, bool uniform, bool has_zero) {
     if (tile_slots < 4u * p.threads) tile_slots = 4u * p.threads;  // kStaged * threads
     size_t floats = (uniform ? 0 : kMaxTableEntries) + 2 * tile_slots;
     floats += tile_rows > static_cast<size_t>(p.threads) ? tile_rows : p.threads;  // bias tile
-    const int group_rows = p.sample_tile >= 8 ? 1 : (p.sample_tile == 4 ? 2 : 4);
+    const int group_rows = p.sample_tile == 4 ? 2 : 4;
     floats += 2 * static_cast<size_t>(group_rows) * p.sample_tile * p.threads;  // per-lane sums, two buffers
     return floats * sizeof(float);
 }
@@ -124,7 +63,11 @@ const Tuning &tuning() {
 
 // Chooses the lane/row decomposition of the chunked kernel; returns false when the
 // layer needs the word kernel (widths or groups that are not multiples of 32 codes,
-// or a scale tile that does not fit in LDS).
+// or a scale tile that does not fit in LDS) or is faster there: short layers, where a workgroup's fixed cost counts, and more
+// samples than four.  fp32 x, 1 / 2 / 4 / 8 samples, us here against us there: INT8 4096 x 4096 8.5 / 12.0 / 19.1 / 26.2
+// against 8.0 / 8.5 / 9.9 / 14.5, 4096 x 14336 16.9 / 19.7 / 26.4 / 49.5 against 24.2 / 26.5 / 30.7 / 44.5, 22016 x 8192 42 /
+// 54 / 73 / 129 against 64 / 70 / 81 / 113; NF4 1024 x 1024 16 / 24 / 41 / 40 against 5.3 / 5.6 / 6.2 / 7.4, 14336 x 4096 17.0 /
+// 22.4 / 33.0 / 62 against 19.7 / 25.0 / 30.8 / 44; 2- and 3-bit codes alike.
 //
 // A row's chunks are spread over `seg` lanes (a power of two up to 64, or whole
 // wavefronts), one chunk per lane, two when a row has more than 512 chunks.  Every
@@ -134,6 +77,7 @@ const Tuning &tuning() {
 bool plan_chunked(int samples, int rows, int width, int group, int groups, int bits, int x_dtype,
                   bool uniform, bool has_zero, Plan &p) {
     if (bits < 2 || width % kChunkCodes != 0) return false;
+    if (samples > kChunkedSamples || static_cast<long long>(rows) * width <= kChunkedWeights) return false;
     if (group % kChunkCodes != 0 && group < width) return false;
     const int chunks_per_row = width / kChunkCodes;
     int c = chunks_per_row > 512 ? 2 : 1;
@@ -164,22 +108,20 @@ bool plan_chunked(int samples, int rows, int width, int group, int groups, int b
     return true;
 }
 
-// Rows [first_row, output_width) through the word-at-a-time kernel.
+// Rows [first_row, output_width) through the word kernel.
 int launch_words(const void *x, int x_dtype, const uint8_t *packed, const void *scales, int scale_dtype,
-                 const float *values, const void *zeros, const void *bias, int bias_dtype, void *y, int samples,
+                 const float *values, int n_values, const void *zeros, const void *bias, int bias_dtype, void *y, int samples,
                  int output_width, int input_width, int group, int bits, int uniform, float grid_min,
                  float grid_step, int first_row, hipStream_t stream) {
-    const int divisor = mk_gcd(bits, 8);
-    WordArgs w;
-    w.x = x; w.packed = packed; w.scales = scales; w.zeros = zeros; w.values = values; w.bias = bias;
-    w.y = y; w.samples = samples; w.rows = output_width; w.width = input_width; w.group = group;
+    WordArgs w{};
+    w.x = x; w.packed = packed; w.scales = scales; w.zeros = zeros; w.values = values; w.n_values = n_values; w.bias = bias;
+    w.y = y; w.samples = samples; w.rows = output_width; w.width = input_width;
     w.groups = mk_cdiv(input_width, group); w.first_row = first_row;
-    w.x_dtype = x_dtype; w.scale_dtype = scale_dtype; w.bias_dtype = bias_dtype;
-    w.bits = bits;
-    w.bytes_per_word = bits / divisor; w.codes_per_word = 8 / divisor; w.uniform = uniform;
+    w.pieces_per_group = group >= input_width ? 0 : group / 16;   // (groups shorter than a row are multiples of sixteen codes)
+    w.row_bytes = static_cast<size_t>(input_width) * bits / 8;
+    w.x_dtype = x_dtype; w.scale_dtype = scale_dtype; w.bias_dtype = bias_dtype; w.uniform = uniform;
     w.grid_min = grid_min; w.grid_step = grid_step;
-    dim3 grid(mk_cdiv(output_width - first_row, 4), mk_cdiv(samples, 8));
-    hipLaunchKernelGGL(packed_matvec_words_kernel, grid, dim3(256), 0, stream, w);
+    mk_matvec::words_launch(w, bits, stream);
     MK_LAUNCH_CHECK("mk_packed_matvec");
     return MK_OK;
 }
@@ -301,7 +243,7 @@ extern "C" int mk_packed_matvec(const void *x, int x_dtype, const uint8_t *packe
         }
     }
     if (done_rows < output_width)
-        return launch_words(x, x_dtype, packed, scales, scale_dtype, values, zeros, bias, bias_dtype, y, samples,
+        return launch_words(x, x_dtype, packed, scales, scale_dtype, values, n_values, zeros, bias, bias_dtype, y, samples,
                             output_width, input_width, group, bits, uniform, grid_min, grid_step, done_rows, stream);
     return MK_OK;
 }
@@ -384,7 +326,7 @@ extern "C" int mk_packed_matvec_group(const void *const *x, int x_dtype, int cou
             covered += more;
         }
         if (covered < output_widths[i])
-            if (int status = launch_words(x[i], x_dtype, packed[i], scales[i], scale_dtype, values, members.member[i].zeros,
+            if (int status = launch_words(x[i], x_dtype, packed[i], scales[i], scale_dtype, values, n_values, members.member[i].zeros,
                                           members.member[i].bias, bias_dtype, y[i], samples, output_widths[i],
                                           input_width, group, bits, uniform, grid_min, grid_step, covered, stream))
                 return status;

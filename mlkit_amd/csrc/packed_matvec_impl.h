@@ -153,6 +153,24 @@ inline int resident_workgroups(Kernel kernel, int threads, size_t dynamic_lds, s
 }
 
 // Pair-table kernel (packed_matvec_pairs.hip): 2-, 3- and 4-bit codes of any scalar grid.
+// packed_matvec_words.hip: rows [first_row, rows) of any layout that mk_packed_layout_supported takes.
+struct WordArgs {
+    const void *x;
+    const uint8_t *packed;
+    const void *scales;
+    const void *zeros;
+    const float *values;
+    const void *bias;
+    void *y;
+    size_t row_bytes;
+    int samples, rows, width, groups, first_row;
+    int pieces_per_group;   // sixteens of codes in a scale group; 0: one group per row
+    int n_values, x_dtype, scale_dtype, bias_dtype, uniform;
+    int waves;              // set by the launcher: wavefronts that share four rows
+    float grid_min, grid_step;
+};
+void words_launch(const WordArgs &a, int bits, hipStream_t stream);
+
 bool pairs_accepts(int width, int group, int bits, int x_dtype, int scale_dtype);
 int pairs_launch(const Stream4Args &a, hipStream_t stream);
 int pairs_launch_group(const Stream4Args &shared, Stream4Group &group, const int *member_rows, int *rows_per_tile,
@@ -1082,7 +1100,7 @@ bool dispatch_tile(const MatvecArgs &a, const Plan &p, hipStream_t stream) {
     }
     MK_CASE(1, 1) MK_CASE(2, 1) MK_CASE(4, 1)
     MK_CASE(1, 2) MK_CASE(2, 2)
-    if constexpr (XT != MK_F32) { MK_CASE(8, 1) MK_CASE(4, 2) }
+    if constexpr (XT != MK_F32) { MK_CASE(4, 2) }
 #undef MK_CASE
     return false;
 }

@@ -325,6 +325,26 @@ def test_streaming_kernels_on_rows_that_do_not_fill_a_wavefront(width, bits, val
             check(run_matvec(layer, x), layer, x)
 
 
+@pytest.mark.parametrize("bits,width,group,rows", [
+    (1, 1000, 32, 3), (1, 24, 16, 9), (2, 1004, 64, 6), (3, 24, 16, 2), (3, 1016, 48, 5), (4, 18, 16, 1), (4, 1002, 128, 7), (4, 2050, 64, 33),
+    (5, 4104, 32, 2), (6, 516, 16, 13), (7, 544, 1040, 6), (8, 17, 16, 4), (8, 777, 128, 11), (8, 4099, 64, 3), (8, 2065, 128, 2050)])
+@pytest.mark.parametrize("samples", [1, 2, 3, 8, 9])
+@pytest.mark.parametrize("dtype,relative", [(torch.float32, 2e-6), (torch.float16, 1e-3), (torch.bfloat16, 8e-3)])
+def test_word_kernel_on_ragged_rows(bits, width, group, rows, samples, dtype, relative):
+    """Rows that are no whole chunks or pieces of codes, at any byte; teams of one to eight wavefronts; tables, uniform grids,
+    offsets and biases.  fp32: two roundings per weight and log2(width) + 16 on the way of a sum, against the output range."""
+    if rows > 1000 and (samples not in (1, 9) or dtype != torch.float32):
+        pytest.skip("one small and one large count of samples on the tall layer")
+    uniform = scaling.int_values(bits) if bits > 1 else np.array([-1, 1], dtype=np.float32)
+    table = np.sort(np.random.default_rng(bits).standard_normal(1 << bits)).astype(np.float32)
+    weight = helpers.normal_weight(rows, width, seed=bits + width)
+    for values, asym in ((uniform, False), (uniform, True), (table, False), (table, True)):
+        layer = helpers.quantised_layer(weight, values, bits=bits, group=group, integer=bits > 1 and values is uniform, asym=asym)
+        x = helpers.activations(samples, width, seed=samples, dtype=dtype)
+        bias = helpers.activations(1, rows, seed=18)[0].to(dtype) if asym else None
+        check(run_matvec(layer, x, bias=bias), layer, x, bias, relative=relative)
+
+
 @pytest.mark.parametrize("name", WIDTHS)
 @pytest.mark.parametrize("out_dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("width", [256, 288, 264])
