@@ -4,8 +4,8 @@
 //             (+ zero[n, k/group]),  every operation a separate fp32 operation.
 //
 // Rows that are whole multiples of 32 codes are decoded a chunk of 32 codes (BITS dwords)
-// per thread: a few wide loads, 32 values from registers, wide stores.  Other layouts take
-// the word kernel: one thread per packing word (the fewest whole bytes holding whole codes).
+// per thread: a few wide loads, 32 values from registers, wide stores.  Other layouts go in
+// pieces of sixteen codes at any byte.
 //
 // Replaces the reference's Triton kernel `decode_rows`
 // (kernels/packed_linear.py:229-276 in /root/reference/src/mlkit).
@@ -13,6 +13,8 @@
 #include "packed_matvec_impl.h"
 
 namespace {
+
+using mk_matvec::kPieceCodes;
 
 struct DecodeArgs {
     const uint8_t *packed;
@@ -22,7 +24,7 @@ struct DecodeArgs {
     void *out;
     int rows, width, group, groups;
     int scale_dtype, out_dtype;
-    int bits, bytes_per_word, codes_per_word, uniform, n_values;
+    int uniform, n_values;
     float grid_min, grid_step;
     int chunks_per_group_shift;   // log2(group / 32) when that is a power of two (31: one group per row), else -1
     const long long *row_index;   // null, or the source row of every output row (a gather of rows)
@@ -37,34 +39,82 @@ __device__ __forceinline__ size_t source_row_of(const DecodeArgs &a, size_t row)
     return wanted >= 0 && wanted < a.source_rows ? static_cast<size_t>(wanted) : 0;
 }
 
-__global__ void packed_decode_kernel(const DecodeArgs a) {
-    const int row_words = a.width / a.codes_per_word;
-    const size_t total = static_cast<size_t>(a.rows) * row_words;
-    const uint64_t mask = (1ull << a.bits) - 1ull;
-    for (size_t word = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; word < total;
-         word += static_cast<size_t>(gridDim.x) * blockDim.x) {
-        const size_t row = word / row_words;
-        const int word_in_row = static_cast<int>(word - row * row_words);
+// Rows that are not whole chunks.  A thread takes a piece of sixteen codes -- 2 BITS bytes, which lie inside one scale group for
+// every layout that mk_packed_layout_supported takes -- and writes sixteen values side by side; a row's last piece, where it
+// is not whole, goes code by code.
+template <int BITS, int OUT>
+__global__ void __launch_bounds__(256) packed_decode_pieces_kernel(const DecodeArgs a) {
+    __shared__ float table[1 << BITS];
+    if (!a.uniform) {
+        for (int i = threadIdx.x; i < (1 << BITS); i += blockDim.x) table[i] = i < a.n_values ? a.values[i] : 0.0f;
+        __syncthreads();
+    }
+    const uint32_t row_pieces = static_cast<uint32_t>((a.width + kPieceCodes - 1) / kPieceCodes);
+    const size_t row_bytes = static_cast<size_t>(a.width) * BITS / 8, total = static_cast<size_t>(a.rows) * row_pieces;
+    for (size_t index = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; index < total; index += static_cast<size_t>(gridDim.x) * blockDim.x) {
+        const size_t row = total < (1ull << 32) ? static_cast<uint32_t>(index) / row_pieces : index / row_pieces;   // (uniform: a division of 32 bits)
+        const int first = static_cast<int>(index - row * row_pieces) * kPieceCodes;
         const size_t from = source_row_of(a, row);
-        const uint8_t *source = a.packed + (from * row_words + word_in_row) * a.bytes_per_word;
-        uint64_t bits = 0;
-        for (int b = 0; b < a.bytes_per_word; ++b) bits |= static_cast<uint64_t>(source[b]) << (8 * b);
-        for (int i = 0; i < a.codes_per_word; ++i) {
-            const int k = word_in_row * a.codes_per_word + i;
-            const uint32_t code = static_cast<uint32_t>((bits >> (i * a.bits)) & mask);
-            const size_t slot = from * a.groups + k / a.group;
-            float weight;
-            if (a.uniform) {
-                const float stepped = __fmul_rn(static_cast<float>(code), a.grid_step);
-                weight = __fadd_rn(a.grid_min, stepped);
-            } else {
-                weight = a.values[code];
+        const uint8_t *source = a.packed + from * row_bytes + static_cast<size_t>(first) * BITS / 8;
+        const size_t slot = from * a.groups + (a.group < a.width ? static_cast<uint32_t>(first) / static_cast<uint32_t>(a.group) : 0u);
+        const float scale = mk_load_as_float(a.scales, slot, a.scale_dtype), zero = a.zeros ? mk_load_as_float(a.zeros, slot, a.scale_dtype) : 0.0f;
+        auto value_of = [&](uint32_t code) __attribute__((always_inline)) -> float {
+            float weight = a.uniform ? __fadd_rn(a.grid_min, __fmul_rn(static_cast<float>(code), a.grid_step)) : table[code];
+            weight = __fmul_rn(weight, scale);
+            return a.zeros ? __fadd_rn(weight, zero) : weight;
+        };
+        if (first + kPieceCodes > a.width) {
+            for (int k = 0; first + k < a.width; ++k) {
+                const int bit = k * BITS;
+                uint32_t word = source[bit >> 3];
+                if ((bit & 7) + BITS > 8) word |= static_cast<uint32_t>(source[(bit >> 3) + 1]) << 8;
+                mk_store_from_float(a.out, row * a.width + first + k, OUT, value_of((word >> (bit & 7)) & ((1u << BITS) - 1u)));
             }
-            weight = __fmul_rn(weight, mk_load_as_float(a.scales, slot, a.scale_dtype));
-            if (a.zeros) weight = __fadd_rn(weight, mk_load_as_float(a.zeros, slot, a.scale_dtype));
-            mk_store_from_float(a.out, row * a.width + k, a.out_dtype, weight);
+            continue;
+        }
+        uint32_t words[mk_matvec::kPieceWords<BITS>];
+        mk_matvec::load_piece<BITS>(words, source);
+        float value[kPieceCodes];
+#pragma unroll
+        for (int k = 0; k < kPieceCodes; ++k) value[k] = value_of(mk_matvec::piece_code<BITS>(words, k));
+        const size_t at = row * a.width + first;
+        if constexpr (OUT == MK_F32) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                mk_matvec::Words4 four;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) four[i] = __float_as_uint(value[4 * q + i]);
+                reinterpret_cast<mk_matvec::Words4 *>(static_cast<float *>(a.out) + at)[q] = four;
+            }
+        } else {
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                mk_matvec::Words4 four;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float low = value[8 * q + 2 * i], high = value[8 * q + 2 * i + 1];
+                    if constexpr (OUT == MK_F16) {
+                        const mk_h2 halves = {static_cast<_Float16>(low), static_cast<_Float16>(high)};
+                        four[i] = __builtin_bit_cast(uint32_t, halves);
+                    } else {
+                        four[i] = static_cast<uint32_t>(mk_float_to_bf16(low)) | (static_cast<uint32_t>(mk_float_to_bf16(high)) << 16);
+                    }
+                }
+                reinterpret_cast<mk_matvec::Words4 *>(static_cast<uint16_t *>(a.out) + at)[q] = four;
+            }
         }
     }
+}
+
+template <int BITS>
+void launch_pieces(const DecodeArgs &a, hipStream_t stream) {
+    const size_t pieces = static_cast<size_t>(a.rows) * mk_cdiv(a.width, kPieceCodes);
+    size_t blocks = (pieces + 255) / 256;
+    if (blocks > 256u * 64u) blocks = 256u * 64u;
+    const dim3 grid(static_cast<unsigned>(blocks)), block(256);
+    if (a.out_dtype == MK_F32) hipLaunchKernelGGL((packed_decode_pieces_kernel<BITS, MK_F32>), grid, block, 0, stream, a);
+    else if (a.out_dtype == MK_F16) hipLaunchKernelGGL((packed_decode_pieces_kernel<BITS, MK_F16>), grid, block, 0, stream, a);
+    else hipLaunchKernelGGL((packed_decode_pieces_kernel<BITS, MK_BF16>), grid, block, 0, stream, a);
 }
 
 
@@ -214,10 +264,9 @@ int decode_rows(const uint8_t *packed, const void *scales, int scale_dtype, cons
     DecodeArgs a;
     a.packed = packed; a.scales = scales; a.zeros = zeros; a.values = values; a.out = out;
     a.rows = output_rows; a.width = input_width; a.group = group; a.groups = mk_cdiv(input_width, group);
-    a.scale_dtype = scale_dtype; a.out_dtype = out_dtype; a.bits = bits;
+    a.scale_dtype = scale_dtype; a.out_dtype = out_dtype;
     a.row_index = row_index; a.source_rows = source_rows;
-    const int divisor = mk_gcd(bits, 8);
-    a.bytes_per_word = bits / divisor; a.codes_per_word = 8 / divisor; a.uniform = uniform;
+    a.uniform = uniform;
     a.grid_min = grid_min; a.grid_step = grid_step;
     a.n_values = n_values;
     a.chunks_per_group_shift = -1;
@@ -246,10 +295,16 @@ int decode_rows(const uint8_t *packed, const void *scales, int scale_dtype, cons
         MK_LAUNCH_CHECK(name);
         return MK_OK;
     }
-    const size_t words = static_cast<size_t>(output_rows) * (input_width / a.codes_per_word);
-    size_t blocks = (words + 255) / 256;
-    if (blocks > 256u * 32u) blocks = 256u * 32u;
-    hipLaunchKernelGGL(packed_decode_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, a);
+    switch (bits) {
+        case 1: launch_pieces<1>(a, stream); break;
+        case 2: launch_pieces<2>(a, stream); break;
+        case 3: launch_pieces<3>(a, stream); break;
+        case 4: launch_pieces<4>(a, stream); break;
+        case 5: launch_pieces<5>(a, stream); break;
+        case 6: launch_pieces<6>(a, stream); break;
+        case 7: launch_pieces<7>(a, stream); break;
+        default: launch_pieces<8>(a, stream); break;
+    }
     MK_LAUNCH_CHECK(name);
     return MK_OK;
 }

@@ -555,6 +555,43 @@ __device__ __forceinline__ uint32_t code_at(const CodeChunk<BITS> &c, int k) {
     return __builtin_amdgcn_alignbit(c.w[(word + 1) % BITS], c.w[word], shift) & mask;
 }
 
+// Sixteen codes, 2 BITS bytes, at any byte.
+constexpr int kPieceCodes = 16;
+template <int BITS>
+constexpr int kPieceWords = (BITS + 1) / 2 + 1;
+
+typedef uint32_t Words4 __attribute__((ext_vector_type(4), aligned(1)));
+typedef uint32_t Words2 __attribute__((ext_vector_type(2), aligned(1)));
+typedef uint32_t Words1 __attribute__((aligned(1)));
+typedef uint16_t Halves1 __attribute__((aligned(1)));
+
+template <int BITS>
+__device__ __forceinline__ void load_piece(uint32_t (&words)[kPieceWords<BITS>], const uint8_t *from) {
+    constexpr int kBytes = 2 * BITS;
+    int at = 0;
+    if constexpr (kBytes >= 16) {
+        const Words4 four = *reinterpret_cast<const Words4 *>(from);
+        words[0] = four.x; words[1] = four.y; words[2] = four.z; words[3] = four.w;
+        at = 4;
+    } else {
+        if constexpr (kBytes >= 8) {
+            const Words2 two = *reinterpret_cast<const Words2 *>(from);
+            words[0] = two.x; words[1] = two.y;
+            at = 2;
+        }
+        if constexpr ((kBytes & 7) >= 4) words[at] = *reinterpret_cast<const Words1 *>(from + 4 * at), ++at;
+        if constexpr ((kBytes & 3) >= 2) words[at] = *reinterpret_cast<const Halves1 *>(from + 4 * at), ++at;
+    }
+    words[at] = 0;   // (a code that ends with the piece's last bit reads one word further)
+}
+
+// Code k (0..15) of a piece, k a compile-time constant after unrolling.
+template <int BITS>
+__device__ __forceinline__ uint32_t piece_code(const uint32_t (&words)[kPieceWords<BITS>], int k) {
+    const int bit = k * BITS, word = bit >> 5, shift = bit & 31;
+    return (shift + BITS <= 32 ? words[word] >> shift : __builtin_amdgcn_alignbit(words[word + 1], words[word], shift)) & ((1u << BITS) - 1u);
+}
+
 // sum_k T[code_k] * x_k for one chunk and MT samples; T = identity (uniform grids,
 // the affine map is applied once per chunk by the caller) or the LDS table.
 template <int BITS, int XT, int MT, bool UNIFORM>

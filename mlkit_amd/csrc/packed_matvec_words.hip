@@ -5,38 +5,14 @@
 
 namespace {
 
-using mk_matvec::lane_exchange;
+using mk_matvec::load_piece;
+using mk_matvec::piece_code;
 using mk_matvec::transposed_value_of_lane;
 using mk_matvec::transposed_wave_sum;
 using mk_matvec::WordArgs;
+using mk_matvec::Words4;
 
-constexpr int kRows = 4, kPiece = 16, kMaxWaves = 8;   // rows and codes of a lane's turn; wavefronts of a workgroup
-
-typedef uint32_t Words4 __attribute__((ext_vector_type(4), aligned(1)));
-typedef uint32_t Words2 __attribute__((ext_vector_type(2), aligned(1)));
-typedef uint32_t Words1 __attribute__((aligned(1)));
-typedef uint16_t Halves1 __attribute__((aligned(1)));
-
-// 2 BITS bytes from any address.
-template <int BITS>
-__device__ __forceinline__ void load_piece(uint32_t (&words)[(BITS + 1) / 2 + 1], const uint8_t *from) {
-    constexpr int kBytes = 2 * BITS;
-    int at = 0;
-    if constexpr (kBytes >= 16) {
-        const Words4 four = *reinterpret_cast<const Words4 *>(from);
-        words[0] = four.x; words[1] = four.y; words[2] = four.z; words[3] = four.w;
-        at = 4;
-    } else {
-        if constexpr (kBytes >= 8) {
-            const Words2 two = *reinterpret_cast<const Words2 *>(from);
-            words[0] = two.x; words[1] = two.y;
-            at = 2;
-        }
-        if constexpr ((kBytes & 7) >= 4) words[at] = *reinterpret_cast<const Words1 *>(from + 4 * at), ++at;
-        if constexpr ((kBytes & 3) >= 2) words[at] = *reinterpret_cast<const Halves1 *>(from + 4 * at), ++at;
-    }
-    words[at] = 0;   // (a code that ends with the piece's last bit reads one word further)
-}
+constexpr int kRows = 4, kPiece = mk_matvec::kPieceCodes, kMaxWaves = 8;   // rows and codes of a lane's turn; wavefronts of a workgroup
 
 template <int XT>
 __device__ __forceinline__ void load_values(float (&value)[kPiece], const void *x, size_t index) {
@@ -98,7 +74,7 @@ __global__ void __launch_bounds__(64 * kMaxWaves) words_kernel(const WordArgs a)
     for (int i = 0; i < kSums; ++i) sums[i] = 0.0f;
     const int pieces = a.width / kPiece, stride = 64 * a.waves;
     for (int piece = 64 * place + lane; piece < pieces; piece += stride) {
-        uint32_t words[kRows][(BITS + 1) / 2 + 1];
+        uint32_t words[kRows][mk_matvec::kPieceWords<BITS>];
         float scale[kRows], zero[kRows], weight[kRows][kPiece];
         const uint32_t group = a.pieces_per_group > 0 ? static_cast<uint32_t>(piece) / static_cast<uint32_t>(a.pieces_per_group) : 0;
 #pragma unroll
@@ -111,9 +87,7 @@ __global__ void __launch_bounds__(64 * kMaxWaves) words_kernel(const WordArgs a)
         for (int r = 0; r < kRows; ++r)
 #pragma unroll
             for (int k = 0; k < kPiece; ++k) {
-                const int bit = k * BITS, word = bit >> 5, shift = bit & 31;
-                const uint32_t code = (shift + BITS <= 32 ? words[r][word] >> shift : __builtin_amdgcn_alignbit(words[r][word + 1], words[r][word], shift))
-                                      & ((1u << BITS) - 1u);
+                const uint32_t code = piece_code<BITS>(words[r], k);
                 const float value = a.uniform ? a.grid_min + static_cast<float>(code) * a.grid_step : table[code];   // uniform
                 weight[r][k] = a.zeros ? value * scale[r] + zero[r] : value * scale[r];
             }

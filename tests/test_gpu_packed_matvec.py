@@ -392,6 +392,37 @@ def test_packed_decode_full_layer_matches_matvec_input():
     np.testing.assert_allclose((x.cuda().float() @ dense.float().T).cpu().numpy(), fused, rtol=2e-3, atol=2e-3)
 
 
+@pytest.mark.parametrize("bits,width,group", [
+    (1, 1000, 32), (2, 1004, 64), (3, 24, 16), (3, 1016, 48), (4, 18, 16), (4, 1002, 128), (5, 520, 32), (6, 516, 16), (7, 1064, 112),
+    (8, 17, 16), (8, 777, 128)])
+@pytest.mark.parametrize("out_dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_decoding_rows_that_are_no_whole_chunks(bits, width, group, out_dtype):
+    """Pieces of sixteen codes at any byte and what is left of a row behind them: the oracle's values and their rounding, all
+    rows and a gather of some (twice the same one, the last, and two outside, which read row 0)."""
+    from mlkit_amd import native
+    from mlkit_amd.kernels import packed_linear
+
+    uniform = scaling.int_values(bits) if bits > 1 else np.array([-1, 1], dtype=np.float32)
+    table = np.sort(np.random.default_rng(bits).standard_normal(1 << bits)).astype(np.float32)
+    weight = helpers.normal_weight(21, width, seed=bits, scale=1.0)
+    for values, asym in ((uniform, False), (uniform, True), (table, True)):
+        layer = helpers.quantised_layer(weight, values, bits=bits, group=group, integer=bits > 1 and values is uniform, asym=asym)
+        tensors = helpers.to_device(layer)
+        grid, minimum, step = helpers.uniform_grid(layer["values"])
+        expected = torch.from_numpy(layer["dense"]).to(out_dtype)
+        dense = torch.empty((21, width), dtype=out_dtype, device="cuda")
+        packed_linear.decode(tensors["packed"], tensors["scales"], tensors["values"], tensors["zeros"], dense, layer["group"],
+                             packed_linear.layout_for(bits, width, layer["group"]), grid, minimum, step)
+        assert torch.equal(dense.cpu(), expected)
+        wanted = torch.tensor([3, 20, 3, -1, 21, -22], device="cuda")
+        some = torch.empty((6, width), dtype=out_dtype, device="cuda")
+        native.check(native.library().mk_packed_decode_rows(
+            tensors["packed"].data_ptr(), tensors["scales"].data_ptr(), native.dtype_code(tensors["scales"]), tensors["values"].data_ptr(),
+            tensors["values"].numel(), native.pointer(tensors["zeros"]), wanted.data_ptr(), 6, some.data_ptr(), native.dtype_code(some), 21,
+            width, layer["group"], bits, int(grid), minimum, step, native.current_stream(some.device)))
+        assert torch.equal(some.cpu(), expected[[3, 20, 3, 20, 0, 0]])
+
+
 @pytest.mark.parametrize("bits,values,integer", [(4, INT4, True), (2, scaling.int_values(2), True),
                                                  (3, scaling.int_values(3), True), (4, scaling.NF4_VALUES, False)])
 @pytest.mark.parametrize("scale_dtype", [torch.float16, torch.bfloat16])
