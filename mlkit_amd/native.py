@@ -164,6 +164,7 @@ SIGNATURES: dict[str, tuple[Any, list[Any]]] = {
 }
 
 _library: ctypes.CDLL | None = None
+_layer_call: tuple | None = None
 
 
 class NativeLibraryMissing(RuntimeError):
@@ -190,6 +191,21 @@ def library() -> ctypes.CDLL:
             function.argtypes = argtypes
         _library = loaded
     return _library
+
+
+def layer_call(layer: "PackedLayer", scales: Tensor, bias: Tensor | None):
+    """The native call of one packed layer whose launch arguments are ``layer`` (``packed_call.cpp``)."""
+    global _layer_call
+    if _layer_call is None:
+        try:
+            from mlkit_amd._packed_call import PackedCall
+        except ImportError as error:
+            raise NativeLibraryMissing(
+                "mlkit_amd._packed_call is missing: build it with `python -m mlkit_amd.build`") from error
+        _layer_call = (PackedCall, *(ctypes.cast(entry, _c_void_p).value for entry in
+                                     (library().mk_packed_layer_matvec, library().mk_packed_layer_matmul)))
+    call, matvec, matmul = _layer_call
+    return call(layer, scales, bias, matvec, matmul)
 
 
 def last_error() -> str:

@@ -344,6 +344,72 @@ class Attention(nn.Module):
         return self.o_proj(mixed)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("bias", [False, True])
+def test_a_bound_layer_calls_natively_and_falls_back(dtype, bias):
+    """The first call goes through Python and binds the native one: both give the same bytes, and whatever is not the plain
+    call (strides, a mode, a replaced buffer, a gradient, a wrong width) still takes the Python path."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    torch.manual_seed(31)
+    linear = nn.Linear(256, 48, bias=bias, device="cuda", dtype=dtype)
+    layer = mk.PackedLinear(linear, mk.int(4, 64, asym=True)(linear.weight.detach()))
+
+    def first(x):
+        layer._launch = None
+        return layer(x)
+
+    shapes = [(256,), (1, 256), (2, 4, 256), (0, 256), (1, 9, 256), (40, 256)]
+    with torch.no_grad():
+        for shape in shapes:
+            x = torch.randn(shape, device="cuda", dtype=dtype)
+            expected, again = first(x), layer(x)
+            assert again.dtype == expected.dtype and again.shape == shape[:-1] + (48,) and torch.equal(again, expected)
+        x = torch.randn(6, 256, device="cuda", dtype=dtype)
+        expected = first(x)
+        native_call = layer._launch[5]
+        assert torch.equal(native_call.matvec(x, layer._buffers, 8), expected)
+        if dtype != torch.float32:
+            assert torch.equal(native_call.matmul(x, layer._buffers, 8), layer._product(x, 6))
+        else:
+            assert native_call.matmul(x, layer._buffers, 8) is None
+        strided = torch.empty(256, 6, device="cuda", dtype=dtype).t().copy_(x)
+        for other in (strided, x[:, :128], x.double(), x.cpu(), x[:0], "x"):
+            assert native_call.matvec(other, layer._buffers, 8) is None
+        assert native_call.matvec(x, layer._buffers, 5) is None
+        assert torch.equal(layer(strided), expected) and torch.equal(layer(nn.Parameter(x)), expected)
+        with TorchDispatchMode():
+            assert native_call.matvec(x, layer._buffers, 8) is None
+        for wrong, error in ((x[:, :128], ValueError), (x.cpu(), ValueError)):
+            with pytest.raises(error):
+                layer(wrong)
+        with pytest.raises(RuntimeError):
+            torch.func.vmap(lambda row: native_call.matvec(row, layer._buffers, 8) or layer(row))(x)
+        # every buffer is compared in every call
+        for name in ("packed", "scales", "values", "zeros", "bias"):
+            held = layer._buffers[name]
+            assert torch.equal(layer(x), expected)
+            if held is not None:
+                layer._buffers[name] = held.clone()
+                assert layer._launch[5].matvec(x, layer._buffers, 8) is None and torch.equal(layer(x), expected)
+                layer._buffers[name] = held
+        layer.scales.data = layer.scales.data * 2   # the same tensor object with other memory
+        doubled = layer(x)
+        assert not torch.equal(doubled, expected) and torch.equal(doubled, first(x))
+        layer.scales = layer.scales / 2
+        assert torch.equal(layer(x), expected)
+        stream = torch.cuda.Stream()
+        stream.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(stream):
+            elsewhere = layer(x)
+        torch.cuda.current_stream().wait_stream(stream)
+        assert torch.equal(elsewhere, expected)
+    with torch.inference_mode():
+        assert layer(x).is_inference()
+    with pytest.raises(RuntimeError, match="autograd"):
+        layer(x.clone().requires_grad_())
+
+
 def test_sibling_layers_share_one_launch():
     """optimize(group_siblings=True): q / k / v (same parent, same input width and codec) are
     linked; the model's output equals the ungrouped packed model bit for bit, for fp16 rows 1..8,
