@@ -3,19 +3,21 @@
 // error-feedback tile that rounds blocks of `dimension` columns.
 //
 // One wavefront owns a row (or a vector): its 64 lanes share out the codebook entries -- four
-// E8P magnitude patterns per lane, or every 64th codeword -- and the winner is found by a
-// reduction over (cost, index) in which the lower index wins ties, which is what a search in
-// ascending order with a strict comparison returns; the reduction moves values between lanes
-// with vector-ALU lane moves only.  Costs are formed in fp32 without fused multiply-adds,
-// coordinates in ascending order.  The magnitude patterns, and any codebook of up to 48 KiB,
-// are staged in LDS once per workgroup.
+// E8P magnitude patterns per lane, or every 64th codeword -- and the winner is the entry of the
+// smallest cost, the lower index on ties, which is what a search in ascending order with a
+// strict comparison returns.  Costs are formed in fp32 without fused multiply-adds (but where
+// the product is exact), coordinates in ascending order.  The magnitude patterns, and any
+// codebook of up to 48 KiB, are staged in LDS once per workgroup.
+//
+// What is done for each entry takes every lane; what is done once for a coordinate (its
+// distance to either coset, its square, the winner's signs, its reconstruction and deviation)
+// takes one lane per coordinate, and what is one number for the row is scalar.
 //
 // In the feedback tile everything a row needs of the tile lives in the wavefront's registers,
-// lane l holding columns l, l + 64, ...: weights, corrections, scales on the way in,
-// reconstructions and codes on the way out (read and written with coalesced accesses before
-// and after the block loop).  A block's values are read out of them with wavefront-uniform
-// lane reads.  Inside the loop the only memory traffic is the block's coefficient rows,
-// requested before its search so that their latency hides behind it.
+// lane l holding columns 2 l and 2 l + 1 (and, in tiles of more than 128 columns, those 128
+// further).  A block's values are read out of them with wavefront-uniform lane reads, its
+// coefficient rows are requested before its search so that their latency hides behind it, and
+// reconstructions, deviations and codes wait in LDS for coalesced writes.
 // An E8P point is rebuilt from its pattern, sign bits and coset instead of being fetched from
 // the 2 MiB table.
 //
@@ -35,144 +37,140 @@ constexpr int kStagedBytes = 48 * 1024;
 
 extern __shared__ __align__(16) float staged[];
 
-// The value lane `lane ^ (1 << STAGE)` holds (DPP inside rows of 16 lanes, v_permlane16_swap /
-// v_permlane32_swap across rows).
-template <int STAGE>
-__device__ __forceinline__ int partner(int bits, int lane) {
-    if constexpr (STAGE == 0) return __builtin_amdgcn_mov_dpp(bits, 0xB1, 0xf, 0xf, true);   // quad_perm [1,0,3,2]
-    else if constexpr (STAGE == 1) return __builtin_amdgcn_mov_dpp(bits, 0x4E, 0xf, 0xf, true);   // quad_perm [2,3,0,1]
-    else if constexpr (STAGE == 2) {
-        int moved = __builtin_amdgcn_update_dpp(bits, bits, 0x104, 0xf, 0x5, false);   // row_shl:4 into lanes 0-3, 8-11
-        return __builtin_amdgcn_update_dpp(moved, bits, 0x114, 0xf, 0xa, false);       // row_shr:4 into lanes 4-7, 12-15
-    } else if constexpr (STAGE == 3) return __builtin_amdgcn_mov_dpp(bits, 0x128, 0xf, 0xf, true);  // row_ror:8
-    else if constexpr (STAGE == 4) {
-        const auto swapped = __builtin_amdgcn_permlane16_swap(bits, bits, false, false);
-        return (lane & 16) ? swapped[0] : swapped[1];
-    } else {
-        const auto swapped = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);
-        return (lane & 32) ? swapped[0] : swapped[1];
-    }
-}
-
-template <int STAGE>
-__device__ __forceinline__ void best_of_pair(float &cost, int &index, int lane) {
-    const float other_cost = __builtin_bit_cast(float, partner<STAGE>(__builtin_bit_cast(int, cost), lane));
-    const int other_index = partner<STAGE>(index, lane);
-    const bool take = other_cost < cost || (other_cost == cost && other_index < index);
-    cost = take ? other_cost : cost;
-    index = take ? other_index : index;
-}
-
-// The smaller cost wins, the smaller index on equal costs; every lane receives the result.
-__device__ __forceinline__ void wave_best(float &cost, int &index, int lane) {
-    best_of_pair<0>(cost, index, lane);
-    best_of_pair<1>(cost, index, lane);
-    best_of_pair<2>(cost, index, lane);
-    best_of_pair<3>(cost, index, lane);
-    best_of_pair<4>(cost, index, lane);
-    best_of_pair<5>(cost, index, lane);
-}
-
-// v_readlane with a wavefront-uniform lane index.
-__device__ __forceinline__ float lane_value(float value, int lane) {
+__device__ __forceinline__ float lane_value(float value, int lane) {   // v_readlane: `lane` is wavefront-uniform
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, value), lane));
 }
 
-// This lane's four magnitude patterns (pattern lane + 64 j), their squared norms and, in bit 31, the parity of their sums.
+template <int CONTROL, int ROWS = 0xf>
+__device__ __forceinline__ int moved(int bits) {
+    return __builtin_amdgcn_update_dpp(bits, bits, CONTROL, ROWS, 0xf, ROWS == 0xf);
+}
+
+// The smallest of the 64 lanes' values, none of them NaN: as integers of the same order, for which a lane move and a minimum
+// are one instruction.
+__device__ __forceinline__ float wave_minimum(float value) {
+    int key = __builtin_bit_cast(int, value);
+    key ^= (key >> 31) & 0x7fffffff;
+    key = min(key, moved<0x128>(key));        // row_ror:8, 4, 2, 1
+    key = min(key, moved<0x124>(key));
+    key = min(key, moved<0x122>(key));
+    key = min(key, moved<0x121>(key));
+    key = min(key, moved<0x142, 0xa>(key));   // row_bcast:15 into rows 1 and 3
+    key = min(key, moved<0x143, 0xc>(key));   // row_bcast:31 into rows 2 and 3
+    key = __builtin_amdgcn_readlane(key, 63);
+    return __builtin_bit_cast(float, key ^ ((key >> 31) & 0x7fffffff));
+}
+
+// This lane's four magnitude patterns (pattern lane + 64 j), their squared norms, what a flip of their cheapest coordinate
+// is to be multiplied by when the signs are even, and the parities of their sums (bit `lane` of parity[j]).
 struct LanePatterns {
     float value[kPatternsPerLane][8];
-    float norm[kPatternsPerLane];
-    uint32_t parity[kPatternsPerLane];
+    float norm[kPatternsPerLane], factor[kPatternsPerLane];
+    uint64_t parity[kPatternsPerLane];
 };
 
-// `patterns`: the 256 x 8 table in LDS.
+struct __attribute__((packed, aligned(4))) Pair {   // one 8-byte load at any float's address
+    float value[2];
+};
+
+struct __attribute__((packed, aligned(4))) Quad {
+    float value[4];
+};
+
+// `patterns`: the 256 x 8 table in global memory (not in LDS: these loads and the staging are in flight together).
 __device__ __forceinline__ void load_patterns(LanePatterns &p, const float *patterns, int lane) {
+#pragma unroll
+    for (int j = 0; j < kPatternsPerLane; ++j)
+#pragma unroll
+        for (int d = 0; d < 8; d += 4) {
+            const Quad quad = *reinterpret_cast<const Quad *>(patterns + (lane + 64 * j) * 8 + d);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) p.value[j][d + i] = quad.value[i];
+        }
 #pragma unroll
     for (int j = 0; j < kPatternsPerLane; ++j) {
         float norm = 0.0f, total = 0.0f;   // (a sum of half-integers: exact)
 #pragma unroll
         for (int d = 0; d < 8; ++d) {
-            const float value = patterns[(lane + 64 * j) * 8 + d];
-            p.value[j][d] = value;
+            const float value = p.value[j][d];
             total += value;
             norm = __fadd_rn(norm, __fmul_rn(value, value));
         }
+        const bool odd = static_cast<int>(total) & 1;
         p.norm[j] = norm;
-        p.parity[j] = static_cast<uint32_t>(static_cast<int>(total)) << 31;
+        p.factor[j] = odd ? 4.0f : 0.0f;
+        p.parity[j] = __ballot(odd);
     }
 }
 
-// Code of the E8P point nearest to v, and the point itself (all lanes hold the same v and
-// receive the same answer).  For either coset every lane scores its four patterns -- the flip of the
-// cheapest coordinate priced in when the pattern's parity disagrees with the signs of v -- the
-// wavefront agrees on the winner of both (index 256 coset + pattern, so that the -1/4 coset stays on a tie),
-// and only then are the winner's parity correction and its first cheapest coordinate worked out, from its row of
-// the table in LDS.
-__device__ __forceinline__ int nearest_lattice_code(const float (&v)[8], const LanePatterns &p, const float *patterns,
-                                                    int lane, float (&point)[8]) {
-    float cost = __builtin_inff();
-    int winner = 0;
+// Code of the E8P point nearest to the vector whose coordinate `lane & 7` is `own`, and that coordinate of the point.  For
+// either coset every lane scores its four patterns -- the flip of the cheapest coordinate priced in when the pattern's parity
+// disagrees with the signs of the vector -- and the first (coset, j, lane) of the smallest cost wins: the lowest index
+// 256 coset + 64 j + lane, so that the -1/4 coset stays on a tie.  Only then are the winner's parity correction and its first
+// cheapest coordinate worked out.
+__device__ __forceinline__ int nearest_lattice_code(float own, const LanePatterns &p, const float *patterns, int lane, float &point) {
+    // lanes 0 to 7 stand for the coset of -1/4, lanes 8 to 15 for that of +1/4
+    const float centered_here = __fsub_rn(own, (lane & 8) ? 0.25f : -0.25f);
+    const float absolute_here = __builtin_fabsf(centered_here), square = __fmul_rn(centered_here, centered_here);
+    const uint32_t below = static_cast<uint32_t>(__ballot(centered_here < 0.0f));   // (a difference of equal numbers is +0)
+    float squares = square;   // lanes 7 and 15: the sum in ascending order
+#pragma unroll
+    for (int d = 1; d < 8; ++d) squares = __fadd_rn(__builtin_bit_cast(float, moved<0x111>(__builtin_bit_cast(int, squares))), square);   // row_shr:1
+    float cost[2 * kPatternsPerLane], smallest = __builtin_inff();
 #pragma unroll
     for (int coset = 0; coset < 2; ++coset) {
-        const float shift = coset == 0 ? -0.25f : 0.25f;
-        float absolute[8], squares = 0.0f;
-        uint32_t signs = 0;   // bit 31: the parity of the negative coordinates
+        const float sum = lane_value(squares, 8 * coset + 7);
+        const float odd = (__builtin_popcount((below >> (8 * coset)) & 255u) & 1) ? 4.0f : 0.0f;
+        float absolute[8];
 #pragma unroll
-        for (int d = 0; d < 8; ++d) {
-            const float centered = __fsub_rn(v[d], shift);
-            absolute[d] = __builtin_fabsf(centered);
-            signs ^= __float_as_uint(centered);   // (a difference of unequal numbers is not -0, of equal ones +0)
-            squares = __fadd_rn(squares, __fmul_rn(centered, centered));
-        }
+        for (int d = 0; d < 8; ++d) absolute[d] = lane_value(absolute_here, 8 * coset + d);
 #pragma unroll
         for (int j = 0; j < kPatternsPerLane; ++j) {
-            float dots = 0.0f, cheapest = __builtin_inff();
+            float dots = __fmul_rn(absolute[0], p.value[j][0]), cheapest = dots;
 #pragma unroll
-            for (int d = 0; d < 8; ++d) {
+            for (int d = 1; d < 8; ++d) {
                 const float product = __fmul_rn(absolute[d], p.value[j][d]);
                 dots = __fadd_rn(dots, product);
                 cheapest = __builtin_fminf(cheapest, product);
             }
-            const bool mismatch = static_cast<int>(signs ^ p.parity[j]) < 0;
-            float candidate = __fsub_rn(__fadd_rn(squares, p.norm[j]), __fmul_rn(2.0f, dots));
-            candidate = __fadd_rn(candidate, mismatch ? __fmul_rn(4.0f, cheapest) : 0.0f);
-            if (candidate < cost) {  // ascending index within the lane
-                cost = candidate;
-                winner = 256 * coset + lane + 64 * j;
-            }
+            // products with 2 and 4 are exact; 0 times the cheapest adds nothing (it is finite wherever the rest is)
+            float candidate = __builtin_fmaf(-2.0f, dots, __fadd_rn(sum, p.norm[j]));
+            candidate = __builtin_fmaf(__builtin_fabsf(__fsub_rn(p.factor[j], odd)), cheapest, candidate);
+            cost[kPatternsPerLane * coset + j] = candidate;
+            smallest = __builtin_fminf(smallest, candidate);   // (NaN is never the smaller)
         }
     }
-    wave_best(cost, winner, lane);
-    // no cost compares below infinity (NaN): pattern 0, no sign bits, the +1/4 coset
-    const bool found = cost < __builtin_inff();
-    const int pattern = found ? winner & 255 : 0;
-    const float shift = found && winner < 256 ? -0.25f : 0.25f;
-    float row[8], total = 0.0f, cheapest = __builtin_inff();
-    int axis = 0, negatives = 0, sign_bits = 0;
+    smallest = wave_minimum(smallest);
+    // no cost below infinity (NaN): pattern 0, no sign bits, the +1/4 coset
+    const bool found = smallest < __builtin_inff();
+    uint64_t lanes = 1;
+    int slot = kPatternsPerLane;
 #pragma unroll
-    for (int d = 0; d < 8; ++d) {
-        row[d] = patterns[pattern * 8 + d];
-        total += row[d];
-        const float centered = __fsub_rn(v[d], shift);
-        const int negative = centered < 0.0f ? 1 : 0;
-        negatives += negative;
-        if (d < 7) sign_bits |= negative << d;
-        const float product = __fmul_rn(__builtin_fabsf(centered), row[d]);
-        if (product < cheapest) {  // the first minimum
-            cheapest = product;
-            axis = d;
+    for (int k = 2 * kPatternsPerLane - 1; k >= 0; --k) {
+        const uint64_t equal = __ballot(cost[k] == smallest);
+        if (found && equal) {
+            lanes = equal;
+            slot = k;
         }
     }
-    const int parity = static_cast<int>(total) & 1;
-    const int flipped = (parity != (negatives & 1) && axis < 7) ? (1 << axis) : 0;
-    const int signs = found ? sign_bits ^ flipped : 0;
-    const int eighth = (__builtin_popcount(signs) + parity) & 1;
-#pragma unroll
-    for (int d = 0; d < 8; ++d) {
-        const int negative = d < 7 ? (signs >> d) & 1 : eighth;
-        point[d] = __fadd_rn(negative ? -row[d] : row[d], shift);
-    }
-    return found ? pattern * 128 + signs + (winner < 256 ? 32768 : 0) : 0;
+    const int holder = __builtin_ctzll(lanes), j = slot & (kPatternsPerLane - 1), pattern = 64 * j + holder;
+    const uint64_t odd = j == 0 ? p.parity[0] : j == 1 ? p.parity[1] : j == 2 ? p.parity[2] : p.parity[3];
+    const int parity = static_cast<int>(odd >> holder) & 1;
+    const float shift = slot < kPatternsPerLane ? -0.25f : 0.25f;
+    const float row = patterns[pattern * 8 + (lane & 7)];
+    const float centered = __fsub_rn(own, shift), product = __fmul_rn(__builtin_fabsf(centered), row);
+    const int magnitude = __builtin_bit_cast(int, product);   // (not negative: ordered as integers)
+    int cheapest = min(magnitude, moved<0xB1>(magnitude));    // quad_perm [1,0,3,2]
+    cheapest = min(cheapest, moved<0x4E>(cheapest));          // quad_perm [2,3,0,1]
+    cheapest = min(cheapest, moved<0x141>(cheapest));         // row_half_mirror
+    const int axis = __builtin_ctz(static_cast<uint32_t>(__ballot(magnitude == cheapest)) | 256u);   // the first minimum
+    const uint32_t negative = static_cast<uint32_t>(__ballot(centered < 0.0f)) & 255u;
+    const bool flips = parity != (__builtin_popcount(negative) & 1) && axis < 7;
+    const uint32_t signs = found ? (negative & 127u) ^ (flips ? 1u << axis : 0u) : 0u;
+    const uint32_t all = signs | ((__builtin_popcount(signs) + parity) & 1) << 7;
+    const uint32_t minus = (all << (31 - (lane & 7))) & 0x80000000u;
+    point = __fadd_rn(__uint_as_float(__float_as_uint(row) ^ minus), shift);
+    return found ? pattern * 128 + static_cast<int>(signs) + (slot < kPatternsPerLane ? 32768 : 0) : 0;
 }
 
 // Index of the nearest of `count` codewords of DIM floats (lowest index on ties).
@@ -193,18 +191,33 @@ __device__ __forceinline__ int nearest_codeword(const float (&v)[DIM], const flo
             index = entry;
         }
     }
-    wave_best(cost, index, lane);
-    return index < count ? index : 0;  // no cost compared below infinity (NaN inputs): the first codeword
+    const float smallest = wave_minimum(cost);
+    if (!(smallest < __builtin_inff())) return 0;  // no cost compared below infinity (NaN inputs): the first codeword
+    uint64_t lanes = __ballot(cost == smallest);
+    int best = 0x7fffffff;
+    do {   // one lane but for ties
+        best = min(best, __builtin_amdgcn_readlane(index, __builtin_ctzll(lanes)));
+        lanes &= lanes - 1;
+    } while (lanes);
+    return best;
 }
 
-// Copies the workgroup's table into LDS: the magnitude patterns of the lattice, or the whole
-// codebook when STAGED says it fits.
+// The workgroup's table, and its copy into LDS: the magnitude patterns of the lattice, or the whole
+// codebook when STAGED says it fits.  Nothing waits here; a barrier has to follow.
 template <int DIM, bool LATTICE, bool STAGED>
-__device__ __forceinline__ void stage_table(const float *codebook, int codebook_size) {
+__device__ __forceinline__ const float *stage_table(const float *codebook, int codebook_size) {
     const float *source = LATTICE ? codebook + static_cast<size_t>(codebook_size) * 8 : codebook;
-    const int floats = LATTICE ? kPatternFloats : (STAGED ? codebook_size * DIM : 0);
-    for (int i = threadIdx.x; i < floats; i += blockDim.x) staged[i] = source[i];
-    __syncthreads();
+    if constexpr (LATTICE) {
+#pragma unroll
+        for (int i = 0; i < kPatternFloats / (4 * 64 * kWaveRows); ++i) {
+            const int at = 4 * (threadIdx.x + 64 * kWaveRows * i);
+            *reinterpret_cast<Quad *>(staged + at) = *reinterpret_cast<const Quad *>(source + at);
+        }
+    } else if constexpr (STAGED) {
+        for (int i = 2 * threadIdx.x; i < codebook_size * DIM; i += 2 * 64 * kWaveRows)   // (DIM is even)
+            *reinterpret_cast<Pair *>(staged + i) = *reinterpret_cast<const Pair *>(source + i);
+    }
+    return source;
 }
 
 struct NearestArgs {
@@ -217,24 +230,23 @@ struct NearestArgs {
 
 template <int DIM, bool LATTICE, bool STAGED>
 __global__ void __launch_bounds__(256) vector_nearest_kernel(const NearestArgs a) {
-    stage_table<DIM, LATTICE, STAGED>(a.codebook, a.count);
+    const float *table = stage_table<DIM, LATTICE, STAGED>(a.codebook, a.count);
     const int lane = threadIdx.x & 63;
     const long long wave = static_cast<long long>(blockIdx.x) * (blockDim.x >> 6) + (threadIdx.x >> 6);
     const long long waves = static_cast<long long>(gridDim.x) * (blockDim.x >> 6);
     LanePatterns patterns;
-    if constexpr (LATTICE) load_patterns(patterns, staged, lane);
+    if constexpr (LATTICE) load_patterns(patterns, table, lane);
+    __syncthreads();
     for (long long vector = wave; vector < a.vectors_count; vector += waves) {
-        float v[DIM];
-#pragma unroll
-        for (int d = 0; d < DIM; ++d) v[d] = a.vectors[vector * DIM + d];
         int code;
         if constexpr (LATTICE) {
-            float point[8];
-            code = nearest_lattice_code(v, patterns, staged, lane, point);
-        } else if constexpr (STAGED) {
-            code = nearest_codeword<DIM>(v, staged, a.count, lane);
+            float point;
+            code = nearest_lattice_code(a.vectors[vector * 8 + (lane & 7)], patterns, staged, lane, point);
         } else {
-            code = nearest_codeword<DIM>(v, a.codebook, a.count, lane);
+            float v[DIM];
+#pragma unroll
+            for (int d = 0; d < DIM; ++d) v[d] = a.vectors[vector * DIM + d];
+            code = nearest_codeword<DIM>(v, STAGED ? staged : a.codebook, a.count, lane);
         }
         if (lane == 0) a.codes[vector] = code;
     }
@@ -246,138 +258,142 @@ struct VectorTileArgs {
     float *deviation_t;   // null, or [width, rows]: original - output, for the trailing updates
     int32_t *encoded;
     int rows, width, region_start, tile_start, tile_width, group, groups_per_row, codebook_size;
-    int whole_quads;   // a lane's four coefficients of a row are one aligned load
+    int whole_rows;   // four rows' deviations of a column are one aligned store
 };
 
-// A tile of up to 256 columns in a wavefront's registers: lane l holds columns 4 l .. 4 l + 3 in
-// slots 0 .. 3, so a block of 4, 8 or 16 columns (which starts at a multiple of 4) occupies
-// whole lanes and every slot index below is a compile-time constant.
-constexpr int kPerLane = 4;
+constexpr int kSpan = 128;       // columns that the wavefront's pairs cover
+constexpr int kSpans = 2;        // of them in the widest tile
 
-// Element d of the block at `local` (wavefront-uniform) out of such registers.
-template <int DIM>
-__device__ __forceinline__ float block_element(const float (&values)[kPerLane], int local, int d) {
-    if constexpr (DIM == 2) {  // a pair sits in slots 0-1 or 2-3 of one lane
-        const float low = lane_value(values[d], local >> 2), high = lane_value(values[2 + d], local >> 2);
-        return (local & 2) ? high : low;
-    } else {
-        return lane_value(values[d & 3], (local >> 2) + (d >> 2));
-    }
-}
-
-// Coefficient rows of the block at `local` for the lane's columns.  Columns that are not behind the block (or past the
-// tile) receive numbers too: nothing reads the corrections of a rounded column again.
-template <int DIM>
-__device__ __forceinline__ void request_rows(float (&rows)[DIM][kPerLane], const VectorTileArgs &a, int local, int lane) {
+// Coefficient rows of the block at `local` for the lane's columns in span HALF and behind it.  Columns that are not behind
+// the block (or past the tile, which is even) receive numbers too: nothing reads the corrections of a rounded column again.
+template <int DIM, int SPANS, int HALF>
+__device__ __forceinline__ void request_rows(float (&rows)[DIM][2 * SPANS], const VectorTileArgs &a, int local, int lane) {
     const float *first = a.coeff + static_cast<size_t>(a.tile_start + local) * a.width + a.tile_start;
-    if (a.whole_quads) {   // uniform
-        const int column = min(kPerLane * lane, a.tile_width - kPerLane);
+#pragma unroll
+    for (int h = HALF; h < SPANS; ++h) {
+        const int column = min(kSpan * h + 2 * lane, a.tile_width - 2);
 #pragma unroll
         for (int d = 0; d < DIM; ++d) {
-            const float4 four = *reinterpret_cast<const float4 *>(first + static_cast<size_t>(d) * a.width + column);
-            rows[d][0] = four.x; rows[d][1] = four.y; rows[d][2] = four.z; rows[d][3] = four.w;
+            const Pair pair = *reinterpret_cast<const Pair *>(first + static_cast<size_t>(d) * a.width + column);
+            rows[d][2 * h] = pair.value[0];
+            rows[d][2 * h + 1] = pair.value[1];
         }
-    } else {
-#pragma unroll
-        for (int d = 0; d < DIM; ++d)
-#pragma unroll
-            for (int s = 0; s < kPerLane; ++s)
-                rows[d][s] = first[static_cast<size_t>(d) * a.width + min(kPerLane * lane + s, a.tile_width - 1)];
     }
 }
 
-// Bound by vector-ALU issue along a row's chain of blocks, with two wavefronts per SIMD at 2048 rows.  128 columns of 2048
-// rows on E8P: 48 us; 67 with a reduction and a rebuilt point for each coset, a division per column of a block in every
-// lane, and the next block's coefficient rows fetched value by value.
-template <int DIM, bool LATTICE, bool STAGED>
-__global__ void __launch_bounds__(64 * kWaveRows) round_vector_tile_kernel(const VectorTileArgs a) {
-    stage_table<DIM, LATTICE, STAGED>(a.codebook, a.codebook_size);
-    const int lane = threadIdx.x & 63;
-    const int row = blockIdx.x * kWaveRows + (threadIdx.x >> 6);
-    if (row >= a.rows) return;  // whole wavefronts leave; nothing below synchronises the workgroup
-    const size_t row_base = static_cast<size_t>(row) * a.width;
-    LanePatterns patterns;
-    if constexpr (LATTICE) load_patterns(patterns, staged, lane);
+// A row's share of a tile: its columns in registers, and what waits in LDS to be written.
+template <int SPANS>
+struct RowTile {
+    float corrections[2 * SPANS], weights[2 * SPANS], scales[2 * SPANS];
+    float *restored, *deviations;   // [tile columns]
+    int *codes;                     // [tile blocks]
+};
 
-    float corrections[kPerLane], weights[kPerLane], scale_at[kPerLane], restored[kPerLane];
-    int codes_at[2] = {0, 0};  // one code per block, block b in lane b % 64: at most 128 blocks (pairs) in a tile
-#pragma unroll
-    for (int s = 0; s < kPerLane; ++s) {
-        const int column = kPerLane * lane + s;
-        const bool inside = column < a.tile_width;
-        const size_t at = row_base + a.tile_start + (inside ? column : 0);
-        corrections[s] = inside ? a.feedback[at] : 0.0f;
-        weights[s] = inside ? a.original[at] : 0.0f;
-        const int group = (a.tile_start + (inside ? column : 0) - a.region_start) / a.group;
-        scale_at[s] = a.scales[static_cast<size_t>(row) * a.groups_per_row + group];
-        restored[s] = 0.0f;
-    }
-    for (int local = 0; local < a.tile_width; local += DIM) {
-        float along[DIM][kPerLane];
-        request_rows<DIM>(along, a, local, lane);   // on their way during the search
+// The blocks of span HALF, one after another.
+template <int DIM, bool LATTICE, bool STAGED, int SPANS, int HALF>
+__device__ __forceinline__ void round_span(RowTile<SPANS> &t, const VectorTileArgs &a, const LanePatterns &patterns, const float *original, int lane) {
+    const int end = min(a.tile_width, kSpan * (HALF + 1));
+    const int mine = lane & (DIM - 1);
+    for (int local = kSpan * HALF; local < end; local += DIM) {
+        float along[DIM][2 * SPANS];
+        request_rows<DIM, SPANS, HALF>(along, a, local, lane);   // on their way during the search
+        const float weight = original[local + mine];
         __builtin_amdgcn_sched_barrier(0);
 
-        const float scale = block_element<DIM>(scale_at, local, 0);  // a block lies inside one scale group
-        float weight[DIM], normalized[DIM], quotients[kPerLane];
-        // every lane divides its own columns: four divisions for a block's two lanes, not one per column
+        const int holder = (local - kSpan * HALF) >> 1;   // the lane with the block's first pair
+        const float scale = lane_value(t.scales[2 * HALF], holder);  // a block lies inside one scale group
+        float quotients[2];   // every lane divides its own columns
 #pragma unroll
-        for (int s = 0; s < kPerLane; ++s) quotients[s] = __fdiv_rn(__fadd_rn(weights[s], corrections[s]), scale_at[s]);
-#pragma unroll
-        for (int d = 0; d < DIM; ++d) {
-            weight[d] = block_element<DIM>(weights, local, d);
-            normalized[d] = block_element<DIM>(quotients, local, d);
-        }
+        for (int s = 0; s < 2; ++s)
+            quotients[s] = __fdiv_rn(__fadd_rn(t.weights[2 * HALF + s], t.corrections[2 * HALF + s]), t.scales[2 * HALF + s]);
         int code;
-        float word[DIM];
+        float word;   // the lane's coordinate
         if constexpr (LATTICE) {
-            code = nearest_lattice_code(normalized, patterns, staged, lane, word);
-        } else if constexpr (STAGED) {
-            code = nearest_codeword<DIM>(normalized, staged, a.codebook_size, lane);
-#pragma unroll
-            for (int d = 0; d < DIM; ++d) word[d] = staged[code * DIM + d];
+            const int from = 4 * (holder + (mine >> 1));
+            const float low = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(from, __builtin_bit_cast(int, quotients[0])));
+            const float high = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(from, __builtin_bit_cast(int, quotients[1])));
+            code = nearest_lattice_code((lane & 1) ? high : low, patterns, staged, lane, word);
         } else {
-            code = nearest_codeword<DIM>(normalized, a.codebook, a.codebook_size, lane);
+            float normalized[DIM];
 #pragma unroll
-            for (int d = 0; d < DIM; ++d) word[d] = a.codebook[static_cast<size_t>(code) * DIM + d];
+            for (int d = 0; d < DIM; ++d) normalized[d] = lane_value(quotients[d & 1], holder + (d >> 1));
+            const float *table = STAGED ? staged : a.codebook;
+            code = nearest_codeword<DIM>(normalized, table, a.codebook_size, lane);
+            word = table[static_cast<size_t>(code) * DIM + mine];
         }
-        float deviation[DIM];
+        const float reconstruction = __fmul_rn(word, scale), deviation = __fsub_rn(weight, reconstruction);
+        t.restored[local + mine] = reconstruction;   // (lanes of one coordinate write the same)
+        t.deviations[local + mine] = deviation;
+        t.codes[local / DIM] = code;
+        float shared[DIM];
 #pragma unroll
-        for (int d = 0; d < DIM; ++d) {
-            const float reconstruction = __fmul_rn(word[d], scale);
-            deviation[d] = __fsub_rn(weight[d], reconstruction);
-            if constexpr (DIM == 2) {
-                const bool holds = lane == (local >> 2);
-                restored[d] = holds && !(local & 2) ? reconstruction : restored[d];
-                restored[2 + d] = holds && (local & 2) ? reconstruction : restored[2 + d];
+        for (int d = 0; d < DIM; ++d) shared[d] = lane_value(deviation, d);
+#pragma unroll
+        for (int s = 2 * HALF; s < 2 * SPANS; ++s) {
+            float pushed = __fmul_rn(shared[0], along[0][s]);
+#pragma unroll
+            for (int d = 1; d < DIM; ++d) pushed = __fadd_rn(pushed, __fmul_rn(shared[d], along[d][s]));
+            t.corrections[s] = __fadd_rn(t.corrections[s], pushed);
+        }
+    }
+}
+
+// SPANS spans of 128 columns.  Bound by vector-ALU issue along a row's chain of blocks, with two wavefronts per SIMD at 2048
+// rows.  128 columns of 2048 rows on E8P: 30 us; 48 with four columns in each of 32 lanes, coefficients in 32 loads a block,
+// costs and indexes reduced together, and a winner worked out by every lane for all coordinates.
+template <int DIM, bool LATTICE, bool STAGED, int SPANS>
+__global__ void __launch_bounds__(64 * kWaveRows) round_vector_tile_kernel(const VectorTileArgs a) {
+    __shared__ __align__(16) float restored[kWaveRows][kSpan * SPANS], deviations[kWaveRows][kSpan * SPANS];
+    __shared__ int codes[kWaveRows][kSpan * SPANS / DIM];
+    const float *table = stage_table<DIM, LATTICE, STAGED>(a.codebook, a.codebook_size);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int first_row = blockIdx.x * kWaveRows;
+    const int row = min(first_row + wave, a.rows - 1);   // wavefronts behind the last row do its work again and write nothing
+    const size_t row_base = static_cast<size_t>(row) * a.width;
+    RowTile<SPANS> t;
+    t.restored = restored[wave];
+    t.deviations = deviations[wave];
+    t.codes = codes[wave];
+#pragma unroll
+    for (int h = 0; h < SPANS; ++h) {
+        const int column = kSpan * h + 2 * lane;   // (a tile is even: a pair lies inside or outside)
+        const bool inside = column < a.tile_width;
+        const size_t at = row_base + a.tile_start + (inside ? column : 0);
+        const Pair feedback = *reinterpret_cast<const Pair *>(a.feedback + at), weights = *reinterpret_cast<const Pair *>(a.original + at);
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            t.corrections[2 * h + s] = inside ? feedback.value[s] : 0.0f;
+            t.weights[2 * h + s] = inside ? weights.value[s] : 0.0f;
+            const int group = (a.tile_start + (inside ? column + s : 0) - a.region_start) / a.group;
+            t.scales[2 * h + s] = a.scales[static_cast<size_t>(row) * a.groups_per_row + group];
+        }
+    }
+    LanePatterns patterns;
+    if constexpr (LATTICE) load_patterns(patterns, table, lane);
+    __syncthreads();
+    const float *original = a.original + row_base + a.tile_start;
+    round_span<DIM, LATTICE, STAGED, SPANS, 0>(t, a, patterns, original, lane);
+    if constexpr (SPANS > 1) round_span<DIM, LATTICE, STAGED, SPANS, SPANS - 1>(t, a, patterns, original, lane);
+
+    __syncthreads();
+    if (first_row + wave < a.rows) {
+        for (int column = lane; column < a.tile_width; column += 64) a.output[row_base + a.tile_start + column] = restored[wave][column];
+        int32_t *encoded = a.encoded + static_cast<size_t>(row) * (a.width / DIM) + a.tile_start / DIM;
+        for (int block = lane; block < a.tile_width / DIM; block += 64) encoded[block] = codes[wave][block];
+    }
+    if (a.deviation_t) {
+        for (int column = threadIdx.x; column < a.tile_width; column += 64 * kWaveRows) {
+            float *target = a.deviation_t + static_cast<size_t>(a.tile_start + column) * a.rows + first_row;
+            if (a.whole_rows) {
+                static_assert(kWaveRows == 4, "one float4 of a column's rows");
+                *reinterpret_cast<float4 *>(target) = make_float4(deviations[0][column], deviations[1][column], deviations[2][column], deviations[3][column]);
             } else {
-                restored[d & 3] = lane == (local >> 2) + (d >> 2) ? reconstruction : restored[d & 3];
+#pragma unroll
+                for (int r = 0; r < kWaveRows; ++r)
+                    if (first_row + r < a.rows) target[r] = deviations[r][column];
             }
         }
-        const int block = local / DIM;
-        const bool keeps = lane == (block & 63);
-        codes_at[0] = keeps && block < 64 ? code : codes_at[0];
-        codes_at[1] = keeps && block >= 64 ? code : codes_at[1];
-#pragma unroll
-        for (int s = 0; s < kPerLane; ++s) {
-            float pushed = __fmul_rn(deviation[0], along[0][s]);
-#pragma unroll
-            for (int d = 1; d < DIM; ++d) pushed = __fadd_rn(pushed, __fmul_rn(deviation[d], along[d][s]));
-            corrections[s] = __fadd_rn(corrections[s], pushed);
-        }
     }
-#pragma unroll
-    for (int s = 0; s < kPerLane; ++s) {
-        const int column = kPerLane * lane + s;
-        if (column < a.tile_width) {
-            a.output[row_base + a.tile_start + column] = restored[s];
-            if (a.deviation_t) a.deviation_t[static_cast<size_t>(a.tile_start + column) * a.rows + row] = __fsub_rn(weights[s], restored[s]);
-        }
-    }
-    const int blocks = a.tile_width / DIM;
-    int32_t *codes = a.encoded + static_cast<size_t>(row) * (a.width / DIM) + a.tile_start / DIM;
-#pragma unroll
-    for (int c = 0; c < 2; ++c)
-        if (64 * c + lane < blocks) codes[64 * c + lane] = codes_at[c];
 }
 
 // LDS a launch needs: the pattern table, or the codebook when it is staged.
@@ -431,8 +447,8 @@ int mk_round_vector_tile(const float *original, const float *feedback, const flo
     MK_REQUIRE(tile_start >= 0 && tile_width >= 1 && tile_start + tile_width <= width && tile_start >= region_start,
                MK_ERR_INVALID, "mk_feedback_round_vector_tile: columns [%d, %d) lie outside a row of %d", tile_start,
                tile_start + tile_width, width);
-    MK_REQUIRE(tile_width <= 64 * kPerLane, MK_ERR_UNSUPPORTED,
-               "mk_feedback_round_vector_tile: at most %d columns per call (got %d)", 64 * kPerLane, tile_width);
+    MK_REQUIRE(tile_width <= kSpan * kSpans, MK_ERR_UNSUPPORTED,
+               "mk_feedback_round_vector_tile: at most %d columns per call (got %d)", kSpan * kSpans, tile_width);
     MK_REQUIRE(width % dimension == 0 && tile_start % dimension == 0 && tile_width % dimension == 0 &&
                    group % dimension == 0,
                MK_ERR_INVALID, "mk_feedback_round_vector_tile: rows, tiles and scale groups must hold whole codewords");
@@ -440,19 +456,23 @@ int mk_round_vector_tile(const float *original, const float *feedback, const flo
                "mk_feedback_round_vector_tile: the lattice search needs the 65536-point table of 8 coordinates");
     VectorTileArgs a{original, feedback, coeff, scales, codebook, output, deviation_t, encoded, rows, width, region_start, tile_start,
                      tile_width, group, groups_per_row, codebook_size,
-                     width % 4 == 0 && tile_start % 4 == 0 && tile_width % 4 == 0 && (reinterpret_cast<uintptr_t>(coeff) & 15u) == 0};
+                     rows % kWaveRows == 0 && (reinterpret_cast<uintptr_t>(deviation_t) & 15u) == 0};
     const dim3 grid(mk_cdiv(rows, kWaveRows)), block(64 * kWaveRows);
     const bool staged_codebook = !lattice && fits_in_lds(codebook_size, dimension);
     const size_t lds = lattice ? kPatternFloats * sizeof(float)
                                : (staged_codebook ? static_cast<size_t>(codebook_size) * dimension * sizeof(float) : 0);
-#define MK_TILE(DIM)                                                                                                \
-    if (staged_codebook) hipLaunchKernelGGL((round_vector_tile_kernel<DIM, false, true>), grid, block, lds, stream, a); \
-    else hipLaunchKernelGGL((round_vector_tile_kernel<DIM, false, false>), grid, block, 0, stream, a)
-    if (lattice) hipLaunchKernelGGL((round_vector_tile_kernel<8, true, false>), grid, block, lds, stream, a);
-    else if (dimension == 2) { MK_TILE(2); }
-    else if (dimension == 4) { MK_TILE(4); }
-    else if (dimension == 8) { MK_TILE(8); }
-    else { MK_TILE(16); }
+#define MK_TILE(...)                                                                                                   \
+    if (tile_width <= kSpan) hipLaunchKernelGGL((round_vector_tile_kernel<__VA_ARGS__, 1>), grid, block, lds, stream, a); \
+    else hipLaunchKernelGGL((round_vector_tile_kernel<__VA_ARGS__, kSpans>), grid, block, lds, stream, a)
+#define MK_TILE_CODEBOOK(DIM)                             \
+    if (staged_codebook) { MK_TILE(DIM, false, true); }   \
+    else { MK_TILE(DIM, false, false); }
+    if (lattice) { MK_TILE(8, true, false); }
+    else if (dimension == 2) { MK_TILE_CODEBOOK(2) }
+    else if (dimension == 4) { MK_TILE_CODEBOOK(4) }
+    else if (dimension == 8) { MK_TILE_CODEBOOK(8) }
+    else { MK_TILE_CODEBOOK(16) }
+#undef MK_TILE_CODEBOOK
 #undef MK_TILE
     MK_LAUNCH_CHECK("mk_feedback_round_vector_tile");
     return MK_OK;

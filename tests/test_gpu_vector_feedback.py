@@ -94,6 +94,43 @@ def test_codebook_search_matches_oracle_codes(entries, dimension, count):
         assert codes[20] == 4 and codes[21] == 11
 
 
+@pytest.mark.parametrize("entries,dimension", [(5, 2), (64, 4), (65, 8), (300, 16), (2000, 8)])
+def test_codebook_search_takes_the_lowest_of_equal_codewords(entries, dimension):
+    """Equal codewords in several lanes, in one lane (64 apart), and all of them at once."""
+    from mlkit_amd.kernels import lattice_search
+
+    rng = np.random.default_rng(entries)
+    codebook = np.round(rng.standard_normal((entries, dimension)) * 2).astype(F32)
+    codebook[entries // 2:] = codebook[:entries - entries // 2]
+    samples = np.concatenate([codebook, np.round(rng.standard_normal((200, dimension)) * 4).astype(F32) / 2])
+    distances = ((samples[:, None, :].astype(np.float64) - codebook[None]) ** 2).sum(-1)   # exact: small multiples of 1/4
+    np.testing.assert_array_equal(host(lattice_search.nearest(dev(samples), dev(codebook))), distances.argmin(1))
+    same = np.broadcast_to(codebook[:1], codebook.shape).copy()
+    np.testing.assert_array_equal(host(lattice_search.nearest(dev(samples), dev(same))), 0)
+
+
+@pytest.mark.parametrize("rows", [1, 6, 8])
+@pytest.mark.parametrize("region_start,tile_start,tile_width,group", [(0, 0, 2, 4), (2, 4, 130, 6), (0, 126, 128, 64), (2, 2, 256, 10)])
+def test_round_vector_tile_on_edges_of_its_spans(rows, region_start, tile_start, tile_width, group):
+    """Pairs of columns where a tile fills no span of 128, or begins at no multiple of four."""
+    from mlkit_amd.kernels import error_feedback
+
+    rng = np.random.default_rng(tile_width + rows)
+    width = 262
+    weight, feedback = (rng.standard_normal((rows, width)).astype(F32) * F32(scale) for scale in (1.0, 0.1))
+    coeff = np.triu(rng.standard_normal((width, width)), 1).astype(F32) * F32(0.1)
+    codebook = rng.standard_normal((33, 2)).astype(F32)
+    scales = (0.5 + rng.random((rows, -(-(width - region_start) // group)))).astype(F32)
+    expected_out, expected_codes = np.zeros_like(weight), np.zeros((rows, width // 2), dtype=np.int32)
+    options = dict(region_start=region_start, tile_start=tile_start, tile_width=tile_width, group=group, dimension=2, lattice=False)
+    oracle_lattice.round_vector_tile(weight, feedback, coeff, scales, codebook, expected_out, expected_codes, **options)
+    output, encoded = torch.zeros((rows, width), device="cuda"), torch.zeros((rows, width // 2), device="cuda", dtype=torch.int32)
+    error_feedback.round_vector_tile(dev(weight), dev(feedback), dev(coeff), dev(scales), dev(codebook), output, encoded,
+                                     codebook_size=33, **options)
+    np.testing.assert_array_equal(host(encoded), expected_codes)
+    np.testing.assert_array_equal(host(output), expected_out)
+
+
 def test_nearest_returns_codewords_or_indices_and_handles_other_dimensions():
     codebook = torch.randn(50, 8, device="cuda")
     samples = torch.randn(200, 8, device="cuda")
