@@ -34,6 +34,7 @@ struct BlockArgs {
 };
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 __device__ __forceinline__ float lane_value(float x, int lane) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), lane));
@@ -67,15 +68,22 @@ constexpr int kColumnFloats = kTile + 4;        // a tile column in LDS (16-byte
 // k = 4 (lane / 16) + i and a tile is read as an operand exactly as it is held: one 16-byte LDS read.  A panel's sixteen
 // products are summed first and subtracted in one addition, so an entry is rounded at most 7 + 15 times on its way (128
 // times in a running accumulator, which left the coefficients of 1024 columns 4.1e-7 from 64 bits; now 2.6e-7, 3.3e-7
-// with the two-column kernel below).
+// with PAIRS).
+//
+// PAIRS: two rows at a time -- both are finished, then an entry loses fma(u_j, u_j, u_{j+1} u_{j+1}) in one subtraction, pair by
+// pair -- in the elimination as on the matrix cores, where a product of 16 x 16 x 1 in four blocks takes row j + 1 of a tile
+// times the wavefront's three tiles and a second one adds row j.  The order of additions that the coefficients of vector grids
+// are worked out in: a code that a last bit of a coefficient turns takes the rest of its row along when it stands for eight
+// weights, and conversions stay what they were, bit for bit.
 //
 // What bounds the kernel is the chain of 128 pivots: a panel takes about 4000 cycles, 1550 of them elimination (up to 2700
 // while the other set's products share the SIMD), 700 the products it waits for.  One copy of the code serves all panels, since
 // a launch runs it once and instruction fetches would show.  A block with 768 columns beside it, called back to back: 17.9 us;
 // with one set of four wavefronts doing all of it in turn 24.9 (2200 cycles a panel went into the stores alone, and as many
 // into products that nobody waited for yet).  The rows' factors as row broadcasts instead of scalars, with the diagonal tile
-// in all lanes: 26.8 (the broadcasts do not become part of the multiply-adds).  A pair of columns per barrier: 48.
-template <bool ROW>
+// in all lanes: 26.8 (the broadcasts do not become part of the multiply-adds).  With PAIRS 28.6 (between others, 64 to 1920
+// columns beside the block); 48.3 with 64 entries of the block in each of 256 threads and a barrier for every pair.
+template <bool ROW, bool PAIRS>
 __global__ void __launch_bounds__(2 * kThreads, 2) cholesky_block_kernel(const BlockArgs a) {
     __builtin_amdgcn_s_setprio(3);   // in front of a trailing update that runs beside it
     __shared__ __align__(16) float panel[2][kTiles + kWaves][kTile][kColumnFloats];   // [buffer][tile column][column][row]
@@ -156,21 +164,60 @@ __global__ void __launch_bounds__(2 * kThreads, 2) cholesky_block_kernel(const B
             auto operand = [&](int tile_column) __attribute__((always_inline)) -> f32x4 {
                 return *reinterpret_cast<const f32x4 *>(&tiles[tile_column][column][4 * quarter]);
             };
-            // what the next elimination waits for: tile row s + 1
-            const f32x4 next = operand(s + 1), u_left = operand(left_column), u_right = operand(right_column), u_beside = operand(ROW ? wave + kTiles : wave);
-            f32x4 from_left = {}, from_right = {}, from_beside = {};
+            // PAIRS: the panel's values of a column; lanes of quarter 0, 1 and 2 hold those of the three tiles' columns
+            auto column_of = [&](float (&values)[kTile], int tile_column) __attribute__((always_inline)) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                from_left = __builtin_amdgcn_mfma_f32_16x16x4f32(next[i], u_left[i], from_left, 0, 0, 0);
-                from_right = __builtin_amdgcn_mfma_f32_16x16x4f32(next[i], u_right[i], from_right, 0, 0, 0);
-                if constexpr (ROW) from_beside = __builtin_amdgcn_mfma_f32_16x16x4f32(next[i], u_beside[i], from_beside, 0, 0, 0);
+                for (int i = 0; i < 4; ++i) {
+                    const f32x4 four = reinterpret_cast<const f32x4 *>(tiles[tile_column][column])[i];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) values[4 * i + k] = four[k];
+                }
+            };
+            float columns[PAIRS ? kTile : 1];
+            if constexpr (PAIRS) column_of(columns, quarter == 1 ? right_column : ROW && quarter == 2 ? wave + kTiles : left_column);
+            auto pairs_from = [&](int r, f32x4 &on_left, f32x4 &on_right, f32x4 &on_beside) __attribute__((always_inline)) {
+                float rows[kTile];
+                column_of(rows, r);
+#pragma unroll
+                for (int k = 0; k < kTile; k += 2) {
+                    f32x16 sum = {};   // of row k + 1, then of row k
+                    sum = __builtin_amdgcn_mfma_f32_16x16x1f32(rows[k + 1], columns[k + 1], sum, 0, 0, 0);
+                    sum = __builtin_amdgcn_mfma_f32_16x16x1f32(rows[k], columns[k], sum, 0, 0, 0);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        on_left[i] += sum[i];
+                        on_right[i] += sum[4 + i];
+                        if constexpr (ROW) on_beside[i] += sum[8 + i];
+                    }
+                }
+            };
+            // what the next elimination waits for: tile row s + 1
+            const f32x4 u_left = operand(left_column), u_right = operand(right_column), u_beside = operand(ROW ? wave + kTiles : wave);
+            f32x4 from_left = {}, from_right = {}, from_beside = {};
+            if constexpr (PAIRS) {
+#pragma unroll
+                for (int r = 1; r < kTiles; ++r)
+                    if (r == s + 1) {   // uniform
+                        if (r < kWaves) from_left = left[r];
+                        from_right = right[r];
+                        if constexpr (ROW) from_beside = beside[r];
+                    }
+                pairs_from(s + 1, from_left, from_right, from_beside);
+            } else {
+                const f32x4 next = operand(s + 1);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    from_left = __builtin_amdgcn_mfma_f32_16x16x4f32(next[i], u_left[i], from_left, 0, 0, 0);
+                    from_right = __builtin_amdgcn_mfma_f32_16x16x4f32(next[i], u_right[i], from_right, 0, 0, 0);
+                    if constexpr (ROW) from_beside = __builtin_amdgcn_mfma_f32_16x16x4f32(next[i], u_beside[i], from_beside, 0, 0, 0);
+                }
             }
 #pragma unroll
             for (int r = 1; r < kTiles; ++r)
                 if (r == s + 1) {   // uniform
-                    if (r < kWaves) left[r] += from_left;
-                    right[r] += from_right;
-                    if constexpr (ROW) beside[r] += from_beside;
+                    if (r < kWaves) left[r] = PAIRS ? from_left : left[r] + from_left;
+                    right[r] = PAIRS ? from_right : right[r] + from_right;
+                    if constexpr (ROW) beside[r] = PAIRS ? from_beside : beside[r] + from_beside;
                     publish(r);
                 }
             __syncthreads();
@@ -179,6 +226,11 @@ __global__ void __launch_bounds__(2 * kThreads, 2) cholesky_block_kernel(const B
 #pragma unroll
             for (int r = 2; r < kTiles; ++r) {
                 if (r <= s + 1) continue;   // uniform, as all the conditions here
+                if constexpr (PAIRS) {
+                    f32x4 unused = {};
+                    pairs_from(r, r < kWaves ? left[r] : unused, right[r], beside[r]);
+                    continue;
+                }
                 const f32x4 row_operand = operand(r);
                 auto products = [&](f32x4 u) __attribute__((always_inline)) -> f32x4 {
                     f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -238,23 +290,46 @@ __global__ void __launch_bounds__(2 * kThreads, 2) cholesky_block_kernel(const B
             pivot = lane == j ? value[j] : pivot;
             return __builtin_amdgcn_rsqf(lane_value(value[j], j));   // accurate to an ulp; an IEEE square root and division would double the chain
         };
-        float reciprocal = reciprocal_root(0);
+        if constexpr (PAIRS) {
+            float reciprocal = reciprocal_root(0);
 #pragma unroll
-        for (int j = 0; j < kTile; ++j) {
-            value[j] *= reciprocal;
-            if (j + 1 < kTile) {   // the next pivot's chain first: the rest of this step hides its latency
-                value[j + 1] = __builtin_fmaf(-lane_value(value[j], j + 1), value[j], value[j + 1]);
-                reciprocal = reciprocal_root(j + 1);
+            for (int j = 0; j < kTile; j += 2) {
+                value[j] *= reciprocal;
+                const float link = lane_value(value[j], j + 1);
+                value[j + 1] = __builtin_fmaf(-link, value[j], value[j + 1]);
+                value[j + 1] *= reciprocal_root(j + 1);
+                auto take = [&](int i) __attribute__((always_inline)) {   // one rounding for the pair's sum, one for the difference
+                    const float first = lane_value(value[j], i), second = lane_value(value[j + 1], i);
+                    value[i] -= __builtin_fmaf(first, value[j], second * value[j + 1]);
+                };
+                if (j + 2 < kTile) {
+                    take(j + 2);
+                    reciprocal = reciprocal_root(j + 2);
+                }
+#pragma unroll
+                for (int i = j + 3; i < kTile; ++i) take(i);
+                if ((j & 3) == 2 && quarter > 0 && own != s && (ROW || quarter < 3)) keep(j / 4, j / 4 + 1);
+                __builtin_amdgcn_sched_barrier(0);
             }
-            float factors[kTile];
+        } else {
+            float reciprocal = reciprocal_root(0);
 #pragma unroll
-            for (int i = j + 2; i < kTile; ++i) factors[i] = lane_value(value[j], i);
+            for (int j = 0; j < kTile; ++j) {
+                value[j] *= reciprocal;
+                if (j + 1 < kTile) {   // the next pivot's chain first: the rest of this step hides its latency
+                    value[j + 1] = __builtin_fmaf(-lane_value(value[j], j + 1), value[j], value[j + 1]);
+                    reciprocal = reciprocal_root(j + 1);
+                }
+                float factors[kTile];
 #pragma unroll
-            for (int i = j + 2; i < kTile; ++i) value[i] = __builtin_fmaf(-factors[i], value[j], value[i]);
-            // (the diagonal tile later: another wavefront may still have to read it as it was)
-            if ((j & 3) == 3 && quarter > 0 && own != s && (ROW || quarter < 3)) keep(j / 4, j / 4 + 1);
-            // step by step: put off, as the compiler would have it, the updates of a row are one dependent chain
-            __builtin_amdgcn_sched_barrier(0);
+                for (int i = j + 2; i < kTile; ++i) factors[i] = lane_value(value[j], i);
+#pragma unroll
+                for (int i = j + 2; i < kTile; ++i) value[i] = __builtin_fmaf(-factors[i], value[j], value[i]);
+                // (the diagonal tile later: another wavefront may still have to read it as it was)
+                if ((j & 3) == 3 && quarter > 0 && own != s && (ROW || quarter < 3)) keep(j / 4, j / 4 + 1);
+                // step by step: put off, as the compiler would have it, the updates of a row are one dependent chain
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
         const uint64_t accepted = __builtin_amdgcn_ballot_w64(static_cast<uint32_t>(__float_as_int(pivot)) - 1u < 0x7f7fffffu);   // positive and finite
         const uint32_t refused = ~static_cast<uint32_t>(accepted) & 0xffffu;
@@ -291,206 +366,6 @@ __global__ void __launch_bounds__(2 * kThreads, 2) cholesky_block_kernel(const B
             }
         }
     }
-}
-
-// ---- the same, two columns per step ------------------------------------------------------------
-//
-// The order of additions that the coefficients of vector grids are worked out in.  Kept for them although it takes twice as
-// long (48 against 25 us with 768 columns beside the block): a code that a last bit of a coefficient turns takes the rest of
-// its row along when it stands for eight weights, and conversions stay what they were, bit for bit.
-
-constexpr int kSub = kBlock / 16;
-constexpr int kRowFloats = 2 * kBlock;   // a published row: the block's columns, then the columns carried beside it
-
-// Columns 16 SIXTEEN ... 16 SIXTEEN + 15 of the factorisation below, two per step (their rows
-// sit in register row SIXTEEN of their owners).  False after a pivot that is not positive and
-// finite, which every thread sees in the same step.
-//
-// A step takes rows j and j + 1 as the updates of columns < j left them (`pivot_rows`), and
-// every thread derives what it needs of the two finished rows itself:
-//   U[j][k]     = A[j][k] / sqrt(A[j][j])
-//   U[j+1][k]   = (A[j+1][k] - U[j][j+1] U[j][k]) / sqrt(A[j+1][j+1] - U[j][j+1]^2)
-// and subtracts both outer products from its sub-block: one LDS round trip and one barrier
-// per two columns.
-//
-// ROW: the workgroup also carries 128 columns to the right of the block (`beside`), which take
-// the same row operations and so become U_jj^-T A_jr, the block row of the factor.
-template <int SIXTEEN, bool ROW, int BT>
-__device__ __forceinline__ bool sixteen_steps(const BlockArgs &a, float (&mine)[kSub][kSub], float (&beside)[kSub][BT],
-                                              float (&pivot_rows)[2][2][kRowFloats], int tx, int ty) {
-#pragma unroll 1
-    for (int lane = 0; lane < 16; lane += 2) {
-        const int j = 16 * SIXTEEN + lane;
-        const float *first = pivot_rows[(j >> 1) & 1][0], *second = pivot_rows[(j >> 1) & 1][1];
-        const float pivot = first[j];
-        if (!(pivot > 0.0f) || !(pivot - pivot == 0.0f)) {
-            if (threadIdx.x == 0) *a.status = a.first_column + j + 1;
-            return false;
-        }
-        // (one v_rsq_f32, accurate to an ulp; the IEEE square root and division were a fifth of a step's chain)
-        const float reciprocal = __builtin_amdgcn_rsqf(pivot);
-        const float link = first[j + 1] * reciprocal;                 // U[j][j+1]
-        const float next_pivot = second[j + 1] - link * link;
-        if (!(next_pivot > 0.0f) || !(next_pivot - next_pivot == 0.0f)) {
-            if (threadIdx.x == 0) *a.status = a.first_column + j + 2;
-            return false;
-        }
-        const float next_reciprocal = __builtin_amdgcn_rsqf(next_pivot);
-        // Register rows below SIXTEEN hold only rows <= j (finished); register columns below
-        // SIXTEEN only columns < j, which for the rows still changing lie below the diagonal
-        // (never read): neither takes part, so a step costs 2 (8 - SIXTEEN)^2 multiply-adds.
-        float rows_first[kSub], rows_second[kSub], columns_first[kSub], columns_second[kSub];
-#pragma unroll
-        for (int u = SIXTEEN; u < kSub; ++u) {
-            const int i = ty + 16 * u, k = tx + 16 * u;
-            const float upper = first[i] * reciprocal;                                   // U[j][i]
-            const float lower = (second[i] - link * upper) * next_reciprocal;            // U[j+1][i]
-            rows_first[u] = i > j + 1 ? upper : 0.0f;   // zero keeps rows <= j + 1 as they are
-            rows_second[u] = i > j + 1 ? lower : 0.0f;
-            columns_first[u] = first[k] * reciprocal;                                    // U[j][k]
-            columns_second[u] = (second[k] - link * columns_first[u]) * next_reciprocal; // U[j+1][k]
-        }
-        float beside_first[BT], beside_second[BT];
-        if constexpr (ROW) {
-#pragma unroll
-            for (int v = 0; v < BT; ++v) {
-                const int c = kBlock + tx + 16 * v;
-                beside_first[v] = first[c] * reciprocal;
-                beside_second[v] = (second[c] - link * beside_first[v]) * next_reciprocal;
-            }
-        }
-        // The two rows' owners keep the finished rows.
-        if (ty == lane) {
-#pragma unroll
-            for (int v = SIXTEEN; v < kSub; ++v) mine[SIXTEEN][v] = columns_first[v];
-            if constexpr (ROW) {
-#pragma unroll
-                for (int v = 0; v < BT; ++v) beside[SIXTEEN][v] = beside_first[v];
-            }
-        }
-        if (ty == lane + 1) {
-#pragma unroll
-            for (int v = SIXTEEN; v < kSub; ++v) mine[SIXTEEN][v] = columns_second[v];
-            if constexpr (ROW) {
-#pragma unroll
-                for (int v = 0; v < BT; ++v) beside[SIXTEEN][v] = beside_second[v];
-            }
-        }
-#pragma unroll
-        for (int u = SIXTEEN; u < kSub; ++u) {
-#pragma unroll
-            for (int v = SIXTEEN; v < kSub; ++v)
-                mine[u][v] -= rows_first[u] * columns_first[v] + rows_second[u] * columns_second[v];
-            if constexpr (ROW) {
-#pragma unroll
-                for (int v = 0; v < BT; ++v)
-                    beside[u][v] -= rows_first[u] * beside_first[v] + rows_second[u] * beside_second[v];
-            }
-        }
-        // Rows j + 2 and j + 3 have all their updates now: their owners publish them.
-        float (*next)[kRowFloats] = pivot_rows[((j >> 1) + 1) & 1];
-        if (lane < 14) {
-            if (ty == lane + 2 || ty == lane + 3) {
-#pragma unroll
-                for (int v = SIXTEEN; v < kSub; ++v) next[ty - lane - 2][tx + 16 * v] = mine[SIXTEEN][v];   // columns < j are not read
-                if constexpr (ROW) {
-#pragma unroll
-                    for (int v = 0; v < BT; ++v) next[ty - lane - 2][kBlock + tx + 16 * v] = beside[SIXTEEN][v];
-                }
-            }
-        } else if constexpr (SIXTEEN + 1 < kSub) {
-            if (ty < 2) {
-#pragma unroll
-                for (int v = SIXTEEN + 1; v < kSub; ++v) next[ty][tx + 16 * v] = mine[SIXTEEN + 1][v];
-                if constexpr (ROW) {
-#pragma unroll
-                    for (int v = 0; v < BT; ++v) next[ty][kBlock + tx + 16 * v] = beside[SIXTEEN + 1][v];
-                }
-            }
-        }
-        __syncthreads();
-    }
-    return true;
-}
-
-// In: the upper triangle of a symmetric positive definite block.  Out: U with block = U^T U
-// in the upper triangle, zeros below it.  A pivot that is not positive (or not finite)
-// records its column and leaves the block unspecified.
-//
-// Right-looking, two columns per step.  The block lives in registers for the whole
-// factorisation: thread (ty, tx) of a 16 x 16 grid owns entries (ty + 16 u, tx + 16 v),
-// an 8 x 8 sub-block.  Per step only the two pivot rows travel: the threads that own them
-// put them (as updated so far) into one of two LDS buffers, one barrier later every thread
-// reads the entries it needs, finishes the two rows for itself and subtracts their outer
-// products from its sub-block.  Rows up to the pivot rows are masked out of the update by
-// zero factors, so finished rows keep their values.
-// BT: sixteenths of 128 columns a workgroup carries beside the block (8: 128 columns, 4: 64).
-template <bool ROW, int BT>
-__global__ void __launch_bounds__(kThreads) cholesky_pairs_kernel(const BlockArgs a) {
-    __shared__ float pivot_rows[2][2][kRowFloats];   // [buffer][row j, row j + 1][column]
-    __shared__ int failed;
-    const int n = a.size;
-    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-    if (threadIdx.x == 0) failed = *a.status != 0;   // an earlier block already failed: do nothing
-    float mine[kSub][kSub], beside[kSub][BT];
-    constexpr int kBeside = 16 * BT;
-    // ROW: workgroup b carries columns kBeside b ... kBeside (b + 1) - 1 of the block row; every workgroup
-    // factors the block itself (from the matrix, which nobody overwrites: the factor goes to
-    // `factor_out`), and the first one stores it.
-    const int beside_first_column = n + kBeside * blockIdx.x;
-#pragma unroll
-    for (int u = 0; u < kSub; ++u)
-#pragma unroll
-        for (int v = 0; v < kSub; ++v) {
-            const int row = ty + 16 * u, column = tx + 16 * v;
-            const bool inside = row < n && column < n && column >= row;
-            const float loaded = a.matrix[(inside ? row : 0) * a.leading + (inside ? column : 0)];
-            // Outside the block: an identity diagonal keeps every pivot of the padding at one.
-            mine[u][v] = inside ? loaded : (row == column ? 1.0f : 0.0f);
-            if (v < BT) {
-                beside[u][v] = 0.0f;
-                if constexpr (ROW) {
-                    const bool present = row < n && kBeside * static_cast<int>(blockIdx.x) + column < a.row_columns;
-                    const float carried = a.matrix[(present ? row : 0) * a.leading + (present ? beside_first_column + column : 0)];
-                    beside[u][v] = present ? carried : 0.0f;
-                }
-            }
-        }
-    if (ty < 2) {
-#pragma unroll
-        for (int v = 0; v < kSub; ++v) {
-            pivot_rows[0][ty][tx + 16 * v] = mine[0][v];
-            if constexpr (ROW) {
-                if (v < BT) pivot_rows[0][ty][kBlock + tx + 16 * v] = beside[0][v];
-            }
-        }
-    }
-    __syncthreads();
-    if (failed) return;
-
-    // All 128 columns run (the padding is an identity): no data-dependent exit other than a bad pivot.
-    bool good = sixteen_steps<0, ROW, BT>(a, mine, beside, pivot_rows, tx, ty);
-    good = good && sixteen_steps<1, ROW, BT>(a, mine, beside, pivot_rows, tx, ty);
-    good = good && sixteen_steps<2, ROW, BT>(a, mine, beside, pivot_rows, tx, ty);
-    good = good && sixteen_steps<3, ROW, BT>(a, mine, beside, pivot_rows, tx, ty);
-    good = good && sixteen_steps<4, ROW, BT>(a, mine, beside, pivot_rows, tx, ty);
-    good = good && sixteen_steps<5, ROW, BT>(a, mine, beside, pivot_rows, tx, ty);
-    good = good && sixteen_steps<6, ROW, BT>(a, mine, beside, pivot_rows, tx, ty);
-    good = good && sixteen_steps<7, ROW, BT>(a, mine, beside, pivot_rows, tx, ty);
-    if (!good) return;
-    float *factor = ROW ? a.factor_out : a.matrix;
-    const long long factor_leading = ROW ? kBlock : a.leading;
-#pragma unroll
-    for (int u = 0; u < kSub; ++u)
-#pragma unroll
-        for (int v = 0; v < kSub; ++v) {
-            const int row = ty + 16 * u, column = tx + 16 * v;
-            if (blockIdx.x == 0 && row < n && column < n) factor[row * factor_leading + column] = column >= row ? mine[u][v] : 0.0f;
-            if constexpr (ROW) {
-                if (v < BT && row < n && kBeside * static_cast<int>(blockIdx.x) + column < a.row_columns)
-                    a.matrix[row * a.leading + beside_first_column + column] = beside[u][v];
-            }
-        }
 }
 
 }  // namespace
@@ -605,9 +480,9 @@ extern "C" int mk_cholesky_block(float *matrix, long long leading, int size, int
     if (int refused = check_block(matrix, leading, size, first_column, row_columns, factor_out, status)) return refused;
     BlockArgs a{matrix, leading, size, first_column, status, row_columns, factor_out};
     if (row_columns > 0)
-        hipLaunchKernelGGL((cholesky_block_kernel<true>), dim3(mk_cdiv(row_columns, kCarried)), dim3(2 * kThreads), 0, stream, a);
+        hipLaunchKernelGGL((cholesky_block_kernel<true, false>), dim3(mk_cdiv(row_columns, kCarried)), dim3(2 * kThreads), 0, stream, a);
     else
-        hipLaunchKernelGGL((cholesky_block_kernel<false>), dim3(1), dim3(2 * kThreads), 0, stream, a);
+        hipLaunchKernelGGL((cholesky_block_kernel<false, false>), dim3(1), dim3(2 * kThreads), 0, stream, a);
     MK_LAUNCH_CHECK("mk_cholesky_block");
     return MK_OK;
 }
@@ -617,14 +492,10 @@ extern "C" int mk_cholesky_block_pairs(float *matrix, long long leading, int siz
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     if (int refused = check_block(matrix, leading, size, first_column, row_columns, factor_out, status)) return refused;
     BlockArgs a{matrix, leading, size, first_column, status, row_columns, factor_out};
-    // 64 columns per workgroup while that still fits one workgroup per CU (a step then costs a
-    // third less arithmetic); 128 beyond.
-    if (row_columns > 256 * 64)
-        hipLaunchKernelGGL((cholesky_pairs_kernel<true, 8>), dim3(mk_cdiv(row_columns, 128)), dim3(kThreads), 0, stream, a);
-    else if (row_columns > 0)
-        hipLaunchKernelGGL((cholesky_pairs_kernel<true, 4>), dim3(mk_cdiv(row_columns, 64)), dim3(kThreads), 0, stream, a);
+    if (row_columns > 0)
+        hipLaunchKernelGGL((cholesky_block_kernel<true, true>), dim3(mk_cdiv(row_columns, kCarried)), dim3(2 * kThreads), 0, stream, a);
     else
-        hipLaunchKernelGGL((cholesky_pairs_kernel<false, 4>), dim3(1), dim3(kThreads), 0, stream, a);
+        hipLaunchKernelGGL((cholesky_block_kernel<false, true>), dim3(1), dim3(2 * kThreads), 0, stream, a);
     MK_LAUNCH_CHECK("mk_cholesky_block_pairs");
     return MK_OK;
 }

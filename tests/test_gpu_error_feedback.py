@@ -447,6 +447,48 @@ def test_a_factored_block_is_as_close_to_64_bits_as_the_two_column_kernel(beside
     assert error["mk_cholesky_block"] <= error["mk_cholesky_block_pairs"], error
 
 
+@pytest.mark.parametrize("size,beside", [(1, 3), (2, 0), (16, 64), (17, 65), (37, 5), (112, 1), (128, 0), (128, 130)])
+def test_pairs_of_rows_are_taken_in_their_order(size, beside):
+    """`mk_cholesky_block_pairs`, bit for bit: an entry loses fma(u_j, v_j, u_{j+1} v_{j+1}) for one pair of rows after another.
+    Replayed with the factor's own rows (sums in extended precision: one more rounding, at 2^-40 of a 24-bit one); only the
+    reciprocal root of a pivot is the device's, one of the numbers within two ulps."""
+    f32, wide = np.float32, np.longdouble
+    rng = np.random.default_rng(size + beside)
+    width = size + beside
+    inputs = rng.standard_normal((2 * width + 8, width))
+    matrix = (inputs.T @ inputs / inputs.shape[0] + 0.05 * np.eye(width)).astype(f32)
+    factor, row, status = block_factor(matrix, size, entry="mk_cholesky_block_pairs")
+    assert status == 0 and not np.tril(factor, -1).any()
+    upper = factor if not beside else np.concatenate([factor, row], 1)
+
+    def fused(a, b, c):
+        return (wide(a) * wide(b) + wide(c)).astype(f32)
+
+    rest = matrix[:size].copy()
+    for j in range(0, size, 2):
+        for k in range(j, min(j + 2, size)):
+            rest[k, k:] = rest[k, k:] if k == j else fused(-upper[j, k], upper[j, k:], rest[k, k:])
+            root = f32(1 / np.sqrt(np.float64(rest[k, k])))
+            near = [root, *(np.nextafter(root, f32(end)) for end in (0, 2 * root))]
+            near += [np.nextafter(near[1], f32(0)), np.nextafter(near[2], f32(2 * root))]
+            assert any(np.array_equal((rest[k, k:] * r).astype(f32), upper[k, k:]) for r in near), k
+        if j + 1 < size:
+            last = (upper[j + 1, :size, None] * upper[j + 1, None]).astype(f32)
+            rest[j + 2:] -= fused(upper[j, :size, None], upper[j, None], last)[j + 2:]
+
+
+@pytest.mark.parametrize("beside", [0, 65])
+@pytest.mark.parametrize("column", [0, 1, 15, 16, 47, 100, 127])
+def test_pairs_of_rows_report_the_first_refused_pivot(column, beside):
+    rng = np.random.default_rng(column)
+    width = 128 + beside
+    matrix = (rng.standard_normal((width, width)) * 0.01).astype(np.float32)
+    matrix = matrix + matrix.T + np.diag(np.full(width, 4, dtype=np.float32))
+    matrix[column, column] = -1.0
+    matrix[127, 127] = -1.0
+    assert block_factor(matrix, 128, first=256, entry="mk_cholesky_block_pairs")[2] == 256 + column + 1
+
+
 @pytest.mark.parametrize("column", [0, 1, 15, 16, 47, 100, 126])
 @pytest.mark.parametrize("value", [-1.0, float("nan"), float("inf")])
 def test_a_factored_block_names_its_bad_pivot(column, value):
