@@ -31,36 +31,56 @@ constexpr int kExchangeFloats = (VALUES * (GROUPS / 2) + GROUPS) * COLUMNS;   //
 // Up to 2048 rows bound by HBM.  Neighbouring workgroups share 128-byte lines, so they are given to one XCD, whose L2 has
 // the line: workgroup b takes column group (b % 8) * groups_per_xcd + b / 8.
 //
-// 14336 columns of 1024 / 2048 / 4096 fp32 values, signs before or behind: 20 / 40 / 145 us (from bf16 17 / 33 / 146), against
-// 63 + 63 us for torch's strided copies around the row transform at 1024, 119 + 119 at 2048 and 255 + 255 at 4096.  4096 rows
-// run at 3.2 TB/s, bound by latency: 144 registers keep a second workgroup off the compute unit, and held to 128 the kernel
-// spills (206 us); 16 columns a workgroup take 151 us.  With the signs behind read from memory as they are needed 25 / 47 /
-// 177 us; multiplied in a pass of their own 22 / 43 / 147.
-template <int COLUMNS, int GROUPS, int VALUES, int SOURCE>
-__global__ void __launch_bounds__(COLUMNS * GROUPS) fwht_columns_kernel(const ColumnArgs a) {
+// 14336 columns of 1024 / 2048 / 4096 fp32 values, signs before or behind: 20 / 39 / 122 us (from bf16 17 / 33 / 108), against
+// 63 + 63 us for torch's strided copies around the row transform at 1024, 119 + 119 at 2048 and 255 + 255 at 4096.  At 4096
+// rows 16 columns a workgroup of 1024 threads, in 103 registers; 8 columns take 145 (each line of 128 bytes is then fetched by
+// four workgroups), and 180 with two workgroups on a compute unit (their lines leave the L2 before the neighbours come).
+// 41 KB of LDS at least keep a fourth workgroup away at 1024 rows for the same reason (22 us with it).  Signs before, read by
+// every thread for itself instead of through LDS: 44 at 2048 rows, 127 at 4096.
+//
+// OFFSET: the type of a thread's byte offset, 32 bits wherever the matrix has fewer bytes.
+template <int COLUMNS, int GROUPS, int VALUES, int SOURCE, typename OFFSET>
+__global__ void __launch_bounds__(COLUMNS * GROUPS, 4) fwht_columns_kernel(const ColumnArgs a) {
     constexpr int kHeld = VALUES / GROUPS;         // the k of a thread behind the exchange
     constexpr int kHalf = VALUES / 2, kHalfGroups = GROUPS / 2;
     constexpr int kSignStride = GROUPS + 4;        // signs of one k, its groups side by side
     extern __shared__ __align__(16) float exchange[];
-    float *const signs = exchange + kExchangeFloats<COLUMNS, GROUPS, VALUES>;
+    constexpr int kElement = SOURCE == MK_F32 ? 4 : 2;
+    constexpr int kSigns = VALUES / COLUMNS;       // a thread's share of the signs
+    static_assert(VALUES * kSignStride <= kExchangeFloats<COLUMNS, GROUPS, VALUES> && GROUPS * (VALUES + 4) <= kExchangeFloats<COLUMNS, GROUPS, VALUES>,
+                  "the signs take the exchange's place");
     const int group = static_cast<int>(blockIdx.x & 7) * a.groups_per_xcd + static_cast<int>(blockIdx.x >> 3);
     if (group >= a.groups) return;   // whole workgroups
     const int local = threadIdx.x & (COLUMNS - 1), g = threadIdx.x / COLUMNS;
     const int half = __builtin_amdgcn_readfirstlane(g / kHalfGroups);   // a wavefront's groups lie in one half
     const int column = group * COLUMNS + local;
     const bool inside = column < a.columns;
-    const size_t from = inside ? column : a.columns - 1;
-    float value[2][kHalf];   // [k / kHalf][k % kHalf]
-#pragma unroll
-    for (int k = 0; k < VALUES; ++k)
-        value[k / kHalf][k % kHalf] = mk_load_as_float(a.source, static_cast<size_t>(g * VALUES + k) * a.columns + from, SOURCE);
-    if (a.signs_after) {   // uniform; a thread's rows lie VALUES apart, their signs are turned to lie side by side
-        for (int row = threadIdx.x; row < GROUPS * VALUES; row += COLUMNS * GROUPS)
-            signs[(row % VALUES) * kSignStride + row / VALUES] = a.signs_after[row];   // (read behind the exchange's barriers)
-    }
+    const char *source = static_cast<const char *>(a.source);
+    const OFFSET from = (static_cast<OFFSET>(g * VALUES) * a.columns + (inside ? column : a.columns - 1)) * kElement;
+    float sign[kSigns];
     if (a.signs_before) {   // uniform
 #pragma unroll
-        for (int k = 0; k < VALUES; ++k) value[k / kHalf][k % kHalf] *= a.signs_before[g * VALUES + k];
+        for (int i = 0; i < kSigns; ++i) sign[i] = a.signs_before[threadIdx.x + i * COLUMNS * GROUPS];
+    }
+    float value[2][kHalf];   // [k / kHalf][k % kHalf]
+#pragma unroll
+    for (int k = 0; k < VALUES; ++k, source += static_cast<size_t>(a.columns) * kElement)   // (a uniform row and the thread's
+        value[k / kHalf][k % kHalf] = mk_load_as_float(source + from, 0, SOURCE);           // offset: one address register)
+    if (a.signs_before) {   // (through LDS: read by each thread for itself they are as many loads again)
+#pragma unroll
+        for (int i = 0; i < kSigns; ++i) {
+            const int row = threadIdx.x + i * COLUMNS * GROUPS;
+            exchange[row / VALUES * (VALUES + 4) + row % VALUES] = sign[i];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < VALUES; k += 4) {
+            const float4 four = *reinterpret_cast<const float4 *>(exchange + g * (VALUES + 4) + k);
+            const float along[4] = {four.x, four.y, four.z, four.w};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) value[(k + j) / kHalf][(k + j) % kHalf] *= along[j];
+        }
+        __syncthreads();   // the exchange takes their place
     }
     auto butterfly = [](float &first, float &second) __attribute__((always_inline)) {
         const float low = first, high = second;
@@ -109,36 +129,62 @@ __global__ void __launch_bounds__(COLUMNS * GROUPS) fwht_columns_kernel(const Co
             }
 #pragma unroll
     for (int i = 0; i < kHalf; ++i) butterfly(value[0][i], value[1][i]);
+#pragma unroll
+    for (int i = 0; i < VALUES; ++i) value[i / kHalf][i % kHalf] *= a.scale;
+    if (a.signs_after) {   // uniform; a thread's rows lie VALUES apart, their signs are turned to lie side by side
+        __syncthreads();   // the exchange has been read
+#pragma unroll
+        for (int i = 0; i < kSigns; ++i) {
+            const int row = threadIdx.x + i * COLUMNS * GROUPS;
+            exchange[(row % VALUES) * kSignStride + row / VALUES] = a.signs_after[row];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int i = 0; i < kHalf; i += 4) {   // four groups of one k
+                const float4 sign = *reinterpret_cast<const float4 *>(exchange + (g * kHeld + i / kHalfGroups) * kSignStride + h * kHalfGroups + i % kHalfGroups);
+                const float along[4] = {sign.x, sign.y, sign.z, sign.w};
+#pragma unroll
+                for (int j = 0; j < 4; ++j) value[h][i + j] *= along[j];
+            }
+    }
     if (!inside) return;
+    const OFFSET to = (static_cast<OFFSET>(g * kHeld) * a.columns + column) * 4;
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int i = 0; i < kHalf; i += 4) {
-            const int k = g * kHeld + i / kHalfGroups, of = h * kHalfGroups + i % kHalfGroups;   // of ... of + 3: four groups of one k
-            float4 sign = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
-            if (a.signs_after) sign = *reinterpret_cast<const float4 *>(signs + k * kSignStride + of);
-            const float along[4] = {sign.x, sign.y, sign.z, sign.w};
+        for (int m = 0; m < kHeld; ++m) {
+            char *target = reinterpret_cast<char *>(a.target) + (static_cast<size_t>(h * kHalfGroups) * VALUES + m) * a.columns * 4;
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                a.target[static_cast<size_t>((of + j) * VALUES + k) * a.columns + column] = value[h][i + j] * a.scale * along[j];
+            for (int of = 0; of < kHalfGroups; ++of, target += static_cast<size_t>(VALUES) * a.columns * 4)
+                *reinterpret_cast<float *>(target + to) = value[h][m * kHalfGroups + of];
         }
+}
+
+template <int COLUMNS, int GROUPS, int VALUES, int SOURCE, typename OFFSET>
+void launch_columns_of(const ColumnArgs &a, hipStream_t stream) {
+    constexpr size_t needed = kExchangeFloats<COLUMNS, GROUPS, VALUES> * sizeof(float), lds = needed < 41 * 1024 ? 41 * 1024 : needed;
+    static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void *>(&fwht_columns_kernel<COLUMNS, GROUPS, VALUES, SOURCE, OFFSET>),
+                                                          hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    static_cast<void>(allowed);   // a refusal shows in the launch
+    hipLaunchKernelGGL((fwht_columns_kernel<COLUMNS, GROUPS, VALUES, SOURCE, OFFSET>), dim3(8 * a.groups_per_xcd), dim3(COLUMNS * GROUPS), lds, stream, a);
 }
 
 template <int COLUMNS, int GROUPS, int VALUES, int SOURCE>
 void launch_columns(ColumnArgs a, hipStream_t stream) {
     a.groups = mk_cdiv(a.columns, COLUMNS);
     a.groups_per_xcd = mk_cdiv(a.groups, 8);
-    constexpr size_t lds = (kExchangeFloats<COLUMNS, GROUPS, VALUES> + VALUES * (GROUPS + 4)) * sizeof(float);
-    static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void *>(&fwht_columns_kernel<COLUMNS, GROUPS, VALUES, SOURCE>),
-                                                          hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    static_cast<void>(allowed);   // a refusal shows in the launch
-    hipLaunchKernelGGL((fwht_columns_kernel<COLUMNS, GROUPS, VALUES, SOURCE>), dim3(8 * a.groups_per_xcd), dim3(COLUMNS * GROUPS), lds, stream, a);
+    if (4ull * GROUPS * VALUES * a.columns < (1ull << 32)) launch_columns_of<COLUMNS, GROUPS, VALUES, SOURCE, uint32_t>(a, stream);
+    else launch_columns_of<COLUMNS, GROUPS, VALUES, SOURCE, uint64_t>(a, stream);
 }
 
 template <int SOURCE>
 void launch_rows(const ColumnArgs &a, int rows, hipStream_t stream) {
+    // 4096 rows: 16 columns a workgroup where half the compute units get one (3072 columns 22 us, 30 with 8; 1000: 18 and 14)
     if (rows == 1024) launch_columns<16, 32, 32, SOURCE>(a, stream);
     else if (rows == 2048) launch_columns<16, 32, 64, SOURCE>(a, stream);
+    else if (a.columns >= 2048) launch_columns<16, 64, 64, SOURCE>(a, stream);
     else launch_columns<8, 64, 64, SOURCE>(a, stream);
 }
 

@@ -319,6 +319,23 @@ def test_columns_and_rows_run_their_stages_in_one_order(rows, dtype):
         assert torch.equal(device_transforms.rotate_columns(matrix, signs=signs, inverse=inverse), expected)
 
 
+@pytest.mark.parametrize("rows,columns", [(4096, 2047), (4096, 2048), (4096, 2061), (2048, 2049), (4096, 262147)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_columns_at_the_edges_of_their_workgroups(rows, columns, dtype):
+    """Both sides of the rule for 8 or 16 columns a workgroup, and a matrix whose bytes take offsets of more than 32 bits: signs
+    that are any numbers, scattered columns and the last ones, bit for bit the transform of rows."""
+    from mlkit_amd.quantization import transforms as device_transforms
+
+    generator = torch.Generator(device="cuda").manual_seed(columns)
+    signs = torch.randn((rows,), device="cuda", generator=generator)
+    looked_at = torch.cat([torch.arange(0, columns, 211), torch.arange(columns - 40, columns)]).cuda()
+    matrix = torch.randn((rows, columns), device="cuda", generator=generator, dtype=dtype)
+    rows_of = matrix[:, looked_at].float().T.contiguous()
+    for inverse in (False, True):
+        out = device_transforms.rotate_columns(matrix, signs=signs, inverse=inverse)[:, looked_at]
+        assert torch.equal(out, device_transforms.rotate(rows_of, signs=signs, inverse=inverse).T)
+
+
 @pytest.mark.parametrize("rows", [2, 3])
 def test_columns_of_a_very_wide_matrix(rows):
     """More columns than a launch has workgroups in its second dimension (65535 tiles of 64)."""
