@@ -464,6 +464,11 @@ int mk_hessian_reversed(const float *source, float *target, int width, const lon
  * lower factor's columns by its diagonal, flip back, contiguous copy). */
 int mk_unit_upper_from_factor(const float *factor, float *out, int width, void *stream);
 
+/* The coefficients for steps of 2, 4, 8 or 16 columns, of which the width holds a whole number: R blockdiag(R)^-1 with
+ * R[a][b] = U[w-1-b][w-1-a]; the factor below its diagonal is not read.  [width, width] fp32, distinct.
+ * Replaces: quantization/algorithms/error_feedback.py:76-83 (the triangular solve of the block columns). */
+int mk_blocks_upper_from_factor(const float *factor, float *out, int width, int step, void *stream);
+
 /* Index of the nearest codeword for `count` vectors of `dimension` (2, 4, 8 or 16) fp32
  * coordinates: the smallest sum over ascending coordinates of squared differences, the
  * lowest index on ties.  codebook: [codebook_size, dimension] fp32.  With lattice != 0 the

@@ -111,8 +111,6 @@ def _factor_in_place(matrix: Tensor, status: Tensor, factored: Tensor, pairs: bo
             slot = factored[start // FACTORIZATION_BLOCK]
             native.check(factor_block(matrix[start, start:].data_ptr(), width, stop - start, start, beside,
                                       slot.data_ptr() if beside else None, status.data_ptr(), raw_stream))
-        if pairs:   # the diagonal block's lower triangle holds leftovers of the products above
-            matrix[panel_start:panel_stop, panel_start:panel_stop].triu_()
         if panel_stop == width:
             break
         if width - panel_stop < LOOK_AHEAD_WIDTH:   # too little left for what the events cost
@@ -292,8 +290,8 @@ def feedback_coefficients(hessian: Tensor, step: int, *, damp: float = 0.01,
 def _coefficients_on_kernels(hessian: Tensor, step: int, damp: float, permutation: Tensor | None) -> tuple[Tensor, int]:
     """The same on a HIP device for matrices of 128 columns and more (1024 for steps of several): one pass writes the
     reversed, damped matrix where it is factored (``mk_hessian_reversed``), the blocked
-    factorisation runs, and for ``step == 1`` one pass turns the factor into the coefficients
-    (``mk_unit_upper_from_factor``)."""
+    factorisation runs, and one pass turns the factor into the coefficients (``mk_unit_upper_from_factor``, for steps of 2
+    to 16 columns ``mk_blocks_upper_from_factor``)."""
     from mlkit_amd import native
 
     width, device = hessian.shape[0], hessian.device
@@ -309,8 +307,10 @@ def _coefficients_on_kernels(hessian: Tensor, step: int, damp: float, permutatio
                                                  addend.data_ptr(), native.current_stream(device)))
 
     def read(factor: Tensor, status: int) -> tuple[Tensor, int]:
-        if step != 1 or status != 0:
-            return _coefficients_of(factor.T, status, step)
+        if status != 0 or not (step == 1 or _block_steps(factor, step)):
+            return _coefficients_of(factor.triu().T, status, step)   # (below its diagonal are leftovers of the products)
+        if step > 1:
+            return _block_coefficients(factor, step), 0
         coefficients = torch.empty_like(factor)
         native.check(library.mk_unit_upper_from_factor(factor.data_ptr(), coefficients.data_ptr(), width,
                                                        native.current_stream(device)))
@@ -319,11 +319,29 @@ def _coefficients_on_kernels(hessian: Tensor, step: int, damp: float, permutatio
     return _with_upper_factor(fill, read, width, device, pairs=step > 1)
 
 
+def _block_steps(factor: Tensor, step: int) -> bool:
+    """Whether one kernel makes the coefficients for steps of several columns."""
+    return factor.is_cuda and factor.dtype == torch.float32 and step in (2, 4, 8, 16) and factor.shape[0] % step == 0
+
+
+def _block_coefficients(upper: Tensor, step: int) -> Tensor:
+    """``R blockdiag(R)^-1`` from the upper factor of the index-reversed matrix (whose lower triangle may hold anything)."""
+    from mlkit_amd import native
+
+    upper = upper.contiguous()
+    coefficients = torch.empty_like(upper)
+    native.check(native.library().mk_blocks_upper_from_factor(upper.data_ptr(), coefficients.data_ptr(), upper.shape[0], step,
+                                                              native.current_stream(upper.device)))
+    return coefficients
+
+
 def _coefficients_of(lower: Tensor, status: int, step: int) -> tuple[Tensor, int]:
     """``R blockdiag(R)^-1`` from the lower factor of the index-reversed matrix."""
     width = lower.shape[0]
     if status != 0:
         return lower.clone(), status
+    if _block_steps(lower, step):
+        return _block_coefficients(lower.T, step), 0
     if step == 1:
         lower = lower / lower.diagonal().clone()
         return lower.flip(0, 1).contiguous(), 0

@@ -477,6 +477,30 @@ def test_pairs_of_rows_are_taken_in_their_order(size, beside):
             rest[j + 2:] -= fused(upper[j, :size, None], upper[j, None], last)[j + 2:]
 
 
+@pytest.mark.parametrize("step", [2, 4, 8, 16])
+@pytest.mark.parametrize("width", [16, 64, 80, 208, 1008])
+def test_block_coefficients_are_those_of_a_forward_substitution(width, step):
+    """`mk_blocks_upper_from_factor`: R blockdiag(R)^-1 by x_j = (r_j - x_0 d_0j - ...) / d_jj, fused and in ascending order (in
+    extended precision here, rounded once each), whatever lies below the factor's diagonal."""
+    from mlkit_amd.quantization import feedback
+
+    f32, wide = np.float32, np.longdouble
+    rng = np.random.default_rng(width + step)
+    upper = np.triu(rng.standard_normal((width, width)) * 0.3).astype(f32)
+    upper[np.arange(width), np.arange(width)] = 0.5 + rng.random(width).astype(f32)
+    r = upper.T[::-1, ::-1]
+    expected = np.zeros_like(r)
+    for first in range(0, width, step):
+        for j in range(first, first + step):
+            rest = r[:, j].copy()
+            for k in range(first, j):
+                rest = (wide(rest) - wide(expected[:, k]) * wide(r[k, j])).astype(f32)
+            expected[:, j] = rest / r[j, j]
+    junk = upper + np.tril(np.full((width, width), np.nan, dtype=f32), -1)
+    out = host(feedback._block_coefficients(dev(junk), step))
+    np.testing.assert_array_equal(out, expected)
+
+
 @pytest.mark.parametrize("beside", [0, 65])
 @pytest.mark.parametrize("column", [0, 1, 15, 16, 47, 100, 127])
 def test_pairs_of_rows_report_the_first_refused_pivot(column, beside):
