@@ -302,7 +302,7 @@ int mk_basis_product(const float *source, float *target, const float *basis, lon
  * replaces the block in place, zeros below the diagonal.  With row_columns > 0 the
  * row_columns columns to the right of the block, in the same rows, take the same elimination
  * and become U^-T times themselves (the block row of the factor), in place, one workgroup
- * per 128 of them; the block itself is then left untouched and U goes to `factor_out`
+ * per 64 of them; the block itself is then left untouched and U goes to `factor_out`
  * (size rows of 128 floats), because every workgroup reads the block.
  * *status (device memory, zero before the first block) receives 1 + first_column + j if
  * pivot j is not positive and finite, as torch.linalg.cholesky_ex reports it; a block

@@ -18,7 +18,7 @@ from torch import nn
 
 from mlkit_amd.models import Model
 from mlkit_amd.quantization.core import layer_seed
-from mlkit_amd.quantization.transforms import OnlineRotation, rht
+from mlkit_amd.quantization.transforms import OnlineRotation, randomized_weight
 
 ROTATED_LAYER_NAMES = ("o_proj", "down_proj")
 
@@ -71,7 +71,7 @@ class Rotate:
                     continue
                 seed = layer_seed(name, self.seed)
                 block = self.block if self.block and layer.in_features % self.block == 0 and layer.in_features > self.block else None
-                layer.weight.copy_(rht(layer.weight.float(), seed=seed, block=block).to(layer.weight.dtype))
+                layer.weight.copy_(randomized_weight(layer.weight.float(), seed=seed, block=block).to(layer.weight.dtype))
                 descriptor = {"kind": "rotation", "name": name, "seed": seed}
                 if block is not None:
                     descriptor["block"] = block

@@ -23,19 +23,23 @@ struct ProductArgs {
 
 constexpr int kThreads = 256;
 constexpr int kMaxOrder = 8192;
+constexpr int kChainOrder = 256;         // bases up to here keep one chain of multiply-adds (the bits of a thread per column)
 constexpr long long kShortLaunch = 256;  // workgroups of 128 x 128 values
 
 // target[r, f', p] = sum_f mix[f', f] source[r, f, p] as a matrix product: f' down, f along the sum, the pairs (r, p) across.
 // A workgroup of four wavefronts (SUB x SUB products of 32 x 32 x 2 each, DOWN of the wavefronts one below the other) owns 64 x 64,
 // 64 x 256 or 128 x 128 of them; DEPTH f at a time go through LDS, the next ones on their way in registers.  A chunk's blocks of one r lie side by side in memory,
 // whatever the power, and threads take them in that order.  Sums run over ascending f from zero, the fused multiply-add chain
-// of the kernels for smaller bases bit for bit.
+// of the kernels for smaller bases bit for bit.  PARTIAL: 64 f at a time, their sums added up behind that, for bases of more than
+// kChainOrder rows, whose rounding would otherwise grow with the chain (380 rows: 3.5e-7 from 64 bits, the library's product 1.8e-7
+// to 3.5e-7; so 1.5e-7).
 //
 // The tiles of one pair of columns go to one XCD, whose L2 then has the source for all but the first of them.  Bound by memory
 // for bases of up to about 100 rows, by the fp32 matrix cores beyond.  5120 rows as 44 blocks of 64: 44 us (114 with the basis
 // in registers, 22 at copy rate); 3840 rows as 104 blocks of 8: 21 us and 4608 as 204 of 32: 190 us (64 TFLOP/s), against 620 us
-// and 7.6 ms with a thread per column of blocks; 2048 rows as 1040 blocks of 8: 470 us.
-template <int SUB, int DOWN, int DEPTH>
+// and 7.6 ms with a thread per column of blocks; 2048 rows as 1040 blocks of 8: 590 us (470 as one
+// chain).
+template <int SUB, int DOWN, int DEPTH, bool PARTIAL>
 __global__ void __launch_bounds__(kThreads, 2) basis_product_kernel(const ProductArgs a) {
     constexpr int kRows = 32 * SUB * DOWN, kColumns = 32 * SUB * (4 / DOWN);
     constexpr int kLogDepth = DEPTH == 16 ? 4 : 5;
@@ -103,13 +107,13 @@ __global__ void __launch_bounds__(kThreads, 2) basis_product_kernel(const Produc
             left[buffer][f][out] = left_held[i];
         }
     };
-    f32x16 sums[SUB][SUB];
-#pragma unroll
-    for (int i = 0; i < SUB; ++i)
-#pragma unroll
-        for (int j = 0; j < SUB; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) sums[i][j][r] = 0.0f;
+    f32x16 sums[SUB][SUB], totals[PARTIAL ? SUB : 1][SUB];
+    auto clear = [](auto &tiles) __attribute__((always_inline)) {
+        for (auto &row : tiles)
+            for (f32x16 &tile : row) tile = f32x16{};
+    };
+    clear(sums);
+    clear(totals);
     fetch(0);
     keep(0);
     __syncthreads();
@@ -130,6 +134,15 @@ __global__ void __launch_bounds__(kThreads, 2) basis_product_kernel(const Produc
 #pragma unroll
                 for (int j = 0; j < SUB; ++j) sums[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(l.of[i], r.of[j], sums[i][j], 0, 0, 0);
         }
+        if constexpr (PARTIAL) {
+            if (((first + DEPTH) & 63) == 0 || !more) {   // uniform
+#pragma unroll
+                for (int i = 0; i < SUB; ++i)
+#pragma unroll
+                    for (int j = 0; j < SUB; ++j) totals[i][j] += sums[i][j];
+                clear(sums);
+            }
+        }
         if (more) keep(buffer ^ 1);
         __syncthreads();
     }
@@ -147,7 +160,7 @@ __global__ void __launch_bounds__(kThreads, 2) basis_product_kernel(const Produc
             if (out >= a.order) continue;
             Values value;
 #pragma unroll
-            for (int j = 0; j < SUB; ++j) value.of[j] = sums[i][j][r];
+            for (int j = 0; j < SUB; ++j) value.of[j] = PARTIAL ? totals[PARTIAL ? i : 0][j][r] : sums[i][j][r];
             if (a.signs_after) {   // uniform
                 const Values sign = *reinterpret_cast<const Values *>(a.signs_after + (static_cast<long long>(out) << a.log_power) + p);
 #pragma unroll
@@ -164,7 +177,10 @@ int launch(ProductArgs a, hipStream_t stream) {
     a.column_tiles = ((a.rows << a.log_power) + kColumns - 1) / kColumns;
     const long long groups = (a.column_tiles + 7) / 8 * 8 * a.row_tiles;
     MK_REQUIRE(groups < (1ll << 31), MK_ERR_UNSUPPORTED, "mk_basis_mix: too many rows");
-    hipLaunchKernelGGL((basis_product_kernel<SUB, DOWN, DEPTH>), dim3(static_cast<unsigned>(groups)), dim3(kThreads), 0, stream, a);
+    if (a.order > kChainOrder)
+        hipLaunchKernelGGL((basis_product_kernel<SUB, DOWN, DEPTH, true>), dim3(static_cast<unsigned>(groups)), dim3(kThreads), 0, stream, a);
+    else
+        hipLaunchKernelGGL((basis_product_kernel<SUB, DOWN, DEPTH, false>), dim3(static_cast<unsigned>(groups)), dim3(kThreads), 0, stream, a);
     return MK_OK;
 }
 
@@ -174,7 +190,7 @@ int mk_basis_product_launch(const float *source, float *target, const float *bas
                             const float *signs_after, hipStream_t stream) {
     const ProductArgs a{source, target, basis, signs_after, rows, order, log_power, transpose, 0, 0};
     // A launch that leaves most of the GPU idle waits for memory once per chunk: small tiles, deep chunks (19 rows as 380 blocks
-    // of 16: 21 us, 50 on the large tiles; 512 as 108 of 16: 11 and 21; from 256 large tiles on both take as long).
+    // of 16: 24 us, 50 on the large tiles; 512 as 108 of 16: 11 and 21; from 256 large tiles on both take as long).
     if (((rows << log_power) + 127) / 128 * mk_cdiv(order, 128) <= kShortLaunch) return launch<1, 2, 32>(a, stream);
     if (order <= 64) return launch<2, 1, 16>(a, stream);
     return launch<2, 2, 16>(a, stream);

@@ -253,6 +253,16 @@ def randomized_transform(value: Tensor, *, seed: int = 0, inverse: bool = False,
     return rotate(value, inverse=inverse, signs=signs, block=block)
 
 
+def randomized_weight(weight: Tensor, *, seed: int, block: int | None = None) -> Tensor:
+    """``randomized_transform`` of an FP32 weight that is quantized afterwards.  Bases of more than 256 rows keep the product of
+    tensor operations here: a last bit of a rotated weight turns codes, and conversions stay what they were."""
+    order, power, basis = transform_factor(weight.shape[-1])
+    if block is not None or order <= MAXIMUM_KERNEL_ORDER_SHORT_BLOCKS:
+        return randomized_transform(weight, seed=seed, block=block)
+    signs = _cached_signs(weight.shape[-1], seed, weight.device)
+    return _structured_on_host(weight * signs, order, power, basis, False)
+
+
 class OnlineRotation:
     """``rht(value, seed=seed)`` for the forward pre-hook of a rotated layer: the same result
     with the per-call work reduced to one allocation and one library call (the launch

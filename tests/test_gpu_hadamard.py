@@ -319,6 +319,27 @@ def test_columns_and_rows_run_their_stages_in_one_order(rows, dtype):
         assert torch.equal(device_transforms.rotate_columns(matrix, signs=signs, inverse=inverse), expected)
 
 
+@pytest.mark.parametrize("width,rows", [(6080, 1), (6080, 19), (6080, 300), (8320, 5), (8320, 900)])
+def test_large_bases_sum_in_parts(width, rows):
+    """Bases of more than 256 rows: 64 products at a time, then their sums.  Both roundings walk at random, so the error is about
+    2^-24 sqrt(64 / 3 + parts / 3) over the terms' spread, and the transform's stages add a little: 2.2e-7 covers both widths,
+    where one chain gives 3.5e-7 and 5.5e-7.  A weight that is quantized behind it keeps the product of tensor operations."""
+    from mlkit_amd.quantization import transforms as device_transforms
+
+    generator = torch.Generator(device="cuda").manual_seed(width + rows)
+    value = torch.randn((rows, width), device="cuda", generator=generator)
+    order, power, basis = device_transforms.transform_factor(width)
+    assert order > 256
+    points = torch.ones((1, 1), device="cuda", dtype=torch.float64)
+    while points.shape[0] < power:
+        points = torch.cat([torch.cat([points, points], 1), torch.cat([points, -points], 1)])
+    exact = torch.matmul(basis.cuda().double(), value.double().reshape(rows, order, power) @ points / power**0.5).reshape(rows, width)
+    assert (device_transforms.rotate(value) - exact).norm() <= 2.2e-7 * exact.norm()
+    signs = device_transforms.random_signs(width, 3, "cuda")
+    kept = device_transforms._structured_on_host(value * signs, order, power, basis, False)
+    assert torch.equal(device_transforms.randomized_weight(value, seed=3), kept)
+
+
 @pytest.mark.parametrize("rows,columns", [(4096, 2047), (4096, 2048), (4096, 2061), (2048, 2049), (4096, 262147)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
 def test_columns_at_the_edges_of_their_workgroups(rows, columns, dtype):
