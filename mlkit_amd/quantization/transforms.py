@@ -143,6 +143,12 @@ def _rotate_blocks_separately(value: Tensor, block: int, inverse: bool, signs: T
     return out * after if after is not None else out
 
 
+def _rotated_dtype(dtype: torch.dtype, signs: Tensor | None, order: int) -> torch.dtype:
+    """The type of a rotation's result.  Bases of more than 256 rows have what the same tensor operations give (FP32 signs make
+    FP32 of 16 bits); the kernels for smaller ones keep the value's own."""
+    return dtype if signs is None or order <= MAXIMUM_KERNEL_ORDER_SHORT_BLOCKS else torch.promote_types(dtype, signs.dtype)
+
+
 def rotate(value: Tensor, *, inverse: bool = False, signs: Tensor | None = None, block: int | None = None) -> Tensor:
     """``structured_transform`` with optional fused sign flips: forward ``T(value * signs)``,
     inverse ``T^-1(value) * signs``.  Two launches at most on a HIP device.  ``block``: T
@@ -159,10 +165,8 @@ def rotate(value: Tensor, *, inverse: bool = False, signs: Tensor | None = None,
         return out * signs if signs is not None and inverse else out
     from mlkit_amd.kernels import hadamard as kernel
 
-    result_dtype = value.dtype
+    result_dtype = _rotated_dtype(value.dtype, signs, order)
     if signs is not None:
-        if order > MAXIMUM_KERNEL_ORDER_SHORT_BLOCKS:   # (as in tensor operations, which such bases took: FP32 signs make FP32 of 16 bits)
-            result_dtype = torch.promote_types(value.dtype, signs.dtype)
         signs = signs.to(device=value.device, dtype=torch.float32).contiguous()
     before, after = (None, signs) if inverse else (signs, None)
     value = value.contiguous()
@@ -211,12 +215,13 @@ def rotate_columns(matrix: Tensor, *, signs: Tensor, inverse: bool = False) -> T
 
 def rotate_columns_in_type(matrix: Tensor, *, signs: Tensor, inverse: bool = False) -> Tensor:
     """The same with the result ``rotate(matrix.T).T`` has for a 16-bit matrix: one of its type where the row kernels take
-    its columns, and whatever the stages in tensor operations make of it where they do not."""
+    its columns as at most 256 blocks, and whatever the stages in tensor operations make of it elsewhere."""
     if matrix.dtype not in (torch.float16, torch.bfloat16) or not columns_on_kernel(matrix, signs):
         return rotate_columns(matrix, signs=signs, inverse=inverse)
-    if not _order_on_kernel(*transform_factor(matrix.shape[0])[:2]):
+    order, power, _ = transform_factor(matrix.shape[0])
+    if not _order_on_kernel(order, power):
         return rotate(matrix.T.contiguous(), inverse=inverse, signs=signs).T
-    return rotate_columns(matrix, signs=signs, inverse=inverse).to(matrix.dtype)
+    return rotate_columns(matrix, signs=signs, inverse=inverse).to(_rotated_dtype(matrix.dtype, signs, order))
 
 
 def _structured_on_host(value: Tensor, order: int, power: int, basis: Tensor | None, inverse: bool) -> Tensor:

@@ -368,7 +368,8 @@ def test_columns_of_a_very_wide_matrix(rows):
     assert torch.equal(device_transforms.rotate_columns(matrix, signs=signs), expected)
 
 
-@pytest.mark.parametrize("rows", [64, 1024, 4099, 33000])   # 33000: past the row kernels, in tensor operations
+# 1472 and 6080: bases of 368 and 380 rows; 33000: past the row kernels, in tensor operations
+@pytest.mark.parametrize("rows", [64, 1024, 1472, 4099, 6080, 33000])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32, torch.float64])
 def test_a_rotated_basis_is_entered_in_fp32(rows, dtype):
     """Whatever type a weight has, the inner quantizer sees the rotation of its fp32 numbers, and a reconstruction that
