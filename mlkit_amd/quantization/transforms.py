@@ -25,8 +25,8 @@ def _order_on_kernel(order: int, power: int) -> bool:
     return order <= (MAXIMUM_KERNEL_ORDER if power >= 4 else MAXIMUM_KERNEL_ORDER_SHORT_BLOCKS)
 
 
-def _on_kernel(value: Tensor) -> bool:
-    tracked = torch.is_grad_enabled() and value.requires_grad
+def _on_kernel(value: Tensor, signs: Tensor | None = None) -> bool:
+    tracked = torch.is_grad_enabled() and (value.requires_grad or (signs is not None and signs.requires_grad))
     return value.is_cuda and value.dtype in _KERNEL_DTYPES and not tracked and value.shape[-1] <= MAXIMUM_KERNEL_WIDTH
 
 
@@ -129,7 +129,7 @@ def _rotate_blocks_separately(value: Tensor, block: int, inverse: bool, signs: T
         raise ValueError(f"blocks of {block} values do not tile a width of {width} as powers of two")
     before, after = (None, signs) if inverse else (signs, None)
     blocks = value.reshape(*value.shape[:-1], width // block, block)
-    if _on_kernel(value) and block <= MAXIMUM_KERNEL_WIDTH:
+    if _on_kernel(value, signs) and block <= MAXIMUM_KERNEL_WIDTH:
         from mlkit_amd.kernels import hadamard as kernel
 
         def as_kernel_signs(vector):
@@ -158,7 +158,7 @@ def rotate(value: Tensor, *, inverse: bool = False, signs: Tensor | None = None,
     if block is not None:
         return _rotate_blocks_separately(value, block, inverse, signs)
     order, power, basis = transform_factor(value.shape[-1])
-    if not (_on_kernel(value) and power <= MAXIMUM_KERNEL_WIDTH and _order_on_kernel(order, power)):
+    if not (_on_kernel(value, signs) and power <= MAXIMUM_KERNEL_WIDTH and _order_on_kernel(order, power)):
         if signs is not None and not inverse:
             value = value * signs
         out = _structured_on_host(value, order, power, basis, inverse)

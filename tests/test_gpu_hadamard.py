@@ -443,6 +443,30 @@ def test_rotations_with_bases_of_more_than_256_rows(width, rows, dtype):
             assert (out.double() - expected).norm() <= allowed * expected.norm()
 
 
+@pytest.mark.parametrize("width", [64, 896, 6080])   # no basis, and bases of 28 and 380 rows
+@pytest.mark.parametrize("inverse", [False, True])
+def test_trained_signs_receive_their_gradient(width, inverse):
+    """Rows, columns and separate blocks of a value that needs no gradient itself.  A gradient is a sum over five rows of
+    products of a probe and a rotated value, each within the width's rounding of 64 bits."""
+    from mlkit_amd.quantization import transforms as device_transforms
+    from mlkit_amd.quantization.codecs import deterministic_signs
+
+    value, probe = torch.randn((2, 5, width), device="cuda")
+    signs = deterministic_signs(width, 3, value.device).requires_grad_()
+    exact = signs.detach().double().requires_grad_()
+
+    def turned(matrix, **options):
+        return device_transforms.rotate_columns(matrix.T, **options).T
+
+    def in_blocks(matrix, **options):
+        return device_transforms.rotate(matrix, block=32, **options)
+
+    for rotated in (device_transforms.rotate, turned, in_blocks):
+        expected, = torch.autograd.grad((rotated(value.double(), inverse=inverse, signs=exact) * probe.double()).sum(), exact)
+        given, = torch.autograd.grad((rotated(value, inverse=inverse, signs=signs) * probe).sum(), signs)
+        assert (given.double() - expected).norm() <= width * 2.0**-24 * expected.norm()
+
+
 @pytest.mark.parametrize("rows,columns", [(1, 1), (3, 70), (64, 64), (65, 4), (100, 132), (260, 68)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 def test_turning_a_matrix(rows, columns, dtype):
