@@ -21,13 +21,19 @@ MAXIMUM_KERNEL_ORDER = 8192               # of mk_basis_product
 MAXIMUM_KERNEL_ORDER_SHORT_BLOCKS = 256   # of mk_basis_mix, which alone takes blocks of one or two values
 
 
-def _order_on_kernel(order: int, power: int) -> bool:
-    return order <= (MAXIMUM_KERNEL_ORDER if power >= 4 else MAXIMUM_KERNEL_ORDER_SHORT_BLOCKS)
-
-
 def _on_kernel(value: Tensor, signs: Tensor | None = None) -> bool:
     tracked = torch.is_grad_enabled() and (value.requires_grad or (signs is not None and signs.requires_grad))
     return value.is_cuda and value.dtype in _KERNEL_DTYPES and not tracked and value.shape[-1] <= MAXIMUM_KERNEL_WIDTH
+
+
+def _order_on_kernel(order: int, power: int, value: Tensor, signs: Tensor | None) -> bool:
+    """Bases of more than 256 rows keep the tensor operations for signs that those take and the kernels do not: other shapes
+    than one sign per column, other devices, and more than 32 bits."""
+    if order <= MAXIMUM_KERNEL_ORDER_SHORT_BLOCKS:
+        return True
+    return order <= MAXIMUM_KERNEL_ORDER and power >= 4 and (signs is None or (
+        signs.shape == value.shape[-1:] and signs.device == value.device
+        and torch.promote_types(value.dtype, signs.dtype) in _KERNEL_DTYPES))
 
 
 def hadamard(value: Tensor, *, normalize: bool = True) -> Tensor:
@@ -158,7 +164,7 @@ def rotate(value: Tensor, *, inverse: bool = False, signs: Tensor | None = None,
     if block is not None:
         return _rotate_blocks_separately(value, block, inverse, signs)
     order, power, basis = transform_factor(value.shape[-1])
-    if not (_on_kernel(value, signs) and power <= MAXIMUM_KERNEL_WIDTH and _order_on_kernel(order, power)):
+    if not (_on_kernel(value, signs) and power <= MAXIMUM_KERNEL_WIDTH and _order_on_kernel(order, power, value, signs)):
         if signs is not None and not inverse:
             value = value * signs
         out = _structured_on_host(value, order, power, basis, inverse)
@@ -219,7 +225,7 @@ def rotate_columns_in_type(matrix: Tensor, *, signs: Tensor, inverse: bool = Fal
     if matrix.dtype not in (torch.float16, torch.bfloat16) or not columns_on_kernel(matrix, signs):
         return rotate_columns(matrix, signs=signs, inverse=inverse)
     order, power, _ = transform_factor(matrix.shape[0])
-    if not _order_on_kernel(order, power):
+    if not _order_on_kernel(order, power, matrix.T, signs):
         return rotate(matrix.T.contiguous(), inverse=inverse, signs=signs).T
     return rotate_columns(matrix, signs=signs, inverse=inverse).to(_rotated_dtype(matrix.dtype, signs, order))
 

@@ -467,6 +467,33 @@ def test_trained_signs_receive_their_gradient(width, inverse):
         assert (given.double() - expected).norm() <= width * 2.0**-24 * expected.norm()
 
 
+@pytest.mark.parametrize("width", [1472, 6080])   # bases of 368 and 380 rows
+@pytest.mark.parametrize("inverse", [False, True])
+def test_large_bases_take_the_signs_that_tensor_operations_take(width, inverse):
+    """Signs of 64 bits (which come after an FP32 transform on the way back), one for all columns and one for each value; too few
+    are refused."""
+    from mlkit_amd.quantization import transforms as device_transforms
+    from mlkit_amd.quantization.codecs import deterministic_signs
+
+    value = torch.randn((3, width), device="cuda")
+    signs = deterministic_signs(width, 3, value.device)
+
+    def exact(matrix, given):
+        return device_transforms.rotate(matrix.double(), inverse=inverse, signs=given)
+
+    def close(out, expected, step):
+        return (out.double() - expected).norm() <= width * step * expected.norm()
+
+    wide = device_transforms.rotate(value, inverse=inverse, signs=signs.double())
+    assert wide.dtype == torch.float64 and close(wide, exact(value, signs.double()), 2.0**-24 if inverse else 2.0**-53)
+    columns = device_transforms.rotate_columns_in_type(value.half().T, inverse=inverse, signs=signs.double())
+    assert columns.dtype == torch.float64
+    for given in (torch.tensor(-1.0, device="cuda"), signs * torch.tensor([[1.0], [-1.0], [1.0]], device="cuda")):
+        assert close(device_transforms.rotate(value, inverse=inverse, signs=given), exact(value, given), 2.0**-24)
+    with pytest.raises(RuntimeError):
+        device_transforms.rotate(value, inverse=inverse, signs=signs[:16].contiguous())
+
+
 @pytest.mark.parametrize("rows,columns", [(1, 1), (3, 70), (64, 64), (65, 4), (100, 132), (260, 68)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 def test_turning_a_matrix(rows, columns, dtype):
