@@ -100,6 +100,9 @@ def mix_blocks(value: Tensor, basis: Tensor, *, transpose: bool, signs_after: Te
     order, power = value.shape[-2], value.shape[-1]
     if basis.shape != (order, order) or basis.dtype != torch.float32 or not basis.is_contiguous():
         raise ValueError("basis must be a contiguous FP32 [order, order] matrix")
+    if signs_after is not None and (signs_after.dtype != torch.float32 or not signs_after.is_contiguous()
+                                    or signs_after.numel() != order * power):
+        raise ValueError("sign vectors must be contiguous FP32 with order * power entries")
     output = torch.empty_like(value)
     rows = value.numel() // (order * power)
     if order > LARGE_ORDER and power >= 4 and value.data_ptr() % 16 == 0:

@@ -494,6 +494,15 @@ def test_large_bases_take_the_signs_that_tensor_operations_take(width, inverse):
         device_transforms.rotate(value, inverse=inverse, signs=signs[:16].contiguous())
 
 
+def test_mixing_refuses_signs_of_another_length():
+    from mlkit_amd.kernels import hadamard
+
+    value, basis = torch.randn((2, 40, 8), device="cuda"), torch.randn((40, 40), device="cuda")
+    for signs in (torch.ones(8, device="cuda"), torch.ones(40 * 8, device="cuda").half(), torch.ones(2 * 40 * 8, device="cuda")[::2]):
+        with pytest.raises(ValueError, match="sign vectors"):
+            hadamard.mix_blocks(value, basis, transpose=False, signs_after=signs)
+
+
 @pytest.mark.parametrize("rows,columns", [(1, 1), (3, 70), (64, 64), (65, 4), (100, 132), (260, 68)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 def test_turning_a_matrix(rows, columns, dtype):
