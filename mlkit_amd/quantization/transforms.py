@@ -9,8 +9,10 @@ FP32 / FP16 / BF16 tensors on a HIP device run ``mk_fwht`` (one launch per tenso
 Host tensors and tensors that track gradients use the stage-by-stage tensor operations.
 """
 
+import collections
 import functools
 import math
+import threading
 
 import torch
 from torch import Tensor
@@ -116,11 +118,56 @@ def transform_factor(width: int) -> tuple[int, int, Tensor | None]:
     return odd, power, matrix.float()
 
 
-@functools.lru_cache(maxsize=64)
-def _basis_on(width: int, device: torch.device) -> Tensor:
+class LargeBases:
+    """Bases of more than 256 rows on their devices (0.6 MB for 6080 columns, 256 MB at most): those used last, ``budget`` bytes
+    of them or one.  What a captured graph reads stays, since it is replayed with the address."""
+
+    def __init__(self, budget: int) -> None:
+        self.budget = budget
+        self._lock = threading.Lock()
+        self._held: collections.OrderedDict[tuple[int, torch.device], Tensor] = collections.OrderedDict()
+        self._captured: dict[tuple[int, torch.device], Tensor] = {}
+
+    @property
+    def held_bytes(self) -> int:
+        return sum(basis.nbytes for basis in self._held.values())
+
+    def __call__(self, width: int, device: torch.device) -> Tensor:
+        key = (width, device)
+        with self._lock:
+            basis = self._held.get(key, self._captured.get(key))
+            if basis is None:
+                basis = self._held[key] = _uploaded_basis(width, device)
+                while len(self._held) > 1 and self.held_bytes > self.budget:
+                    self._held.popitem(last=False)
+            elif key in self._held:
+                self._held.move_to_end(key)
+            if device.type == "cuda":
+                basis.record_stream(torch.cuda.current_stream(device))   # (its memory is free when every stream is done with it)
+                if torch.cuda.is_current_stream_capturing():
+                    self._captured[key] = basis
+        return basis
+
+    def clear(self) -> None:
+        with self._lock:
+            self._held.clear()
+
+
+large_bases = LargeBases(budget=256 << 20)
+
+
+def _uploaded_basis(width: int, device: torch.device) -> Tensor:
     basis = transform_factor(width)[2]
     assert basis is not None
     return basis.to(device).contiguous()
+
+
+_small_basis_on = functools.lru_cache(maxsize=64)(_uploaded_basis)
+
+
+def _basis_on(width: int, device: torch.device) -> Tensor:
+    large = transform_factor(width)[0] > MAXIMUM_KERNEL_ORDER_SHORT_BLOCKS
+    return large_bases(width, device) if large else _small_basis_on(width, device)
 
 
 ONE_LAUNCH_ROWS = 256

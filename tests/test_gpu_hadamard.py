@@ -494,6 +494,27 @@ def test_large_bases_take_the_signs_that_tensor_operations_take(width, inverse):
         device_transforms.rotate(value, inverse=inverse, signs=signs[:16].contiguous())
 
 
+def test_a_captured_rotation_keeps_its_large_basis():
+    """Replays after the cache was emptied and the memory it gave back was written over, against the eager result."""
+    from mlkit_amd.quantization import transforms as device_transforms
+
+    width = 6080
+    value = torch.randn((3, width), device="cuda")
+    expected = device_transforms.rht(value, seed=5)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = device_transforms.rht(value, seed=5)
+    device_transforms.large_bases.clear()
+    torch.cuda.synchronize()
+    for _ in range(3):
+        written = [torch.full((380 * 380,), float("nan"), device="cuda") for _ in range(8)]
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, expected) and len(written) == 8
+        assert torch.equal(device_transforms.rht(value, seed=5), expected)
+
+
 def test_mixing_refuses_signs_of_another_length():
     from mlkit_amd.kernels import hadamard
 

@@ -541,3 +541,21 @@ def test_only_the_main_thread_captures_factorisations(monkeypatch):
     captured = ask(2048)
     assert captured[0] is None and captured[1] is captured[2] is not None and len(made) == 1
     feedback.clear_factor_graphs()
+
+
+def test_large_bases_are_bounded_by_their_bytes():
+    from mlkit_amd.quantization import transforms
+
+    bytes_of = {width: transforms.transform_factor(width)[2].nbytes for width in (1472, 4992, 6080)}
+    bases = transforms.LargeBases(budget=bytes_of[1472] + bytes_of[6080])
+    device = torch.device("cpu")
+    for width in (1472, 4992, 1472):
+        assert torch.equal(bases(width, device), transforms.transform_factor(width)[2])
+    bases(6080, device)   # 4992 goes, used longer ago than 1472
+    assert bases.held_bytes == bases.budget and {width for width, _ in bases._held} == {1472, 6080}
+    small = transforms.LargeBases(budget=1)
+    for width in (1472, 4992):
+        small(width, device)
+        assert small.held_bytes == bytes_of[width]   # the one in use
+    small.clear()
+    assert small.held_bytes == 0
