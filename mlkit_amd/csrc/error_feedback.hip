@@ -965,12 +965,14 @@ __global__ void __launch_bounds__(kUpdateThreads, 2) block_update_kernel(const U
 // computed once.  Rows and columns beyond the matrix are read from its last ones and not written.
 //
 // VEC: rows of both operands start on 16-byte boundaries and move in 16-byte pieces; otherwise in
-// single floats (four times the instructions, which the matrix products hide).  Bound by the fp32 matrix cores.  All
-// updates of a sweep of 1000 x 2777 / 704 x 1384 / 3001 x 8184, whose tiles are not whole: 0.25 / 0.08 / 2.59 ms (107 TFLOP/s
+// single floats (four times the instructions, which the matrix products hide).  Bound by the fp32 matrix cores.  WHOLE: no
+// tile reaches past the rows or the columns; a kernel of its own, since one that also holds the edges spends more on addresses
+// and on guarded stores with a wait each (11008 columns: 214 against 219 us, the kernel of small tiles below 9.5 against 11.5).
+// All updates of a sweep of 1000 x 2777 / 704 x 1384 / 3001 x 8184, whose tiles are not whole: 0.25 / 0.08 / 2.59 ms (107 TFLOP/s
 // in the wide ones of the last), against 1.21 / 0.39 / 4.08 with the kernel above.
 constexpr int kDeviationStride = kTileRows;  // floats per k row in LDS
 
-template <bool VEC>
+template <bool VEC, bool WHOLE>
 __global__ void __launch_bounds__(kUpdateThreads, 2) block_update_from_deviations_kernel(const UpdateArgs a) {
     // Two buffers per operand, each a variable of its own: the compiler then sees that the
     // transfer into one buffer cannot touch the buffer being read, and does not wait for it.
@@ -989,7 +991,7 @@ __global__ void __launch_bounds__(kUpdateThreads, 2) block_update_from_deviation
     const int wave_row = (wave >> 1) * 64, wave_column = (wave & 1) * 64;
     const int chunks_per_chain = a.chain_width / kDepthChunk;
     const int steps = a.chains * chunks_per_chain;
-    const bool inside = row0 + kTileRows <= a.rows && column0 + kTileColumns <= a.column_end;   // uniform
+    const bool inside = WHOLE || (row0 + kTileRows <= a.rows && column0 + kTileColumns <= a.column_end);   // uniform
 
     // Operands go from global memory straight into LDS: one wavefront instruction moves two
     // consecutive k rows of a tile (2 x 128 floats = 64 lanes x 16 bytes, lane l's bytes at
@@ -1000,11 +1002,11 @@ __global__ void __launch_bounds__(kUpdateThreads, 2) block_update_from_deviation
 #pragma unroll
     for (int half = 0; half < kHalves; ++half) {
         const int along = half * 64 + (lane & (kPieceLanes - 1)) * kPiece;
-        left_lane[half] = (VEC ? static_cast<uint32_t>(lane >> 5) * a.rows : 0u) + min(row0 + along, a.rows - kPiece);
-        right_lane[half] = (VEC ? static_cast<uint32_t>(lane >> 5) * a.width : 0u) + min(column0 + along, a.width - kPiece);
+        left_lane[half] = (VEC ? static_cast<uint32_t>(lane >> 5) * a.rows : 0u) + (WHOLE ? along : min(row0 + along, a.rows - kPiece));
+        right_lane[half] = (VEC ? static_cast<uint32_t>(lane >> 5) * a.width : 0u) + (WHOLE ? along : min(column0 + along, a.width - kPiece));
     }
-    const float *left_tile = a.deviation_t;     // + k * rows
-    const float *right_tile = a.coeff;          // + k * width
+    const float *left_tile = a.deviation_t + (WHOLE ? row0 : 0);   // + k * rows
+    const float *right_tile = a.coeff + (WHOLE ? column0 : 0);     // + k * width
 
     // This lane's cell of every 32 x 32 MFMA tile: rows (lane / 32) * 4 + ..., column lane % 32.
     const uint32_t cell_lane = static_cast<uint32_t>((lane >> 5) * 4) * a.width + (lane & 31);
@@ -1146,7 +1148,7 @@ constexpr int kSmallTile = 64;
 
 constexpr int kSmallDepth = 64;  // k rows per step: half a chain, two LDS buffers of 2 x 16 KB
 
-template <bool VEC>
+template <bool VEC, bool WHOLE>
 __global__ void __launch_bounds__(kUpdateThreads) block_update_small_tile_kernel(const UpdateArgs a) {
     __shared__ __attribute__((aligned(16))) float deviation_even[kSmallDepth][kSmallTile];     // [k][row]
     __shared__ __attribute__((aligned(16))) float deviation_odd[kSmallDepth][kSmallTile];
@@ -1161,19 +1163,19 @@ __global__ void __launch_bounds__(kUpdateThreads) block_update_small_tile_kernel
     const int column0 = a.column_begin + (large - large_row * a.column_tiles) * kTileColumns + (quarter & 1) * kSmallTile;
     const int wave_row = (wave >> 1) * 32, wave_column = (wave & 1) * 32;
 
-    if (row0 >= a.rows || column0 >= a.column_end) return;   // a quarter outside the matrix (uniform)
-    const bool inside = row0 + kSmallTile <= a.rows && column0 + kSmallTile <= a.column_end;   // uniform
+    if (!WHOLE && (row0 >= a.rows || column0 >= a.column_end)) return;   // a quarter outside the matrix (uniform)
+    const bool inside = WHOLE || (row0 + kSmallTile <= a.rows && column0 + kSmallTile <= a.column_end);   // uniform
 
     // One instruction moves four k rows of a tile (4 x 64 floats; lane l's 16 bytes land at
     // 16 l from the uniform LDS address), or one; per step a wavefront moves k rows 16 wave ... 16 wave + 15.
     constexpr int kPiece = VEC ? 4 : 1, kPieceLanes = VEC ? 16 : 64, kRowsAtOnce = VEC ? 4 : 1;
     const int along = (lane & (kPieceLanes - 1)) * kPiece;
-    const uint32_t left_lane = (VEC ? static_cast<uint32_t>(lane >> 4) * a.rows : 0u) + min(row0 + along, a.rows - kPiece);
-    const uint32_t right_lane = (VEC ? static_cast<uint32_t>(lane >> 4) * a.width : 0u) + min(column0 + along, a.width - kPiece);
+    const uint32_t left_lane = (VEC ? static_cast<uint32_t>(lane >> 4) * a.rows : 0u) + (WHOLE ? along : min(row0 + along, a.rows - kPiece));
+    const uint32_t right_lane = (VEC ? static_cast<uint32_t>(lane >> 4) * a.width : 0u) + (WHOLE ? along : min(column0 + along, a.width - kPiece));
     auto fetch = [&](int step, auto odd) __attribute__((always_inline)) {
         const size_t k_base = static_cast<size_t>(a.first_column + step * kSmallDepth + wave * 16);  // chains are adjacent
-        const float *left = a.deviation_t + k_base * a.rows;
-        const float *right = a.coeff + k_base * a.width;
+        const float *left = a.deviation_t + (WHOLE ? row0 : 0) + k_base * a.rows;
+        const float *right = a.coeff + (WHOLE ? column0 : 0) + k_base * a.width;
 #pragma unroll
         for (int one = 0; one < 16; one += kRowsAtOnce) {
             const int k = wave * 16 + one;
@@ -1251,13 +1253,16 @@ int launch_update(UpdateArgs a, hipStream_t stream) {
     const bool staged = a.deviation_t && a.chain_width % kDepthChunk == 0 && a.chain_width / kDepthChunk >= 4;
     // (rows of both operands in 16-byte pieces)
     const bool pieces = aligned(a.deviation_t) && aligned(a.coeff) && a.rows % 4 == 0 && a.width % 4 == 0 && a.column_begin % 4 == 0;
+    const bool whole_tiles = pieces && a.rows % kTileRows == 0 && (a.column_end - a.column_begin) % kTileColumns == 0;
     const auto launch_large = [&](unsigned count) {
-        if (pieces) hipLaunchKernelGGL((block_update_from_deviations_kernel<true>), dim3(count), dim3(kUpdateThreads), 0, stream, a);
-        else hipLaunchKernelGGL((block_update_from_deviations_kernel<false>), dim3(count), dim3(kUpdateThreads), 0, stream, a);
+        if (whole_tiles) hipLaunchKernelGGL((block_update_from_deviations_kernel<true, true>), dim3(count), dim3(kUpdateThreads), 0, stream, a);
+        else if (pieces) hipLaunchKernelGGL((block_update_from_deviations_kernel<true, false>), dim3(count), dim3(kUpdateThreads), 0, stream, a);
+        else hipLaunchKernelGGL((block_update_from_deviations_kernel<false, false>), dim3(count), dim3(kUpdateThreads), 0, stream, a);
     };
     const auto launch_small = [&](unsigned count) {
-        if (pieces) hipLaunchKernelGGL((block_update_small_tile_kernel<true>), dim3(count * 4), dim3(kUpdateThreads), 0, stream, a);
-        else hipLaunchKernelGGL((block_update_small_tile_kernel<false>), dim3(count * 4), dim3(kUpdateThreads), 0, stream, a);
+        if (whole_tiles) hipLaunchKernelGGL((block_update_small_tile_kernel<true, true>), dim3(count * 4), dim3(kUpdateThreads), 0, stream, a);
+        else if (pieces) hipLaunchKernelGGL((block_update_small_tile_kernel<true, false>), dim3(count * 4), dim3(kUpdateThreads), 0, stream, a);
+        else hipLaunchKernelGGL((block_update_small_tile_kernel<false, false>), dim3(count * 4), dim3(kUpdateThreads), 0, stream, a);
     };
     // (launches that leave most of the GPU idle with 128 x 128 tiles)
     const unsigned tiles = grid.x * grid.y;
