@@ -344,6 +344,23 @@ class Attention(nn.Module):
         return self.o_proj(mixed)
 
 
+def test_the_first_call_of_a_layer_is_native(monkeypatch):
+    """It binds the arguments and uses them; the same bytes as the call through Python."""
+    linear = nn.Linear(256, 48, device="cuda", dtype=torch.float16)
+    layer = mk.PackedLinear(linear, mk.nf4(64)(linear.weight.detach()))
+    x = torch.randn(3, 256, device="cuda", dtype=torch.float16)
+    expected = torch.empty(3, 48, device="cuda", dtype=torch.float16)
+    layer._matvec(x, expected, 3)
+    layer._launch = None
+
+    def refused(*arguments):
+        raise AssertionError("the call through Python")
+
+    monkeypatch.setattr(mk.PackedLinear, "_matvec", refused)
+    with torch.no_grad():
+        assert torch.equal(layer(x), expected) and torch.equal(layer(x), expected)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("bias", [False, True])
 def test_a_bound_layer_calls_natively_and_falls_back(dtype, bias):
