@@ -23,9 +23,6 @@ using mk_matvec::MatvecArgs;
 using mk_matvec::Plan;
 using mk_matvec::WordArgs;
 
-constexpr int kChunkedSamples = 4;                   // the chunked kernel's (plan_chunked)
-constexpr long long kChunkedWeights = 1ll << 25;
-
 int next_pow2(int v) {
     int p = 1;
     while (p < v) p <<= 1;
@@ -40,7 +37,7 @@ size_t lds_bytes_for(const Plan &p, int groups, bool uniform, bool has_zero) {
     if (tile_slots < 4u * p.threads) tile_slots = 4u * p.threads;  // kStaged * threads
     size_t floats = (uniform ? 0 : kMaxTableEntries) + 2 * tile_slots;
     floats += tile_rows > static_cast<size_t>(p.threads) ? tile_rows : p.threads;  // bias tile
-    const int group_rows = p.sample_tile == 4 ? 2 : 4;
+    const int group_rows = p.sample_tile >= 8 ? 1 : (p.sample_tile == 4 ? 2 : 4);
     floats += 2 * static_cast<size_t>(group_rows) * p.sample_tile * p.threads;  // per-lane sums, two buffers
     return floats * sizeof(float);
 }
@@ -61,13 +58,39 @@ const Tuning &tuning() {
     return values;
 }
 
+// Whether the chunked kernel beats the word kernel, whose workgroups cost less to start and whose rows share the activations: on
+// larger layers of few samples.  us here against us there, codes that mostly no cache holds:
+// * one sample beyond 2^24 weights -- INT8 with fp32 x 4096 x 4096 10.2 / 10.1, 4096 x 6144 12.0 / 15.6, 8192 x 4096 13.9 / 17.5, 22016 x
+//   8192 43 / 72; fp32 scales under fp16 x: INT8 10.4 / 9.9, 12.0 / 15.4, 14.8 / 17.0, 3-bit codebook 13.3 / 10.3, 13.3 / 15.8, 15.0 /
+//   17.5 -- but beyond 2^25 for tables of two and four bits, which the word kernel unpacks in the fewest steps (NF4 with fp32 x
+//   13.1 / 8.5, 13.8 / 12.9, 15.2 / 14.3, 46 / 56);
+// * two samples from 2^24 likewise with bf16 x (NF4 4096 x 6144 16.7 / 22.3, 8192 x 4096 19.1 / 21.2), with fp16 x unless on such a
+//   table (2-bit grid 13.1 / 15.0, 17.0 / 16.7; NF4 16.4 / 14.4, 19.0 / 16.6), and with fp32 x on even grids in rows of more than 4096
+//   codes (INT8 15.5 / 16.7, 3 bits 4096 x 8192 14.2 / 16.0, but 8192 x 4096 17.5 / 16.4);
+// * two otherwise, three and four from 2^25 (NF4 with fp32 x, two: 4096 x 6144 17.2 / 15.1, 4096 x 11008 18.5 / 21.7; INT8, four: 8192 x
+//   4096 27.7 / 21.7, 4096 x 11008 23.9 / 30.0, 11008 x 4096 30.4 / 28.2);
+// * more only in rows of at least 8192 codes on even grids: fp32 x and up to seven bits from 3 * 2^24 weights (3 bits, eight samples:
+//   4096 x 11008 40 / 39, 8192 x 8192 48 / 53, 22016 x 8192 116 / 132; INT8 53 / 54 and 132 / 133), fp16 x and four bits from 2^25
+//   (4096 x 11008 26 / 28, 4096 x 14336 28 / 35); eight samples of 16 bits take 4 to 11 times as long otherwise;
+// * rows of more than 16384 codes, where a thread holds two chunks, on even grids with one and two samples from 3 * 2^24, with
+//   bf16 x from 2^25 (INT8 with fp32 x, one: 2048 x 18432 21.4 / 20.1, 4096 x 18432 22.9 / 32.7; 3 bits with bf16 x, one and two: 2048 x
+//   18432 18.9 / 19.8 and 21.6 / 28.8; NF4 62 / 18 and 75 / 28, INT8 with four samples 65 / 45).
+bool chunked_is_faster(int samples, int rows, int width, int bits, int x_dtype, bool uniform) {
+    const long long weights = static_cast<long long>(rows) * width, unit = 1ll << 24;
+    if (width > 16384) return uniform && samples <= 2 && weights > (x_dtype == MK_BF16 ? 2 : 3) * unit;
+    if (samples <= 2) {
+        const bool quick_table = !uniform && (bits == 2 || bits == 4);
+        const bool early = samples == 1 ? !quick_table : x_dtype == MK_BF16 || (x_dtype == MK_F16 ? !quick_table : uniform && width > 4096);
+        return weights > (early ? 1 : 2) * unit;
+    }
+    if (samples <= 4) return weights > 2 * unit;
+    if (!uniform || width < 8192) return false;
+    return x_dtype == MK_F32 ? bits < 8 && weights > 3 * unit : x_dtype == MK_F16 && bits == 4 && weights > 2 * unit;
+}
+
 // Chooses the lane/row decomposition of the chunked kernel; returns false when the
 // layer needs the word kernel (widths or groups that are not multiples of 32 codes,
-// or a scale tile that does not fit in LDS) or is faster there: short layers, where a workgroup's fixed cost counts, and more
-// samples than four.  fp32 x, 1 / 2 / 4 / 8 samples, us here against us there: INT8 4096 x 4096 8.5 / 12.0 / 19.1 / 26.2
-// against 8.0 / 8.5 / 9.9 / 14.5, 4096 x 14336 16.9 / 19.7 / 26.4 / 49.5 against 24.2 / 26.5 / 30.7 / 44.5, 22016 x 8192 42 /
-// 54 / 73 / 129 against 64 / 70 / 81 / 113; NF4 1024 x 1024 16 / 24 / 41 / 40 against 5.3 / 5.6 / 6.2 / 7.4, 14336 x 4096 17.0 /
-// 22.4 / 33.0 / 62 against 19.7 / 25.0 / 30.8 / 44; 2- and 3-bit codes alike.
+// or a scale tile that does not fit in LDS) or is faster there.
 //
 // A row's chunks are spread over `seg` lanes (a power of two up to 64, or whole
 // wavefronts), one chunk per lane, two when a row has more than 512 chunks.  Every
@@ -77,7 +100,7 @@ const Tuning &tuning() {
 bool plan_chunked(int samples, int rows, int width, int group, int groups, int bits, int x_dtype,
                   bool uniform, bool has_zero, Plan &p) {
     if (bits < 2 || width % kChunkCodes != 0) return false;
-    if (samples > kChunkedSamples || static_cast<long long>(rows) * width <= kChunkedWeights) return false;
+    if (!chunked_is_faster(samples, rows, width, bits, x_dtype, uniform)) return false;
     if (group % kChunkCodes != 0 && group < width) return false;
     const int chunks_per_row = width / kChunkCodes;
     int c = chunks_per_row > 512 ? 2 : 1;

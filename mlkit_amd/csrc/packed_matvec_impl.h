@@ -1136,8 +1136,8 @@ bool dispatch_tile(const MatvecArgs &a, const Plan &p, hipStream_t stream) {
         return true;                                                  \
     }
     MK_CASE(1, 1) MK_CASE(2, 1) MK_CASE(4, 1)
-    MK_CASE(1, 2) MK_CASE(2, 2)
-    if constexpr (XT != MK_F32) { MK_CASE(4, 2) }
+    if constexpr (UNIFORM) { MK_CASE(1, 2) MK_CASE(2, 2) }
+    if constexpr (XT == MK_F16 && BITS == 4 && UNIFORM) { MK_CASE(8, 1) }
 #undef MK_CASE
     return false;
 }

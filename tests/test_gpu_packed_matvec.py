@@ -345,6 +345,47 @@ def test_word_kernel_on_ragged_rows(bits, width, group, rows, samples, dtype, re
         check(run_matvec(layer, x, bias=bias), layer, x, bias, relative=relative)
 
 
+@pytest.mark.parametrize("bits,uniform,dtype,rows,width,samples", [
+    (8, True, torch.float32, 4096, 4096, (1, 2, 3)),              # 2^24 weights: all words
+    (8, True, torch.float32, 4101, 4096, (1, 2)),                 # beyond: one sample in chunks, and rows behind the last tile
+    (3, True, torch.float32, 2055, 8192, (1, 2, 4)),              # two in rows of more than 4096 codes
+    (4, False, torch.float32, 2055, 8192, (1, 2)),                # tables of four bits wait for 2^25
+    (4, False, torch.float32, 4101, 8192, (1, 2, 3, 4, 5)),
+    (2, False, torch.float16, 2055, 8192, (1, 2)),
+    (3, False, torch.float16, 2055, 8192, (1, 2, 4)),
+    (8, True, torch.float16, 4101, 8192, (1, 4, 8)),
+    (4, False, torch.bfloat16, 2055, 8192, (1, 2)),
+    (4, True, torch.float16, 4101, 8192, (3, 4, 5, 7, 8, 11)),    # eight samples a pass
+    (4, True, torch.bfloat16, 4101, 8192, (3, 8)),
+    (5, True, torch.float32, 6155, 8192, (3, 5, 8)),              # 3 * 2^24: more than four samples, four a pass
+    (6, True, torch.float32, 2741, 18432, (1, 2, 3, 8)),          # two chunks a thread
+    (8, False, torch.float32, 2741, 18432, (1, 2))])
+def test_layers_around_the_limits_of_the_chunked_kernel(bits, uniform, dtype, rows, width, samples):
+    """Both sides of every limit between the chunked and the word kernel, against products in 64 bits with the decoded weight
+    (fp32 scales under 16-bit x, which the table kernels leave to these two).  Tolerances as for the word kernel."""
+    from mlkit_amd.kernels import packed_linear
+
+    generator = torch.Generator(device="cuda").manual_seed(bits + rows)
+    packed = torch.randint(0, 256, (rows * width * bits // 8,), dtype=torch.uint8, device="cuda", generator=generator)
+    scales = (torch.rand((rows, width // 64), device="cuda", generator=generator) + 0.5).half()
+    if dtype != torch.float32:
+        scales = scales.float()
+    values = torch.linspace(-1.0, 1.0, 1 << bits, device="cuda")
+    minimum, step = -1.0, 2.0 / ((1 << bits) - 1)
+    layout = packed_linear.layout_for(bits, width, 64)
+    dense = torch.empty((rows, width), device="cuda")
+    packed_linear.decode(packed, scales, values, None, dense, 64, layout, uniform, minimum, step)
+    relative = {torch.float32: 2e-6, torch.float16: 1e-3, torch.bfloat16: 8e-3}[dtype]
+    bias = torch.randn(rows, device="cuda", generator=generator).to(dtype)
+    for count in samples:
+        x = torch.randn((count, width), device="cuda", generator=generator).to(dtype)
+        y = torch.empty((count, rows), device="cuda", dtype=dtype)
+        packed_linear.matrix_vector(x, packed, scales, values, None, bias, y, 64, layout, uniform_grid=uniform, grid_minimum=minimum,
+                                    grid_step=step)
+        expected = x.double() @ dense.double().T + bias.double()
+        assert (y.double() - expected).abs().max() <= relative * expected.abs().max(), count
+
+
 @pytest.mark.parametrize("name", WIDTHS)
 @pytest.mark.parametrize("out_dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("width", [256, 288, 264])
