@@ -609,9 +609,14 @@ struct MixArgs {
 // (dynamically indexed registers would live in scratch memory); consecutive lanes take
 // consecutive p, and the basis entries are wavefront-uniform scalar loads.
 constexpr int kMaxOrder = 256;
-// A wavefront's registers hold the basis; the kernel of basis_products.hip beyond (5120 x 2816 as 20 blocks: 44 us here, 54
-// there; 2816 x 5120 as 44 blocks 114 us with two register tiles, 44 there).
-constexpr int kMaxRegisterOrder = 32;
+// Up to 32 rows a wavefront's registers hold the basis; beyond, the kernel of basis_products.hip (5120 x 2816 as 20 blocks: 44 us
+// here, 54 there; 2816 x 5120 as 44 blocks 114 us with two register tiles, 44 there), and three register tiles at most for what
+// that one does not take, blocks of one or two values and unaligned tensors: 64 rows as 60 / 92 blocks of two 11 / 22 us, 4096 rows 39 /
+// 83, against 210 / 485 and 215 / 496 with a thread per column.  Those win again on many rows of such short blocks, whose
+// wavefronts are nearly empty here (65536 rows as 33 / 60 blocks of two 76 / 232 against 334 / 389; 92 1034 against 761).
+constexpr int kMaxInRegisters = 32, kMaxRegisterOrder = 96;
+constexpr long long kManyRows = 32768;
+constexpr int kManyRowsOrder = 72;
 
 __global__ void __launch_bounds__(256) basis_mix_kernel(const MixArgs a) {
     extern __shared__ float columns_tile[];  // [order][blockDim.x]
@@ -635,25 +640,28 @@ __global__ void __launch_bounds__(256) basis_mix_kernel(const MixArgs a) {
     }
 }
 
-// The same product on the fp32 matrix cores for bases of up to 32 rows.  One wavefront
-// owns 32 adjacent columns p of one row r: the basis (zero-padded to 32 rows) is
+// The same product on the fp32 matrix cores for bases of up to 96 rows.  One wavefront
+// owns 32 adjacent columns p of one row r: the basis (zero-padded to TILES x 32 rows) is
 // the left operand, kept in registers; the right operand comes straight from global memory,
 // lanes 0..31 reading 32 adjacent p of block f and lanes 32..63 of block f + 1, so no LDS is
 // involved.  v_mfma_f32_32x32x2_f32 accumulates over ascending f from zero, which equals
 // the fused multiply-add chain of basis_mix_kernel bit for bit.
+template <int TILES>
 __global__ void __launch_bounds__(256) basis_mix_mfma_kernel(const MixArgs a) {
-    constexpr int kMaxPairs = kMaxRegisterOrder / 2;
+    constexpr int kMaxPairs = TILES * 16;   // k-pairs of a basis padded to TILES x 32
     const int lane = threadIdx.x & 63;
     const int half = lane >> 5, within = lane & 31;
     const int pairs = (a.order + 1) >> 1;
-    float left[kMaxPairs];   // mix[within][2 q + half]
+    float left[TILES][kMaxPairs];   // mix[32 t + within][2 q + half]
 #pragma unroll
-    for (int q = 0; q < kMaxPairs; ++q) {
-        const int in = 2 * q + half;
-        const bool inside = within < a.order && in < a.order;
-        const int index = a.transpose ? in * a.order + within : within * a.order + in;
-        left[q] = inside ? a.basis[inside ? index : 0] : 0.0f;
-    }
+    for (int t = 0; t < TILES; ++t)
+#pragma unroll
+        for (int q = 0; q < kMaxPairs; ++q) {
+            const int out = 32 * t + within, in = 2 * q + half;
+            const bool inside = out < a.order && in < a.order;
+            const int index = a.transpose ? in * a.order + out : out * a.order + in;
+            left[t][q] = inside ? a.basis[inside ? index : 0] : 0.0f;
+        }
     const int tiles_per_row = (a.power + 31) >> 5;
     const long long total = a.rows * tiles_per_row;
     const long long first = static_cast<long long>(blockIdx.x) * (blockDim.x >> 6) + (threadIdx.x >> 6);
@@ -671,29 +679,33 @@ __global__ void __launch_bounds__(256) basis_mix_mfma_kernel(const MixArgs a) {
             const float loaded = a.source[base + static_cast<size_t>(inside ? in : 0) * a.power];
             right[q] = inside ? loaded : 0.0f;
         }
-        mk_mix16 sums;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) sums[r] = 0.0f;
+        for (int t = 0; t < TILES; ++t) {
+            mk_mix16 sums;
 #pragma unroll
-        for (int q = 0; q < kMaxPairs; ++q)
-            if (q < pairs) sums = __builtin_amdgcn_mfma_f32_32x32x2f32(left[q], right[q], sums, 0, 0, 0);
+            for (int r = 0; r < 16; ++r) sums[r] = 0.0f;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int out = (r >> 2) * 8 + half * 4 + (r & 3);
-            if (out < a.order && column_ok) {
-                float value = sums[r];
-                if (a.signs_after) value *= a.signs_after[out * a.power + p];
-                a.target[base + static_cast<size_t>(out) * a.power] = value;
+            for (int q = 0; q < kMaxPairs; ++q)
+                if (q < pairs) sums = __builtin_amdgcn_mfma_f32_32x32x2f32(left[t][q], right[q], sums, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int out = 32 * t + (r >> 2) * 8 + half * 4 + (r & 3);
+                if (out < a.order && column_ok) {
+                    float value = sums[r];
+                    if (a.signs_after) value *= a.signs_after[out * a.power + p];
+                    a.target[base + static_cast<size_t>(out) * a.power] = value;
+                }
             }
         }
     }
 }
 
+template <int TILES>
 void launch_mix_mfma(const MixArgs &a, hipStream_t stream) {
     const long long tiles = a.rows * ((a.power + 31) / 32);
     long long blocks = (tiles + 3) / 4;
     if (blocks > 256 * 16) blocks = 256 * 16;
-    hipLaunchKernelGGL(basis_mix_mfma_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, a);
+    hipLaunchKernelGGL(basis_mix_mfma_kernel<TILES>, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, a);
 }
 
 }  // namespace
@@ -788,7 +800,7 @@ extern "C" int mk_basis_mix(const float *source, float *target, const float *bas
     MK_REQUIRE(source && target && basis, MK_ERR_INVALID, "mk_basis_mix: null tensor pointer");
     MK_REQUIRE(source != target, MK_ERR_INVALID, "mk_basis_mix: source and target must not alias");
     const auto aligned = [](const void *pointer) { return (reinterpret_cast<uintptr_t>(pointer) & 15u) == 0; };
-    if (order > kMaxRegisterOrder && power >= 4 && (power & (power - 1)) == 0 && aligned(source) && aligned(target) && aligned(signs_after)) {
+    if (order > kMaxInRegisters && power >= 4 && (power & (power - 1)) == 0 && aligned(source) && aligned(target) && aligned(signs_after)) {
         int log_power = 0;
         while ((1 << log_power) < power) ++log_power;
         if (int status = mk_basis_product_launch(source, target, basis, rows, order, log_power, transpose, signs_after, stream)) return status;
@@ -796,8 +808,11 @@ extern "C" int mk_basis_mix(const float *source, float *target, const float *bas
         return MK_OK;
     }
     MixArgs a{source, target, basis, signs_after, rows, order, power, transpose};
-    if (order <= kMaxRegisterOrder) {
-        launch_mix_mfma(a, stream);
+    const bool by_thread = order > kMaxRegisterOrder || (order > kMaxInRegisters && order <= kManyRowsOrder && power <= 2 && rows >= kManyRows);
+    if (!by_thread) {
+        if (order <= 32) launch_mix_mfma<1>(a, stream);
+        else if (order <= 64) launch_mix_mfma<2>(a, stream);
+        else launch_mix_mfma<3>(a, stream);
     } else {
         // One LDS column of `order` floats per thread: fewer threads for larger bases (64 KB).
         const int threads = order <= 128 ? 128 : 64;

@@ -89,7 +89,7 @@ def turned(matrix: Tensor) -> Tensor:
     return output
 
 
-LARGE_ORDER = 256   # of mk_basis_mix
+REGISTER_ORDER, LARGE_ORDER = 32, 256   # of mk_basis_mix: without the kernel for large bases, and the most it takes
 
 
 def mix_blocks(value: Tensor, basis: Tensor, *, transpose: bool, signs_after: Tensor | None = None) -> Tensor:
@@ -105,12 +105,10 @@ def mix_blocks(value: Tensor, basis: Tensor, *, transpose: bool, signs_after: Te
         raise ValueError("sign vectors must be contiguous FP32 with order * power entries")
     output = torch.empty_like(value)
     rows = value.numel() // (order * power)
-    if order > LARGE_ORDER and power >= 4 and value.data_ptr() % 16 == 0:
-        product = native.library().mk_basis_product
-        if signs_after is not None and signs_after.data_ptr() % 16:
-            signs_after = signs_after.clone()
-    else:
-        product = native.library().mk_basis_mix
+    if order > REGISTER_ORDER and signs_after is not None and signs_after.data_ptr() % 16:
+        signs_after = signs_after.clone()   # (the kernel for large bases loads whole quads)
+    large = order > LARGE_ORDER and power >= 4 and value.data_ptr() % 16 == 0
+    product = native.library().mk_basis_product if large else native.library().mk_basis_mix
     native.check(product(
         value.data_ptr(), output.data_ptr(), basis.data_ptr(), rows, order, power, int(transpose),
         native.pointer(signs_after), native.current_stream(device),

@@ -515,6 +515,29 @@ def test_a_captured_rotation_keeps_its_large_basis():
         assert torch.equal(device_transforms.rht(value, seed=5), expected)
 
 
+@pytest.mark.parametrize("order", [33, 64, 65, 72, 73, 96, 97])
+@pytest.mark.parametrize("rows,power", [(1, 1), (9, 2), (33000, 1), (70, 4), (3, 64)])
+@pytest.mark.parametrize("transpose", [False, True])
+def test_mixing_short_blocks_and_unaligned_tensors(order, rows, power, transpose):
+    """What the kernel for large bases does not take: register tiles or a thread per column, every
+    sum within its rounding bound of 64 bits, and the bits of the kernel for large bases."""
+    from mlkit_amd.kernels import hadamard
+
+    generator = torch.Generator(device="cuda").manual_seed(rows + order)
+    storage = torch.randn(rows * order * power + 1, device="cuda", generator=generator)
+    basis = torch.randn((order, order), device="cuda", generator=generator)
+    signs = (torch.rand(order * power + 1, device="cuda", generator=generator) < 0.5).float()[1:] * 2 - 1
+    value = storage[1:].view(rows, order, power) if power >= 4 else storage[:-1].view(rows, order, power)
+    mix = (basis.T if transpose else basis).double()
+    bound = (order + 1) * 2.0**-24 * torch.matmul(mix.abs(), value.double().abs())
+    expected = torch.matmul(mix, value.double())
+    out = hadamard.mix_blocks(value, basis, transpose=transpose)
+    assert ((out.double() - expected).abs() <= bound).all()
+    assert torch.equal(hadamard.mix_blocks(value, basis, transpose=transpose, signs_after=signs), out * signs.view(order, power))
+    if power >= 4:   # the kernel for large bases sums in the same order
+        assert torch.equal(out, hadamard.mix_blocks(value.clone(), basis, transpose=transpose))
+
+
 def test_mixing_refuses_signs_of_another_length():
     from mlkit_amd.kernels import hadamard
 
