@@ -322,7 +322,8 @@ int mk_cholesky_block_pairs(float *matrix, long long leading, int size, int firs
  * mk_factor_block_rows: at most 128 rows r from row_first on, every column c >= row_first; k_stop - k_first a multiple of
  * 128.  one_chain != 0: each sum is one chain of additions over ascending k, otherwise four that are added up.
  * mk_factor_trailing: any number of rows, the columns c >= r (values below the diagonal are left or changed); k_stop -
- * k_first a multiple of 64.  leave_room != 0: the launch leaves every compute unit room for kernels on another stream.
+ * k_first a multiple of 64.  leave_room != 0: a launch of 128 x 128 tiles (1024 of them or more) leaves every compute unit
+ * room for kernels on another stream; smaller launches, whose tiles of 64 x 64 end soon, ignore it.
  * Replaces: part of torch.linalg.cholesky_ex, quantization/algorithms/error_feedback.py:37-83. */
 int mk_factor_block_rows(float *matrix, int width, int k_first, int k_stop, int row_first, int row_stop, int one_chain,
                          void *stream);

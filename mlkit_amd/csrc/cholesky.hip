@@ -2,17 +2,17 @@
 //
 // The error-feedback coefficients are U blockdiag(U)^-1 for the damped Hessian H = U^T U
 // (K up to 16384).  The library factorisation spends most of its time in its small
-// unblocked panel kernel, so the blocked algorithm is driven from the host with library
-// matrix products for the trailing updates, and this file supplies the rest: a workgroup
-// factors a diagonal block of at most 128 x 128 in registers and, on request, carries 64
-// columns of the block's rows through the same elimination, which makes them the factor's
-// block row (one workgroup per 64 columns; no triangular solve is needed).
+// unblocked panel kernel, so the blocked algorithm is driven from the host; its products are
+// those of factor_products.hip, and this file supplies the rest: a workgroup factors a
+// diagonal block of at most 128 x 128 in registers and, on request, carries 64 columns of the
+// block's rows through the same elimination, which makes them the factor's block row (one workgroup per 64 columns; no triangular solve is needed).
 //
 // Replaces the `torch.linalg.cholesky_ex` call of `feedback_coefficients`
 // (quantization/algorithms/error_feedback.py:37-83 in /root/reference/src/mlkit) for large
-// matrices on the device; mk_hessian_reversed and mk_unit_upper_from_factor are the tensor
-// operations in front of it and behind it (:55-66 index reversal and damping, :72-75 division
-// by the diagonal and reversal back), one pass over the matrix each.
+// matrices on the device; mk_hessian_reversed, mk_unit_upper_from_factor and
+// mk_blocks_upper_from_factor are the tensor operations in front of it and behind it (:55-66
+// index reversal and damping, :72-83 division by the diagonal or its blocks and reversal
+// back), one pass over the matrix each.
 
 #include "mk_common.h"
 

@@ -39,8 +39,8 @@ __device__ __forceinline__ T *element_at(T *uniform, uint32_t bytes) {
 // products' operands ahead; with SPLIT the four wavefronts of a workgroup take a quarter of the k each and their sums meet in
 // LDS.  Without, sums are one chain over ascending k (what the library's kernels compute, bit for bit).
 //
-// Bound by latency where the matrix is narrow: the seven products of 896 columns 5 us each (8 us, and 78 and 48 where the
-// library chose one workgroup); 14 us with 10880 columns beside 128 k.  32 x 64 values a workgroup from 4096 columns on, where
+// Bound by latency where the matrix is narrow: the three products of 896 columns 4.4 us each (library products 8, and 78 and 48
+// where one workgroup was chosen); 14 us with 10880 columns beside 128 k.  32 x 64 values a workgroup from 4096 columns on, where
 // the operands that all workgroups read together count (32 x 32 below: twice the workgroups, half their chain).
 template <int R, int C, bool SPLIT, int S>
 __global__ void __launch_bounds__(kThreads, 3) block_rows_kernel(const ProductArgs a) {
@@ -164,7 +164,8 @@ constexpr int kDepth = 16, kBuffers = 4, kBand = 8;
 // empty.  360 columns behind a panel of 1024: 22 us on 64 x 64 tiles, 75 on 128 x 128.
 constexpr int kLargeTiles = 1024;
 // Beyond the 64 KB of its buffers: one workgroup per compute unit, beside which a workgroup of the block kernel finds room.
-// Without, block kernels wait for tiles to end: 11008 columns in 6.5 ms instead of 6.2, 8184 in 3.47 instead of 3.40.
+// Without, block kernels wait for tiles to end: 11008 columns in 6.5 ms instead of 6.2, 8184 in 3.47 instead of 3.40.  (Tiles of
+// 64 x 64 take 32 KB and end soon.)
 constexpr size_t kRoomBeside = 20 * 1024;
 
 struct TrailingArgs {

@@ -152,7 +152,6 @@ inline int resident_workgroups(Kernel kernel, int threads, size_t dynamic_lds, s
     return value;
 }
 
-// Pair-table kernel (packed_matvec_pairs.hip): 2-, 3- and 4-bit codes of any scalar grid.
 // packed_matvec_words.hip: rows [first_row, rows) of any layout that mk_packed_layout_supported takes.
 struct WordArgs {
     const void *x;
@@ -171,6 +170,7 @@ struct WordArgs {
 };
 void words_launch(const WordArgs &a, int bits, hipStream_t stream);
 
+// Pair-table kernel (packed_matvec_pairs.hip): 2- to 8-bit codes of any scalar grid.
 bool pairs_accepts(int width, int group, int bits, int x_dtype, int scale_dtype);
 int pairs_launch(const Stream4Args &a, hipStream_t stream);
 int pairs_launch_group(const Stream4Args &shared, Stream4Group &group, const int *member_rows, int *rows_per_tile,
