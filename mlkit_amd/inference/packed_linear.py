@@ -288,14 +288,13 @@ class PackedLinear(nn.Module):
     # -- forward -----------------------------------------------------------------------------
 
     def forward(self, inputs: Tensor) -> Tensor:
-        compiling, unbound = torch.compiler.is_compiling(), False
+        compiling = torch.compiler.is_compiling()
         if not compiling and self._rotation is None and self._siblings is None:
             # The plain call in one native function, once the checks below have let one through and bound it (the layers of a
             # small model wait for the host: 896 to 128 values, one row, 8.1 us of host a call through ctypes and 5.0 through
             # this); None is whatever else comes, and all of that is decided below.
             launch = self._launch
-            unbound = launch is None
-            if not unbound and launch[5] is not None:
+            if launch is not None and launch[5] is not None:
                 output = launch[5].matvec(inputs, self._buffers, self.maximum_fused_rows)
                 if output is not None:
                     return output
@@ -320,7 +319,7 @@ class PackedLinear(nn.Module):
             return functional.linear(inputs, self.weight.to(inputs.dtype), self.bias)
         if inputs.requires_grad and torch.is_grad_enabled():
             raise RuntimeError("packed CUDA inference does not support autograd")
-        if unbound:
+        if not compiling and self._rotation is None and self._siblings is None and self._launch is None:
             launch = self._bound_arguments()
             if launch[5] is not None:
                 output = launch[5].matvec(inputs, self._buffers, rows)

@@ -494,6 +494,7 @@ def test_large_bases_take_the_signs_that_tensor_operations_take(width, inverse):
         device_transforms.rotate(value, inverse=inverse, signs=signs[:16].contiguous())
 
 
+@torch.inference_mode()   # (where an earlier capture of the process may have left the random generator's state)
 def test_a_captured_rotation_keeps_its_large_basis():
     """Replays after the cache was emptied and the memory it gave back was written over, against the eager result."""
     from mlkit_amd.quantization import transforms as device_transforms
