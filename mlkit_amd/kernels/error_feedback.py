@@ -184,10 +184,14 @@ def sweep(
 
 def _kept_deviations(rows: int, width: int, block: int, device: torch.device) -> Tensor | None:
     """Room for the column-major deviations of finished columns, which the trailing updates multiply: those after tiles of
-    128 columns or more in whole chunks of 32 (shorter ones work them out again from weights and reconstruction)."""
+    128 columns or more in whole chunks of 32.  Shorter ones, and matrices that leave no memory for it, work them out again from
+    weights and reconstruction, with the same results."""
     if width <= block or block < 128 or block % 32:
         return None
-    return torch.empty((width, rows), device=device, dtype=torch.float32)
+    try:
+        return torch.empty((width, rows), device=device, dtype=torch.float32)
+    except torch.OutOfMemoryError:
+        return None
 
 
 def vector_sweep(

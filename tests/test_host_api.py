@@ -559,3 +559,15 @@ def test_large_bases_are_bounded_by_their_bytes():
         assert small.held_bytes == bytes_of[width]   # the one in use
     small.clear()
     assert small.held_bytes == 0
+
+
+def test_a_sweep_goes_without_kept_deviations_where_memory_is_short(monkeypatch):
+    from mlkit_amd.kernels import error_feedback
+
+    def refused(*arguments, **options):
+        raise torch.OutOfMemoryError("no room")
+
+    device = torch.device("cpu")
+    assert error_feedback._kept_deviations(5, 1000, 128, device).shape == (1000, 5)
+    monkeypatch.setattr(error_feedback.torch, "empty", refused)
+    assert error_feedback._kept_deviations(5, 1000, 128, device) is None
