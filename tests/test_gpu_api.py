@@ -344,27 +344,31 @@ class Attention(nn.Module):
         return self.o_proj(mixed)
 
 
-def test_the_first_call_of_a_layer_is_native(monkeypatch):
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("bias", [False, True])
+def test_the_first_call_of_a_layer_is_native(dtype, bias, monkeypatch):
     """It binds the arguments and uses them; the same bytes as the call through Python."""
-    linear = nn.Linear(256, 48, device="cuda", dtype=torch.float16)
-    layer = mk.PackedLinear(linear, mk.nf4(64)(linear.weight.detach()))
-    x = torch.randn(3, 256, device="cuda", dtype=torch.float16)
-    expected = torch.empty(3, 48, device="cuda", dtype=torch.float16)
-    layer._matvec(x, expected, 3)
-    layer._launch = None
+    linear = nn.Linear(256, 48, bias=bias, device="cuda", dtype=dtype)
+    layer = mk.PackedLinear(linear, mk.int(4, 64, asym=True)(linear.weight.detach()))
+    inputs = [torch.randn(shape, device="cuda", dtype=dtype) for shape in ((256,), (1, 256), (2, 4, 256))]
+    expected = [torch.empty(x.shape[:-1] + (48,), device="cuda", dtype=dtype) for x in inputs]
+    for x, y in zip(inputs, expected):
+        layer._matvec(x, y, x.numel() // 256)
 
     def refused(*arguments):
         raise AssertionError("the call through Python")
 
     monkeypatch.setattr(mk.PackedLinear, "_matvec", refused)
     with torch.no_grad():
-        assert torch.equal(layer(x), expected) and torch.equal(layer(x), expected)
+        for x, y in zip(inputs, expected):
+            layer._launch = None
+            assert torch.equal(layer(x), y) and torch.equal(layer(x), y)
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("bias", [False, True])
 def test_a_bound_layer_calls_natively_and_falls_back(dtype, bias):
-    """The first call goes through Python and binds the native one: both give the same bytes, and whatever is not the plain
+    """The first call binds the native one: later ones give the same bytes, and whatever is not the plain
     call (strides, a mode, a replaced buffer, a gradient, a wrong width) still takes the Python path."""
     from torch.utils._python_dispatch import TorchDispatchMode
 

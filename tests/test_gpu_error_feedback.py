@@ -212,10 +212,11 @@ def test_update_from_kept_deviations_equals_the_recomputing_update(rows, width, 
     assert torch.equal(updated[:, :begin], feedback[:, :begin])
 
 
-@pytest.mark.parametrize("rows,width", [(1, 260), (3, 389), (63, 516), (130, 641), (129, 1157), (260, 1284), (517, 2049), (1029, 3076)])
+@pytest.mark.parametrize("rows,width", [(1, 260), (3, 389), (63, 516), (130, 641), (129, 1157), (260, 1284), (517, 2049), (1029, 3076),
+                                        (128, 640), (256, 1284), (1024, 3072)])
 def test_sweep_with_kept_deviations_equals_the_one_without(rows, width):
-    """Rows and columns that fill no whole tile, on 16-byte boundaries and off them: the kernels that read the kept
-    deviations (64 x 64 and 128 x 128 tiles) against the one that works them out again, bit for bit."""
+    """Rows and columns that fill no whole tile, on 16-byte boundaries and off them, and whole ones: the kernels that read the
+    kept deviations (64 x 64 and 128 x 128 tiles) against the one that works them out again, bit for bit."""
     from mlkit_amd import native
 
     generator = torch.Generator(device="cuda").manual_seed(rows * width)
